@@ -325,3 +325,123 @@ def tolerance(case):
     if case["kind"] in ("append", "copy"):
         return "exact"
     return {"rel": 3e-6, "max": 4e-5}
+
+
+def _blocks(x, half_scale):
+    """x (f32, rows of 256) as int8 codes times a scale of every 32 values, back in 64 bits."""
+    b = x.reshape(*x.shape[:-1], HD // 32, 32)
+    amax = b.abs().amax(-1, keepdim=True)
+    # quotients through 64 bits: rounded once, as IEEE division does
+    scale = torch.where(amax > 0, (amax.double() / 127.0).float(), torch.ones_like(amax))
+    if half_scale:
+        scale = torch.where(amax > 0, scale.half().float().clamp_min(2.0 ** -14), scale)
+    t = (b.double() / scale.double()).float().clamp(-127.0, 127.0)
+    code = torch.trunc(t + torch.copysign(torch.full_like(t, 0.5), t))
+    return (code.double() * scale.double()).reshape(x.shape)
+
+
+def _kept(x, layout, is_k):
+    """What the cache holds of f32 rows."""
+    if layout == "i8h" or (layout == "q8v" and not is_k):
+        return _blocks(x, layout == "i8h")
+    h = x.half().double()
+    return torch.where(h.abs() < 2.0 ** -14, torch.zeros_like(h), h)
+
+
+def _norm_rotate(x, gamma, at):
+    """RMSNorm and the rotary of the first N_ROT values; x [n, ..., d], at [n] positions; f32 between the steps."""
+    x = x.double()
+    y = (x / torch.sqrt((x * x).mean(-1, keepdim=True) + EPS) * gamma.double()).float().double()
+    half = N_ROT // 2
+    inv = torch.tensor([FREQ ** (-2.0 * i / N_ROT) for i in range(half)], dtype=torch.float64, device=x.device)
+    angle = (at.double()[:, None] * inv).reshape(at.numel(), *([1] * (x.dim() - 2)), half)
+    cos, sin = torch.cos(angle).float().double(), torch.sin(angle).float().double()
+    a, b = y[..., :half], y[..., half:N_ROT]
+    return torch.cat([a * cos - b * sin, a * sin + b * cos, y[..., N_ROT:]], -1).float()
+
+
+def _attend(q, k, v, seen, n_kv, gate):
+    """q [T, n_q, HD], k and v [C, n_kv, HD] in 64 bits, seen [T, C] or None (all)."""
+    tokens, n_q = q.shape[:2]
+    group = n_q // n_kv
+    out = torch.empty_like(q)
+    for h in range(n_kv):
+        keys, values = k[:, h].t().contiguous(), v[:, h].contiguous()
+        step = max(1, (1 << 27) // (keys.shape[1] * group))
+        for t in range(0, tokens, step):
+            rows = q[t:t + step, h * group:(h + 1) * group]
+            s = (rows.reshape(-1, HD) @ keys / 16.0).reshape(rows.shape[0], group, -1)
+            if seen is not None:
+                s = s.masked_fill(~seen[t:t + step, None, :], float("-inf"))
+            p = torch.softmax(s, -1).reshape(-1, keys.shape[1])
+            out[t:t + step, h * group:(h + 1) * group] = (p @ values).reshape(rows.shape)
+    return out if gate is None else out * torch.sigmoid(gate.double())
+
+
+def exact(case, seed):
+    """The attention outputs in 64 bits over what the cache holds; everything else that a pass returns is bytes or
+    whole numbers.  The draws repeat those of prepare(), in its order."""
+    kind, layers, n_kv, layout = case["kind"], case["layers"], case["n_kv"], case["layout"]
+    if kind in ("append", "copy"):
+        return None
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+
+    held = _ints(case["ctx"] if kind == "decode" else case["prefix"])
+    tokens = [1] * len(held) if kind == "decode" else _ints(case["tokens"])
+    cache = []
+    for _ in range(layers):
+        rows = []
+        for h in held:
+            k, v = [randn(0, n_kv, HD)], [randn(0, n_kv, HD)]
+            for at in range(0, h, 16384):
+                n = min(16384, h - at)
+                k.append(randn(n, n_kv, HD))
+                v.append(randn(n, n_kv, HD))
+            rows.append((torch.cat(k), torch.cat(v)))
+        cache.append(rows)
+    total, n_q = sum(tokens), case["n_q"]
+    dt = torch.float16 if case.get("source") == "f16" else torch.float32
+    new_k = [randn(total, n_kv, HD).to(dt).float() for _ in range(layers)]
+    new_v = [randn(total, n_kv, HD).to(dt).float() for _ in range(layers)]
+    form = case.get("form", case.get("source"))
+    gamma = 1.0 + 0.1 * randn(HD) if form in ("kprep", "select") else None
+    q = [randn(total, n_q, HD) for _ in range(layers)]
+    gate = [randn(total, n_q, HD) for _ in range(layers)] if case["gate"] else None
+    if form == "select":
+        pooled = [[randn(h // BLOCK + 1, IDX_DIM) for h in held] for _ in range(layers)]
+        tail = [randn(len(held), BLOCK - 1, IDX_DIM) for _ in range(layers)]
+        idx_k = [randn(len(held), IDX_DIM) for _ in range(layers)]
+        idx_q = [randn(len(held), IDX_HEADS, IDX_DIM) for _ in range(layers)]
+        idx_gamma = 1.0 + 0.1 * randn(IDX_DIM)
+    out = torch.empty(layers, total, n_q, HD, dtype=torch.float64, device="cuda")
+    for layer in range(layers):
+        first = 0
+        for i, (h, t) in enumerate(zip(held, tokens)):
+            mine = slice(first, first + t)
+            first += t
+            k, v = new_k[layer][mine], new_v[layer][mine]
+            if form == "kprep":
+                k = _norm_rotate(k, gamma, torch.arange(h, h + t, device="cuda"))
+            k = _kept(torch.cat([cache[layer][i][0], k]), layout, True)
+            v = _kept(torch.cat([cache[layer][i][1], v]), layout, False)
+            seen = None
+            if kind == "prefill":
+                seen = torch.arange(h + t, device="cuda")[None, :] <= torch.arange(h, h + t, device="cuda")[:, None]
+            if form == "select":
+                keys = pooled[layer][i]
+                if (h + 1) % BLOCK == 0:
+                    raw = torch.cat([tail[layer][i], idx_k[layer][i][None]])
+                    mean = ((raw[0] / BLOCK + raw[1] / BLOCK) + raw[2] / BLOCK) + raw[3] / BLOCK
+                    keys[h // BLOCK] = _norm_rotate(mean[None], idx_gamma, torch.tensor([h // BLOCK * BLOCK], device="cuda"))[0]
+                n = (h + 1) // BLOCK
+                score = (idx_q[layer][i].double() @ keys[:n].double().t().contiguous()).clamp_min(0.0).sum(0)
+                chosen = torch.sort(score, descending=True, stable=True).indices[:TOPK]
+                chosen = torch.unique(torch.cat([chosen, torch.tensor([h // BLOCK], device="cuda")]))
+                cells = (chosen[:, None] * BLOCK + torch.arange(BLOCK, device="cuda")).reshape(-1)
+                cells = cells[cells <= h]
+                k, v = k[cells], v[cells]
+            out[layer, mine] = _attend(q[layer][mine].double(), k, v, seen, n_kv, gate[layer][mine] if gate else None)
+    return (out, None, None, None, None) if form == "select" else (out, None)
