@@ -1347,7 +1347,19 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
     a.gate_head_stride = gate_head_stride;
     a.scale = scale;
     a.out = out_dev;
-    BKV_HIP(launch_prefill_attn(p, layer, b, a, (int32_t)rows_per_wg, S(stream)));
+    PrefillSplit split;
+    bool cut = plan_prefill_split(p, b, (int32_t)rows_per_wg, (int32_t)group, split);
+    if (cut && stream) {
+        // a captured call stays uncut: its replays would share the workspace with whatever runs beside them
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        cut = hipStreamIsCapturing(S(stream), &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+        if (!cut) (void)hipGetLastError();
+    }
+    if (cut) {
+        st = order_workspace(p->attn_ws, S(stream));
+        if (st != BKV_OK) return st;
+    }
+    BKV_HIP(launch_prefill_attn(p, layer, b, a, (int32_t)rows_per_wg, cut ? &split : nullptr, S(stream)));
     return BKV_OK;
 }
 

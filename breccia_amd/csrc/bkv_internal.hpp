@@ -256,8 +256,20 @@ struct PrefillBatch {
 };
 // query rows one work-group owns, given how many 64-row work-groups the call's chunks would make
 int32_t prefill_rows_per_wg(int32_t layout, int64_t wgs_of_64_rows, int32_t n_cu);
+// How a call whose row blocks leave most of the chip idle is cut: the page walks of an entry's
+// longest blocks (its last ones) in ranges of at most pps pages, a work-group each.
+struct PrefillSplit {
+    int32_t pps;                           // even
+    int32_t n_cut[BKV_MAX_BATCH];          // row blocks of the entry that are cut
+    int32_t splits[BKV_MAX_BATCH];         // ranges of its longest block
+    int32_t wg_base[BKV_MAX_BATCH + 1];    // work-groups of the entries before; [n] = total
+    int32_t unit_base[BKV_MAX_BATCH + 1];  // their cut (row block, kv head) units; [n] = total
+    int32_t slot_base[BKV_MAX_BATCH];      // their partial results, in row blocks
+};
+// False where the call is better off uncut.  A cut call uses the pool's split-K workspace.
+bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows_per_wg, int32_t group, PrefillSplit& s);
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
-                               int32_t rows_per_wg, hipStream_t stream);
+                               int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream);
 
 hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_dev, int32_t n_pairs,
                             hipStream_t stream);

@@ -43,6 +43,7 @@
 // without the exponent: both K and V become hi/lo image pairs, and the scores are
 // K_hi.q_hi + K_hi.q_lo + K_lo.q_hi.
 #include <algorithm>
+#include <type_traits>
 
 #include "bkv_internal.hpp"
 #include "lane_groups.hpp"
@@ -83,6 +84,21 @@ struct PrefillKernelParams {
     int32_t by_xcd;  // work-groups are dealt to the chip's 8 dies so that each die sees few (entry, kv head) units
 };
 
+// A cut call: a work-group walks one range of its block's pages and leaves a partial result,
+// prefill_merge_kernel puts the ranges of a row together.
+struct PrefillSplitParams : PrefillKernelParams {
+    PrefillSplit s;
+    float* part_o;   // [slot][row of the block][256], relative to the range's own softmax reference
+    float* part_ml;  // [slot][row of the block][reference, denominator]
+};
+
+// Ranges of a block that walks `pages` pages, and the (even) pages of each: evened out, none empty.
+__host__ __device__ __forceinline__ int split_ranges(int pages, int pps, int max_splits, int& each) {
+    const int n = min((pages + pps - 1) / pps, max_splits);
+    each = ((pages + n - 1) / n + 1) & ~1;
+    return (pages + each - 1) / each;
+}
+
 // The chip is 8 dies (XCDs), each with an L2 of its own, and work-group i runs on die i % 8.
 // Every work-group of one (entry, kv head) unit walks the same K/V pages, so the dies are given
 // whole units: with 8 or more units, die x serves units x, x + 8, ...; with fewer, unit u is
@@ -98,6 +114,13 @@ __device__ __forceinline__ f4 mfma32(h8 a, h8 b, f4 c) {
 __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
     hi = (_Float16)x;
     lo = (_Float16)(x - (float)hi);
+}
+
+// sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91)
+__device__ __forceinline__ float sigmoid(float x) {
+    if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
+    const float ex = expf(x);
+    return ex / (1.0f + ex);
 }
 
 // What a thread carries of one page between its fetch and its deposit into LDS.
@@ -134,8 +157,10 @@ struct PrefillLds {
 // WAVES: waves of a work-group, 16 query rows each.  Eight share every page image they put into LDS
 // among 128 rows (one work-group per compute unit); four (f16 pools only, two work-groups per
 // compute unit) spread a small chunk over twice as many compute units.
-template <int LAY, int WAVES = 8>
-__global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(const PrefillKernelParams P) {
+// SPLIT: a work-group walks one range of its block's pages and leaves a partial result.
+template <int LAY, int WAVES = 8, bool SPLIT = false>
+__global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
+    const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams> P) {
     static_assert(WAVES == 8 || (WAVES == 4 && LAY == BKV_LAYOUT_F16), "the quantised images are dequantised by 512 threads");
     constexpr bool Q8V = LAY == BKV_LAYOUT_Q8V;
     constexpr bool I8H = LAY == BKV_LAYOUT_I8H;
@@ -145,7 +170,22 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
     constexpr int kRowsPerWg = kRowsPerWave * kWavesPerWg;
     // ---- which (entry, kv head, block of 64 query rows) ---------------------------------
     int e = 0, kvh, idx;  // idx: which of the unit's blocks, in dispatch order
-    if (P.by_xcd) {
+    int range = 0;       // which range of the block's pages
+    bool cut = false;    // the block is cut at all
+    if constexpr (SPLIT) {
+        while (e + 1 < P.b.n && (int)blockIdx.x >= P.s.wg_base[e + 1]) ++e;
+        int rem = (int)blockIdx.x - P.s.wg_base[e];
+        const int in_ranges = P.s.n_cut[e] * P.n_kv * P.s.splits[e];
+        cut = rem < in_ranges;
+        if (cut) {
+            range = rem % P.s.splits[e];
+            rem /= P.s.splits[e];
+        } else {
+            rem -= in_ranges;
+        }
+        kvh = rem % P.n_kv;
+        idx = rem / P.n_kv + (cut ? 0 : P.s.n_cut[e]);
+    } else if (P.by_xcd) {
         const int units = P.b.n * P.n_kv;
         const int x = (int)blockIdx.x % kXcds;
         int j = (int)blockIdx.x / kXcds;
@@ -199,11 +239,22 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
     // the last token any row of this wave belongs to bounds the page walk
     const int last_row = min(row0 + kRowsPerWave, n_rows) - 1;
     const int pos_max = wave_live ? P.b.pos0[e] + last_row / P.group : -1;
-    const int n_pages = wave_live ? pos_max / kPage + 1 : 0;
+    int n_pages = wave_live ? pos_max / kPage + 1 : 0;
     // pages the work-group walks: those of its last row
     const int wg_last_row = min(rb * kRowsPerWg + kRowsPerWg, n_rows) - 1;
     const int wg_pos_max = P.b.pos0[e] + wg_last_row / P.group;
-    const int wg_pages = wg_pos_max / kPage + 1;
+    int wg_pages = wg_pos_max / kPage + 1;
+    int first_pg = 0;
+    if constexpr (SPLIT) {
+        if (cut) {
+            int each;
+            const int ranges = split_ranges(wg_pages, P.s.pps, P.s.splits[e], each);
+            if (range >= ranges) return;  // the entry's longest block has more
+            first_pg = range * each;
+            wg_pages = min(wg_pages, first_pg + each);
+            n_pages = min(n_pages, wg_pages);
+        }
+    }
 
     typedef const __attribute__((address_space(4))) int32_t* table_ptr;
     const table_ptr bt = (table_ptr)(uintptr_t)(P.tables + (size_t)P.b.row[e] * (size_t)P.max_pages_per_seq);
@@ -460,16 +511,19 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
         pm = max_over_lane_groups(pm);
         const bool moved = pm > m_run + kSlack;  // m_run = -inf at the start: any finite maximum moves it
         const float m_new = moved ? pm : m_run;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);  // 1, or 0 at the start
+        // a range may hold no live cell for a row (it begins past the row's position): its reference
+        // stays at -inf, and the weights of its dead cells are taken against 0
+        const float m_at = SPLIT && m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_at);  // 1, or 0 at the start
         float pv[8];
         float psum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const float ww = r < 4 ? wa[r & 3] : wb[r & 3];
-            pv[r] = __builtin_amdgcn_exp2f(ww - m_new);
+            pv[r] = __builtin_amdgcn_exp2f(ww - m_at);
             if constexpr (Q8V) {
                 const float tt = r < 4 ? ta[r & 3] : tb[r & 3];
-                psum += __builtin_amdgcn_exp2f(tt - m_new);
+                psum += __builtin_amdgcn_exp2f(tt - m_at);
             } else {
                 psum += pv[r];
             }
@@ -519,15 +573,15 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
     // one in the staging registers (past the end they carry the last page again).
     PageStage<LAY> stage_a, stage_b;
     const int last_pg = wg_pages - 1;
-    fetch(0, stage_a);
-    fetch(min(1, last_pg), stage_b);
+    fetch(first_pg, stage_a);
+    fetch(min(first_pg + 1, last_pg), stage_b);
     deposit(0, stage_a);
     deposit(1, stage_b);
-    fetch(min(2, last_pg), stage_a);
-    fetch(min(3, last_pg), stage_b);
+    fetch(min(first_pg + 2, last_pg), stage_a);
+    fetch(min(first_pg + 3, last_pg), stage_b);
     __syncthreads();
-    for (int pg = 0; pg < wg_pages; pg += 2) {
-        const int buf = pg & 2;  // 0 or 2
+    for (int pg = first_pg; pg < wg_pages; pg += 2) {
+        const int buf = (pg - first_pg) & 2;  // 0 or 2
         if (pg < n_pages) process_pair(pg, buf);
         deposit(buf ^ 2, stage_a);  // pages pg + 2, pg + 3
         deposit((buf ^ 2) + 1, stage_b);
@@ -540,6 +594,17 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
     // ---- normalise, gate, store ---------------------------------------------------------------------
     l_run = sum_over_lane_groups(l_run);
     if (!row_live) return;
+    if constexpr (SPLIT) {
+        if (cut) {
+            const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
+            const size_t at = slot * kRowsPerWg + wave * kRowsPerWave + c;
+            float* po = P.part_o + at * kHd + 4 * g;
+#pragma unroll
+            for (int t = 0; t < 16; ++t) *reinterpret_cast<f4*>(po + 16 * t) = o[t];
+            if (g == 0) *reinterpret_cast<float2*>(P.part_ml + at * 2) = make_float2(m_run, l_run);
+            return;
+        }
+    }
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     float* op = P.out + ((size_t)(P.b.src0[e] + tok) * P.n_q + head) * kHd;
     const float* gp = P.gate ? P.gate + (size_t)(P.b.src0[e] + tok) * P.gate_tok_stride +
@@ -552,21 +617,87 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(con
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             y[r] = o[t][r] * inv;
-            if (gp) {
-                // sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91)
-                const float gt = gp[d0 + r];
-                float sg;
-                if (gt >= 0.0f) {
-                    sg = 1.0f / (1.0f + expf(-gt));
-                } else {
-                    const float ex = expf(gt);
-                    sg = ex / (1.0f + ex);
-                }
-                y[r] *= sg;
-            }
+            if (gp) y[r] *= sigmoid(gp[d0 + r]);
         }
         *reinterpret_cast<float4*>(op + d0) = make_float4(y[0], y[1], y[2], y[3]);
     }
+}
+
+// The ranges of a cut block's rows put together: one wave per row, lane d4 owns head-dim elements
+// 4 d4 .. 4 d4 + 3; lane s holds range s's reference and denominator (at most 64 ranges).  Bound by
+// the latency of its two trips to memory, so the partial rows are requested eight at a time before
+// the references are looked at.
+constexpr int kMergeWaves = 4;
+constexpr int kMergeInFlight = 8;
+__global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(const PrefillSplitParams P, int32_t rows_per_wg) {
+    const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kMergeWaves + (int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    int unit = w / rows_per_wg;
+    const int r = w - unit * rows_per_wg;
+    if (unit >= P.s.unit_base[P.b.n]) return;
+    int e = 0;
+    while (unit >= P.s.unit_base[e + 1]) ++e;
+    unit -= P.s.unit_base[e];
+    const int kvh = unit % P.n_kv;
+    const int n_rows = P.b.n_tok[e] * P.group;
+    const int rb = (n_rows + rows_per_wg - 1) / rows_per_wg - 1 - unit / P.n_kv;
+    const int row = rb * rows_per_wg + r;
+    if (row >= n_rows) return;
+    const int wg_last_row = min(rb * rows_per_wg + rows_per_wg, n_rows) - 1;
+    int each;
+    const int ranges = split_ranges((P.b.pos0[e] + wg_last_row / P.group) / kPage + 1, P.s.pps, P.s.splits[e], each);
+    const size_t at = ((size_t)P.s.slot_base[e] + (size_t)unit * P.s.splits[e]) * rows_per_wg + r;
+    const float* po = P.part_o + at * kHd + 4 * lane;
+    const size_t step = (size_t)rows_per_wg * kHd;
+    f4 v[kMergeInFlight];
+#pragma unroll
+    for (int u = 0; u < kMergeInFlight; ++u)
+        if (u < ranges) v[u] = *reinterpret_cast<const f4*>(po + u * step);
+    float2 ml = make_float2(-INFINITY, 0.0f);
+    if (lane < ranges) ml = *reinterpret_cast<const float2*>(P.part_ml + (at + (size_t)lane * rows_per_wg) * 2);
+    const int tok = row / P.group, head = kvh * P.group + row % P.group;
+    const size_t out_row = (size_t)(P.b.src0[e] + tok);
+    float4 gt = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (P.gate) {
+        const float* gp = P.gate + out_row * P.gate_tok_stride + (size_t)head * P.gate_head_stride + 4 * lane;
+        gt = make_float4(gp[0], gp[1], gp[2], gp[3]);
+    }
+    // the first range holds cell 0, which every row attends: the maximum is finite
+    float mx = ml.x;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float wt = __builtin_amdgcn_exp2f(ml.x - mx);
+    float l = wt * ml.y;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
+    f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < ranges; s += kMergeInFlight) {
+        if (s > 0) {
+#pragma unroll
+            for (int u = 0; u < kMergeInFlight; ++u)
+                if (s + u < ranges) v[u] = *reinterpret_cast<const f4*>(po + (s + u) * step);
+        }
+#pragma unroll
+        for (int u = 0; u < kMergeInFlight; ++u)
+            if (s + u < ranges) acc += v[u] * __shfl(wt, s + u, 64);
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    float4 y = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+    if (P.gate) y = make_float4(y.x * sigmoid(gt.x), y.y * sigmoid(gt.y), y.z * sigmoid(gt.z), y.w * sigmoid(gt.w));
+    *reinterpret_cast<float4*>(P.out + (out_row * P.n_q + head) * kHd + 4 * lane) = y;
+}
+
+template <int LAY, int WAVES>
+hipError_t launch_split(bkv_pool* p, const PrefillSplitParams& kp, hipStream_t stream) {
+    constexpr int kRows = WAVES * kRowsPerWave;
+    launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<LAY, WAVES, true>,
+                  dim3((unsigned)kp.s.wg_base[kp.b.n]), dim3(64 * WAVES), 0, stream, kp);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    const unsigned rows = (unsigned)kp.s.unit_base[kp.b.n] * kRows;
+    launch_staged(p, BKV_STAGE_ATTN_MERGE, prefill_merge_kernel, dim3(rows / kMergeWaves), dim3(64 * kMergeWaves), 0,
+                  stream, kp, (int32_t)kRows);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -579,9 +710,70 @@ int32_t prefill_rows_per_wg(int32_t layout, int64_t wgs_of_64_rows, int32_t n_cu
     return wgs_of_64_rows > 2 * (int64_t)(n_cu > 0 ? n_cu : 256) ? 8 * kRowsPerWave : 4 * kRowsPerWave;
 }
 
+// Cuts the page walks of a small call's row blocks into ranges; false where the call is better off
+// uncut.  A row block's walk is a serial chain: 1.4 us a page pair on f16 pools when the compute unit
+// has nothing else (2.3-3.6 us on the quantised ones), and a call of a few blocks is as long as its longest
+// chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups, 34 us).  Cutting
+// pays for a second kernel (4-9 us, by the partial rows it reads), so:
+// - only calls that leave half of the compute units idle are cut (the merge's traffic grows with the rows);
+// - a range has at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several;
+// - the chain has to lose 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured
+//   31.1 us uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
+// - one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer than
+//   8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8.
+// Before / after, us a layer: 41 tokens behind 517 cells 37 / 24.6, 100 behind 8000 374 / 57, 200 behind
+// 3000 with q8_0 V 262 / 64, 300 behind 1000 on an int8 pool 125 / 55.
+bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s) {
+    const int32_t n_kv = p->g.n_kv;
+    const int n_cu = p->n_cu > 0 ? p->n_cu : 256;
+    if ((int64_t)b.wg_base[b.n] * 2 > n_cu) return false;
+    const bool f16 = p->g.layout == BKV_LAYOUT_F16;
+    const int64_t least = f16 ? 3 : 2, gain = f16 ? 10 : 5;
+    const int64_t room = (int64_t)p->max_wgs * 8 / rows;  // partial results the workspace holds
+    int64_t work = 0;
+    int32_t longest = 0;
+    const auto pairs_of = [&](int i, int32_t blk) {
+        const int32_t last_row = std::min((blk + 1) * rows, b.n_tok[i] * group) - 1;
+        return ((b.pos0[i] + last_row / group) / kPage + 2) / 2;
+    };
+    const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
+    for (int i = 0; i < b.n; ++i) {
+        const int32_t nb = blocks_of(i);
+        for (int32_t k = 0; k < nb; ++k) work += (int64_t)pairs_of(i, k) * n_kv;
+        if (nb) longest = std::max(longest, pairs_of(i, nb - 1));
+    }
+    int64_t most = std::min<int64_t>(room, n_cu);
+    if (f16 && work > 8 * most) most = std::min<int64_t>(room, 2 * n_cu);
+    int64_t each = std::max<int64_t>({least, (work + most - 1) / most, (longest + 63) / 64});
+    for (;; each += std::max<int64_t>(1, each / 8)) {
+        if (longest < each + gain) return false;
+        int64_t wgs = 0, units = 0, slots = 0;
+        for (int i = 0; i < b.n; ++i) {
+            const int32_t nb = blocks_of(i);
+            int32_t cut = 0;
+            while (cut < nb && pairs_of(i, nb - 1 - cut) > each) ++cut;
+            const int64_t ranges = cut ? (pairs_of(i, nb - 1) + each - 1) / each : 1;
+            s.n_cut[i] = cut;
+            s.splits[i] = (int32_t)ranges;
+            s.unit_base[i] = (int32_t)units;
+            s.slot_base[i] = (int32_t)slots;
+            s.wg_base[i] = (int32_t)wgs;
+            units += (int64_t)cut * n_kv;
+            slots += cut * n_kv * ranges;
+            wgs += cut * n_kv * ranges + (int64_t)(nb - cut) * n_kv;
+        }
+        s.unit_base[b.n] = (int32_t)units;
+        s.wg_base[b.n] = (int32_t)wgs;
+        if (wgs <= most) break;
+    }
+    s.pps = (int32_t)each * 2;
+    return true;
+}
+
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
-                               int32_t rows_per_wg, hipStream_t stream) {
-    PrefillKernelParams kp;
+                               int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream) {
+    PrefillSplitParams sp;
+    PrefillKernelParams& kp = sp;
     kp.b = b;
     kp.kpool = p->k_layer[(size_t)layer];
     kp.vpool = p->v_layer[(size_t)layer];
@@ -598,6 +790,15 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
     kp.scale_log2e = a.scale * kLog2e;
     int32_t grid = b.wg_base[b.n];
     if (grid == 0) return hipSuccess;
+    if (split) {
+        kp.by_xcd = 0;
+        sp.s = *split;
+        sp.part_o = p->part_o;
+        sp.part_ml = p->part_ml;
+        if (p->g.layout == BKV_LAYOUT_Q8V) return launch_split<BKV_LAYOUT_Q8V, 8>(p, sp, stream);
+        if (p->g.layout == BKV_LAYOUT_I8H) return launch_split<BKV_LAYOUT_I8H, 8>(p, sp, stream);
+        return launch_split<BKV_LAYOUT_F16, 4>(p, sp, stream);
+    }
     // Deal the work-groups to the dies by unit where that costs little: the grid then holds 8 x the
     // longest die's share, and work-groups past a shorter die's share leave at once.
     kp.by_xcd = 0;
