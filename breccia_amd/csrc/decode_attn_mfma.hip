@@ -36,91 +36,109 @@ __device__ __forceinline__ void split_hi_lo(float x, _Float16& hi, _Float16& lo)
     lo = (_Float16)(x - (float)hi);
 }
 
-// q fragments of head c of the kv head (heads past the group stay zero): lane (c, g) holds
-// q[head][32 m + 8 g + 0..7], m = 0..7, as a high and a low f16 part
-__device__ __forceinline__ void load_q_fragments(const AttnKernelParams& P, int e, int kvh, int c, int g,
-                                                 half8 (&qhi)[8], half8 (&qlo)[8]) {
-    const bool head_live = c < P.group;
-    const float* qp = P.q + ((size_t)e * P.n_q + (size_t)kvh * P.group + (head_live ? c : 0)) * kHd + g * 8;
+// q fragments of head c of the kv head: lane (c, g) holds q[head][32 m + 8 g + 0..7], m = 0..7, as a high and
+// a low f16 part.  The waves of a work-group need the same fragments, and splitting the 64 values of a lane
+// into 128 halves took each of them a microsecond of issue at the head of a launch that may last eight; so
+// wave w requests and splits fragments 2 w and 2 w + 1 only, and the waves trade them through LDS.  They are
+// requested ahead of the first pages: loads return in order, and waiting for q must not wait for those.
+// Columns past the group are zeros: nothing of them is stored, but matrix cores that multiply zeros draw less
+// power (16 int8 sequences of 8k to 128k at 8 heads a group: 275 us, against 288 with head 0 repeated there).
+constexpr int kQFragsPerWave = 8 / kWaves;
+struct QFragLds {
+    half8 part[8][2][64];  // [fragment][high, low][lane]
+};
+struct QRaw {
+    float4 x[kQFragsPerWave][2];
+};
+__device__ __forceinline__ void request_q(const AttnKernelParams& P, int e, int kvh, int wave, int c, int g, QRaw& q) {
+    const float* qp = P.q + ((size_t)e * P.n_q + (size_t)kvh * P.group + (c < P.group ? c : 0)) * kHd + g * 8;
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        float x[8];
-        const float4 a = *reinterpret_cast<const float4*>(qp + m * 32);
-        const float4 b = *reinterpret_cast<const float4*>(qp + m * 32 + 4);
-        x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
-        x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+    for (int i = 0; i < kQFragsPerWave; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            q.x[i][j] = *reinterpret_cast<const float4*>(qp + (wave * kQFragsPerWave + i) * 32 + 4 * j);
+}
+__device__ __forceinline__ void trade_q(const QRaw& q, QFragLds& L, int wave, int lane, bool head_live, half8 (&qhi)[8], half8 (&qlo)[8]) {
+#pragma unroll
+    for (int i = 0; i < kQFragsPerWave; ++i) {
+        const float x[8] = {q.x[i][0].x, q.x[i][0].y, q.x[i][0].z, q.x[i][0].w,
+                            q.x[i][1].x, q.x[i][1].y, q.x[i][1].z, q.x[i][1].w};
+        half8 h, l;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             _Float16 hi, lo;
             split_hi_lo(head_live ? x[j] : 0.0f, hi, lo);
-            qhi[m][j] = hi;
-            qlo[m][j] = lo;
+            h[j] = hi;
+            l[j] = lo;
         }
+        L.part[wave * kQFragsPerWave + i][0][lane] = h;
+        L.part[wave * kQFragsPerWave + i][1][lane] = l;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        qhi[m] = L.part[m][0][lane];
+        qlo[m] = L.part[m][1][lane];
     }
 }
 
 constexpr int kOwStride = kHd + 4;  // floats per head in the wave-merge staging
 
-// Shared tail of the MFMA decode kernels: wave totals, then every wave stages its scaled O in
-// LDS and each wave sums one quarter of the columns over the four stagings and writes it as the
-// work-group's partial (m, l, O) in the layout the merge kernel reads.
+// Shared tail of the MFMA decode kernels: every wave stages its O and its (m, l) in LDS, then each wave
+// sums one quarter of the columns over the four stagings, every staging at the scale of its distance to the
+// common maximum, and writes it as the work-group's partial (m, l, O) in the layout the merge kernel reads.
 // o[h][t][r] of lane (c, g) is out[head c][128 h + 8 (4 g + r) + t].
 struct MfmaFoldLds {
     float ow[kWaves][16][kOwStride];
-    float wave_m[kWaves][16];
-    float wave_l[kWaves][16];
+    float wave_m[16][kWaves];
+    float wave_l[16][kWaves];
 };
 
 __device__ __forceinline__ void mfma_fold_and_store(const AttnKernelParams& P, MfmaFoldLds& L, int wg, int wave,
                                                     int c, int g, f4 (&o)[2][8], float m_run, float l_run) {
     auto& ow = L.ow;
-    auto& wave_m = L.wave_m;
-    auto& wave_l = L.wave_l;
+    const int hg = P.group;
     l_run = sum_over_lane_groups(l_run);
-    if (g == 0) {
-        wave_m[wave][c] = m_run;
-        wave_l[wave][c] = l_run;
-    }
-    __syncthreads();
-    float mx = wave_m[0][c];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) mx = fmaxf(mx, wave_m[w][c]);
-    float lsum = 0.0f;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-        const float mw = wave_m[w][c];
-        lsum = fmaf(mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw - mx), wave_l[w][c], lsum);
-    }
-    {
-        const float f = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mx);
+    if (c < hg) {  // columns past the group are nobody's
+        if (g == 0) {
+            L.wave_m[c][wave] = m_run;
+            L.wave_l[c][wave] = l_run;
+        }
         // element (h, r, t) of a lane is out[head c][128 h + 8 (4 g + r) + t]: 8 consecutive floats per (h, r)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 float* d = &ow[wave][c][128 * h + 8 * (4 * g + r)];
-                *reinterpret_cast<f4*>(d) = f4{o[h][0][r] * f, o[h][1][r] * f, o[h][2][r] * f, o[h][3][r] * f};
-                *reinterpret_cast<f4*>(d + 4) = f4{o[h][4][r] * f, o[h][5][r] * f, o[h][6][r] * f, o[h][7][r] * f};
+                *reinterpret_cast<f4*>(d) = f4{o[h][0][r], o[h][1][r], o[h][2][r], o[h][3][r]};
+                *reinterpret_cast<f4*>(d + 4) = f4{o[h][4][r], o[h][5][r], o[h][6][r], o[h][7][r]};
             }
     }
     __syncthreads();
     // wave w sums columns [64 w, 64 w + 64): lane (c, g) takes 4 columns at 4 c of heads g, g + 4, ...
-    const int hg = P.group;
+    const int col = 64 * wave + 4 * c;
 #pragma unroll
     for (int hp = 0; hp < 16; hp += 4) {
         const int head = hp + g;
         if (hp >= hg) break;
         if (head < hg) {
-            const int col = 64 * wave + 4 * c;
-            f4 acc = *reinterpret_cast<const f4*>(&ow[0][head][col]);
+            const f4 m = *reinterpret_cast<const f4*>(&L.wave_m[head][0]);
+            const f4 l = *reinterpret_cast<const f4*>(&L.wave_l[head][0]);
+            const float mx = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
+            f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            float lsum = 0.0f;
 #pragma unroll
-            for (int w = 1; w < kWaves; ++w) acc += *reinterpret_cast<const f4*>(&ow[w][head][col]);
+            for (int w = 0; w < kWaves; ++w) {
+                const float f = m[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[w] - mx);
+                acc += *reinterpret_cast<const f4*>(&ow[w][head][col]) * f;
+                lsum = fmaf(f, l[w], lsum);
+            }
             *reinterpret_cast<f4*>(P.part_o + ((size_t)wg * hg + head) * kHd + col) = acc;
+            if (wave == 0 && c == 0) {
+                P.part_ml[((size_t)wg * hg + head) * 2 + 0] = mx;
+                P.part_ml[((size_t)wg * hg + head) * 2 + 1] = lsum;
+            }
         }
-    }
-    if (wave == 0 && g == 0 && c < hg) {
-        P.part_ml[((size_t)wg * hg + c) * 2 + 0] = mx;
-        P.part_ml[((size_t)wg * hg + c) * 2 + 1] = lsum;
     }
 }
 
@@ -147,7 +165,11 @@ __device__ __forceinline__ void k_pair_home(const v4u& lo_rows, const v4u& hi_ro
 template <bool STEP, bool SEL = false, bool DESC = false>
 __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnKernelParams P) {
     static_assert(!(STEP && SEL), "the fused step attends the dense selection");
+    // the q fragments on their way between the waves lie where the fold staging will be
     __shared__ __attribute__((aligned(16))) MfmaFoldLds lds;
+    QFragLds& q_lds = *reinterpret_cast<QFragLds*>(&lds.ow[0][0][0]);
+    static_assert(sizeof(QFragLds) <= sizeof(lds.ow), "the staging holds the q fragments");
+    __shared__ __attribute__((aligned(16))) v4u new_row[STEP ? 64 : 1];  // STEP: the row of cell pos, K then V
 
     // ---- which (entry, kv head, page range); one work-group per unit (no head chunks) --------
     const int unit = blockIdx.x;
@@ -224,6 +246,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
         return reinterpret_cast<const v4u*>(rows + (size_t)r * (kHd * 2) + (size_t)(h * 128 + c * 8) * 2);
     };
 
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
     int pg = pg0 + wave;
     v4u kf[8], vf[2][4];
     RowRuns<SEL> cur{};
@@ -245,12 +270,15 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
             for (int r = 0; r < 4; ++r) vf[h][r] = __builtin_nontemporal_load(v_addr(vp, h, r));
     }
 
+    half8 qhi[8], qlo[8];
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
+    __syncthreads();  // a wave without pages goes straight to the fold
+
     // STEP: the wave that will hold the page of cell pos (in its last iteration) takes the new row now,
     // while its first pages are on their way: lane l < 32 converts slice l (8 values) of the K row, lane
     // 32 + l slice l of the V row, stores it into the pool (whole rows, 16 bytes a lane) and parks it in
-    // the wave's part of the fold staging, which nothing else uses before the loop is over.  Fetched at
-    // the last page instead, the row would add a trip to memory to the end of that work-group's walk.
-    v4u* const new_row = reinterpret_cast<v4u*>(&lds.ow[wave][0][0]);
+    // LDS.  Fetched at the last page instead, the row would add a trip to memory to the end of that
+    // work-group's walk.
     if constexpr (STEP) {
         const int last = n_pages - 1;
         if (last >= pg0 && last < pg1 && ((last - pg0) & (kWaves - 1)) == wave) {
@@ -268,9 +296,6 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         }
     }
-
-    half8 qhi[8], qlo[8];
-    load_q_fragments(P, e, kvh, c, g, qhi, qlo);
 
     // O^T accumulators: o[h][t][r] = out[head c][128 h + 8 (4 g + r) + t]
     f4 o[2][8];
@@ -529,6 +554,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     // one slot per wave; the fold staging of the epilogue reuses the memory
     constexpr int kRing = kWaves * kI8hSlot > (int)sizeof(MfmaFoldLds) ? kWaves * kI8hSlot : (int)sizeof(MfmaFoldLds);
     __shared__ __attribute__((aligned(16))) uint8_t ring[kRing];
+    // the q fragments on their way between the waves lie behind the slots
+    static_assert(kWaves * kI8hSlot + sizeof(QFragLds) <= sizeof(MfmaFoldLds), "slots and q fragments fit the fold staging");
+    QFragLds& q_lds = *reinterpret_cast<QFragLds*>(ring + kWaves * kI8hSlot);
     constexpr int kRow = row_bytes_of(kRowI8H);  // 272
     // STEP: the new K row and the new V row of the entry, encoded; one wave of a work-group at most
     __shared__ __attribute__((aligned(16))) uint8_t parked[STEP ? 2 * kRow : 16];
@@ -588,6 +616,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
         unit_src(i, P.vpool, u);
         i8h_unit_fetch<SEL>(u, lane, v_regs);
     };
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
     if (SEL || n_steps > 0) fetch(0);  // a selection list's first units before its length is known
 
     // STEP: the wave that will hold the page of cell pos (in its last step) takes the new rows before the
@@ -617,7 +648,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     }
 
     half8 qhi[8], qlo[8];
-    load_q_fragments(P, e, kvh, c, g, qhi, qlo);
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
 
     if constexpr (STEP) {
         if (takes_new_row) {
@@ -872,6 +903,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     constexpr int kWaveLds = kQ8vUnit;
     constexpr int kLds = kWaves * kWaveLds > (int)sizeof(MfmaFoldLds) ? kWaves * kWaveLds : (int)sizeof(MfmaFoldLds);
     __shared__ __attribute__((aligned(16))) uint8_t smem[kLds];
+    // the q fragments on their way between the waves lie behind the slots
+    static_assert(kWaves * kWaveLds + sizeof(QFragLds) <= sizeof(MfmaFoldLds), "slots and q fragments fit the fold staging");
+    QFragLds& q_lds = *reinterpret_cast<QFragLds*>(smem + kWaves * kWaveLds);
     // STEP: the new row of the entry, encoded (512 bytes of K, 288 of V); one wave of a work-group at most
     __shared__ __attribute__((aligned(16))) uint8_t parked[STEP ? 512 + kQ8vRow : 16];
 
@@ -942,6 +976,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     };
     // the page in flight: K in the fragment registers, refilled as they are used up; the V unit requested
     // while the page before is multiplied
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
     v4u kf[8];
     Q8vUnitRegs v_regs;
     if (SEL || n_steps > 0) {  // a selection list's first units before its length is known
@@ -991,7 +1028,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     }
 
     half8 qhi[8], qlo[8];
-    load_q_fragments(P, e, kvh, c, g, qhi, qlo);
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
 
     if constexpr (STEP) {
         if (takes_new_row) {
