@@ -317,6 +317,7 @@ struct KPrepParams {
     const int32_t* positions;  // optional: rotary position of cell c; null = c itself
     float eps;
     int32_t n_rot, max_pos;
+    uint32_t inv_kv32;  // ceil(2^32 / n_kv) (0 for one head): row / n_kv as a multiplication
 };
 
 constexpr int kPrepRows = 16;  // (token, kv head) rows per work-group
@@ -348,8 +349,12 @@ __device__ __forceinline__ void rotate_pair(float& lo, float& hi, float c32, flo
 
 // HD: the head dim as a compile-time constant (the index arithmetic of every loop divides by it),
 // or 0 for the value in the geometry.
-template <int LAYOUT, int HD>
-__global__ __launch_bounds__(kBlock) void append_kprep_kernel(AppendBatch b, MoveGeom g,
+// AHEAD (head dim 256): for calls with many rows.  What the later phases read -- the thread's rotary pairs, its
+// groups of V, its gamma -- is requested with the K rows, so that the phases between the barriers wait for one
+// trip to memory instead of one each, and scaling reads four rows at a time.  4 x 16384 tokens: f16 81 -> 77 us
+// (5.2 TB/s), q8_0 V 82 -> 72, int8 80 -> 69; 2 x 512: 8.9 -> 7.6, 9.6 -> 8.5, 9.9 -> 9.1.
+template <int LAYOUT, int HD, bool AHEAD>
+__global__ __launch_bounds__(kBlock, AHEAD ? 5 : 1) void append_kprep_kernel(AppendBatch b, MoveGeom g,
                                                               KPrepParams kp,
                                                               uint8_t* __restrict__ kpool,
                                                               uint8_t* __restrict__ vpool,
@@ -371,52 +376,138 @@ __global__ __launch_bounds__(kBlock) void append_kprep_kernel(AppendBatch b, Mov
     const size_t src_base = ((size_t)b.src0[s] * g.n_kv + (size_t)r0) * (size_t)hd;
     const int tid = threadIdx.x;
 
-    // rows of one sequence are contiguous in the source: one coalesced sweep
-    for (int idx = tid; idx < nrows * hd / 4; idx += kBlock) {
-        const v4u w = ld_stream(k + src_base + (size_t)idx * 4);
-        const int row = (idx * 4) / hd, col = (idx * 4) % hd;
-        *reinterpret_cast<v4u*>(prep_lds + row * stride + col) = w;
+    static_assert(!AHEAD || HD == 256, "the index arithmetic of AHEAD is for 256 values a row");
+    const int half = kp.n_rot / 2;
+    const int lpr = hd / 8;  // 8-value groups of a row
+    uint64_t* const row_s = reinterpret_cast<uint64_t*>(inv_s + kPrepRows);
+    int32_t* const pos_s = reinterpret_cast<int32_t*>(row_s + kPrepRows);
+    constexpr int kVGroups = AHEAD ? kPrepRows * 256 / 8 / kBlock : 1;   // 8-value groups of a thread
+    constexpr int kPairs = AHEAD ? 2 : 1;                                // rotary pairs requested ahead
+    // AHEAD: in the rotary phase thread t has row t % 16 and pairs t / 16 + 16 i (all 64 lanes of a wave in banks
+    // of their own); this is its row's cell and rotary position
+    const int my_row = min(tid & (kPrepRows - 1), nrows - 1), my_col = tid / kPrepRows;
+    unsigned my_cell = 0, my_kvh = 0;
+    int my_pos = 0;
+    float v_ahead[kVGroups][8];
+    float2 cs_ahead[kPairs];
+    float gamma = 0.0f;
+    if constexpr (AHEAD) {
+        // no branches around the loads (the compiler waits for a load at the end of its branch): indices
+        // past the rows are clamped to the last and what they read is dropped
+        v4u kk[kPrepRows * 256 / 4 / kBlock];
+#pragma unroll
+        for (int i = 0; i < kPrepRows * 256 / 4 / kBlock; ++i)
+            kk[i] = ld_stream(k + src_base + (size_t)min(tid + i * kBlock, nrows * 64 - 1) * 4);
+        gamma = kp.gamma[tid];
+#pragma unroll
+        for (int i = 0; i < kVGroups; ++i)
+            load8(v + src_base + (size_t)min(tid + i * kBlock, nrows * 32 - 1) * 8, v_ahead[i]);
+        const unsigned r = (unsigned)(r0 + my_row);
+        const unsigned t = kp.inv_kv32 ? __umulhi(r, kp.inv_kv32) : r;
+        my_cell = (unsigned)b.pos0[s] + t;
+        my_kvh = r - t * (unsigned)g.n_kv;
+        const int64_t pos = kp.positions ? (int64_t)kp.positions[my_cell] : (int64_t)my_cell;
+        my_pos = (int)(pos < 0 ? 0 : (pos > kp.max_pos - 1 ? kp.max_pos - 1 : pos));
+        // without a rotary there may be no table: any address that can be read stands in
+        const float2* const cs = half > 0 ? reinterpret_cast<const float2*>(kp.table) + (size_t)my_pos * half
+                                          : reinterpret_cast<const float2*>(kp.gamma);
+#pragma unroll
+        for (int i = 0; i < kPairs; ++i) cs_ahead[i] = cs[max(min(my_col + 16 * i, half - 1), 0)];
+#pragma unroll
+        for (int i = 0; i < kPrepRows * 256 / 4 / kBlock; ++i) {
+            const int idx = tid + i * kBlock;
+            if (idx < nrows * 64) *reinterpret_cast<v4u*>(prep_lds + (idx >> 6) * stride + (idx & 63) * 4) = kk[i];
+        }
+    } else {
+        // rows of one sequence are contiguous in the source: one coalesced sweep
+        for (int idx = tid; idx < nrows * hd / 4; idx += kBlock) {
+            const v4u w = ld_stream(k + src_base + (size_t)idx * 4);
+            const int row = (idx * 4) / hd, col = (idx * 4) % hd;
+            *reinterpret_cast<v4u*>(prep_lds + row * stride + col) = w;
+        }
     }
     __syncthreads();
     // While the first lanes sum their rows, a second wave works out where the rows go: the pool row
     // of (sequence row r) = (token, kv head) and the token's rotary position.
-    uint64_t* const row_s = reinterpret_cast<uint64_t*>(inv_s + kPrepRows);
-    int32_t* const pos_s = reinterpret_cast<int32_t*>(row_s + kPrepRows);
     if (tid < nrows) {
         const double ss = row_sum_squares(prep_lds + tid * stride, hd);
         inv_s[tid] = 1.0 / sqrt(ss / (double)hd + (double)kp.eps);
     } else if (tid >= 64 && tid - 64 < nrows) {
-        const unsigned r = (unsigned)(r0 + tid - 64);
-        const unsigned cell = (unsigned)b.pos0[s] + r / (unsigned)g.n_kv;
-        const unsigned kvh = r % (unsigned)g.n_kv;
-        const int32_t phys = tables[(size_t)b.row[s] * (size_t)g.max_pages_per_seq + (size_t)(cell >> kPageShift)];
-        row_s[tid - 64] = (((uint64_t)phys * g.n_kv + kvh) << kPageShift) + (uint64_t)(cell & kPageMask);
-        int64_t pos = kp.positions ? (int64_t)kp.positions[cell] : (int64_t)cell;
-        pos = pos < 0 ? 0 : (pos > kp.max_pos - 1 ? kp.max_pos - 1 : pos);
-        pos_s[tid - 64] = (int32_t)pos;
+        if constexpr (!AHEAD) {
+            const unsigned r = (unsigned)(r0 + tid - 64);
+            my_cell = (unsigned)b.pos0[s] + r / (unsigned)g.n_kv;
+            my_kvh = r % (unsigned)g.n_kv;
+        }
+        const int32_t phys = tables[(size_t)b.row[s] * (size_t)g.max_pages_per_seq + (size_t)(my_cell >> kPageShift)];
+        row_s[tid - 64] = (((uint64_t)phys * g.n_kv + my_kvh) << kPageShift) + (uint64_t)(my_cell & kPageMask);
+        if constexpr (!AHEAD) {
+            int64_t pos = kp.positions ? (int64_t)kp.positions[my_cell] : (int64_t)my_cell;
+            pos = pos < 0 ? 0 : (pos > kp.max_pos - 1 ? kp.max_pos - 1 : pos);
+            pos_s[tid - 64] = (int32_t)pos;
+        }
     }
     __syncthreads();
-    for (int idx = tid; idx < nrows * hd; idx += kBlock) {
-        const int row = idx / hd, col = idx % hd;
-        float* d = prep_lds + row * stride + col;
-        *d = (float)((double)*d * inv_s[row] * (double)kp.gamma[col]);
-    }
-    __syncthreads();
-    const int half = kp.n_rot / 2;
-    for (int idx = tid; idx < nrows * half; idx += kBlock) {
-        const int row = idx / half, j = idx % half;
-        const float2 cs = reinterpret_cast<const float2*>(kp.table)[(size_t)pos_s[row] * half + j];
-        float* d = prep_lds + row * stride;
-        rotate_pair(d[j], d[j + half], cs.x, cs.y);
+    if constexpr (AHEAD) {
+        // thread t has column t of every row; four rows at a time, so that their reads are on their way together
+#pragma unroll
+        for (int r = 0; r < kPrepRows; r += 4) {
+            if (r >= nrows) break;
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                x[i] = (float)((double)prep_lds[(r + i) * stride + tid] * inv_s[r + i] * (double)gamma);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (r + i < nrows) prep_lds[(r + i) * stride + tid] = x[i];
+        }
+        __syncthreads();
+        if ((tid & (kPrepRows - 1)) < nrows) {
+            float* d = prep_lds + my_row * stride;
+#pragma unroll
+            for (int i = 0; i < kPairs; ++i) {
+                const int j = my_col + 16 * i;
+                if (j < half) rotate_pair(d[j], d[j + half], cs_ahead[i].x, cs_ahead[i].y);
+            }
+            for (int j = my_col + 16 * kPairs; j < half; j += 16) {
+                const float2 cs = reinterpret_cast<const float2*>(kp.table)[(size_t)my_pos * half + j];
+                rotate_pair(d[j], d[j + half], cs.x, cs.y);
+            }
+        }
+    } else {
+        for (int idx = tid; idx < nrows * hd; idx += kBlock) {
+            const int row = idx / hd, col = idx % hd;
+            float* d = prep_lds + row * stride + col;
+            *d = (float)((double)*d * inv_s[row] * (double)kp.gamma[col]);
+        }
+        __syncthreads();
+        for (int idx = tid; idx < nrows * half; idx += kBlock) {
+            const int row = idx / half, j = idx % half;
+            const float2 cs = reinterpret_cast<const float2*>(kp.table)[(size_t)pos_s[row] * half + j];
+            float* d = prep_lds + row * stride;
+            rotate_pair(d[j], d[j + half], cs.x, cs.y);
+        }
     }
     __syncthreads();
 
     const auto pool_row = [&](int row) -> size_t { return (size_t)row_s[row]; };
-    const int lpr = hd / 8;  // 8-value groups of a row
+    // every 8-value group of the thread: group(index, its values of V)
+    const auto each_group = [&](auto group) {
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int i = 0; i < kVGroups; ++i)
+                if (tid + i * kBlock < nrows * lpr) group(tid + i * kBlock, v_ahead[i]);
+        } else {
+            for (int idx = tid; idx < nrows * lpr; idx += kBlock) {
+                float vx[8];
+                load8(v + src_base + (size_t)idx * 8, vx);
+                group(idx, vx);
+            }
+        }
+    };
 
     if (LAYOUT == BKV_LAYOUT_F16) {
         // K from LDS, V straight from the source rows
-        for (int idx = tid; idx < nrows * lpr; idx += kBlock) {
+        each_group([&](int idx, const float (&y)[8]) {
             const int row = (idx * 8) / hd, col = (idx * 8) % hd;
             const float* x = prep_lds + row * stride + col;
             v4u o;
@@ -425,14 +516,12 @@ __global__ __launch_bounds__(kBlock) void append_kprep_kernel(AppendBatch b, Mov
             o.z = pack2(x[4], x[5]);
             o.w = pack2(x[6], x[7]);
             st_stream(reinterpret_cast<uint16_t*>(kpool) + pool_row(row) * (size_t)hd + col, o);
-            float y[8];
-            load8(v + src_base + (size_t)idx * 8, y);
             o.x = pack2(y[0], y[1]);
             o.y = pack2(y[2], y[3]);
             o.z = pack2(y[4], y[5]);
             o.w = pack2(y[6], y[7]);
             st_stream(reinterpret_cast<uint16_t*>(vpool) + pool_row(row) * (size_t)hd + col, o);
-        }
+        });
         return;
     }
     // Quantised rows, as in append_quant_kernel: a lane encodes 8 consecutive values (the four lanes of a
@@ -442,13 +531,11 @@ __global__ __launch_bounds__(kBlock) void append_kprep_kernel(AppendBatch b, Mov
     const int blocks = hd / 32;
     const uint32_t row_bytes = LAYOUT == BKV_LAYOUT_Q8V ? (uint32_t)blocks * 36u : (uint32_t)hd + (uint32_t)blocks * 2u;
     uint8_t* const v_image = image + (LAYOUT == BKV_LAYOUT_I8H ? kPrepRows * row_bytes : 0u);
-    for (int idx = tid; idx < nrows * lpr; idx += kBlock) {
+    each_group([&](int idx, float (&vx)[8]) {
         const int row = idx / lpr, li = idx - row * lpr;
         const int blk = li >> 2, quarter = li & 3;
         const float* kxp = prep_lds + row * stride + li * 8;
         const float4 ka = *reinterpret_cast<const float4*>(kxp), kb = *reinterpret_cast<const float4*>(kxp + 4);
-        float vx[8];
-        load8(v + src_base + (size_t)idx * 8, vx);
         if (LAYOUT == BKV_LAYOUT_Q8V) {
             v4u o;
             o.x = pack2(ka.x, ka.y);
@@ -477,7 +564,7 @@ __global__ __launch_bounds__(kBlock) void append_kprep_kernel(AppendBatch b, Mov
                 *reinterpret_cast<uint16_t*>(vr + hd + blk * 2) = (uint16_t)vs;
             }
         }
-    }
+    });
     __syncthreads();
     constexpr uint32_t kPiece = HD == 256 ? 16u : 4u;
     if (LAYOUT == BKV_LAYOUT_I8H) image_rows_out<kPiece>(image, kpool, row_s, nrows, row_bytes, tid);
@@ -720,22 +807,32 @@ hipError_t launch_append_kprep(bkv_pool* p, int32_t layer, const AppendBatch& b,
                                const float* table, int32_t n_rot, int32_t max_pos,
                                const int32_t* positions, hipStream_t stream) {
     const MoveGeom g = move_geom(p);
-    const KPrepParams kp{gamma, table, positions, eps, n_rot, max_pos};
+    const KPrepParams kp{gamma, table, positions, eps, n_rot, max_pos,
+                         g.n_kv > 1 ? (uint32_t)(((1ull << 32) + (uint64_t)g.n_kv - 1) / (uint64_t)g.n_kv) : 0u};
     const int rows = max_tok * g.n_kv;
     dim3 grid((unsigned)((rows + kPrepRows - 1) / kPrepRows), (unsigned)b.n);
+    // AHEAD from 16 whole tiles on (32 tiles: 8.8 -> 7.8 us); for the few rows of a decode step the longer
+    // preamble costs more than the trips it saves (8 tokens: 5.6 -> 6.9 us).  Its row / n_kv is exact while
+    // row * n_kv < 2^32.
+    int64_t tiles = 0;
+    for (int i = 0; i < b.n; ++i) tiles += (int64_t)b.n_tok[i] * g.n_kv / kPrepRows;
+    const bool ahead = g.hd == 256 && tiles >= 16 && (int64_t)rows * g.n_kv < (1ll << 32);
     const size_t lds = (size_t)kPrepRows * (g.hd + 4) * sizeof(float) +
                        kPrepRows * (sizeof(double) + sizeof(uint64_t) + sizeof(int32_t));
     uint8_t* kpl = p->k_layer[(size_t)layer];
     uint8_t* vpl = p->v_layer[(size_t)layer];
-    const auto launch = [&](auto layout_tag, auto hd_tag) {
-        launch_staged(p, BKV_STAGE_APPEND_KPREP, append_kprep_kernel<decltype(layout_tag)::value, decltype(hd_tag)::value>,
+    const auto launch = [&](auto layout_tag, auto hd_tag, auto ahead_tag) {
+        launch_staged(p, BKV_STAGE_APPEND_KPREP,
+                      append_kprep_kernel<decltype(layout_tag)::value, decltype(hd_tag)::value, decltype(ahead_tag)::value>,
                       grid, dim3(kBlock), (uint32_t)lds, stream, b, g, kp, kpl, vpl, (const int32_t*)p->table_dev, k, v);
     };
     const auto by_hd = [&](auto layout_tag) {
-        if (g.hd == 256)
-            launch(layout_tag, std::integral_constant<int, 256>{});
+        if (ahead)
+            launch(layout_tag, std::integral_constant<int, 256>{}, std::true_type{});
+        else if (g.hd == 256)
+            launch(layout_tag, std::integral_constant<int, 256>{}, std::false_type{});
         else
-            launch(layout_tag, std::integral_constant<int, 0>{});
+            launch(layout_tag, std::integral_constant<int, 0>{}, std::false_type{});
     };
     switch (p->g.layout) {
         case BKV_LAYOUT_F16:

@@ -216,3 +216,38 @@ def test_errors_come_before_any_launch():
         device_sync()
     z.free()
     prep.free()
+
+
+@pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H])
+@pytest.mark.parametrize("n_kv, n_rot, tokens, with_positions", [
+    (1, 64, [15, 255], False),          # one head; fifteen tiles of whole rows in all: just below the path for many rows
+    (1, 64, [256, 3], True),            # sixteen whole tiles, and a sequence of three rows beside them
+    (3, 2, [90, 1], False),             # rows divided by three; one rotary pair
+    (4, 256, [80, 7, 33], True),        # every value rotated: pairs beyond the two requested ahead
+])
+def test_many_rows_in_one_call_are_bit_exact(n_kv, n_rot, tokens, with_positions, layout):
+    rng = np.random.Generator(np.random.PCG64(900 + n_rot + layout))
+    gamma = (1.0 + 0.3 * rng.standard_normal(HD)).astype(np.float32)
+    pos0 = [5 * i for i in range(len(tokens))]
+    cells = 1024
+    positions = rng.integers(-3, 700, size=cells).astype(np.int32) if with_positions else None
+    prep = Prep(gamma, max_pos=600, n_rot=n_rot, positions=positions)
+    with Twin(n_pages=128, n_kv=n_kv, layout=layout, max_seqs=4) as tw:
+        seqs = [tw.pool.seq_create() for _ in tokens]
+        for s, p0, t in zip(seqs, pos0, tokens):
+            tw.pool.seq_reserve(s, p0 + t)
+        ks = [rng.standard_normal((t, n_kv, HD)).astype(np.float32) for t in tokens]
+        vs = [rng.standard_normal((t, n_kv, HD)).astype(np.float32) for t in tokens]
+        kd = DeviceBuffer.from_numpy(np.concatenate([k.reshape(-1) for k in ks]))
+        vd = DeviceBuffer.from_numpy(np.concatenate([v.reshape(-1) for v in vs]))
+        tw.pool.append_kprep(0, seqs, pos0, tokens, kd, vd, prep.gd, EPS, prep.td, n_rot, prep.max_pos, prep.pd)
+        device_sync()
+        for s, p0, k, v, t in zip(seqs, pos0, ks, vs, tokens):
+            at = p0 + np.arange(t)
+            at = np.clip(at if positions is None else positions[at], 0, prep.max_pos - 1)
+            want = oracle.k_prep(k, n_kv, HD, gamma, EPS, prep.table, n_rot, at)
+            assert tw.images[0].append(tw.pool.block_table(s), p0, want, v, capacity_cells=tw.pool.seq_capacity(s)) == 0
+        tw.assert_pools_equal()
+        kd.free()
+        vd.free()
+    prep.free()
