@@ -504,9 +504,9 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
         // Cell 0 is live for every query, so from the first pair on the reference m_run is finite.
         // It follows the running maximum lazily: it moves only when a pair's maximum passes it by
         // more than kSlack (weights then reach 2^kSlack at most, far inside f16 and f32), which after
-        // the first pairs is rare -- and every move costs a rescale of the 64 accumulators.  The
-        // q8_0 weights multiply values of up to 2^8, so there the reference is the maximum itself.
-        constexpr float kSlack = Q8V ? 0.0f : 6.0f;
+        // the first pairs is rare -- and every move costs a rescale of the 64 accumulators.  (q8_0 weights
+        // multiply values of up to 2^8: products of up to 2^14, summed in f32.)
+        constexpr float kSlack = 6.0f;
         float pm = fmaxf(fmaxf(fmaxf(wa[0], wa[1]), fmaxf(wa[2], wa[3])), fmaxf(fmaxf(wb[0], wb[1]), fmaxf(wb[2], wb[3])));
         pm = max_over_lane_groups(pm);
         const bool moved = pm > m_run + kSlack;  // m_run = -inf at the start: any finite maximum moves it
