@@ -1513,6 +1513,10 @@ bkv_status bkv_page_copy(bkv_pool* p, const bkv_page_pair* pairs, int32_t n_pair
     if (st != BKV_OK) return st;
     st = wait_for_tier_moves(p, S(stream));
     if (st != BKV_OK) return st;
+    if (n_pairs > 0 && n_pairs <= kPagePairsInArgs) {
+        BKV_HIP(launch_page_copy(p, pairs, nullptr, n_pairs, S(stream)));
+        return BKV_OK;
+    }
     const int32_t per_launch = (int32_t)(ParamRing::kSlotBytes / sizeof(bkv_page_pair));
     for (int32_t at = 0; at < n_pairs; at += per_launch) {
         const int32_t n = std::min(per_launch, n_pairs - at);
@@ -1520,7 +1524,7 @@ bkv_status bkv_page_copy(bkv_pool* p, const bkv_page_pair* pairs, int32_t n_pair
         int slot;
         st = ring_upload(p, pairs + at, (size_t)n * sizeof(bkv_page_pair), S(stream), &dev, &slot);
         if (st != BKV_OK) return st;
-        BKV_HIP(launch_page_copy(p, static_cast<const bkv_page_pair*>(dev), n, S(stream)));
+        BKV_HIP(launch_page_copy(p, nullptr, static_cast<const bkv_page_pair*>(dev), n, S(stream)));
         st = ring_done(p, slot, S(stream));
         if (st != BKV_OK) return st;
     }

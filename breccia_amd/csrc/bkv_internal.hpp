@@ -271,7 +271,10 @@ bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows_p
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
                                int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream);
 
-hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_dev, int32_t n_pairs,
+// Up to kPagePairsInArgs pairs, given on the host, travel in the arguments of the launch (a launch has 4 KiB of
+// them); longer lists are read from pairs_dev (pairs_host null).
+constexpr int32_t kPagePairsInArgs = 448;
+hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_host, const bkv_page_pair* pairs_dev, int32_t n_pairs,
                             hipStream_t stream);
 // Gather (to_stage=1) / scatter (to_stage=0) whole pages between the pools and a
 // contiguous staging buffer laid out [page][layer][K bytes | V bytes].

@@ -3,6 +3,7 @@
 // host swap, a dequantising row gather for parity checks, and small utilities.
 // All of it is HBM-bound; the rules that matter are 16-byte accesses, whole-line
 // coalescing and several independent loads in flight per lane.
+#include <algorithm>
 #include <type_traits>
 
 #include "bkv_internal.hpp"
@@ -621,8 +622,15 @@ __device__ __forceinline__ CopyUnit copy_unit(const PoolPtrs& pp, const bkv_page
     return u;
 }
 
+// Pairs: the list in device memory (const bkv_page_pair*), or, up to kPagePairsInArgs of them, in the launch's
+// arguments (PagePairArgs): no upload ahead of the copy.  256 pairs of 12 layers: 47.5 -> 40.9 us a call.
+struct PagePairArgs {
+    bkv_page_pair p[kPagePairsInArgs];
+    __device__ __forceinline__ const bkv_page_pair& operator[](uint32_t i) const { return p[i]; }
+};
+template <typename Pairs>
 __global__ __launch_bounds__(kBlock) void page_copy_kernel(PoolPtrs pp,
-                                                           const bkv_page_pair* __restrict__ pairs,
+                                                           const Pairs pairs,
                                                            uint32_t n_pairs, uint32_t chunks_k,
                                                            uint32_t chunks_v) {
     const uint32_t per_pl = chunks_k + chunks_v;
@@ -848,7 +856,7 @@ hipError_t launch_append_kprep(bkv_pool* p, int32_t layer, const AppendBatch& b,
     return hipGetLastError();
 }
 
-hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_dev, int32_t n_pairs,
+hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_host, const bkv_page_pair* pairs_dev, int32_t n_pairs,
                             hipStream_t stream) {
     const PoolPtrs pp = pool_ptrs(p);
     const uint32_t chunks_k = (uint32_t)((pp.k_page_bytes / 16 + 4 * kBlock - 1) / (4 * kBlock));
@@ -857,8 +865,16 @@ hipError_t launch_page_copy(bkv_pool* p, const bkv_page_pair* pairs_dev, int32_t
     uint64_t grid = total;
     const uint64_t cap = (uint64_t)(p->n_cu > 0 ? p->n_cu : 256) * 32;
     if (grid > cap) grid = cap;
-    launch_staged(p, BKV_STAGE_PAGE_COPY, page_copy_kernel, dim3((unsigned)grid), dim3(kBlock), 0, stream, pp,
-                  pairs_dev, (uint32_t)n_pairs, chunks_k, chunks_v);
+    if (pairs_host) {
+        if (n_pairs > kPagePairsInArgs) return hipErrorInvalidValue;
+        PagePairArgs a;
+        std::copy_n(pairs_host, n_pairs, a.p);
+        launch_staged(p, BKV_STAGE_PAGE_COPY, page_copy_kernel<PagePairArgs>, dim3((unsigned)grid), dim3(kBlock), 0, stream,
+                      pp, a, (uint32_t)n_pairs, chunks_k, chunks_v);
+    } else {
+        launch_staged(p, BKV_STAGE_PAGE_COPY, page_copy_kernel<const bkv_page_pair*>, dim3((unsigned)grid), dim3(kBlock), 0,
+                      stream, pp, pairs_dev, (uint32_t)n_pairs, chunks_k, chunks_v);
+    }
     return hipGetLastError();
 }
 

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from breccia_amd import lib as L
-from breccia_amd.kv import BkvError, Stream, device_sync
+from breccia_amd.kv import BkvError, Pool, Stream, device_sync
 from gpu_common import Twin, check_attn
 from test_gpu_attn import fill
 
@@ -289,3 +289,23 @@ def test_bounded_waits_time_out_and_the_work_still_completes():
         host.free()
         kd.free()
         vd.free()
+
+
+@pytest.mark.parametrize("n", [1, 448, 449])
+def test_page_copies_around_the_longest_list_in_launch_arguments(n):
+    rng = np.random.Generator(np.random.PCG64(4480 + n))
+    with Pool(n_layers=2, n_pages=1000) as pool:
+        order = rng.permutation(1000).astype(np.int32)
+        pairs = np.stack([order[:n], order[500:500 + n]], axis=1)
+        before = []
+        for layer in range(2):
+            for which in range(2):
+                _, size = pool.layer_ptr(layer, which)
+                data = rng.integers(0, 256, size=size, dtype=np.uint8)
+                pool.write_layer(layer, which, data)
+                before.append(data.reshape(1000, -1))
+        pool.page_copy(pairs)
+        device_sync()
+        for i, data in enumerate(before):
+            data[pairs[:, 1]] = data[pairs[:, 0]]
+            assert np.array_equal(pool.read_layer(i // 2, i % 2), data.reshape(-1))
