@@ -629,7 +629,7 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
 // the references are looked at.
 constexpr int kMergeWaves = 4;
 constexpr int kMergeInFlight = 8;
-__global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(const PrefillSplitParams P, int32_t rows_per_wg) {
+__global__ __launch_bounds__(64 * kMergeWaves, 4) void prefill_merge_kernel(const PrefillSplitParams P, int32_t rows_per_wg) {
     const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kMergeWaves + (int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     int unit = w / rows_per_wg;
@@ -649,12 +649,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(const P
     const size_t at = ((size_t)P.s.slot_base[e] + (size_t)unit * P.s.splits[e]) * rows_per_wg + r;
     const float* po = P.part_o + at * kHd + 4 * lane;
     const size_t step = (size_t)rows_per_wg * kHd;
+    // (past the last range its row is read again and dropped: a load behind a branch is waited for there)
+    const auto part_row = [&](int i) { return *reinterpret_cast<const f4*>(po + min(i, ranges - 1) * step); };
     f4 v[kMergeInFlight];
 #pragma unroll
-    for (int u = 0; u < kMergeInFlight; ++u)
-        if (u < ranges) v[u] = *reinterpret_cast<const f4*>(po + u * step);
-    float2 ml = make_float2(-INFINITY, 0.0f);
-    if (lane < ranges) ml = *reinterpret_cast<const float2*>(P.part_ml + (at + (size_t)lane * rows_per_wg) * 2);
+    for (int u = 0; u < kMergeInFlight; ++u) v[u] = part_row(u);
+    float2 ml = *reinterpret_cast<const float2*>(P.part_ml + (at + (size_t)min(lane, ranges - 1) * rows_per_wg) * 2);
+    if (lane >= ranges) ml = make_float2(-INFINITY, 0.0f);
     const int tok = row / P.group, head = kvh * P.group + row % P.group;
     const size_t out_row = (size_t)(P.b.src0[e] + tok);
     float4 gt = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -671,15 +672,14 @@ __global__ __launch_bounds__(64 * kMergeWaves) void prefill_merge_kernel(const P
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
     f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < ranges; s += kMergeInFlight) {
-        if (s > 0) {
-#pragma unroll
-            for (int u = 0; u < kMergeInFlight; ++u)
-                if (s + u < ranges) v[u] = *reinterpret_cast<const f4*>(po + (s + u) * step);
-        }
+    for (int s = 0;;) {
 #pragma unroll
         for (int u = 0; u < kMergeInFlight; ++u)
             if (s + u < ranges) acc += v[u] * __shfl(wt, s + u, 64);
+        s += kMergeInFlight;
+        if (s >= ranges) break;
+#pragma unroll
+        for (int u = 0; u < kMergeInFlight; ++u) v[u] = part_row(s + u);
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     float4 y = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
