@@ -256,7 +256,7 @@ struct PrefillBatch {
 };
 // query rows one work-group owns, given how many 64-row work-groups the call's chunks would make
 int32_t prefill_rows_per_wg(int32_t layout, int64_t wgs_of_64_rows, int32_t n_cu);
-// How a call whose row blocks leave most of the chip idle is cut: the page walks of an entry's
+// How a call whose longest page walks would outlast the rest is cut: the walks of an entry's
 // longest blocks (its last ones) in ranges of at most pps pages, a work-group each.
 struct PrefillSplit {
     int32_t pps;                           // even

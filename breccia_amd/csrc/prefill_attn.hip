@@ -175,13 +175,14 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
     if constexpr (SPLIT) {
         while (e + 1 < P.b.n && (int)blockIdx.x >= P.s.wg_base[e + 1]) ++e;
         int rem = (int)blockIdx.x - P.s.wg_base[e];
-        const int in_ranges = P.s.n_cut[e] * P.n_kv * P.s.splits[e];
-        cut = rem < in_ranges;
+        // uncut blocks first: the longest of them are longer than a range
+        const int blocks = (P.b.n_tok[e] * P.group + kRowsPerWg - 1) / kRowsPerWg;
+        const int uncut = (blocks - P.s.n_cut[e]) * P.n_kv;
+        cut = rem >= uncut;
         if (cut) {
+            rem -= uncut;
             range = rem % P.s.splits[e];
             rem /= P.s.splits[e];
-        } else {
-            rem -= in_ranges;
         }
         kvh = rem % P.n_kv;
         idx = rem / P.n_kv + (cut ? 0 : P.s.n_cut[e]);
@@ -715,19 +716,24 @@ int32_t prefill_rows_per_wg(int32_t layout, int64_t wgs_of_64_rows, int32_t n_cu
 // has nothing else (2.3-3.6 us on the quantised ones), and a call of a few blocks is as long as its longest
 // chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups, 34 us).  Cutting
 // pays for a second kernel (4-9 us, by the partial rows it reads), so:
-// - only calls that leave half of the compute units idle are cut (the merge's traffic grows with the rows);
-// - a range has at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several;
-// - the chain has to lose 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured
-//   31.1 us uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
-// - one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer than
-//   8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8.
-// Before / after, us a layer: 41 tokens behind 517 cells 37 / 24.6, 100 behind 8000 374 / 57, 200 behind
-// 3000 with q8_0 V 262 / 64, 300 behind 1000 on an int8 pool 125 / 55.
+// - a call that leaves half of the compute units idle is cut if
+//   - a range keeps at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several, and
+//   - the chain loses 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured 31.1 us
+//     uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
+//   - into one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer
+//     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8;
+// - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) if its
+//   longest walk is over 1.7 times what an even share of the pairs would be -- cut calls measured 1.45 to
+//   1.75 of that: 900 tokens behind 3000 and 900 from scratch (int8) 383 -> 243 us, 2048 from scratch
+//   201 -> 176, 1500 with 24 heads behind 500 (1.47) 205 and 206.
+// Before / after, us a layer: 41 tokens behind 517 cells 37 / 24, 100 behind 8000 374 / 55, 200 behind
+// 3000 with q8_0 V 262 / 59, 300 behind 1000 on an int8 pool 125 / 48.
 bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s) {
     const int32_t n_kv = p->g.n_kv;
     const int n_cu = p->n_cu > 0 ? p->n_cu : 256;
-    if ((int64_t)b.wg_base[b.n] * 2 > n_cu) return false;
     const bool f16 = p->g.layout == BKV_LAYOUT_F16;
+    const bool idle = (int64_t)b.wg_base[b.n] * 2 <= n_cu;
+    if (!idle && (f16 || b.wg_base[b.n] > 2 * n_cu)) return false;
     const int64_t least = f16 ? 3 : 2, gain = f16 ? 10 : 5;
     const int64_t room = (int64_t)p->max_wgs * 8 / rows;  // partial results the workspace holds
     int64_t work = 0;
@@ -745,6 +751,7 @@ bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows, 
     int64_t most = std::min<int64_t>(room, n_cu);
     if (f16 && work > 8 * most) most = std::min<int64_t>(room, 2 * n_cu);
     int64_t each = std::max<int64_t>({least, (work + most - 1) / most, (longest + 63) / 64});
+    if (!idle && 10 * (int64_t)longest * n_cu < 17 * work) return false;
     for (;; each += std::max<int64_t>(1, each / 8)) {
         if (longest < each + gain) return false;
         int64_t wgs = 0, units = 0, slots = 0;
@@ -764,7 +771,7 @@ bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows, 
         }
         s.unit_base[b.n] = (int32_t)units;
         s.wg_base[b.n] = (int32_t)wgs;
-        if (wgs <= most) break;
+        if (idle ? wgs <= most : slots <= room) break;
     }
     s.pps = (int32_t)each * 2;
     return true;

@@ -49,6 +49,28 @@ def test_cut_chunks_match_the_oracle(n_q, cases, layout):
                 assert rel <= REF_BAR_MAX_REL, (before, i, rel)
 
 
+@pytest.mark.parametrize("layout", [L.LAYOUT_Q8V, L.LAYOUT_I8H])
+def test_an_unbalanced_call_that_fills_the_chip(layout):
+    # 150 and 100 work-groups' worth of rows, walks of 60 to 68 and of 1 to 13 pairs of pages: the long ones are cut
+    rng = np.random.Generator(np.random.PCG64(79))
+    cases = [(0, 400), (1900, 600)]
+    with Twin(n_pages=400, n_kv=2, max_seqs=4, layout=layout) as tw:
+        tw.pool.set_free_order(rng.permutation(400).astype(np.int32))
+        seqs = [tw.pool.seq_create() for _ in cases]
+        for s, (before, t) in zip(seqs, cases):
+            fill(tw, s, before + t, rng, chunk=1024)
+        qs = [rng.standard_normal((t, 32, 256)).astype(np.float32) for _, t in cases]
+        tw.pool.timing_enable(True)
+        outs = prefill(tw, 0, seqs, [b for b, _ in cases], qs, 32)
+        device_sync()
+        tw.pool.timing_enable(False)
+        assert tw.pool.timing_read(L.STAGE_ATTN_MERGE)[0] == 1, "the call was meant to be cut"
+        for s, (before, t), q, out in zip(seqs, cases, qs, outs):
+            for i in (0, 7, 199, t // 2 + 3, t - 1):
+                _, rel = check_attn(out[i], tw.oracle_attend(0, s, before + i, q[i], 32), "chunk at %d, token %d" % (before, i))
+                assert rel <= REF_BAR_MAX_REL, (before, i, rel)
+
+
 def test_a_captured_chunk_replays():
     # a captured call stays uncut (its replays leave the pool's workspace to the calls beside them)
     rng = np.random.Generator(np.random.PCG64(78))
