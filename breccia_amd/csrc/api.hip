@@ -157,6 +157,15 @@ static bkv_status order_workspace(WorkspaceOrder& w, hipStream_t stream) {
     return BKV_OK;
 }
 
+// Whether an event recorded on the stream now would belong to a capture (or break one: the null stream beside
+// a capture of a stream that synchronises with it).
+static bool being_captured(hipStream_t stream) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const hipError_t err = hipStreamIsCapturing(stream, &cs);
+    if (err != hipSuccess) (void)hipGetLastError();
+    return err == hipErrorStreamCaptureImplicit || (err == hipSuccess && cs != hipStreamCaptureStatusNone);
+}
+
 // Block-table updates are scattered on whichever stream brings the next call.  A call on another
 // stream reads the same table: it waits for the last scatter (until that is known to be over).
 // `may_query` false: only the wait is enqueued, no host-side look at the event (for streams that
@@ -284,11 +293,14 @@ static void destroy_device_side(bkv_pool* p) {
     if (p->tiers.done) (void)hipEventDestroy(p->tiers.done);
     if (p->attn_ws.ev) (void)hipEventDestroy(p->attn_ws.ev);
     if (p->sel_ws.ev) (void)hipEventDestroy(p->sel_ws.ev);
+    if (p->chunk_ws.ev) (void)hipEventDestroy(p->chunk_ws.ev);
     if (p->table_sync.ev) (void)hipEventDestroy(p->table_sync.ev);
     if (p->slab) (void)hipFree(p->slab);
     if (p->table_dev) (void)hipFree(p->table_dev);
     if (p->part_o) (void)hipFree(p->part_o);
     if (p->part_ml) (void)hipFree(p->part_ml);
+    if (p->chunk_o) (void)hipFree(p->chunk_o);
+    if (p->chunk_ml) (void)hipFree(p->chunk_ml);
     if (p->sel_scores) (void)hipFree(p->sel_scores);
     if (p->ring.host) (void)hipHostFree(p->ring.host);
     if (p->ring.dev) (void)hipFree(p->ring.dev);
@@ -411,6 +423,8 @@ bkv_status bkv_pool_create(const bkv_pool_desc* d, bkv_pool** out) {
 
     BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->part_o), (uint64_t)p->max_wgs * 8u * 256u * 4u));
     BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->part_ml), (uint64_t)p->max_wgs * 8u * 2u * 4u));
+    BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->chunk_o), (uint64_t)p->max_wgs * 8u * 256u * 4u));
+    BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->chunk_ml), (uint64_t)p->max_wgs * 8u * 2u * 4u));
 
     BKV_TRY(hipHostMalloc(reinterpret_cast<void**>(&p->ring.host),
                           ParamRing::kSlots * ParamRing::kSlotBytes, hipHostMallocDefault));
@@ -431,6 +445,7 @@ bkv_status bkv_pool_create(const bkv_pool_desc* d, bkv_pool** out) {
     // created here rather than on first use: the calls that order work with them create nothing
     BKV_TRY(hipEventCreateWithFlags(&p->attn_ws.ev, hipEventDisableTiming));
     BKV_TRY(hipEventCreateWithFlags(&p->sel_ws.ev, hipEventDisableTiming));
+    BKV_TRY(hipEventCreateWithFlags(&p->chunk_ws.ev, hipEventDisableTiming));
     BKV_TRY(hipEventCreateWithFlags(&p->table_sync.ev, hipEventDisableTiming));
     // this device's copy of the static scratch of bkv_decode_attn_static
     BKV_TRY(attn_static_scratch_init(p->device));
@@ -1364,14 +1379,12 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
     a.out = out_dev;
     PrefillSplit split;
     bool cut = plan_prefill_split(p, b, (int32_t)rows_per_wg, (int32_t)group, split);
-    if (cut && stream) {
-        // a captured call stays uncut: its replays would share the workspace with whatever runs beside them
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        cut = hipStreamIsCapturing(S(stream), &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
-        if (!cut) (void)hipGetLastError();
-    }
+    // A captured call stays uncut: its replays would share the workspace with whatever runs beside them.  So
+    // does one that would be ordered behind a stream that is being captured now.
+    if (cut && stream) cut = !being_captured(S(stream));
+    if (cut && p->chunk_ws.used && p->chunk_ws.last != S(stream)) cut = !being_captured(p->chunk_ws.last);
     if (cut) {
-        st = order_workspace(p->attn_ws, S(stream));
+        st = order_workspace(p->chunk_ws, S(stream));
         if (st != BKV_OK) return st;
     }
     BKV_HIP(launch_prefill_attn(p, layer, b, a, (int32_t)rows_per_wg, cut ? &split : nullptr, S(stream)));

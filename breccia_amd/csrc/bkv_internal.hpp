@@ -114,14 +114,18 @@ struct bkv_pool {
     float* part_o = nullptr;
     float* part_ml = nullptr;
     int32_t max_wgs = 0;
+    // the same for cut chunk calls, as large.  Apart from the decode calls' one: those may be captured, and
+    // must not have to be ordered behind a chunk on a stream outside the capture.
+    float* chunk_o = nullptr;
+    float* chunk_ml = nullptr;
     int32_t live_plans = 0;  // step plans made from this pool and not yet destroyed
     // block selection: f64 indexer scores [entry][block], grown on demand
     double* sel_scores = nullptr;
     uint64_t sel_scores_cap = 0;  // doubles
 
-    // Streams that used the split-K workspace and the score workspace last: a call on another
+    // Streams that used the split-K workspaces and the score workspace last: a call on another
     // stream is ordered behind them first (the workspaces are one per pool).
-    bkv::WorkspaceOrder attn_ws, sel_ws;
+    bkv::WorkspaceOrder attn_ws, sel_ws, chunk_ws;
     // the stream of the last block-table scatter, and the event behind it
     bkv::WorkspaceOrder table_sync;
 
@@ -266,7 +270,7 @@ struct PrefillSplit {
     int32_t unit_base[BKV_MAX_BATCH + 1];  // their cut (row block, kv head) units; [n] = total
     int32_t slot_base[BKV_MAX_BATCH];      // their partial results, in row blocks
 };
-// False where the call is better off uncut.  A cut call uses the pool's split-K workspace.
+// False where the call is better off uncut.  A cut call uses the pool's workspace for chunks.
 bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows_per_wg, int32_t group, PrefillSplit& s);
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
                                int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream);

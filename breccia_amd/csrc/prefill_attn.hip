@@ -800,8 +800,8 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
     if (split) {
         kp.by_xcd = 0;
         sp.s = *split;
-        sp.part_o = p->part_o;
-        sp.part_ml = p->part_ml;
+        sp.part_o = p->chunk_o;
+        sp.part_ml = p->chunk_ml;
         if (p->g.layout == BKV_LAYOUT_Q8V) return launch_split<BKV_LAYOUT_Q8V, 8>(p, sp, stream);
         if (p->g.layout == BKV_LAYOUT_I8H) return launch_split<BKV_LAYOUT_I8H, 8>(p, sp, stream);
         return launch_split<BKV_LAYOUT_F16, 4>(p, sp, stream);

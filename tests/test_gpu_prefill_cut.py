@@ -97,3 +97,43 @@ def test_a_captured_chunk_replays():
         stream.close()
         qd.free()
         od.free()
+
+
+def test_a_cut_chunk_leaves_captures_on_other_streams_alone():
+    # a chunk before the capture of a decode call and one during it, on streams outside the capture
+    rng = np.random.Generator(np.random.PCG64(80))
+    with Twin(n_pages=100, max_seqs=2) as tw:
+        s = tw.pool.seq_create()
+        fill(tw, s, 600, rng, chunk=600)
+        q = rng.standard_normal((30, 16, 256)).astype(np.float32)
+        qd, od = DeviceBuffer.from_numpy(q), DeviceBuffer(q.nbytes)
+        last, cd = DeviceBuffer.from_numpy(q[29]), DeviceBuffer(q[29].nbytes)
+        one, two = Stream(), Stream()
+        device_sync()
+        tw.pool.prefill_attn(0, [s], [570], [30], 16, qd, od, 1.0 / 16.0, stream=one)
+        one.sync()
+        want = od.download(np.float32)
+        graph = Graph(two)
+        tw.pool.decode_attn(0, [s], [599], 16, last, cd, 1.0 / 16.0, stream=two)
+        graph.end()
+        graph_again = Graph(one)  # the stream of the chunk is captured now
+        tw.pool.prefill_attn(0, [s], [570], [30], 16, qd, od, 1.0 / 16.0, stream=one)
+        tw.pool.prefill_attn(0, [s], [570], [30], 16, qd, od, 1.0 / 16.0, stream=two)
+        graph_again.end()
+        two.sync()
+        got = od.download(np.float32)
+        check_attn(got.reshape(q.shape)[29], tw.oracle_attend(0, s, 599, q[29], 16), "chunk beside a capture")
+        for _ in range(3):
+            cd.upload(np.zeros(q[29].shape, np.float32))
+            tw.pool.prefill_attn(0, [s], [570], [30], 16, qd, od, 1.0 / 16.0, stream=one)
+            one.sync()
+            assert np.array_equal(od.download(np.float32), want)
+            graph.launch(two)
+            two.sync()
+            check_attn(cd.download(np.float32).reshape(16, 256), tw.oracle_attend(0, s, 599, q[29], 16), "replayed decode")
+        graph_again.destroy()
+        graph.destroy()
+        for x in (one, two):
+            x.close()
+        for x in (qd, od, last, cd):
+            x.free()
