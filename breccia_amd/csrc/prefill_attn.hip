@@ -36,9 +36,10 @@
 // all eight, on its way into LDS, into two f16 images whose sum is the value to 22 bits
 //   E[cell]    = exponent of the largest of the cell's 8 block scales (clamped to +-120),
 //   a[cell][d] = code * (scale * 2^-E[cell]) = hi + lo,
-// and the softmax runs over logit + E with weights exp2(logit + E - M) (the denominator sums
-// exp2(logit - M)), as in the decode kernel for this layout: the largest terms have weights near
-// 1 whatever the magnitude of their values.  P.V is then hi.p_hi + hi.p_lo + lo.p_hi.
+// and the softmax runs over logit + E with weights exp2(logit + E - M), as in the decode kernel for
+// this layout: the largest terms have weights near 1 whatever the magnitude of their values.  P.V is
+// then hi.p_hi + hi.p_lo + lo.p_hi.  The denominator sums exp2(logit - R), a second exponential of its
+// own: R is M until a sum comes near the end of f32's range, which rows of tiny V (E near -120) lead to.
 // Int8 pools (codes with an f16 scale per 32 values, K and V alike) are dequantised the same way,
 // without the exponent: both K and V become hi/lo image pairs, and the scores are
 // K_hi.q_hi + K_hi.q_lo + K_lo.q_hi.
@@ -306,6 +307,13 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
     for (int t = 0; t < 16; ++t) o[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     float m_run = -INFINITY;  // running max of this lane's query (base-2 logits), same in all 4 g lanes
     float l_run = 0.0f;       // this lane's share (its 4 cells per page) of the denominator
+    // q8_0 V: what l_run is relative to.  Against M its terms reach 2^(120 + kSlack) on rows of tiny V
+    // (E = -120), and a few of them overflow f32; so the denominator has a reference of its own, at or
+    // above M.  It leaves M when a lane's sum passes kMostL, and M meets it again from below.  Checked beside
+    // the branch that rescales the accumulators: the 4096-token prompt of the q8_0 V cache went from 640.8
+    // to 642.9 us with it (649 with a branch of its own).
+    float l_ref = -INFINITY;
+    constexpr float kMostL = 0x1p100f;
 
     // ---- pages through LDS -----------------------------------------------------------------------
     // Rows are padded to 528 bytes so that the 16-byte fragment reads of the 64 lanes spread
@@ -515,19 +523,15 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
         // a range may hold no live cell for a row (it begins past the row's position): its reference
         // stays at -inf, and the weights of its dead cells are taken against 0
         const float m_at = SPLIT && m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_at);  // 1, or 0 at the start
         float pv[8];
         float psum = 0.0f;
+        const float ref = Q8V ? fmaxf(l_ref, m_new) : m_new;
+        const float ref_at = SPLIT && ref == -INFINITY ? 0.0f : ref;
+        const auto tt = [&](int r) { return r < 4 ? ta[r & 3] : tb[r & 3]; };
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
-            const float ww = r < 4 ? wa[r & 3] : wb[r & 3];
-            pv[r] = __builtin_amdgcn_exp2f(ww - m_at);
-            if constexpr (Q8V) {
-                const float tt = r < 4 ? ta[r & 3] : tb[r & 3];
-                psum += __builtin_amdgcn_exp2f(tt - m_at);
-            } else {
-                psum += pv[r];
-            }
+            pv[r] = __builtin_amdgcn_exp2f((r < 4 ? wa[r & 3] : wb[r & 3]) - m_at);
+            psum += Q8V ? __builtin_amdgcn_exp2f(tt(r) - ref_at) : pv[r];
         }
         // p = hi + lo, both rounded to nearest (the matrix cores read f16 subnormals as the numbers
         // they are, so small weights keep their low parts' few bits)
@@ -539,12 +543,33 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
             ph[r] = hi;
             pl[r] = lo;
         }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+        float l_new = l_run + psum;
+        const bool high = Q8V && l_new > kMostL;
+        if (__builtin_amdgcn_ballot_w64(moved || high) != 0) {
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_at);  // 1, or 0 at the start
 #pragma unroll
             for (int t = 0; t < 16; ++t) o[t] *= alpha;
+            if constexpr (Q8V) {
+                l_new = l_run * __builtin_amdgcn_exp2f(l_ref - ref_at) + psum;
+                const float l_was = l_ref;
+                l_ref = ref;
+                if (l_new > kMostL) {
+                    // up to the pair's largest logit (its terms are then 1 at most), and by 2^64 at least
+                    float up = ref_at + 64.0f;
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) up = fmaxf(up, tt(r));
+                    l_new = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) l_new += __builtin_amdgcn_exp2f(tt(r) - up);
+                    l_new += l_run * __builtin_amdgcn_exp2f(l_was - up);
+                    l_ref = up;
+                }
+            } else {
+                l_new = l_run * alpha + psum;
+            }
         }
+        l_run = l_new;
+        m_run = m_new;
 
         // ---- O^T += V^T . P^T over the 32 cells of the pair ----------------------------------------
         // Per tile of 16 output columns one transposing read from either page's image: lane (c, g)
@@ -593,6 +618,18 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
     }
 
     // ---- normalise, gate, store ---------------------------------------------------------------------
+    if constexpr (Q8V) {
+        // the row's four lanes to one reference, the outputs to it too (nearly always M: nothing to do)
+        const float ref = max_over_lane_groups(l_ref);
+        const float ref_at = ref == -INFINITY ? 0.0f : ref;
+        l_run *= __builtin_amdgcn_exp2f(l_ref - ref_at);
+        if (__builtin_amdgcn_ballot_w64(m_run != ref) != 0) {
+            const float down = __builtin_amdgcn_exp2f(m_run - ref_at);
+#pragma unroll
+            for (int t = 0; t < 16; ++t) o[t] *= down;
+        }
+        m_run = ref;
+    }
     l_run = sum_over_lane_groups(l_run);
     if (!row_live) return;
     if constexpr (SPLIT) {

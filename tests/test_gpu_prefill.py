@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from breccia_amd import lib as L
-from breccia_amd.kv import BkvError, DeviceBuffer
+from breccia_amd.kv import BkvError, DeviceBuffer, device_sync
 from gpu_common import REF_BAR_MAX_REL, Twin, check_attn
 from helpers import max_abs
 from test_gpu_attn import fill
@@ -97,6 +97,43 @@ def test_quantised_chunks_across_the_scale_range(v_mag, layout):
         for i in (0, 10, 29):
             want = tw.oracle_attend(0, s, 35 + i, q2[i], 16)
             rel = max_abs(out2[i], want) / float(np.max(np.abs(want)))
+            assert rel <= REF_BAR_MAX_REL, (i, rel)
+
+
+@pytest.mark.parametrize("rise", [0.0, 4.1])
+@pytest.mark.parametrize("n_q, before, tokens, tiny, cut", [
+    (16, 0, 130, 64, 0),        # the first tokens see tiny rows only
+    (16, 70, 60, 64, 0),
+    (16, 600, 41, 64, 1),       # the tiny rows in the first range
+    (16, 3000, 41, 1300, 1),    # in several ranges, some of which hold nothing else
+    (64, 1400, 1100, 1300, 0),  # more than 1024 of them in one walk
+])
+def test_rows_of_tiny_values_leave_the_denominator_finite(n_q, before, tokens, tiny, cut, rise):
+    # q8_0 V: rows whose block scales lie at 2^-125 are weighed at exp2(logit - 120), and the softmax reference is
+    # theirs as long as no larger row follows: the denominator's terms exp2(logit - reference) are then 2^120, and up
+    # to 2^126 where the logits rise by the 6 bits the reference may lag behind (4.1 nats).  A handful of such
+    # terms is past the end of f32's range.
+    rng = np.random.Generator(np.random.PCG64(1022))
+    n = before + tokens
+    with Twin(n_pages=n // 16 + 8, max_seqs=2, layout=L.LAYOUT_Q8V) as tw:
+        s = tw.pool.seq_create()
+        tw.pool.seq_reserve(s, n)
+        k = (0.05 * rng.standard_normal((n, 2, 256))).astype(np.float32)
+        k[:, :, 0] = 0.0
+        k[tiny // 2:tiny, :, 0] = rise
+        v = rng.standard_normal((n, 2, 256)).astype(np.float32)
+        v[:tiny] *= np.float32(3e-36)
+        tw.append(0, [s], [0], [k], [v])
+        q = (0.3 * rng.standard_normal((tokens, n_q, 256))).astype(np.float32)
+        q[:, :, 0] = 16.0
+        tw.pool.timing_enable(True)
+        out = prefill(tw, 0, [s], [before], [q], n_q)[0]
+        device_sync()
+        tw.pool.timing_enable(False)
+        assert tw.pool.timing_read(L.STAGE_ATTN_MERGE)[0] == cut
+        for i in sorted({0, 7, 40, tokens // 2, 63 + tokens // 3, tokens - 1} & set(range(tokens))):
+            want = tw.oracle_attend(0, s, before + i, q[i], n_q)
+            rel = max_abs(out[i], want) / float(np.max(np.abs(want)))
             assert rel <= REF_BAR_MAX_REL, (i, rel)
 
 
