@@ -82,6 +82,18 @@ struct WorkspaceOrder {
     hipEvent_t ev = nullptr;
 };
 
+// Partial results of one cut chunk call at a time.
+struct ChunkWorkspace {
+    float* o = nullptr;   // null: not allocated
+    float* ml = nullptr;
+    bool tried = false;   // to allocate it
+    hipStream_t last = nullptr;  // the stream of the last call
+    uint64_t turn = 0;           // its number among the pool's cut calls, 0 = none yet
+    hipEvent_t done = nullptr;
+    bool recorded = false;  // `done` lies behind the last call: one from another stream can be ordered behind it,
+                            // whatever became of that stream since
+};
+
 // Where the prefix tree's lower tiers keep their pages: a pinned-host arena of slots and a file,
 // slot = one page's bytes of every layer ([layer][K page | V page]).
 struct TierStore {
@@ -115,17 +127,21 @@ struct bkv_pool {
     float* part_ml = nullptr;
     int32_t max_wgs = 0;
     // the same for cut chunk calls, as large.  Apart from the decode calls' one: those may be captured, and
-    // must not have to be ordered behind a chunk on a stream outside the capture.
-    float* chunk_o = nullptr;
-    float* chunk_ml = nullptr;
+    // must not have to be ordered behind a chunk on a stream outside the capture.  Up to four streams have one
+    // each, so that their chunks run side by side as uncut ones do (HIP's default is four hardware queues; more
+    // streams share those); the first is allocated with the pool, the others when a further stream first cuts.
+    static constexpr int kChunkWorkspaces = 4;
+    bkv::ChunkWorkspace chunk_ws[kChunkWorkspaces];
+    uint64_t chunk_turn = 0;
+    bool chunk_many = false;  // cut calls have come from more than one stream
     int32_t live_plans = 0;  // step plans made from this pool and not yet destroyed
     // block selection: f64 indexer scores [entry][block], grown on demand
     double* sel_scores = nullptr;
     uint64_t sel_scores_cap = 0;  // doubles
 
-    // Streams that used the split-K workspaces and the score workspace last: a call on another
+    // Streams that used the split-K workspace and the score workspace last: a call on another
     // stream is ordered behind them first (the workspaces are one per pool).
-    bkv::WorkspaceOrder attn_ws, sel_ws, chunk_ws;
+    bkv::WorkspaceOrder attn_ws, sel_ws;
     // the stream of the last block-table scatter, and the event behind it
     bkv::WorkspaceOrder table_sync;
 
@@ -270,10 +286,11 @@ struct PrefillSplit {
     int32_t unit_base[BKV_MAX_BATCH + 1];  // their cut (row block, kv head) units; [n] = total
     int32_t slot_base[BKV_MAX_BATCH];      // their partial results, in row blocks
 };
-// False where the call is better off uncut.  A cut call uses the pool's workspace for chunks.
+// False where the call is better off uncut.
 bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows_per_wg, int32_t group, PrefillSplit& s);
+// split: null for an uncut call; a cut one leaves its partial results in ws
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
-                               int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream);
+                               int32_t rows_per_wg, const PrefillSplit* split, const ChunkWorkspace* ws, hipStream_t stream);
 
 // Up to kPagePairsInArgs pairs, given on the host, travel in the arguments of the launch (a launch has 4 KiB of
 // them); longer lists are read from pairs_dev (pairs_host null).

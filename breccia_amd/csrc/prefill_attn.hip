@@ -815,7 +815,7 @@ bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows, 
 }
 
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
-                               int32_t rows_per_wg, const PrefillSplit* split, hipStream_t stream) {
+                               int32_t rows_per_wg, const PrefillSplit* split, const ChunkWorkspace* ws, hipStream_t stream) {
     PrefillSplitParams sp;
     PrefillKernelParams& kp = sp;
     kp.b = b;
@@ -837,8 +837,8 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
     if (split) {
         kp.by_xcd = 0;
         sp.s = *split;
-        sp.part_o = p->chunk_o;
-        sp.part_ml = p->chunk_ml;
+        sp.part_o = ws->o;
+        sp.part_ml = ws->ml;
         if (p->g.layout == BKV_LAYOUT_Q8V) return launch_split<BKV_LAYOUT_Q8V, 8>(p, sp, stream);
         if (p->g.layout == BKV_LAYOUT_I8H) return launch_split<BKV_LAYOUT_I8H, 8>(p, sp, stream);
         return launch_split<BKV_LAYOUT_F16, 4>(p, sp, stream);

@@ -17,9 +17,11 @@
  * a Rust wrapper is Send and not Sync).  Different pools may be used from different threads;
  * bkv_last_error and the wait options are the only process-wide state.  What the pool owns and every call shares --
  * the argument ring, the block tables, the split-K and score workspaces, the swap
- * staging -- it orders across streams by itself with events; the order between the
- * caller's own data (an append before the attention that reads its rows, on another
- * stream) is the caller's to keep, as with any work on streams.
+ * staging -- it orders across streams by itself with events, recorded where a call arrives
+ * on another stream than the one before: a stream that decode attention or block selection
+ * was given stays alive until the pool has had such a call on another stream or is
+ * destroyed.  The order between the caller's own data (an append before the attention that
+ * reads its rows, on another stream) is the caller's to keep, as with any work on streams.
  *
  * Reference items each group replaces are cited per declaration; paths are
  * relative to the reference tree, `qsa/` = crates/breccia-kernels/src/qsa/.
@@ -327,7 +329,17 @@ bkv_status bkv_decode_attn_static(bkv_pool *pool, int32_t layer, int32_t n, cons
  * qsa_attn_apply_gqa.comp:53-77) are dequantised once per work-group into two f16 terms whose
  * sum carries code * scale to 22 bits, and so are int8 K blocks.  All three layouts, head_dim
  * 256, 16-cell pages.  Written
- * for chunks of tens to thousands of tokens; a handful of tokens is bkv_decode_attn's case. */
+ * for chunks of tens to thousands of tokens; a handful of tokens is bkv_decode_attn's case.
+ * A call whose longest page walks would outlast the rest of it (few rows, or very unequal
+ * contexts on the quantised layouts) has them cut into ranges: two kernels, with partial results
+ * in a workspace of the pool.  The pool keeps up to four of these (33.8 MB each on 256 compute
+ * units; the first comes with the pool, the others when a further stream brings such a call), so
+ * that the calls of four streams run side by side; calls of more streams share them and are
+ * ordered behind each other by events.  A stream may be destroyed once its work is over.  A call on a
+ * stream that is being captured is never cut, nor is one for which there is no memory.
+ * Which way a call takes follows from its chunks' sizes and places (and, f16 layout, decides
+ * with them how many rows a work-group has): the same chunk alone, in other company or captured
+ * may differ in its last bits; the same call on the same path has the same bits every time. */
 bkv_status bkv_prefill_attn(bkv_pool *pool, int32_t layer, int32_t n_seqs, const int32_t *seqs,
                             const int64_t *pos0, const int32_t *n_tokens, int32_t n_q_head,
                             const float *q_dev, const float *gate_dev, int64_t gate_tok_stride,

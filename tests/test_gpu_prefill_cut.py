@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from breccia_amd import lib as L
-from breccia_amd.kv import DeviceBuffer, Graph, Stream, device_sync
+from breccia_amd.kv import BkvError, DeviceBuffer, Graph, Stream, device_sync
 from gpu_common import REF_BAR_MAX_REL, Twin, check_attn
 from test_gpu_attn import fill
 from test_gpu_prefill import prefill
@@ -51,7 +51,7 @@ def test_cut_chunks_match_the_oracle(n_q, cases, layout):
 
 @pytest.mark.parametrize("layout", [L.LAYOUT_Q8V, L.LAYOUT_I8H])
 def test_an_unbalanced_call_that_fills_the_chip(layout):
-    # 150 and 100 work-groups' worth of rows, walks of 60 to 68 and of 1 to 13 pairs of pages: the long ones are cut
+    # 150 and 100 work-groups' worth of rows, walks of 60 to 79 and of 1 to 13 pairs of pages: the long ones are cut
     rng = np.random.Generator(np.random.PCG64(79))
     cases = [(0, 400), (1900, 600)]
     with Twin(n_pages=400, n_kv=2, max_seqs=4, layout=layout) as tw:
@@ -71,32 +71,144 @@ def test_an_unbalanced_call_that_fills_the_chip(layout):
                 assert rel <= REF_BAR_MAX_REL, (before, i, rel)
 
 
-def test_a_captured_chunk_replays():
-    # a captured call stays uncut (its replays leave the pool's workspace to the calls beside them)
+class Chunk:
+    """Query rows of `t` tokens behind `before` cells of sequence s, and room for their outputs, on the device."""
+
+    def __init__(self, tw, s, before, t, rng, n_q=16):
+        self.tw, self.s, self.before, self.t, self.n_q = tw, s, before, t, n_q
+        self.q = rng.standard_normal((t, n_q, 256)).astype(np.float32)
+        self.qd, self.od = DeviceBuffer.from_numpy(self.q), DeviceBuffer(self.q.nbytes)
+        device_sync()
+
+    def run(self, stream=None):
+        self.tw.pool.prefill_attn(0, [self.s], [self.before], [self.t], self.n_q, self.qd, self.od, 1.0 / 16.0, stream=stream)
+
+    def clear(self):
+        self.od.upload(np.zeros(self.q.shape, np.float32))
+
+    def out(self):
+        return self.od.download(np.float32).reshape(self.q.shape)
+
+    def serial(self):
+        """What the call returns with nothing beside it."""
+        device_sync()
+        self.run()
+        device_sync()
+        out = self.out()
+        self.clear()
+        return out
+
+    def free(self):
+        self.qd.free()
+        self.od.free()
+
+
+def test_a_captured_chunk_stays_uncut():
+    # its replays leave the pool's workspaces to the calls beside them: the bits of the uncut call, next to a cut call
+    # on other inputs that runs at the same time
     rng = np.random.Generator(np.random.PCG64(78))
     with Twin(n_pages=100, max_seqs=2) as tw:
         s = tw.pool.seq_create()
         fill(tw, s, 600, rng, chunk=600)
-        q = rng.standard_normal((30, 16, 256)).astype(np.float32)
-        eager = prefill(tw, 0, [s], [570], [q], 16)[0]
-        qd, od = DeviceBuffer.from_numpy(q), DeviceBuffer(q.nbytes)
-        stream = Stream()
-        graph = Graph(stream)
-        tw.pool.prefill_attn(0, [s], [570], [30], 16, qd, od, 1.0 / 16.0, stream=stream)
+        big = tw.pool.seq_create()
+        fill(tw, big, 900, rng, chunk=900)
+        chunk, other = Chunk(tw, s, 570, 30, rng), Chunk(tw, s, 570, 30, rng)
+        # beside a chunk that fills the chip it is uncut (f16 pools), with the same bits whatever the company
+        uncut = prefill(tw, 0, [s, big], [570, 0], [chunk.q, np.zeros((900, 16, 256), np.float32)], 16)[0]
+        assert not np.array_equal(uncut, chunk.serial()), "cut and uncut differ in some last bit"
+        for i in (0, 29):
+            check_attn(uncut[i], tw.oracle_attend(0, s, 570 + i, chunk.q[i], 16), "token %d" % i)
+        cut = other.serial()
+        one, two = Stream(), Stream()
+        other.run(two)
+        graph = Graph(one)
+        chunk.run(one)
         graph.end()
-        for _ in range(3):
-            od.upload(np.zeros(q.shape, np.float32))
-            graph.launch(stream)
-            again = prefill(tw, 0, [s], [570], [q], 16)[0]
-            assert np.array_equal(again, eager)
+        for _ in range(4):
             device_sync()
-            got = od.download(np.float32).reshape(q.shape)
-            for i in (0, 29):
-                check_attn(got[i], tw.oracle_attend(0, s, 570 + i, q[i], 16), "token %d" % i)
+            chunk.clear()
+            other.clear()
+            graph.launch(one)
+            other.run(two)
+            graph.launch(one)
+            device_sync()
+            assert np.array_equal(chunk.out(), uncut)
+            assert np.array_equal(other.out(), cut)
         graph.destroy()
-        stream.close()
-        qd.free()
-        od.free()
+        for x in (one, two):
+            x.close()
+        for x in (chunk, other):
+            x.free()
+
+
+@pytest.mark.parametrize("n_streams", [2, 6])
+@pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_I8H])
+def test_cut_chunks_on_several_streams_at_once(layout, n_streams):
+    # streams with a workspace of their own and, beyond four, streams that share one: nothing waits on the host
+    # between the calls, and every output has the bits of the same call alone
+    rng = np.random.Generator(np.random.PCG64(81))
+    with Twin(n_pages=300, max_seqs=2, layout=layout) as tw:
+        s = tw.pool.seq_create()
+        fill(tw, s, 3100, rng, chunk=1024)
+        streams = [Stream() for _ in range(n_streams)]
+        chunks = [Chunk(tw, s, 3000 - 37 * i, 60 + 7 * i, rng) for i in range(n_streams)]
+        want = [c.serial() for c in chunks]
+        for _ in range(4):
+            for _ in range(3):
+                for c, x in zip(chunks, streams):
+                    c.run(x)
+            device_sync()
+            for i, (c, w) in enumerate(zip(chunks, want)):
+                assert np.array_equal(c.out(), w), i
+                c.clear()
+            device_sync()
+        for x in streams:
+            x.close()
+        for c in chunks:
+            c.free()
+
+
+def test_cut_chunks_after_their_streams_are_gone():
+    # the streams of earlier chunks are destroyed, another has work left and a third is being captured: the next chunk
+    # neither waits on the host nor disturbs the capture
+    rng = np.random.Generator(np.random.PCG64(82))
+    with Twin(n_pages=100, max_seqs=2) as tw:
+        s = tw.pool.seq_create()
+        fill(tw, s, 600, rng, chunk=600)
+        long, busy = Chunk(tw, s, 0, 600, rng, n_q=64), Stream()
+        chunk, captured = Chunk(tw, s, 570, 30, rng), Chunk(tw, s, 500, 40, rng)
+        want = chunk.serial()
+        capturing = Stream()
+        for _ in range(3):
+            fresh, *gone = [Stream() for _ in range(6)]  # first, so that it is none of the destroyed ones' handles
+            for x in gone:
+                chunk.run(x)
+            for x in gone:
+                x.sync()
+                x.close()
+            for _ in range(300):  # some 0.1 ms each
+                long.run(busy)
+            graph = Graph(capturing)
+            captured.run(capturing)
+            chunk.run(fresh)
+            graph.end()
+            with pytest.raises(BkvError) as ei:
+                busy.wait(1)
+            assert ei.value.status == L.ERR_TIMEOUT, "the call waited for everything on the device"
+            fresh.sync()
+            assert np.array_equal(chunk.out(), want)
+            chunk.clear()
+            graph.launch(capturing)
+            device_sync()
+            for i in (0, 39):
+                check_attn(captured.out()[i], tw.oracle_attend(0, s, 500 + i, captured.q[i], 16), "token %d" % i)
+            captured.clear()
+            graph.destroy()
+            fresh.close()
+        for x in (capturing, busy):
+            x.close()
+        for c in (chunk, captured, long):
+            c.free()
 
 
 def test_a_cut_chunk_leaves_captures_on_other_streams_alone():
