@@ -618,22 +618,14 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     };
     QRaw q_raw;
     request_q(P, e, kvh, wave, c, g, q_raw);
-    __builtin_amdgcn_sched_barrier(0);
-    if (SEL || n_steps > 0) fetch(0);  // a selection list's first units before its length is known
-
     // STEP: the wave that will hold the page of cell pos (in its last step) takes the new rows before the
-    // loop, while its first units are on their way: the raw values are requested ahead of the q fragments
-    // (one wait covers both), then lanes 0..7 encode the K row and lanes 8..15 the V row with the append
-    // kernel's encoder, one lane per 32-value block, into the pool and into two parking rows in LDS.  In
-    // its last step the wave copies a parked row into the unit that has just landed (an LDS move instead
-    // of a trip to memory and an encode at the end of the work-group's walk).
-    const auto wave_lds_fence = [&]() {
-        // the wave's own LDS writes are in order with its later reads; keep the compiler from
-        // moving those reads up
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
+    // loop, while its first units are on their way: the raw values are requested with its part of q, then lanes
+    // 0..7 encode the K row and lanes 8..15 the V row with the append kernel's encoder, one lane per 32-value
+    // block, into the pool and into two parking rows in LDS.  In its last step the wave copies a parked row
+    // into the unit that has just landed (an LDS move instead of a trip to memory and an encode at the end of
+    // the work-group's walk).  Encoded ahead of the trade of the q fragments: beside those, the raw values and
+    // the units in flight no longer fitted the registers (12 bytes of scratch a lane; 64 sequences of 512 to
+    // 4096 cells 36.3 us with it, 35.7 without).
     const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
     float new_x[32];
     if constexpr (STEP) {
@@ -646,10 +638,16 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
             }
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (SEL || n_steps > 0) fetch(0);  // a selection list's first units before its length is known
 
-    half8 qhi[8], qlo[8];
-    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
-
+    const auto wave_lds_fence = [&]() {
+        // the wave's own LDS writes are in order with its later reads; keep the compiler from
+        // moving those reads up
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     if constexpr (STEP) {
         if (takes_new_row) {
             if (lane < 16) {
@@ -669,6 +667,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
             wave_lds_fence();
         }
     }
+
+    half8 qhi[8], qlo[8];
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
 
     f4 o[2][8];
 #pragma unroll
@@ -1005,7 +1006,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    // the raw values are requested ahead of the q fragments (one wait covers both) and encoded after them
+    // the raw values are requested behind the first units and encoded once the q fragments are traded
     const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
     float new_x[32];
     if constexpr (STEP) {
