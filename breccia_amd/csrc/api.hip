@@ -492,7 +492,6 @@ bkv_status bkv_pool_create(const bkv_pool_desc* d, bkv_pool** out) {
     // created here rather than on first use: the calls that order work with them create nothing
     BKV_TRY(hipEventCreateWithFlags(&p->attn_ws.ev, hipEventDisableTiming));
     BKV_TRY(hipEventCreateWithFlags(&p->sel_ws.ev, hipEventDisableTiming));
-    for (ChunkWorkspace& w : p->chunk_ws) BKV_TRY(hipEventCreateWithFlags(&w.done, hipEventDisableTiming | hipEventDisableSystemFence));
     BKV_TRY(hipEventCreateWithFlags(&p->table_sync.ev, hipEventDisableTiming));
     (void)allocate_chunk_workspace(p, p->chunk_ws[0]);  // chunks stay uncut without it
     // this device's copy of the static scratch of bkv_decode_attn_static
@@ -1436,6 +1435,7 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
     }
     BKV_HIP(launch_prefill_attn(p, layer, b, a, (int32_t)rows_per_wg, ws ? &split : nullptr, ws, S(stream)));
     if (ws && p->chunk_many) {
+        if (!ws->done) BKV_HIP(hipEventCreateWithFlags(&ws->done, hipEventDisableTiming | hipEventDisableSystemFence));
         BKV_HIP(hipEventRecord(ws->done, S(stream)));
         ws->recorded = true;
     }
