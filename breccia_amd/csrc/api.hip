@@ -472,6 +472,7 @@ bkv_status bkv_pool_create(const bkv_pool_desc* d, bkv_pool** out) {
 
     BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->part_o), (uint64_t)p->max_wgs * 8u * 256u * 4u));
     BKV_TRY(hipMalloc(reinterpret_cast<void**>(&p->part_ml), (uint64_t)p->max_wgs * 8u * 2u * 4u));
+    (void)allocate_chunk_workspace(p, p->chunk_ws[0]);  // chunks stay uncut without it
 
     BKV_TRY(hipHostMalloc(reinterpret_cast<void**>(&p->ring.host),
                           ParamRing::kSlots * ParamRing::kSlotBytes, hipHostMallocDefault));
@@ -493,7 +494,6 @@ bkv_status bkv_pool_create(const bkv_pool_desc* d, bkv_pool** out) {
     BKV_TRY(hipEventCreateWithFlags(&p->attn_ws.ev, hipEventDisableTiming));
     BKV_TRY(hipEventCreateWithFlags(&p->sel_ws.ev, hipEventDisableTiming));
     BKV_TRY(hipEventCreateWithFlags(&p->table_sync.ev, hipEventDisableTiming));
-    (void)allocate_chunk_workspace(p, p->chunk_ws[0]);  // chunks stay uncut without it
     // this device's copy of the static scratch of bkv_decode_attn_static
     BKV_TRY(attn_static_scratch_init(p->device));
     BKV_TRY(hipDeviceSynchronize());
@@ -1401,7 +1401,8 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
             b.src0[i] = as_given.src0[order[i]];
         }
     }
-    const int64_t rows_per_wg = prefill_rows_per_wg(p->g.layout, wgs, p->n_cu);
+    const bool f16 = p->g.layout == BKV_LAYOUT_F16;
+    const int64_t rows_per_wg = prefill_rows_per_wg(f16, wgs, p->n_cu);
     wgs = 0;
     for (int i = 0; i < n_seqs; ++i) {
         b.wg_base[i] = (int32_t)wgs;
@@ -1425,7 +1426,8 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
     a.scale = scale;
     a.out = out_dev;
     PrefillSplit split;
-    bool cut = plan_prefill_split(p, b, (int32_t)rows_per_wg, (int32_t)group, split);
+    const PrefillPlanLimits lim{f16, p->g.n_kv, p->n_cu, (int64_t)p->max_wgs * 8};
+    bool cut = plan_prefill_split(lim, b, (int32_t)rows_per_wg, (int32_t)group, split);
     // A captured call stays uncut: its replays would share a workspace with whatever runs beside them.
     if (cut && stream) cut = !being_captured(S(stream));
     ChunkWorkspace* ws = nullptr;

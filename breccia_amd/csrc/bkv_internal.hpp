@@ -12,6 +12,7 @@
 #include "../../include/breccia_kv.h"
 #include "allocator.hpp"
 #include "attn_plan.hpp"
+#include "prefill_plan.hpp"
 #include "prefix_tree.hpp"
 
 namespace bkv {
@@ -265,29 +266,7 @@ hipError_t attn_static_scratch_init(int device);
 bool attn_static_scratch(int device, float** o, float** ml);
 hipError_t launch_decode_attn(bkv_pool* p, int32_t layer, const AttnBatch& b, const AttnArgs& a,
                               hipStream_t stream);
-// Prefill attention (prefill_attn.hip): one entry per sequence chunk.
-struct PrefillBatch {
-    int32_t n;
-    int32_t row[BKV_MAX_BATCH];     // block-table row
-    int32_t pos0[BKV_MAX_BATCH];    // position of the chunk's first token
-    int32_t n_tok[BKV_MAX_BATCH];   // tokens of the chunk
-    int32_t src0[BKV_MAX_BATCH];    // first token row in q / out
-    int32_t wg_base[BKV_MAX_BATCH + 1];
-};
-// query rows one work-group owns, given how many 64-row work-groups the call's chunks would make
-int32_t prefill_rows_per_wg(int32_t layout, int64_t wgs_of_64_rows, int32_t n_cu);
-// How a call whose longest page walks would outlast the rest is cut: the walks of an entry's
-// longest blocks (its last ones) in ranges of at most pps pages, a work-group each.
-struct PrefillSplit {
-    int32_t pps;                           // even
-    int32_t n_cut[BKV_MAX_BATCH];          // row blocks of the entry that are cut
-    int32_t splits[BKV_MAX_BATCH];         // ranges of its longest block
-    int32_t wg_base[BKV_MAX_BATCH + 1];    // work-groups of the entries before; [n] = total
-    int32_t unit_base[BKV_MAX_BATCH + 1];  // their cut (row block, kv head) units; [n] = total
-    int32_t slot_base[BKV_MAX_BATCH];      // their partial results, in row blocks
-};
-// False where the call is better off uncut.
-bool plan_prefill_split(const bkv_pool* p, const PrefillBatch& b, int32_t rows_per_wg, int32_t group, PrefillSplit& s);
+// Prefill attention (prefill_attn.hip; the batch and how it is cut: prefill_plan.hpp).
 // split: null for an uncut call; a cut one leaves its partial results in ws
 hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b, const AttnArgs& a,
                                int32_t rows_per_wg, const PrefillSplit* split, const ChunkWorkspace* ws, hipStream_t stream);

@@ -1,0 +1,126 @@
+// How the chunk attention kernel's work is laid out: query rows of a work-group, and the cut of page walks that
+// would outlast the rest of a call.  No HIP types: host-only tests run the same functions.
+#pragma once
+
+#include <algorithm>
+#include <cstdint>
+
+#include "attn_plan.hpp"
+
+namespace bkv {
+
+constexpr int kPrefillPage = 16;         // cells of a page
+constexpr int kPrefillRowsPerWave = 16;  // query rows
+constexpr int kMaxRanges = 64;           // of one row block: the merge kernel has a lane for each
+
+// one entry per sequence chunk
+struct PrefillBatch {
+    int32_t n;
+    int32_t row[kMaxBatch];    // block-table row
+    int32_t pos0[kMaxBatch];   // position of the chunk's first token
+    int32_t n_tok[kMaxBatch];  // tokens of the chunk
+    int32_t src0[kMaxBatch];   // first token row in q / out
+    int32_t wg_base[kMaxBatch + 1];
+};
+
+// How a call whose longest page walks would outlast the rest is cut: the walks of an entry's
+// longest blocks (its last ones) in ranges of at most pps pages, a work-group each.
+struct PrefillSplit {
+    int32_t pps;                       // even
+    int32_t n_cut[kMaxBatch];          // row blocks of the entry that are cut
+    int32_t splits[kMaxBatch];         // ranges of its longest block
+    int32_t wg_base[kMaxBatch + 1];    // work-groups of the entries before; [n] = total
+    int32_t unit_base[kMaxBatch + 1];  // their cut (row block, kv head) units; [n] = total
+    int32_t slot_base[kMaxBatch];      // their partial results, in row blocks
+};
+
+struct PrefillPlanLimits {
+    bool f16;      // the layout: f16 pools, or quantised ones
+    int32_t n_kv;
+    int32_t n_cu;
+    int64_t rows;  // query rows a workspace holds partial results for
+};
+
+// Ranges of a block that walks `pages` pages, and the (even) pages of each: evened out, none empty.
+BKV_HD inline int split_ranges(int pages, int pps, int max_splits, int& each) {
+    const int by_pps = (pages + pps - 1) / pps;
+    const int n = by_pps < max_splits ? by_pps : max_splits;
+    each = ((pages + n - 1) / n + 1) & ~1;
+    return (pages + each - 1) / each;
+}
+
+// Query rows one work-group owns.  f16 pools: 128 when the chunks make more 64-row work-groups than
+// fit the chip at two per compute unit (then sharing the page images among more rows is worth more
+// than spreading out), else 64.
+inline int32_t prefill_rows_per_wg(bool f16, int64_t wgs_of_64_rows, int32_t n_cu) {
+    if (!f16) return 8 * kPrefillRowsPerWave;
+    return wgs_of_64_rows > 2 * (int64_t)(n_cu > 0 ? n_cu : 256) ? 8 * kPrefillRowsPerWave : 4 * kPrefillRowsPerWave;
+}
+
+// Cuts the page walks of a small call's row blocks into ranges; false where the call is better off
+// uncut.  A row block's walk is a serial chain: 1.4 us a page pair on f16 pools when the compute unit
+// has nothing else (2.3-3.6 us on the quantised ones), and a call of a few blocks is as long as its longest
+// chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups, 34 us).  Cutting
+// pays for a second kernel (4-9 us, by the partial rows it reads), so:
+// - a call that leaves half of the compute units idle is cut if
+//   - a range keeps at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several, and
+//   - the chain loses 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured 31.1 us
+//     uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
+//   - into one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer
+//     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8;
+// - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) if its
+//   longest walk is over 1.7 times what an even share of the pairs would be -- cut calls measured 1.45 to
+//   1.75 of that: 900 tokens behind 3000 and 900 from scratch (int8) 383 -> 243 us, 2048 from scratch
+//   201 -> 176, 1500 with 24 heads behind 500 (1.47) 205 and 206.
+// Before / after, us a layer: 41 tokens behind 517 cells 37 / 24, 100 behind 8000 374 / 55, 200 behind
+// 3000 with q8_0 V 262 / 59, 300 behind 1000 on an int8 pool 125 / 48.
+inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s) {
+    const int32_t n_kv = lim.n_kv;
+    const int n_cu = lim.n_cu > 0 ? lim.n_cu : 256;
+    const bool f16 = lim.f16;
+    const bool idle = (int64_t)b.wg_base[b.n] * 2 <= n_cu;
+    if (!idle && (f16 || b.wg_base[b.n] > 2 * n_cu)) return false;
+    const int64_t least = f16 ? 3 : 2, gain = f16 ? 10 : 5;
+    const int64_t room = lim.rows / rows;  // partial results the workspace holds
+    int64_t work = 0;
+    int32_t longest = 0;
+    const auto pairs_of = [&](int i, int32_t blk) {
+        const int32_t last_row = std::min((blk + 1) * rows, b.n_tok[i] * group) - 1;
+        return ((b.pos0[i] + last_row / group) / kPrefillPage + 2) / 2;
+    };
+    const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
+    for (int i = 0; i < b.n; ++i) {
+        const int32_t nb = blocks_of(i);
+        for (int32_t k = 0; k < nb; ++k) work += (int64_t)pairs_of(i, k) * n_kv;
+        if (nb) longest = std::max(longest, pairs_of(i, nb - 1));
+    }
+    int64_t most = std::min<int64_t>(room, n_cu);
+    if (f16 && work > 8 * most) most = std::min<int64_t>(room, 2 * n_cu);
+    int64_t each = std::max<int64_t>({least, (work + most - 1) / most, (longest + kMaxRanges - 1) / kMaxRanges});
+    if (!idle && 10 * (int64_t)longest * n_cu < 17 * work) return false;
+    for (;; each += std::max<int64_t>(1, each / 8)) {
+        if (longest < each + gain) return false;
+        int64_t wgs = 0, units = 0, slots = 0;
+        for (int i = 0; i < b.n; ++i) {
+            const int32_t nb = blocks_of(i);
+            int32_t cut = 0;
+            while (cut < nb && pairs_of(i, nb - 1 - cut) > each) ++cut;
+            const int64_t ranges = cut ? (pairs_of(i, nb - 1) + each - 1) / each : 1;
+            s.n_cut[i] = cut;
+            s.splits[i] = (int32_t)ranges;
+            s.unit_base[i] = (int32_t)units;
+            s.slot_base[i] = (int32_t)slots;
+            s.wg_base[i] = (int32_t)wgs;
+            units += (int64_t)cut * n_kv;
+            slots += cut * n_kv * ranges;
+            wgs += cut * n_kv * ranges + (int64_t)(nb - cut) * n_kv;
+        }
+        s.unit_base[b.n] = (int32_t)units;
+        s.wg_base[b.n] = (int32_t)wgs;
+        if (idle ? wgs <= most : slots <= room) break;
+    }
+    s.pps = (int32_t)each * 2;
+    return true;
+}
+
+}  // namespace bkv

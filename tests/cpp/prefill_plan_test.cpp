@@ -1,0 +1,120 @@
+// How chunk attention cuts its page walks (breccia_amd/csrc/prefill_plan.hpp), over random batches: every cut the
+// planner returns is walked the way the kernels walk it -- work-group index to (entry, row block, kv head, range), and
+// row block to its partial results -- and has to cover every page of every row block once, inside the workspace.
+// Prints what it met and exits 0.
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+#include <vector>
+
+#include "../../breccia_amd/csrc/prefill_plan.hpp"
+
+using namespace bkv;
+
+static void must(bool ok, const char* what, int at) {
+    if (!ok) {
+        std::fprintf(stderr, "FAILED in batch %d: %s\n", at, what);
+        std::exit(1);
+    }
+}
+
+int main(int argc, char** argv) {
+    std::mt19937 rng(argc > 1 ? (unsigned)std::atoi(argv[1]) : 1u);
+    const int batches = argc > 2 ? std::atoi(argv[2]) : 100000;
+    const auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
+    const auto log_pick = [&](double lo, double hi) { return (int)std::lround(lo * std::pow(hi / lo, (rng() % 4096) / 4095.0)); };
+    int cuts = 0, widened = 0, unbalanced = 0, most_ranges = 0;
+    double fullest = 0.0;
+    for (int at = 0; at < batches; ++at) {
+        PrefillPlanLimits lim{};
+        lim.f16 = pick(0, 1);
+        lim.n_kv = 1 << pick(0, 3);
+        lim.n_cu = pick(0, 3) ? 256 : pick(16, 304);
+        lim.rows = 4096 * 8;
+        const int group = pick(1, 16);
+        PrefillBatch b{};
+        b.n = pick(0, 2) ? pick(1, 3) : log_pick(1, kMaxBatch);
+        const int most_tok = log_pick(1, 3000), most_before = log_pick(1, 300000);
+        int64_t wgs64 = 0;
+        for (int i = 0; i < b.n; ++i) {
+            b.n_tok[i] = pick(0, 7) ? log_pick(1, most_tok) : 0;
+            b.pos0[i] = pick(0, 2) ? log_pick(1, most_before) : 0;
+            wgs64 += ((int64_t)b.n_tok[i] * group + 63) / 64 * lim.n_kv;
+        }
+        const int rows = prefill_rows_per_wg(lim.f16, wgs64, lim.n_cu);
+        const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
+        int64_t wgs = 0;
+        for (int i = 0; i < b.n; ++i) {
+            b.wg_base[i] = (int32_t)wgs;
+            wgs += (int64_t)blocks_of(i) * lim.n_kv;
+        }
+        b.wg_base[b.n] = (int32_t)wgs;
+        PrefillSplit s;
+        if (wgs == 0 || !plan_prefill_split(lim, b, rows, group, s)) continue;
+        ++cuts;
+        const int64_t room = lim.rows / rows;
+        must(s.pps > 0 && s.pps % 2 == 0, "an odd range", at);
+        must(s.wg_base[0] == 0 && s.unit_base[0] == 0, "bases begin at zero", at);
+        // pages of the row block `idx` of entry e, blocks counted from the last one
+        const auto pages_of = [&](int e, int idx) {
+            const int rb = blocks_of(e) - 1 - idx;
+            const int last_row = std::min(rb * rows + rows, b.n_tok[e] * group) - 1;
+            return (b.pos0[e] + last_row / group) / kPrefillPage + 1;
+        };
+        std::vector<std::vector<std::vector<int>>> walked(b.n);  // [entry][block, kv head] -> how often each page
+        for (int e = 0; e < b.n; ++e) {
+            must(s.n_cut[e] >= 0 && s.n_cut[e] <= blocks_of(e), "more blocks cut than there are", at);
+            must(s.splits[e] >= 1 && s.splits[e] <= kMaxRanges, "more ranges than the merge has lanes", at);
+            for (int idx = 0; idx < blocks_of(e); ++idx)
+                for (int h = 0; h < lim.n_kv; ++h) walked[e].push_back(std::vector<int>(pages_of(e, idx), 0));
+        }
+        std::vector<char> slot_used(room, 0);
+        int used = 0;
+        for (int wg = 0; wg < s.wg_base[b.n]; ++wg) {
+            int e = 0;
+            while (e + 1 < b.n && wg >= s.wg_base[e + 1]) ++e;
+            int rem = wg - s.wg_base[e], range = 0;
+            const int uncut = (blocks_of(e) - s.n_cut[e]) * lim.n_kv;
+            const bool cut = rem >= uncut;
+            if (cut) {
+                rem -= uncut;
+                range = rem % s.splits[e];
+                rem /= s.splits[e];
+            }
+            const int kvh = rem % lim.n_kv, idx = rem / lim.n_kv + (cut ? 0 : s.n_cut[e]);
+            must(idx < blocks_of(e), "a work-group past the entry's blocks", at);
+            const int pages = pages_of(e, idx);
+            int first = 0, end = pages;
+            if (cut) {
+                int each;
+                const int ranges = split_ranges(pages, s.pps, s.splits[e], each);
+                must(ranges >= 2 && ranges <= s.splits[e] && each % 2 == 0 && each <= s.pps, "a block's ranges", at);
+                most_ranges = std::max(most_ranges, ranges);
+                if (range >= ranges) continue;
+                first = range * each;
+                end = std::min(pages, first + each);
+                const int64_t slot = s.slot_base[e] + (int64_t)(idx * lim.n_kv + kvh) * s.splits[e] + range;
+                must(slot >= 0 && slot < room, "a partial result outside the workspace", at);
+                must(!slot_used[slot], "two ranges in one place", at);
+                slot_used[slot] = 1;
+                used = std::max(used, (int)slot + 1);
+            }
+            must(first < end, "an empty range", at);
+            for (int pg = first; pg < end; ++pg) ++walked[e][(size_t)idx * lim.n_kv + kvh][pg];
+        }
+        for (const auto& entry : walked)
+            for (const auto& block : entry)
+                for (int times : block) must(times == 1, "a page is walked other than once", at);
+        // the merge's units: the cut blocks, entry by entry
+        for (int e = 0; e < b.n; ++e)
+            must(s.unit_base[e + 1] - s.unit_base[e] == s.n_cut[e] * lim.n_kv, "units of the merge", at);
+        fullest = std::max(fullest, (double)used / (double)room);
+        if (lim.f16 && s.wg_base[b.n] > lim.n_cu) ++widened;
+        if (wgs * 2 > lim.n_cu) ++unbalanced;
+    }
+    std::printf("%d cut: %d two work-groups a compute unit, %d unbalanced, up to %d ranges, workspace filled to %.3f\n", cuts, widened,
+                unbalanced, most_ranges, fullest);
+    // the sweep has to reach the planner's ends
+    return cuts > batches / 20 && widened > 100 && unbalanced > 100 && most_ranges >= 63 && fullest > 0.99 ? 0 : 2;
+}

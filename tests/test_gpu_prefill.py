@@ -252,7 +252,8 @@ def test_work_group_width_does_not_change_a_bit():
     # On f16 pools a call whose chunks fill the chip runs work-groups of eight waves (128 query rows
     # share each page image), a smaller one work-groups of four.  A wave's sixteen rows are computed
     # the same way in both, so three chunks in one call (566 work-groups of 64 rows: eight waves) and
-    # the same chunks one call each (four waves) must agree in every bit; the oracle checks a sample.
+    # the same chunks one call each (four waves; each keeps more than half of the chip busy, so that
+    # none has its walks cut) must agree in every bit; the oracle checks a sample.
     rng = np.random.Generator(np.random.PCG64(1234))
     cases = [(100, 700), (37, 650), (515, 900)]
     with Twin(n_pages=200, max_seqs=4) as tw:

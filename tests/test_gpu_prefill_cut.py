@@ -21,15 +21,17 @@ pytestmark = pytest.mark.gpu
     (24, [(0, 239), (4081, 3)]),                         # blocks of one entry uncut beside cut ones
     (6, [(700, 77), (0, 0), (0, 9), (1535, 33)]),        # groups of 3 rows, an empty chunk, a chunk too short to cut
     (2, [(0, 600)]),                                     # ranges past the positions of their block's first rows
+    (16, [(8000, 100)]),                                 # f16: two work-groups a compute unit, the workspace nearly full
+    (2, [(9990, 20)]),                                   # 63 ranges in a row block: the merge has 64 lanes for them
 ])
 def test_cut_chunks_match_the_oracle(n_q, cases, layout):
     rng = np.random.Generator(np.random.PCG64(77 + n_q))
-    with Twin(n_pages=500, max_seqs=4, layout=layout) as tw:
+    with Twin(n_pages=640, max_seqs=4, layout=layout) as tw:
         tw.pool.fill(0xFF)
         for img in tw.images:
             img.k[:] = 0xFF
             img.v[:] = 0xFF
-        tw.pool.set_free_order(rng.permutation(500).astype(np.int32))
+        tw.pool.set_free_order(rng.permutation(640).astype(np.int32))
         seqs = [tw.pool.seq_create() for _ in cases]
         for s, (before, t) in zip(seqs, cases):
             if before + t:
