@@ -3,7 +3,10 @@
 #pragma once
 
 #include <algorithm>
+#include <cstddef>
 #include <cstdint>
+#include <functional>
+#include <vector>
 
 #include "attn_plan.hpp"
 
@@ -57,6 +60,24 @@ inline int32_t prefill_rows_per_wg(bool f16, int64_t wgs_of_64_rows, int32_t n_c
     return wgs_of_64_rows > 2 * (int64_t)(n_cu > 0 ? n_cu : 256) ? 8 * kPrefillRowsPerWave : 4 * kPrefillRowsPerWave;
 }
 
+// When the last of the work-groups is done, in page pairs, if each unit takes the next one as it becomes free.
+// runs: their pairs, in the order of dispatch.
+inline int32_t last_done(const std::vector<int32_t>& runs, int32_t units) {
+    const size_t at_once = std::min(runs.size(), (size_t)units);
+    std::vector<int32_t> free_at(runs.begin(), runs.begin() + (ptrdiff_t)at_once);
+    int32_t last = free_at.empty() ? 0 : *std::max_element(free_at.begin(), free_at.end());
+    if (runs.size() == at_once) return last;
+    const auto later = std::greater<int32_t>();  // a heap, the earliest in front
+    std::make_heap(free_at.begin(), free_at.end(), later);
+    for (size_t i = at_once; i < runs.size(); ++i) {
+        std::pop_heap(free_at.begin(), free_at.end(), later);
+        free_at.back() += runs[i];
+        last = std::max(last, free_at.back());
+        std::push_heap(free_at.begin(), free_at.end(), later);
+    }
+    return last;
+}
+
 // Cuts the page walks of a small call's row blocks into ranges; false where the call is better off
 // uncut.  A row block's walk is a serial chain: 1.4 us a page pair on f16 pools when the compute unit
 // has nothing else (2.3-3.6 us on the quantised ones), and a call of a few blocks is as long as its longest
@@ -68,10 +89,16 @@ inline int32_t prefill_rows_per_wg(bool f16, int64_t wgs_of_64_rows, int32_t n_c
 //     uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
 //   - into one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer
 //     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8;
-// - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) if its
-//   longest walk is over 1.7 times what an even share of the pairs would be -- cut calls measured 1.45 to
-//   1.75 of that: 900 tokens behind 3000 and 900 from scratch (int8) 383 -> 243 us, 2048 from scratch
-//   201 -> 176, 1500 with 24 heads behind 500 (1.47) 205 and 206.
+// - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) of up to
+//   two work-groups a compute unit may be cut, into ranges of an even share of the pairs;
+// - either way the chain has to lose a pair for every 32 partial results the second kernel reads; in the larger calls,
+//   where the ranges come on top of a chip that is nearly busy, for every 24, and for every 19 if they don't all find a
+//   compute unit at once (the chain of a cut call is then the schedule's).  260 calls a layout, random and at the
+//   edges, each measured cut and uncut: a pair less gains 2.5 us (f16 1.4), a partial result costs 0.04 (f16 0.03),
+//   in the larger calls 0.17.  With these lines no call loses more than 4 %, but for 60 chunks of 8 tokens
+//   behind 600 cells (7 %); with a ratio of longest walk to even share (1.7) some lost 41 %: four chunks of 270 from
+//   scratch 38 us uncut, 52 cut; 600 with 48 heads 70 and 79; 32 chunks of 8 behind 250 28 and 31; on the other
+//   side two chunks of 530 60 and 48, 1900 169 and 151, 400 with 48 heads 51 and 45.
 // Before / after, us a layer: 41 tokens behind 517 cells 37 / 24, 100 behind 8000 374 / 55, 200 behind
 // 3000 with q8_0 V 262 / 59, 300 behind 1000 on an int8 pool 125 / 48.
 inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s) {
@@ -84,10 +111,11 @@ inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch&
     const int64_t room = lim.rows / rows;  // partial results the workspace holds
     int64_t work = 0;
     int32_t longest = 0;
-    const auto pairs_of = [&](int i, int32_t blk) {
+    const auto pages_of = [&](int i, int32_t blk) {
         const int32_t last_row = std::min((blk + 1) * rows, b.n_tok[i] * group) - 1;
-        return ((b.pos0[i] + last_row / group) / kPrefillPage + 2) / 2;
+        return (b.pos0[i] + last_row / group) / kPrefillPage + 1;
     };
+    const auto pairs_of = [&](int i, int32_t blk) { return (pages_of(i, blk) + 1) / 2; };
     const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
     for (int i = 0; i < b.n; ++i) {
         const int32_t nb = blocks_of(i);
@@ -97,7 +125,6 @@ inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch&
     int64_t most = std::min<int64_t>(room, n_cu);
     if (f16 && work > 8 * most) most = std::min<int64_t>(room, 2 * n_cu);
     int64_t each = std::max<int64_t>({least, (work + most - 1) / most, (longest + kMaxRanges - 1) / kMaxRanges});
-    if (!idle && 10 * (int64_t)longest * n_cu < 17 * work) return false;
     for (;; each += std::max<int64_t>(1, each / 8)) {
         if (longest < each + gain) return false;
         int64_t wgs = 0, units = 0, slots = 0;
@@ -120,7 +147,25 @@ inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch&
         if (idle ? wgs <= most : slots <= room) break;
     }
     s.pps = (int32_t)each * 2;
-    return true;
+    int64_t partials = 0;
+    std::vector<int32_t> runs;  // of the work-groups, in the order of dispatch
+    runs.reserve((size_t)s.wg_base[b.n]);
+    for (int i = 0; i < b.n; ++i) {
+        const int32_t nb = blocks_of(i);
+        for (int32_t k = s.n_cut[i]; k < nb; ++k) runs.insert(runs.end(), (size_t)n_kv, pairs_of(i, nb - 1 - k));
+        for (int32_t k = 0; k < s.n_cut[i]; ++k) {
+            int even;
+            const int pages = pages_of(i, nb - 1 - k), ranges = split_ranges(pages, s.pps, s.splits[i], even);
+            partials += (int64_t)ranges * n_kv;
+            for (int h = 0; h < n_kv; ++h) {
+                runs.insert(runs.end(), (size_t)(ranges - 1), even / 2);
+                runs.push_back((pages - (ranges - 1) * even + 1) / 2);
+            }
+        }
+    }
+    const int32_t units = f16 ? 2 * n_cu : n_cu;
+    const int32_t chain = last_done(runs, units);
+    return (int64_t)(longest - chain) * (idle ? 32 : (int32_t)runs.size() <= units ? 24 : 19) > partials;
 }
 
 }  // namespace bkv

@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <random>
+#include <utility>
 #include <vector>
 
 #include "../../breccia_amd/csrc/prefill_plan.hpp"
@@ -19,7 +20,42 @@ static void must(bool ok, const char* what, int at) {
     }
 }
 
+// Whether the call's walks are cut: q heads over two kv heads, (cells before, tokens) of its chunks, on 256 compute units.
+static bool is_cut(bool f16, int n_q, const std::vector<std::pair<int, int>>& chunks) {
+    const PrefillPlanLimits lim{f16, 2, 256, 4096 * 8};
+    const int group = n_q / 2;
+    PrefillBatch b{};
+    int64_t wgs64 = 0, wgs = 0;
+    for (const auto& c : chunks) {
+        b.pos0[b.n] = c.first;
+        b.n_tok[b.n++] = c.second;
+        wgs64 += ((int64_t)c.second * group + 63) / 64 * lim.n_kv;
+    }
+    const int rows = prefill_rows_per_wg(f16, wgs64, lim.n_cu);
+    for (int i = 0; i < b.n; ++i) {
+        b.wg_base[i] = (int32_t)wgs;
+        wgs += ((int64_t)b.n_tok[i] * group + rows - 1) / rows * lim.n_kv;
+    }
+    b.wg_base[b.n] = (int32_t)wgs;
+    PrefillSplit s;
+    return plan_prefill_split(lim, b, rows, group, s);
+}
+
+// Calls measured both ways, on either side of the planner's lines.
+static void lines() {
+    using Chunks = std::vector<std::pair<int, int>>;
+    must(!is_cut(false, 16, Chunks(4, {0, 270})), "four chunks of 270: 38 us uncut, 52 cut", -1);
+    must(!is_cut(false, 48, {{0, 600}}), "600 tokens with 48 heads: 70 us uncut, 79 cut", -1);
+    must(!is_cut(false, 16, Chunks(32, {250, 8})), "32 chunks of 8 behind 250: 28 us uncut, 31 cut", -1);
+    must(!is_cut(true, 16, Chunks(16, {500, 30})), "f16, 16 chunks of 30 behind 500: 35 us uncut, 38 cut", -1);
+    must(is_cut(false, 16, Chunks(2, {0, 530})), "two chunks of 530: 60 us uncut, 48 cut", -1);
+    must(is_cut(false, 16, {{0, 1900}}), "1900 tokens: 169 us uncut, 151 cut", -1);
+    must(is_cut(false, 48, {{0, 400}}), "400 tokens with 48 heads: 51 us uncut, 45 cut", -1);
+    must(is_cut(true, 16, {{517, 41}}), "f16, 41 tokens behind 517: 37 us uncut, 24 cut", -1);
+}
+
 int main(int argc, char** argv) {
+    lines();
     std::mt19937 rng(argc > 1 ? (unsigned)std::atoi(argv[1]) : 1u);
     const int batches = argc > 2 ? std::atoi(argv[2]) : 100000;
     const auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
