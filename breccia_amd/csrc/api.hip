@@ -3,7 +3,6 @@
 // before anything reaches the GPU (the reference's contract, crates/breccia-kernels/
 // src/qsa/mod.rs:1108-1116).
 #include <algorithm>
-#include <numeric>
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -1387,28 +1386,9 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
             return fail(BKV_ERR_INVALID, "prefill_attn: more than 2^24 tokens in one call");
     }
     b.n = n_seqs;
-    // the chunks with the longest walks are dispatched first
-    {
-        int32_t order[BKV_MAX_BATCH];
-        std::iota(order, order + n_seqs, 0);
-        const auto end_of = [&](int32_t i) { return pos0[i] + n_tokens[i]; };
-        std::stable_sort(order, order + n_seqs, [&](int32_t i, int32_t j) { return end_of(i) > end_of(j); });
-        const PrefillBatch as_given = b;
-        for (int i = 0; i < n_seqs; ++i) {
-            b.row[i] = as_given.row[order[i]];
-            b.pos0[i] = as_given.pos0[order[i]];
-            b.n_tok[i] = as_given.n_tok[order[i]];
-            b.src0[i] = as_given.src0[order[i]];
-        }
-    }
     const bool f16 = p->g.layout == BKV_LAYOUT_F16;
     const int64_t rows_per_wg = prefill_rows_per_wg(f16, wgs, p->n_cu);
-    wgs = 0;
-    for (int i = 0; i < n_seqs; ++i) {
-        b.wg_base[i] = (int32_t)wgs;
-        wgs += ((int64_t)b.n_tok[i] * group + rows_per_wg - 1) / rows_per_wg * p->g.n_kv;
-    }
-    b.wg_base[n_seqs] = (int32_t)wgs;
+    order_chunks(b, p->g.n_kv, (int32_t)group, (int32_t)rows_per_wg);
     bkv_status st = need_device(p);
     if (st != BKV_OK) return st;
     if (total == 0) return BKV_OK;
@@ -1427,7 +1407,7 @@ bkv_status bkv_prefill_attn(bkv_pool* p, int32_t layer, int32_t n_seqs, const in
     a.out = out_dev;
     PrefillSplit split;
     const PrefillPlanLimits lim{f16, p->g.n_kv, p->n_cu, (int64_t)p->max_wgs * 8};
-    bool cut = plan_prefill_split(lim, b, (int32_t)rows_per_wg, (int32_t)group, split);
+    bool cut = plan_prefill(lim, b, (int32_t)rows_per_wg, (int32_t)group, split);
     // A captured call stays uncut: its replays would share a workspace with whatever runs beside them.
     if (cut && stream) cut = !being_captured(S(stream));
     ChunkWorkspace* ws = nullptr;

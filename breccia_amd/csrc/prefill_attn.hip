@@ -97,8 +97,8 @@ struct PrefillSplitParams : PrefillKernelParams {
 // Every work-group of one (entry, kv head) unit walks the same K/V pages, so the dies are given
 // whole units: with 8 or more units, die x serves units x, x + 8, ...; with fewer, unit u is
 // served by dies u, u + U, ...  A unit's pages then stay in one die's L2 (3 MiB for a 3072-token
-// chunk) instead of every die fetching every unit through the fabric.
-constexpr int kXcds = 8;
+// chunk) instead of every die fetching every unit through the fabric.  (kXcds, and where it is done:
+// prefill_plan.hpp)
 
 // gfx950's double-depth form: 32 contraction steps, 8 halves per lane (k = 8 (lane / 16) + 0..7)
 __device__ __forceinline__ f4 mfma32(h8 a, h8 b, f4 c) {
@@ -765,26 +765,10 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
     // Deal the work-groups to the dies by unit where that costs little: the grid then holds 8 x the
     // longest die's share, and work-groups past a shorter die's share leave at once.
     kp.by_xcd = 0;
-    {
-        const int units = b.n * p->g.n_kv;
-        int64_t longest = 0;
-        if (units >= kXcds) {
-            int64_t share[kXcds] = {};
-            for (int u = 0; u < units; ++u)
-                share[u % kXcds] += ((int64_t)b.n_tok[u / p->g.n_kv] * kp.group + rows_per_wg - 1) / rows_per_wg;
-            for (int x = 0; x < kXcds; ++x) longest = std::max(longest, share[x]);
-        } else {
-            for (int u = 0; u < units; ++u) {
-                const int64_t nb = ((int64_t)b.n_tok[u / p->g.n_kv] * kp.group + rows_per_wg - 1) / rows_per_wg;
-                const int dies = (kXcds - u + units - 1) / units;
-                longest = std::max(longest, (nb + dies - 1) / dies);
-            }
-        }
-        const int64_t by_xcd_grid = longest * kXcds;
-        if (by_xcd_grid <= (int64_t)grid + grid / 4 + kXcds) {
-            kp.by_xcd = 1;
-            grid = (int32_t)by_xcd_grid;
-        }
+    const int64_t share = even_die_share(b, p->g.n_kv, kp.group, rows_per_wg);
+    if (share) {
+        kp.by_xcd = 1;
+        grid = (int32_t)(share * kXcds);
     }
     if (p->g.layout == BKV_LAYOUT_Q8V)
         launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_Q8V>, dim3((unsigned)grid), dim3(512), 0,

@@ -25,20 +25,16 @@ static bool is_cut(bool f16, int n_q, const std::vector<std::pair<int, int>>& ch
     const PrefillPlanLimits lim{f16, 2, 256, 4096 * 8};
     const int group = n_q / 2;
     PrefillBatch b{};
-    int64_t wgs64 = 0, wgs = 0;
+    int64_t wgs64 = 0;
     for (const auto& c : chunks) {
         b.pos0[b.n] = c.first;
         b.n_tok[b.n++] = c.second;
         wgs64 += ((int64_t)c.second * group + 63) / 64 * lim.n_kv;
     }
     const int rows = prefill_rows_per_wg(f16, wgs64, lim.n_cu);
-    for (int i = 0; i < b.n; ++i) {
-        b.wg_base[i] = (int32_t)wgs;
-        wgs += ((int64_t)b.n_tok[i] * group + rows - 1) / rows * lim.n_kv;
-    }
-    b.wg_base[b.n] = (int32_t)wgs;
+    order_chunks(b, lim.n_kv, group, rows);
     PrefillSplit s;
-    return plan_prefill_split(lim, b, rows, group, s);
+    return plan_prefill(lim, b, rows, group, s);
 }
 
 // Calls measured both ways, on either side of the planner's lines.
@@ -54,8 +50,115 @@ static void lines() {
     must(is_cut(true, 16, {{517, 41}}), "f16, 41 tokens behind 517: 37 us uncut, 24 cut", -1);
 }
 
+// When an uncut call on a quantised pool ends, in page pairs, its chunks in the batch's order.
+static int32_t uncut_end(const PrefillBatch& b, int group) {
+    std::vector<int32_t> runs;
+    for (int i = 0; i < b.n; ++i)
+        for (int rb = (b.n_tok[i] * group + 127) / 128 - 1; rb >= 0; --rb) {
+            const int last_row = std::min((rb + 1) * 128, b.n_tok[i] * group) - 1;
+            runs.insert(runs.end(), 2, ((b.pos0[i] + last_row / group) / kPrefillPage + 2) / 2);
+        }
+    return last_done(runs, 256);
+}
+
+// The order of dispatch: every chunk once, with what belongs to it, and no call much worse for it.
+static void order() {
+    std::mt19937 rng(5);
+    const auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
+    const auto log_pick = [&](double lo, double hi) { return (int)std::lround(lo * std::pow(hi / lo, (rng() % 4096) / 4095.0)); };
+    double sum = 0.0, worst = 0.0;
+    int calls = 0;
+    while (calls < 300) {
+        PrefillBatch b{};
+        b.n = pick(2, 16);
+        const int group = 4 * pick(1, 4);
+        int64_t wgs = 0, src = 0;
+        for (int i = 0; i < b.n; ++i) {
+            b.row[i] = i;
+            b.n_tok[i] = log_pick(16, 3000);
+            b.pos0[i] = pick(0, 1) ? log_pick(16, 6000) : 0;
+            b.src0[i] = (int32_t)src;
+            src += b.n_tok[i];
+            wgs += ((int64_t)b.n_tok[i] * group + 127) / 128 * 2;
+        }
+        if (wgs < 200 || wgs > 1500) continue;
+        PrefillBatch o = b;
+        order_chunks(o, 2, group, 128);
+        std::vector<char> seen(b.n, 0);
+        for (int i = 0; i < b.n; ++i) {
+            const int r = o.row[i];
+            must(!seen[r]++ && o.pos0[i] == b.pos0[r] && o.n_tok[i] == b.n_tok[r] && o.src0[i] == b.src0[r], "a chunk's own values", calls);
+        }
+        const double ratio = (double)uncut_end(o, group) / (double)uncut_end(b, group);
+        sum += ratio;
+        worst = std::max(worst, ratio);
+        ++calls;
+    }
+    std::printf("order of dispatch: %.3f of the caller's on average, %.3f at most\n", sum / calls, worst);
+    must(sum / calls < 0.96 && worst < 1.16, "the order of dispatch costs more than it gains", calls);
+}
+
+// Units dealt to the dies, walked the way the kernel does it: every row block of every unit once, no die with far more
+// than its share of the pages.
+static void dies() {
+    std::mt19937 rng(9);
+    const auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
+    const auto log_pick = [&](double lo, double hi) { return (int)std::lround(lo * std::pow(hi / lo, (rng() % 4096) / 4095.0)); };
+    int dealt = 0;
+    double worst = 0.0;
+    for (int at = 0; at < 20000; ++at) {
+        const int n_kv = 1 << pick(0, 3), group = pick(1, 16), rows = pick(0, 1) ? 64 : 128;
+        PrefillBatch b{};
+        b.n = pick(1, 12);
+        const int tok = log_pick(1, 3000), before = log_pick(1, 8000), alike = pick(0, 1);
+        for (int i = 0; i < b.n; ++i) {
+            b.n_tok[i] = alike ? pick(tok / 2, tok) : pick(0, 7) ? log_pick(1, 3000) : 0;
+            b.pos0[i] = alike ? before : pick(0, 1) ? log_pick(1, 8000) : 0;
+        }
+        const int64_t share = even_die_share(b, n_kv, group, rows);
+        if (!share) continue;
+        ++dealt;
+        const int units = b.n * n_kv;
+        const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
+        std::vector<std::vector<int>> seen;
+        for (int u = 0; u < units; ++u) seen.push_back(std::vector<int>(blocks_of(u / n_kv), 0));
+        int64_t pages[kXcds] = {}, all = 0;
+        for (int64_t wg = 0; wg < share * kXcds; ++wg) {
+            const int x = (int)(wg % kXcds);
+            int j = (int)(wg / kXcds), u, idx;
+            if (units >= kXcds) {
+                for (u = x; u < units; u += kXcds) {
+                    const int nb = blocks_of(u / n_kv);
+                    if (j < nb) break;
+                    j -= nb;
+                }
+                if (u >= units) continue;
+                idx = j;
+            } else {
+                u = x % units;
+                idx = j * ((kXcds - u + units - 1) / units) + x / units;
+            }
+            const int i = u / n_kv;
+            if (idx >= blocks_of(i)) continue;
+            ++seen[u][idx];
+            const int last_row = std::min((blocks_of(i) - idx) * rows, b.n_tok[i] * group) - 1;
+            const int walked = (b.pos0[i] + last_row / group) / kPrefillPage + 1;
+            pages[x] += walked;
+            all += walked;
+        }
+        for (const auto& unit : seen)
+            for (int times : unit) must(times == 1, "a row block dealt other than once", at);
+        const double most = (double)*std::max_element(pages, pages + kXcds) * kXcds / (double)std::max<int64_t>(all, 1);
+        if (all > 20000) worst = std::max(worst, most);
+    }
+    std::printf("%d dealt to the dies, the fullest with %.2f of its share of the pages\n", dealt, worst);
+    must(dealt > 1000 && worst < 1.35, "dealing to the dies", -1);
+}
+
 int main(int argc, char** argv) {
     lines();
+    order();
+    dies();
     std::mt19937 rng(argc > 1 ? (unsigned)std::atoi(argv[1]) : 1u);
     const int batches = argc > 2 ? std::atoi(argv[2]) : 100000;
     const auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
@@ -80,14 +183,10 @@ int main(int argc, char** argv) {
         }
         const int rows = prefill_rows_per_wg(lim.f16, wgs64, lim.n_cu);
         const auto blocks_of = [&](int i) { return (b.n_tok[i] * group + rows - 1) / rows; };
-        int64_t wgs = 0;
-        for (int i = 0; i < b.n; ++i) {
-            b.wg_base[i] = (int32_t)wgs;
-            wgs += (int64_t)blocks_of(i) * lim.n_kv;
-        }
-        b.wg_base[b.n] = (int32_t)wgs;
+        order_chunks(b, lim.n_kv, group, rows);
+        const int64_t wgs = b.wg_base[b.n];
         PrefillSplit s;
-        if (wgs == 0 || !plan_prefill_split(lim, b, rows, group, s)) continue;
+        if (wgs == 0 || !plan_prefill(lim, b, rows, group, s)) continue;
         ++cuts;
         const int64_t room = lim.rows / rows;
         must(s.pps > 0 && s.pps % 2 == 0, "an odd range", at);
