@@ -7,7 +7,8 @@
 // With hundreds of query rows per kv head the work is a real matrix product (each K/V row is
 // used by every query row behind it), so it goes to MFMA -- unlike the decode kernel, which
 // is a GEMV per sequence.  A work-group of four waves owns 64 consecutive query rows ((token,
-// head) pairs of one kv head), 16 per wave, and walks the pages 0..page(pos) together: each
+// head) pairs of one kv head), 16 per wave (eight waves and 128 rows where that pays, and on the quantised
+// pools), and walks the pages 0..page(pos) together: each
 // page's K and V rows are fetched from memory once per work-group into LDS (double-buffered,
 // the next page in flight while the current one is multiplied; fetching them per wave ran into
 // the L2's bandwidth), and every wave takes its operand fragments from there.  Per page of 16
@@ -43,6 +44,10 @@
 // Int8 pools (codes with an f16 scale per 32 values, K and V alike) are dequantised the same way,
 // without the exponent: both K and V become hi/lo image pairs, and the scores are
 // K_hi.q_hi + K_hi.q_lo + K_lo.q_hi.
+//
+// A walk is a serial chain.  Where the longest of a call would outlast the rest, walks are cut into ranges, a work-group
+// each, that leave partial results; prefill_merge_kernel puts them together.  Which calls, and the order of
+// dispatch: prefill_plan.hpp.
 #include <algorithm>
 #include <type_traits>
 

@@ -550,7 +550,7 @@ bkv_status bkv_attn_plan(int32_t n_cu, int32_t n_kv_head, int32_t n_q_head, int3
 typedef enum bkv_stage {
     BKV_STAGE_APPEND = 0,
     BKV_STAGE_ATTN_SPLIT = 1, /* split-K online-softmax kernel (the dominant one) */
-    BKV_STAGE_ATTN_MERGE = 2,
+    BKV_STAGE_ATTN_MERGE = 2, /* of decode's split-K ranges, and of the ranges of cut chunk walks */
     BKV_STAGE_PAGE_COPY = 3,
     BKV_STAGE_PREFILL_ATTN = 4, /* chunk attention (bkv_prefill_attn) */
     BKV_STAGE_APPEND_KPREP = 5, /* norm + rotary + append in one kernel */
