@@ -618,28 +618,27 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     };
     QRaw q_raw;
     request_q(P, e, kvh, wave, c, g, q_raw);
-    // STEP: the wave that will hold the page of cell pos (in its last step) takes the new rows before the
-    // loop, while its first units are on their way: the raw values are requested with its part of q, then lanes
-    // 0..7 encode the K row and lanes 8..15 the V row with the append kernel's encoder, one lane per 32-value
-    // block, into the pool and into two parking rows in LDS.  In its last step the wave copies a parked row
-    // into the unit that has just landed (an LDS move instead of a trip to memory and an encode at the end of
-    // the work-group's walk).  Encoded ahead of the trade of the q fragments: beside those, the raw values and
-    // the units in flight no longer fitted the registers (12 bytes of scratch a lane; 64 sequences of 512 to
-    // 4096 cells 36.3 us with it, 35.7 without).
-    const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
-    float new_x[32];
-    if constexpr (STEP) {
-        if (takes_new_row && lane < 16) {
-            const float* src = (lane < 8 ? P.new_k : P.new_v) + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + (lane & 7) * 32;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 a = *reinterpret_cast<const float4*>(src + 4 * j);
-                new_x[4 * j] = a.x, new_x[4 * j + 1] = a.y, new_x[4 * j + 2] = a.z, new_x[4 * j + 3] = a.w;
-            }
-        }
-    }
     __builtin_amdgcn_sched_barrier(0);
     if (SEL || n_steps > 0) fetch(0);  // a selection list's first units before its length is known
+
+    // STEP: the wave that will hold the page of cell pos (in its last step) takes the new rows before the
+    // loop, behind the request of its first units: lanes 0..31 encode the K row and lanes 32..63 the V row, 8
+    // values a lane as in the append kernel, into the pool and into two parking rows in LDS.  In its last step
+    // the wave copies a parked row into the unit that has just landed (an LDS move instead of a trip to memory
+    // and an encode at the end of the work-group's walk).  With 32 values in each of 16 lanes, encoded behind the
+    // trade of the q fragments, the encode was four times as long and the kernel spilled (12 bytes a lane): us a
+    // layer with the merge, one sequence of 4096 cells 12.3 -> 11.0, four short ones 12.5 -> 11.3, 64 of 512 to
+    // 4096 45.7 -> 43.9.
+    const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
+    float new_x[8];
+    if constexpr (STEP) {
+        if (takes_new_row) {
+            const float* src = (lane < 32 ? P.new_k : P.new_v) + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + (lane & 31) * 8;
+            const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+            new_x[0] = a.x, new_x[1] = a.y, new_x[2] = a.z, new_x[3] = a.w;
+            new_x[4] = b.x, new_x[5] = b.y, new_x[6] = b.z, new_x[7] = b.w;
+        }
+    }
 
     const auto wave_lds_fence = [&]() {
         // the wave's own LDS writes are in order with its later reads; keep the compiler from
@@ -650,19 +649,18 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     };
     if constexpr (STEP) {
         if (takes_new_row) {
-            if (lane < 16) {
-                uint32_t w[8], hb;
-                i8h_block_words(new_x, w, hb);
-                const int r = pos & (kPage - 1);
-                const int blk = lane & 7;
-                uint8_t* const pool_row = (lane < 8 ? P.kpool_w : P.vpool_w) + unit_off(n_steps - 1) + (size_t)r * kRow;
-                uint8_t* const rows[2] = {parked + (lane < 8 ? 0 : kRow), pool_row};
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    *reinterpret_cast<v4u*>(rows[t] + blk * 32) = v4u{w[0], w[1], w[2], w[3]};
-                    *reinterpret_cast<v4u*>(rows[t] + blk * 32 + 16) = v4u{w[4], w[5], w[6], w[7]};
-                    *reinterpret_cast<unsigned short*>(rows[t] + kHd + 2 * blk) = (unsigned short)hb;
-                }
+            const uint32_t hb = i8h_scale_bits(quad_max(amax8(new_x)));
+            uint32_t w0, w1;
+            i8h_codes8(new_x, f16_load(hb), w0, w1);
+            const int li = lane & 31;
+            const size_t at = unit_off(n_steps - 1) + (size_t)(pos & (kPage - 1)) * kRow;
+            uint8_t* const pool_row = (lane < 32 ? P.kpool_w : P.vpool_w) + at;
+            uint8_t* const park = parked + (lane < 32 ? 0 : kRow);
+            *reinterpret_cast<v2u*>(pool_row + li * 8) = v2u{w0, w1};
+            *reinterpret_cast<v2u*>(park + li * 8) = v2u{w0, w1};
+            if ((li & 3) == 0) {
+                *reinterpret_cast<unsigned short*>(pool_row + kHd + 2 * (li >> 2)) = (unsigned short)hb;
+                *reinterpret_cast<unsigned short*>(park + kHd + 2 * (li >> 2)) = (unsigned short)hb;
             }
             wave_lds_fence();
         }
@@ -853,7 +851,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 
     // every wave is done with its slot before the fold staging takes their place
     __syncthreads();
-    mfma_fold_and_store(P, *reinterpret_cast<MfmaFoldLds*>(ring), wg, wave, c, g, o, m_run, l_run);
+    // the lane's place from the hardware again: kept over the loop, it was one register too many
+    const int again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    mfma_fold_and_store(P, *reinterpret_cast<MfmaFoldLds*>(ring), wg, wave, again & 15, again >> 4, o, m_run, l_run);
 }
 
 // ---- decode attention on the matrix cores, f16 K and q8_0 V -----------------------------------

@@ -23,8 +23,8 @@ __device__ __forceinline__ float f16_load(uint32_t h) {
 
 // ---- the encoders' primitives, on 8 consecutive values of a 32-value block ----------------
 // The append kernels give a block to four neighbouring lanes (8 values each, so that a wave's
-// loads are contiguous); the attention kernels that take a new row in flight give it to one lane.
-// Both go through these functions, so both store the very same codes.
+// loads are contiguous), and so does the int8 attention kernel that takes a new row in flight; the q8_0 V one
+// gives it to one lane.  All go through these functions, so all store the very same codes.
 
 __device__ __forceinline__ float amax8(const float (&x)[8], float amax = 0.0f) {
 #pragma unroll
@@ -186,19 +186,6 @@ __device__ __forceinline__ void q8v_block_words(const float (&x)[32], uint32_t (
     w[0] = __float_as_uint(scale);
 #pragma unroll
     for (int j = 0; j < 8; ++j) w[1 + j] = c[j];
-}
-
-// One block of the int8 layout: w = 32 x i8, scale_bits = the binary16 code of the scale.
-__device__ __forceinline__ void i8h_block_words(const float (&x)[32], uint32_t (&w)[8], uint32_t& scale_bits) {
-    const uint32_t hb = i8h_scale_bits(amax32(x));
-    const float sh = f16_load(hb);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float y[8] = {x[8 * j], x[8 * j + 1], x[8 * j + 2], x[8 * j + 3],
-                            x[8 * j + 4], x[8 * j + 5], x[8 * j + 6], x[8 * j + 7]};
-        i8h_codes8(y, sh, w[2 * j], w[2 * j + 1]);
-    }
-    scale_bits = hb;
 }
 
 }  // namespace bkv
