@@ -188,7 +188,7 @@ def test_cut_chunks_after_their_streams_are_gone():
             for x in gone:
                 x.sync()
                 x.close()
-            for _ in range(300):  # some 0.1 ms each
+            for _ in range(500):  # some 0.1 ms each
                 long.run(busy)
             graph = Graph(capturing)
             captured.run(capturing)
