@@ -21,6 +21,10 @@ ARCH = "gfx950"
 # Packed-FP32 VALU forms are switched off for every kernel in this library.
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# The chunk attention kernel fills both halves of a wave's register file.  By default every matrix product of
+# such a kernel accumulates in the upper half, which the VALU cannot read; this option lets the register allocator
+# decide, product by product.
+FILE_FLAGS = {"prefill_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _hipcc() -> str:
@@ -47,8 +51,8 @@ def build(verbose: bool = False) -> str:
     objs = []
     for src in SOURCES:
         obj = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc] + HIP_FLAGS + ["-I", os.path.join(HERE, "..", "include"), "-c",
-                                     os.path.join(CSRC, src), "-o", obj]
+        cmd = [hipcc] + HIP_FLAGS + FILE_FLAGS.get(src, []) + ["-I", os.path.join(HERE, "..", "include"), "-c",
+                                                               os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd))
         _run(cmd)

@@ -6,13 +6,9 @@
 //
 // With hundreds of query rows per kv head the work is a real matrix product (each K/V row is
 // used by every query row behind it), so it goes to MFMA -- unlike the decode kernel, which
-// is a GEMV per sequence.  A work-group of four waves owns 64 consecutive query rows ((token,
-// head) pairs of one kv head), 16 per wave (eight waves and 128 rows where that pays, and on the quantised
-// pools), and walks the pages 0..page(pos) together: each
-// page's K and V rows are fetched from memory once per work-group into LDS (double-buffered,
-// the next page in flight while the current one is multiplied; fetching them per wave ran into
-// the L2's bandwidth), and every wave takes its operand fragments from there.  Per page of 16
-// cells and per wave:
+// is a GEMV per sequence.  A work-group of four waves owns 128 consecutive query rows ((token, head) pairs of one kv
+// head), two tiles of 16 a wave, and walks the pages 0..page(pos) together, two at a time.  (Small calls on f16 pools:
+// one tile a wave, 64 rows a work-group, two work-groups a compute unit.)  Per page of 16 cells and per tile:
 //   S^T[cell][query] = K[cell][:] . Q[query][:]        v_mfma_f32_16x16x32_f16, A = K, B = Q
 //   online softmax per query (base 2), P^T in the layout S^T came out in
 //   O^T[d][query]   += V^T[d][cell] . P^T[cell][query]  v_mfma_f32_16x16x32_f16 over the 32 cells of
@@ -22,19 +18,33 @@
 // Both products keep the per-lane query (lane % 16) fixed, so the softmax statistics never
 // move between lanes, and P^T feeds the second product straight from registers.  K and V are
 // exact f16; q and p are f32 values split into a high and a low f16 part (two MFMAs each), so the
-// products carry ~22 significant bits and the result stays at f32-accumulate accuracy.  Pages are
-// walked two at a time: one softmax update and one barrier per pair.
+// products carry ~22 significant bits and the result stays at f32-accumulate accuracy.
+//
+// What bounds it, and the split that follows.  Every fragment that a wave reads from LDS (1 KiB) meets the high and low
+// parts of each of its tiles.  With one tile a wave that is two products, and LDS has to deliver its 128 bytes a clock
+// for the matrix cores to be busy; two tiles halve it.  They need 256 registers for q and the accumulators, so a wave has
+// a SIMD (512 registers) to itself: q in the upper half of the register file, which only matrix products read, everything
+// else in the lower.  Nobody fills such a wave's gaps, hence
+// - a pair's scores are computed a step ahead of their softmax, whose instructions stand between those products;
+// - f16 pages go from memory to LDS without passing through registers (load_to_lds);
+// - every instruction counts, a wave issues one at a time (4 cycles): packed conversions, mixed-precision remainders, page
+//   addresses worked out lane by lane.
+// Against work-groups of eight waves with a tile each, whose steps were not pipelined: 4 chunks of 1024 behind 2048 cells,
+// 16 heads, f16, 334 -> 286 us; a prompt of 4096, 24 heads, q8_0 V, 650 -> 538; three ragged chunks, int8, 175 -> 160; 41
+// tokens behind 517 cells through 12 layers 274 -> 235.  A step takes 3120 cycles on f16 pools, 4930 with q8_0 V; its products
+// alone would take 2048 and 2560.  On f16 pools the clock falls to 2.0 GHz (1200 TFLOP/s issued; registers alone, no
+// loads, reach 1430 there): power is the next bound.  Tried and slower: all of a step as one block, the output a step
+// later (305 us f16); a third pair of pages in LDS (290, 582); chunks of one fragment fenced off from each other (299).
 // The V operand needs, per lane, four cells of one head-dim column of either page: a column of
 // the row-major page image.  gfx950's transposing LDS read (ds_read_b64_tr_b16) delivers exactly
 // that: within a group of 16 lanes, lane L receives element L % 4 of the 8-byte pieces that lanes
 // L / 4, 4 + L / 4, 8 + L / 4 and 12 + L / 4 addressed.  With lane (c, g) addressing row 4 g + c / 4,
 // halves 4 (c % 4) .. of a tile of 16 columns, lane c receives column c of the tile for cells
-// 4 g .. 4 g + 3: the MFMA operand, no regrouping on the VALU.  The V images have rows of 544
-// bytes (8 banks apart: the 64 lanes' 8-byte pieces of such a read tile the banks exactly).
+// 4 g .. 4 g + 3: the MFMA operand, no regrouping on the VALU.
 //
 // Pools with q8_0 V ([f32 scale][32 x i8] blocks, qsa_attn_apply_gqa.comp:53-77) take the same
-// walk with work-groups of eight waves: the threads that fetch a V page dequantise it once for
-// all eight, on its way into LDS, into two f16 images whose sum is the value to 22 bits
+// walk: the threads that fetch a V page dequantise it once for
+// all waves, on its way into LDS, into two f16 images whose sum is the value to 22 bits
 //   E[cell]    = exponent of the largest of the cell's 8 block scales (clamped to +-120),
 //   a[cell][d] = code * (scale * 2^-E[cell]) = hi + lo,
 // and the softmax runs over logit + E with weights exp2(logit + E - M), as in the decode kernel for
@@ -43,7 +53,7 @@
 // own: R is M until a sum comes near the end of f32's range, which rows of tiny V (E near -120) lead to.
 // Int8 pools (codes with an f16 scale per 32 values, K and V alike) are dequantised the same way,
 // without the exponent: both K and V become hi/lo image pairs, and the scores are
-// K_hi.q_hi + K_hi.q_lo + K_lo.q_hi.
+// K_hi.q_hi + K_hi.q_lo + K_lo.q_hi.  The dequantisation of the next pair stands between the P.V products of this one.
 //
 // A walk is a serial chain.  Where the longest of a call would outlast the rest, walks are cut into ranges, a work-group
 // each, that leave partial results; prefill_merge_kernel puts them together.  Which calls, and the order of
@@ -66,8 +76,11 @@ constexpr int kQ8vRow = kHd / 32 * 36;  // bytes of a q8_0 row
 constexpr int kI8hRow = kHd + kHd / 32 * 2;  // bytes of an int8 row: codes, then 8 f16 scales
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLoDown = 1.0f / 2048.0f;  // q's low parts enter the products times 2^11
-constexpr int kLdsRow = kHd + 8;    // halves per row of a K page image in LDS (528 bytes)
-constexpr int kLdsRowV = kHd + 16;  // of a V page image (544 bytes)
+// Two rows of a page image in LDS: 1024 bytes in one piece, as one load of a wave delivers them, and padding.  In the
+// second row neighbouring 16-byte chunks (V: 32-byte pairs of them) have changed places.  With the padding, the rows
+// that a read touches at a time then lie 16 (V: 32) bytes apart modulo the banks.
+constexpr int kLdsRowsK = 1024 + 32;
+constexpr int kLdsRowsV = 1024 + 64;
 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -75,6 +88,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef short tr_s4 __attribute__((__vector_size__(8)));  // what the transposing LDS read returns
 typedef __attribute__((address_space(3))) tr_s4* lds_tr_ptr;
+typedef const __attribute__((address_space(1))) uint8_t* page_ptr;  // said to be global memory: its address goes through integers
 
 struct PrefillKernelParams {
     PrefillBatch b;
@@ -117,57 +131,87 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
 
 // sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91)
 __device__ __forceinline__ float sigmoid(float x) {
-    if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-    const float ex = expf(x);
-    return ex / (1.0f + ex);
+    const float ex = expf(-fabsf(x));
+    const float d = 1.0f + ex;  // 1 .. 2: nothing of a general division's scaling is needed
+    float inv = __builtin_amdgcn_rcpf(d);
+    inv = __builtin_fmaf(__builtin_fmaf(-d, inv, 1.0f), inv, inv);
+    return (x >= 0.0f ? 1.0f : ex) * inv;
 }
 
-// What a thread carries of one page between its fetch and its deposit into LDS.
-template <int LAY>
-struct PageStage;
-template <>
-struct PageStage<BKV_LAYOUT_F16> {
-    v4u k[2], v[2];  // chunks tid (and, in a work-group of 256 threads, tid + 256) of either image
-    int pg;
-};
-// the quantised layouts: thread tid owns row tid / 32, block tid / 4 % 8, codes 8 (tid % 4) .. + 7 of it
-template <>
-struct PageStage<BKV_LAYOUT_Q8V> {
-    v4u k;                   // chunk tid of the f16 K image
-    unsigned scale, c0, c1;  // of V
-    int pg;
-};
-template <>
-struct PageStage<BKV_LAYOUT_I8H> {
-    unsigned kc0, kc1, vc0, vc1;
-    unsigned short kscale, vscale;
-    int pg;
+// two f32 numbers as f16, rounded to nearest
+__device__ __forceinline__ h2m to_f16(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    return __builtin_convertvector(f2{a, b}, h2m);
+}
+// x - (the f16 number hi): one v_fma_mix_f32 takes the f16 operand as it is (minus_one: -1.0f that the compiler
+// cannot see through, a plain subtraction would be preceded by a conversion)
+__device__ __forceinline__ float remainder_of(float x, _Float16 hi, float minus_one) {
+    return __builtin_fmaf((float)hi, minus_one, x);
+}
+// keeps a value where it is computed: between matrix products, not behind the branch that its use stands behind
+template <typename T>
+__device__ __forceinline__ void stay(T& x) {
+    asm volatile("" : "+v"(x));
+}
+// a maximum whose operands are known not to be signalling NaNs; fmaxf would quiet each of them first
+__device__ __forceinline__ float max_of(float a, float b) {
+    asm("v_max_f32 %0, %0, %1" : "+v"(a) : "v"(b));
+    return a;
+}
+
+// 16 bytes a lane straight into LDS: lane l's go to byte lds + 16 l.  Nothing but the vector-memory count says when they
+// have landed; each wave waits for its own ahead of the barrier that publishes them.
+__device__ __forceinline__ void load_to_lds(unsigned lds, page_ptr base, unsigned lane_off) {
+    // (the base came from a VALU instruction, which a vector-memory one must not follow closely: the copy is a scalar
+    // instruction, and the wait state that m0 wants)
+    uint64_t at;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+                 : "=&s"(at)
+                 : "s"(lds), "v"(lane_off), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// the maximum over the four lane groups; the swaps' neighbours and wait states stand in the same block
+__device__ __forceinline__ float max_over_groups(float x) {
+    float a = x, b = x;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0\n\tv_max_f32 %0, %0, %1" : "+v"(a), "+v"(b));
+    b = a;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0\n\tv_max_f32 %0, %0, %1" : "+v"(a), "+v"(b));
+    return a;
+}
+
+// What a thread carries of one pair of quantised pages between its fetch and its deposit into LDS: of row tid / 16,
+// block tid / 2 % 8, the codes of two 16-byte chunks of the f16 images.
+struct CodeStage {
+    uint2 c[2][2];      // [page][chunk]
+    unsigned scale[2];  // q8_0: the f32; int8 pools: the f16's bits
 };
 
 template <int LAY>
 struct PrefillLds {
-    // [buffer][image][16 rows][halves]: K (int8 pools: K high parts, K low parts) and V (quantised
+    // [pair of pages][page][image][pair of rows][...]: K (int8 pools: K high parts, K low parts) and V (quantised
     // pools: V high parts, V low parts)
-    _Float16 kimg[4][LAY == BKV_LAYOUT_I8H ? 2 : 1][kPage][kLdsRow];
-    _Float16 vimg[4][LAY == BKV_LAYOUT_F16 ? 1 : 2][kPage][kLdsRowV];
-    float e[LAY == BKV_LAYOUT_Q8V ? 4 : 1][kPage];  // q8_0 V: E of the buffer's cells
+    uint8_t kimg[2][2][LAY == BKV_LAYOUT_I8H ? 2 : 1][kPage / 2][kLdsRowsK];
+    uint8_t vimg[2][2][LAY == BKV_LAYOUT_F16 ? 1 : 2][kPage / 2][kLdsRowsV];
+    float e[LAY == BKV_LAYOUT_Q8V ? 2 : 1][2][kPage];  // q8_0 V: E of the cells
 };
+// byte of 16-byte chunk `chunk` of row `row` in a page image
+__device__ __forceinline__ int k_at(int row, int chunk) { return (row >> 1) * kLdsRowsK + (row & 1) * 512 + (chunk ^ (row & 1)) * 16; }
+__device__ __forceinline__ int v_at(int row, int chunk) { return (row >> 1) * kLdsRowsV + (row & 1) * 512 + (chunk ^ 2 * (row & 1)) * 16; }
 
-// WAVES: waves of a work-group, 16 query rows each.  Eight share every page image they put into LDS
-// among 128 rows (one work-group per compute unit); four (f16 pools only, two work-groups per
-// compute unit) spread a small chunk over twice as many compute units.
+// TILES: tiles of 16 query rows a wave owns.
 // SPLIT: a work-group walks one range of its block's pages and leaves a partial result.
-template <int LAY, int WAVES = 8, bool SPLIT = false>
-__global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
+template <int LAY, int TILES, bool SPLIT = false>
+__global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams> P) {
-    static_assert(WAVES == 8 || (WAVES == 4 && LAY == BKV_LAYOUT_F16), "the quantised images are dequantised by 512 threads");
     constexpr bool Q8V = LAY == BKV_LAYOUT_Q8V;
     constexpr bool I8H = LAY == BKV_LAYOUT_I8H;
     constexpr bool WIDE = LAY != BKV_LAYOUT_F16;  // V (int8 pools: K too) as two f16 images
-    constexpr int kWavesPerWg = WAVES;
-    constexpr int kThreads = 64 * kWavesPerWg;
-    constexpr int kRowsPerWg = kRowsPerWave * kWavesPerWg;
-    // ---- which (entry, kv head, block of 64 query rows) ---------------------------------
+    constexpr int kWavesPerWg = 4;
+    constexpr int kRows = kRowsPerWave * TILES;
+    constexpr int kRowsPerWg = kRows * kWavesPerWg;
+    // ---- which (entry, kv head, block of query rows) ---------------------------------
     int e = 0, kvh, idx;  // idx: which of the unit's blocks, in dispatch order
     int range = 0;       // which range of the block's pages
     bool cut = false;    // the block is cut at all
@@ -222,24 +266,10 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
     const int lane = threadIdx.x & 63;
     const int c = lane & 15;  // query row of the tile / cell of the page / output column group
     const int g = lane >> 4;  // which quarter of the contraction index this lane feeds
-    const int row0 = rb * kRowsPerWg + wave * kRowsPerWave;
+    const int row0 = rb * kRowsPerWg + wave * kRows;
     // a wave whose rows lie past the end still helps to fetch pages and joins the barriers
     const bool wave_live = row0 < n_rows;
 
-    // this lane's query row
-    const int row = row0 + c;
-    const bool row_live = wave_live && row < n_rows;
-    const int tok = row_live ? row / P.group : 0;
-    const int head = kvh * P.group + (row_live ? row % P.group : 0);
-    // a lane without a query row (past the end of the chunk) walks along with q = 0 and every cell
-    // live: its column of the products is its own, and nothing of it is stored
-    const int pos_q = row_live ? P.b.pos0[e] + tok : 0x7fffffff;
-    // the first position any row of this wave has: pages wholly at or below it need no causal mask
-    const int pos_min = P.b.pos0[e] + (wave_live ? row0 / P.group : 0);
-    // the last token any row of this wave belongs to bounds the page walk
-    const int last_row = min(row0 + kRowsPerWave, n_rows) - 1;
-    const int pos_max = wave_live ? P.b.pos0[e] + last_row / P.group : -1;
-    int n_pages = wave_live ? pos_max / kPage + 1 : 0;
     // pages the work-group walks: those of its last row
     const int wg_last_row = min(rb * kRowsPerWg + kRowsPerWg, n_rows) - 1;
     const int wg_pos_max = P.b.pos0[e] + wg_last_row / P.group;
@@ -252,12 +282,24 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
             if (range >= ranges) return;  // the entry's longest block has more
             first_pg = range * each;
             wg_pages = min(wg_pages, first_pg + each);
-            n_pages = min(n_pages, wg_pages);
         }
     }
+    // this lane's query rows, and the last cell each of them attends here
+    int tok[TILES], head[TILES], last_cell[TILES];
+    bool row_live[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const int row = row0 + t * kRowsPerWave + c;
+        row_live[t] = row < n_rows;
+        tok[t] = row_live[t] ? row / P.group : 0;
+        head[t] = kvh * P.group + (row_live[t] ? row % P.group : 0);
+        // a lane without a query row (past the end of the chunk) walks along with q = 0: its column of
+        // the products is its own, and nothing of it is stored
+        last_cell[t] = min(row_live[t] ? P.b.pos0[e] + tok[t] : 0x7fffffff, wg_pages * kPage - 1);
+    }
+    // the last cell that every row of this wave attends: pages wholly at or below it need no mask
+    const int all_live = min(P.b.pos0[e] + (wave_live ? row0 / P.group : 0), wg_pages * kPage - 1);
 
-    typedef const __attribute__((address_space(4))) int32_t* table_ptr;
-    const table_ptr bt = (table_ptr)(uintptr_t)(P.tables + (size_t)P.b.row[e] * (size_t)P.max_pages_per_seq);
     constexpr int kKRow = I8H ? kI8hRow : kHd * 2;  // bytes of a row in the K pool and in the V pool
     constexpr int kVRow = I8H ? kI8hRow : Q8V ? kQ8vRow : kHd * 2;
     const size_t page_bytes = (size_t)P.n_kv * kPage * kKRow;
@@ -265,22 +307,202 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
     const size_t v_page_bytes = (size_t)P.n_kv * kPage * kVRow;
     const size_t v_head_off = (size_t)kvh * kPage * kVRow;
 
-    // ---- q fragments: lane (c, g) holds q[row][32 m + 8 g + 0..7], m = 0..7, as hi + lo f16 ----
-    h8 qhi[8], qlo[8];
-    {
-        const float* qp = P.q + ((size_t)(P.b.src0[e] + tok) * P.n_q + head) * kHd + g * 8;
+    // ---- requests of the prologue ----------------------------------------------------------------
+    __shared__ __attribute__((aligned(16))) PrefillLds<LAY> L;
+    const int tid = threadIdx.x;
+    const int last_pg = wg_pages - 1;
+    // The table's entries come through the vector path (lane parity picks the page of a pair, past the end the last page
+    // again): a scalar load among LDS reads would have to be waited for together with all of them.
+    const int32_t* table = P.tables + (size_t)P.b.row[e] * (size_t)P.max_pages_per_seq;
+    const auto table_pair = [&](int pg) { return table[min(pg + (lane & 1), last_pg)]; };
+    const int ids_0 = table_pair(first_pg);
+    int ids_v = table_pair(first_pg + 2), ids_k = table_pair(first_pg + 4);  // the pairs whose V and K are asked for next
+    // addresses of a pair's pages, lane by lane as the entries came; pages are then picked from them
+    const auto k_pages = [&](int ids) { return (uint64_t)(uintptr_t)(P.kpool + head_off) + (uint64_t)(unsigned)ids * (unsigned)page_bytes; };
+    const auto v_pages = [&](int ids) { return (uint64_t)(uintptr_t)(P.vpool + v_head_off) + (uint64_t)(unsigned)ids * (unsigned)v_page_bytes; };
+    const auto page_of = [](uint64_t pages, int w) {
+        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)pages, w);
+        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(pages >> 32), w);
+        return (page_ptr)((uint64_t)hi << 32 | lo);
+    };
+
+    // q: lane (c, g) holds q[row][32 m + 8 g + 0..7], m = 0..7.  All of the row is requested at once (a lane without a row
+    // reads the chunk's first one and drops it): behind a branch a fragment, each was waited for before the next was
+    // asked for, a trip to memory each.
+    f4 raw[TILES][16];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const float* qp = P.q + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd + g * 8;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
+    }
+
+    // ---- pages into LDS --------------------------------------------------------------------------
+    // f16 rows go there by themselves: wave w moves rows 4 w .. 4 w + 3 of a page, two rows a load; lane l delivers
+    // chunk l % 32 of the image's row, which is chunk l % 32 or its neighbour of the page's row.
+    const unsigned k_lane = (unsigned)(wave * 2048 + (lane >> 5) * 512 + (((lane & 31) ^ (lane >> 5)) << 4));
+    const unsigned v_lane = (unsigned)(wave * 2048 + (lane >> 5) * 512 + (((lane & 31) ^ (2 * (lane >> 5))) << 4));
+    const auto lds_of = [](const uint8_t* p) { return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p; };
+    const auto load_k = [&](int buf, page_ptr page, int w, int n) {
+        load_to_lds(lds_of(&L.kimg[buf][w][0][2 * wave + n][0]), page, k_lane + n * 1024);
+    };
+    const auto load_v = [&](int buf, page_ptr page, int w, int n) {
+        load_to_lds(lds_of(&L.vimg[buf][w][0][2 * wave + n][0]), page, v_lane + n * 1024);
+    };
+    // Quantised rows travel through registers and become high and low parts on the way.  Of its block's four chunks a
+    // thread takes every other one, blocks 2, 3, 6 and 7 in the other order: eight neighbouring lanes then write eight
+    // chunks that differ modulo the banks.
+    const int c_row = tid >> 4, c_blk = (tid >> 1) & 7;
+    const int c_chunk[2] = {4 * c_blk + (tid & 1) + (c_blk & 2), 4 * c_blk + (tid & 1) + ((c_blk & 2) ^ 2)};
+    const auto fetch_codes = [&](page_ptr page, bool q8, CodeStage& st, int w) {
+        const unsigned row = c_row * (q8 ? kQ8vRow : kI8hRow);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const unsigned at = q8 ? row + c_blk * 36 + 4 + (c_chunk[h] & 3) * 8 : row + c_chunk[h] * 8;
+            st.c[w][h].x = *(const __attribute__((address_space(1))) unsigned*)(page + at);
+            st.c[w][h].y = *(const __attribute__((address_space(1))) unsigned*)(page + (at + 4));
+        }
+        if (q8) st.scale[w] = *(const __attribute__((address_space(1))) unsigned*)(page + (row + c_blk * 36));
+        else st.scale[w] = *(const __attribute__((address_space(1))) unsigned short*)(page + (row + kHd + c_blk * 2));
+    };
+    const auto eight = [](const h2m (&x)[4]) {
+        return h8{x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
+    };
+    // code * scale (7 + 11 significant bits) as hi = f16(code * scale) and the exact remainder (times `up`).  A scale
+    // with exponent field 0 reads as zero, as everywhere.
+    const auto i8h_scale = [](unsigned bits) {
+        return __builtin_bit_cast(_Float16, (unsigned short)((bits & 0x7c00u) == 0 ? 0u : bits));
+    };
+    const auto half_of = [&](unsigned codes, h2m s_hi, h2m s_lo, h2m* hi, h2m* lo) {
+        h2m cd[2];
+        codes_to_f16(codes, cd[0], cd[1]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if constexpr (Q8V) {
+                scaled_hi_lo(cd[i], s_hi, s_lo, hi[i], lo[i]);
+            } else {
+                hi[i] = cd[i] * s_hi;
+                lo[i] = __builtin_elementwise_fma(cd[i], s_hi, -hi[i]);
+            }
+        }
+    };
+    // The deposit of a page in seven parts, which go between matrix products: the scale, then four codes at a time and the
+    // stores of either chunk.
+    h2m put_sh, put_sl, put_hi[4], put_lo[4];
+    const auto store_parts = [&](uint8_t* to_hi, uint8_t* to_lo, int at) {
+        *reinterpret_cast<h8*>(to_hi + at) = eight(put_hi);
+        *reinterpret_cast<h8*>(to_lo + at) = eight(put_lo);
+    };
+    // the low parts of K times 2^11, like those of q: their products with q's high parts join those of q's low parts
+    const auto deposit_k_part = [&](int buf, const CodeStage& st, int w, int part) {
+        if (part == 0) {
+            const _Float16 scale = i8h_scale(st.scale[w]);
+            put_sh = h2m{scale, scale};
+        } else if (part % 3 != 0) {
+            const int h = part / 4, k = (part - 1) % 3;
+            half_of(k ? st.c[w][h].y : st.c[w][h].x, put_sh, put_sl, put_hi + 2 * k, put_lo + 2 * k);
+#pragma unroll
+            for (int i = 2 * k; i < 2 * k + 2; ++i) put_lo[i] *= h2m{(_Float16)2048.0f, (_Float16)2048.0f};
+        } else {
+            store_parts(&L.kimg[buf][w][0][0][0], &L.kimg[buf][w][I8H ? 1 : 0][0][0], k_at(c_row, c_chunk[part / 3 - 1]));
+        }
+    };
+    const auto deposit_v_part = [&](int buf, const CodeStage& st, int w, int part) {
+        if (part == 0) {
+            if constexpr (I8H) {
+                const _Float16 scale = i8h_scale(st.scale[w]);
+                put_sh = h2m{scale, scale};
+            } else {
+                // the largest scale of the row: over the lanes that differ in the block bits (1..3).  (Scales are not
+                // negative: as integers their order is the same, and a NaN among foreign bytes is a large number.)
+                int top = (int)(st.scale[w] & 0x7fffffffu);
+                top = max(top, __builtin_amdgcn_update_dpp(0, top, 0x122, 0xf, 0xf, false));  // row_ror:2
+                top = max(top, __builtin_amdgcn_update_dpp(0, top, 0x124, 0xf, 0xf, false));  // row_ror:4
+                top = max(top, __builtin_amdgcn_update_dpp(0, top, 0x128, 0xf, 0xf, false));  // row_ror:8
+                const int ee = min(max((top >> 23) - 127, -120), 120);
+                _Float16 s_hi, s_lo;
+                split_f16(__builtin_ldexpf(__builtin_bit_cast(float, st.scale[w]), -ee), s_hi, s_lo);
+                put_sh = h2m{s_hi, s_hi}, put_sl = h2m{s_lo, s_lo};
+                L.e[buf][w][c_row] = (float)ee;  // the same number from sixteen lanes
+            }
+        } else if (part % 3 != 0) {
+            const int h = part / 4, k = (part - 1) % 3;
+            half_of(k ? st.c[w][h].y : st.c[w][h].x, put_sh, put_sl, put_hi + 2 * k, put_lo + 2 * k);
+        } else {
+            store_parts(&L.vimg[buf][w][0][0][0], &L.vimg[buf][w][WIDE ? 1 : 0][0][0], v_at(c_row, c_chunk[part / 3 - 1]));
+        }
+    };
+    constexpr int kPutParts = 7;
+    const auto deposit_k = [&](int buf, const CodeStage& st, int w) {
+#pragma unroll
+        for (int part = 0; part < kPutParts; ++part) deposit_k_part(buf, st, w, part);
+    };
+    const auto deposit_v = [&](int buf, const CodeStage& st, int w) {
+#pragma unroll
+        for (int part = 0; part < kPutParts; ++part) deposit_v_part(buf, st, w, part);
+    };
+    // Rows of V past the work-group's last position were never written for these queries and may hold anything (even
+    // NaN): exact zeros, before they meet a zero probability.  Each wave clears what it has put there itself; only the
+    // last pair has such rows.
+    const auto clear_dead_v = [&](int buf, int pg) {
+        if ((pg + 2) * kPage - 1 <= wg_pos_max) return;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const int first = min(pg + w, last_pg) * kPage;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                // f16: rows 4 w .. 4 w + 3, as loaded; quantised: two chunks, as deposited
+                const int row = WIDE ? c_row : 4 * wave + 2 * j + (lane >> 5);
+                const int at = v_at(row, WIDE ? c_chunk[j] : lane & 31);
+                if (first + row > wg_pos_max) {
+#pragma unroll
+                    for (int img = 0; img < (WIDE ? 2 : 1); ++img) *reinterpret_cast<v4u*>(&L.vimg[buf][w][img][0][0] + at) = v4u{0u, 0u, 0u, 0u};
+                }
+            }
+        }
+    };
+
+    CodeStage stage_k, stage_v;
+    // the first two pairs of K and the first of V; the next of either (quantised rows) in registers
+    const auto load_pair_k = [&](int buf, int ids) {
+        const uint64_t at = k_pages(ids);
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const page_ptr page = page_of(at, w);
+            if constexpr (I8H) {
+                fetch_codes(page, false, stage_k, w);
+            } else {
+                load_k(buf, page, w, 0);
+                load_k(buf, page, w, 1);
+            }
+        }
+    };
+    const auto load_pair_v = [&](int buf, int ids) {
+        const uint64_t at = v_pages(ids);
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const page_ptr page = page_of(at, w);
+            if constexpr (WIDE) {
+                fetch_codes(page, Q8V, stage_v, w);
+            } else {
+                load_v(buf, page, w, 0);
+                load_v(buf, page, w, 1);
+            }
+        }
+    };
+    load_pair_k(0, ids_0);
+    load_pair_v(0, ids_0);
+    if constexpr (!I8H) load_pair_k(1, ids_v);
+
+    // ---- q as hi + lo f16 --------------------------------------------------------------------------
+    float minus_one = -1.0f;
+    asm("" : "+v"(minus_one));
+    h8 qhi[TILES][8], qlo[TILES][8];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const float by = row_live[t] ? P.scale_log2e : 0.0f;
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
-            float x[8];
-            if (row_live) {
-                const float4 a = *reinterpret_cast<const float4*>(qp + m * 32);
-                const float4 b = *reinterpret_cast<const float4*>(qp + m * 32 + 4);
-                x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
-                x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) x[j] = 0.0f;
-            }
             // The softmax scale (and the change to base 2) rides on q: one rounding of q, 2^-24
             // relative.  The low parts are kept times 2^11 and their products scaled back in f32
             // (kLoDown), which keeps them out of the f16 subnormals' few bits.  The product is
@@ -289,373 +511,360 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void prefill_attn_kernel(
             // f32, then to f16) -- two numbers that differ by an f16 ulp now and then, which showed as
             // 3e-5 in short contexts.
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                float xs = x[j] * P.scale_log2e;
-                asm("" : "+v"(xs));  // the product as one f32 number: no fusing into the conversions below
-                const _Float16 hi = (_Float16)xs;
-                qhi[m][j] = hi;
-                qlo[m][j] = (_Float16)((xs - (float)hi) * 2048.0f);
+            for (int j = 0; j < 8; j += 2) {
+                float a = raw[t][2 * m + (j >> 2)][j & 3], b = raw[t][2 * m + (j >> 2)][(j & 3) + 1];
+                a = row_live[t] ? a * by : 0.0f;
+                b = row_live[t] ? b * by : 0.0f;
+                asm("" : "+v"(a), "+v"(b));  // the products as f32 numbers: no fusing into the conversions below
+                const h2m hi = to_f16(a, b);
+                const h2m lo = to_f16(remainder_of(a, hi[0], minus_one) * 2048.0f, remainder_of(b, hi[1], minus_one) * 2048.0f);
+                qhi[t][m][j] = hi[0], qhi[t][m][j + 1] = hi[1];
+                qlo[t][m][j] = lo[0], qlo[t][m][j + 1] = lo[1];
             }
         }
     }
 
-    // O^T accumulators: o[tile][r] = out[row][16 tile + 4 g + r]
-    f4 o[16];
+    // O^T accumulators: o[tile][column tile][r] = out[row][16 (column tile) + 4 g + r]
+    f4 o[TILES][16];
 #pragma unroll
-    for (int t = 0; t < 16; ++t) o[t] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = -INFINITY;  // running max of this lane's query (base-2 logits), same in all 4 g lanes
-    float l_run = 0.0f;       // this lane's share (its 4 cells per page) of the denominator
+    for (int t = 0; t < TILES; ++t)
+#pragma unroll
+        for (int d = 0; d < 16; ++d) o[t][d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run[TILES];  // running max of the lane's query (base-2 logits), same in all 4 g lanes
+    float l_run[TILES];  // this lane's share (its 4 cells per page) of the denominator
     // q8_0 V: what l_run is relative to.  Against M its terms reach 2^(120 + kSlack) on rows of tiny V
     // (E = -120), and a few of them overflow f32; so the denominator has a reference of its own, at or
-    // above M.  It leaves M when a lane's sum passes kMostL, and M meets it again from below.  Checked beside
-    // the branch that rescales the accumulators: the 4096-token prompt of the q8_0 V cache went from 640.8
-    // to 642.9 us with it (649 with a branch of its own).
-    float l_ref = -INFINITY;
+    // above M.  It leaves M when a lane's sum passes kMostL, and M meets it again from below.
+    float l_ref[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) m_run[t] = l_ref[t] = -INFINITY, l_run[t] = 0.0f;
     constexpr float kMostL = 0x1p100f;
 
-    // ---- pages through LDS -----------------------------------------------------------------------
-    // Rows are padded to 528 bytes so that the 16-byte fragment reads of the 64 lanes spread
-    // evenly over the banks.  An f16 page image is 512 chunks of 16 bytes: thread t moves chunk
-    // t (+ 256) of it.  Pages are taken two at a time (one softmax update, one
-    // barrier and P.V MFMAs that contract over the 32 cells of the pair): four buffers, the pair
-    // being multiplied and the pair being filled.
-    __shared__ __attribute__((aligned(16))) PrefillLds<LAY> L;
-    const int tid = threadIdx.x;
-    // quantised layouts: this thread's part of a page
-    const int v_row = tid >> 5, v_blk = (tid >> 2) & 7, v_j = tid & 3;
-    const auto fetch = [&](int pg, PageStage<LAY>& st) {
-        const int32_t phys = bt[pg];
-        const uint8_t* kp = P.kpool + (size_t)phys * page_bytes + head_off;
-        const uint8_t* vp = P.vpool + (size_t)phys * v_page_bytes + v_head_off;
-        if constexpr (Q8V) {
-            st.k = *reinterpret_cast<const v4u*>(kp + (size_t)tid * 16);
-            const uint8_t* blk = vp + v_row * kQ8vRow + v_blk * 36;
-            st.scale = *reinterpret_cast<const unsigned*>(blk);
-            st.c0 = *reinterpret_cast<const unsigned*>(blk + 4 + v_j * 8);
-            st.c1 = *reinterpret_cast<const unsigned*>(blk + 8 + v_j * 8);
-            st.pg = pg;
-        } else if constexpr (I8H) {
-            const uint8_t* kr = kp + v_row * kI8hRow;
-            const uint8_t* vr = vp + v_row * kI8hRow;
-            st.kc0 = *reinterpret_cast<const unsigned*>(kr + v_blk * 32 + v_j * 8);
-            st.kc1 = *reinterpret_cast<const unsigned*>(kr + v_blk * 32 + v_j * 8 + 4);
-            st.vc0 = *reinterpret_cast<const unsigned*>(vr + v_blk * 32 + v_j * 8);
-            st.vc1 = *reinterpret_cast<const unsigned*>(vr + v_blk * 32 + v_j * 8 + 4);
-            st.kscale = *reinterpret_cast<const unsigned short*>(kr + kHd + v_blk * 2);
-            st.vscale = *reinterpret_cast<const unsigned short*>(vr + kHd + v_blk * 2);
-            st.pg = pg;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 512 / kThreads; ++j) {
-                st.k[j] = *reinterpret_cast<const v4u*>(kp + (size_t)(tid + j * kThreads) * 16);
-                st.v[j] = *reinterpret_cast<const v4u*>(vp + (size_t)(tid + j * kThreads) * 16);
-            }
-            st.pg = pg;
-        }
-    };
-    const auto deposit = [&](int buf, const PageStage<LAY>& st) {
-        // chunk q of a page image: row q / 32, halves (q % 32) * 8 ..
-        if constexpr (Q8V) {
-            *reinterpret_cast<v4u*>(&L.kimg[buf][0][tid >> 5][(tid & 31) * 8]) = st.k;
-            // Rows past the work-group's last position were never written for these queries and
-            // may hold anything: scale 1 for the row's exponent, zeros for its values.
-            const bool dead = st.pg * kPage + v_row > wg_pos_max;
-            const float sc = __builtin_bit_cast(float, st.scale);
-            // the largest scale of the row: over the lanes that differ in the block bits (2..4)
-            float smax = dead ? 1.0f : sc;
-            smax = fmaxf(smax, dpp_mov<0x124>(smax));  // row_ror:4
-            smax = fmaxf(smax, dpp_mov<0x128>(smax));  // row_ror:8
-            {
-                const LanePair o = swap_rows(smax);
-                smax = fmaxf(o.a, o.b);
-            }
-            int ee = (int)((__builtin_bit_cast(unsigned, smax) >> 23) & 0xffu) - 127;
-            ee = min(max(ee, -120), 120);
-            const float down = __builtin_bit_cast(float, (unsigned)(127 - ee) << 23);  // 2^-E
-            _Float16 s_hi, s_lo;
-            split_f16(dead ? 0.0f : sc * down, s_hi, s_lo);
-            const h2m sh = h2m{s_hi, s_hi}, sl = h2m{s_lo, s_lo};
-            h2m cd[4], hi[4], lo[4];
-            codes_to_f16(st.c0, cd[0], cd[1]);
-            codes_to_f16(st.c1, cd[2], cd[3]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) scaled_hi_lo(cd[i], sh, sl, hi[i], lo[i]);
-            const h8 vh = h8{hi[0][0], hi[0][1], hi[1][0], hi[1][1], hi[2][0], hi[2][1], hi[3][0], hi[3][1]};
-            const h8 vl = h8{lo[0][0], lo[0][1], lo[1][0], lo[1][1], lo[2][0], lo[2][1], lo[3][0], lo[3][1]};
-            *reinterpret_cast<h8*>(&L.vimg[buf][0][v_row][v_blk * 32 + v_j * 8]) = vh;
-            *reinterpret_cast<h8*>(&L.vimg[buf][1][v_row][v_blk * 32 + v_j * 8]) = vl;
-            if ((tid & 31) == 0) L.e[buf][v_row] = (float)ee;
-        } else if constexpr (I8H) {
-            // K: code * scale (7 + 11 significant bits) as hi = f16(code * scale) and the exact
-            // remainder, like V below.  A scale with exponent field 0 reads as zero, as everywhere.
-            {
-                const unsigned short ks = (st.kscale & 0x7c00u) == 0 ? (unsigned short)0 : st.kscale;
-                const _Float16 ksc = __builtin_bit_cast(_Float16, ks);
-                const h2m sh = h2m{ksc, ksc}, sl = h2m{(_Float16)0.0f, (_Float16)0.0f};
-                h2m kd[4], hi[4], lo[4];
-                codes_to_f16(st.kc0, kd[0], kd[1]);
-                codes_to_f16(st.kc1, kd[2], kd[3]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) scaled_hi_lo(kd[i], sh, sl, hi[i], lo[i]);
-                *reinterpret_cast<h8*>(&L.kimg[buf][0][v_row][v_blk * 32 + v_j * 8]) =
-                    h8{hi[0][0], hi[0][1], hi[1][0], hi[1][1], hi[2][0], hi[2][1], hi[3][0], hi[3][1]};
-                *reinterpret_cast<h8*>(&L.kimg[buf][1][v_row][v_blk * 32 + v_j * 8]) =
-                    h8{lo[0][0], lo[0][1], lo[1][0], lo[1][1], lo[2][0], lo[2][1], lo[3][0], lo[3][1]};
-            }
-            // V: code * scale (7 + 11 significant bits) as hi = f16(code * scale) and the exact
-            // remainder; rows past the work-group's last position become zeros
-            const bool dead = st.pg * kPage + v_row > wg_pos_max;
-            const unsigned short vs = (dead || (st.vscale & 0x7c00u) == 0) ? (unsigned short)0 : st.vscale;
-            const _Float16 vsc = __builtin_bit_cast(_Float16, vs);
-            const h2m sh = h2m{vsc, vsc}, sl = h2m{(_Float16)0.0f, (_Float16)0.0f};
-            h2m cd[4], hi[4], lo[4];
-            codes_to_f16(st.vc0, cd[0], cd[1]);
-            codes_to_f16(st.vc1, cd[2], cd[3]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) scaled_hi_lo(cd[i], sh, sl, hi[i], lo[i]);
-            *reinterpret_cast<h8*>(&L.vimg[buf][0][v_row][v_blk * 32 + v_j * 8]) =
-                h8{hi[0][0], hi[0][1], hi[1][0], hi[1][1], hi[2][0], hi[2][1], hi[3][0], hi[3][1]};
-            *reinterpret_cast<h8*>(&L.vimg[buf][1][v_row][v_blk * 32 + v_j * 8]) =
-                h8{lo[0][0], lo[0][1], lo[1][0], lo[1][1], lo[2][0], lo[2][1], lo[3][0], lo[3][1]};
-        } else {
-            // V rows past the work-group's last position were never written for these queries and may
-            // hold anything (even NaN): exact zeros, before they meet a zero probability.  Only the
-            // work-group's last page has such rows.
-            const bool last_page = st.pg * kPage + kPage - 1 > wg_pos_max;
-#pragma unroll
-            for (int j = 0; j < 512 / kThreads; ++j) {
-                const int q = tid + j * kThreads;
-                v4u vv = st.v[j];
-                if (last_page && st.pg * kPage + (q >> 5) > wg_pos_max) vv = v4u{0u, 0u, 0u, 0u};
-                *reinterpret_cast<v4u*>(&L.kimg[buf][0][q >> 5][(q & 31) * 8]) = st.k[j];
-                *reinterpret_cast<v4u*>(&L.vimg[buf][0][q >> 5][(q & 31) * 8]) = vv;
-            }
-        }
-    };
+    // this lane's piece of a transposing V read: row 4 g + c / 4, halves 4 (c % 4) .. of a 16-column tile.  In odd rows
+    // the even tiles have changed places with the odd ones.
+    const int v_row = 4 * g + (c >> 2);
+    const int v_piece = v_at(v_row, 0) + 8 * (c & 3), v_odd = 32 - 64 * (v_row & 1);
+    const int k_piece = k_at(c, g);
 
-    // this lane's piece of a transposing V read: row 4 g + c / 4, halves 4 (c % 4) .. of a 16-column tile
-    const int tr_off = (4 * g + (c >> 2)) * kLdsRowV + 4 * (c & 3);
-    // scores of one page in base 2: s[r] = scale * log2(e) * q[row c] . k[cell 4 g + r], unmasked
-    const auto scores = [&](int buf) -> f4 {
-        const _Float16* ks = &L.kimg[buf][0][0][0];
-        // K: row c, 16 bytes at element 32 m + 8 g (the same split of the head dim as q): the 8
-        // halves of a lane are the 8 contraction steps it feeds to the 32-deep MFMA
-        h8 kf[8];
+    // scores of a pair of pages in base 2, unmasked: [tile][page][r] of cell 4 g + r, in two parts (q's high and q's
+    // low parts)
+    f4 s_hi[TILES][2], s_lo[TILES][2];
+    // chunk i: fragment m = i % 8 of page i / 8.  K: row c, 16 bytes at element 32 m + 8 g (the same split of the head
+    // dim as q): the 8 halves of a lane are the 8 contraction steps it feeds to the 32-deep MFMA
+    h8 kf[16], kl[I8H ? 16 : 1];
+    const auto read_k = [&](int buf, int i) {
+        kf[i] = *reinterpret_cast<const h8*>(&L.kimg[buf][i >> 3][0][0][0] + k_piece + (i & 7) * 64);
+        if constexpr (I8H) kl[i] = *reinterpret_cast<const h8*>(&L.kimg[buf][i >> 3][1][0][0] + k_piece + (i & 7) * 64);
+    };
+    const auto multiply_k = [&](int i) {
+        const f4 zero = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        const int w = i >> 3, m = i & 7;
 #pragma unroll
-        for (int m = 0; m < 8; ++m) kf[m] = *reinterpret_cast<const h8*>(ks + c * kLdsRow + m * 32 + g * 8);
+        for (int t = 0; t < TILES; ++t) s_hi[t][w] = mfma32(kf[i], qhi[t][m], m ? s_hi[t][w] : zero);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) s_lo[t][w] = mfma32(kf[i], qlo[t][m], m ? s_lo[t][w] : zero);
         if constexpr (I8H) {
-            // K = hi + lo: hi meets q's high and low parts, lo q's high parts; three chains
-            const _Float16* kl = &L.kimg[buf][1][0][0];
-            f4 s0 = f4{0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0, s2 = s0;
 #pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                const h8 klo = *reinterpret_cast<const h8*>(kl + c * kLdsRow + m * 32 + g * 8);
-                s0 = mfma32(kf[m], qhi[m], s0);
-                s1 = mfma32(kf[m], qlo[m], s1);
-                s2 = mfma32(klo, qhi[m], s2);
-            }
-            return (s0 + s2) + s1 * kLoDown;
-        } else {
-            // two accumulation chains, q's high parts and q's low parts: an MFMA adds to the sum of the
-            // one before the last, which has left the pipeline by then
-            f4 s0 = f4{0.0f, 0.0f, 0.0f, 0.0f}, s1 = s0;
-#pragma unroll
-            for (int m = 0; m < 8; ++m) {
-                s0 = mfma32(kf[m], qhi[m], s0);
-                s1 = mfma32(kf[m], qlo[m], s1);
-            }
-            return s0 + s1 * kLoDown;
+            for (int t = 0; t < TILES; ++t) s_lo[t][w] = mfma32(kl[i], qhi[t][m], s_lo[t][w]);
         }
     };
 
-    // pages pg and pg + 1 of this wave: scores -> softmax -> accumulate, operands from the LDS
-    // buffers buf and buf + 1.  The second page may lie past the wave's last one: it then counts
-    // as all dead (its buffer holds some finite page of the work-group, or nothing yet).
-    const auto process_pair = [&](int pg, int buf) {
-        const bool second = pg + 1 < n_pages;
-        float ta[4], tb[4];
-        {
-            const f4 sa = scores(buf);
-            f4 sb = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (second) sb = scores(buf + 1);
-            if (second && (pg + 2) * kPage - 1 <= pos_min) {
-                // every cell of the pair is at or below every row's position
+    // Base-2 logits of pages pg and pg + 1 (slots 0..3: the first page's cells 4 g + r, slots 4..7: the second
+    // page's), dead cells at -inf.
+    float x[TILES][8];
+    const auto logits = [&](int pg) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ta[r] = sa[r], tb[r] = sb[r];
-            } else {
+        for (int t = 0; t < TILES; ++t)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int cell = pg * kPage + 4 * g + r;
-                    ta[r] = cell <= pos_q ? sa[r] : -INFINITY;
-                    tb[r] = second && cell + kPage <= pos_q ? sb[r] : -INFINITY;
+            for (int r = 0; r < 8; ++r) x[t][r] = s_hi[t][r >> 2][r & 3] + s_lo[t][r >> 2][r & 3] * kLoDown;
+        if ((pg + 2) * kPage - 1 > all_live) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const int cell = (pg + (r >> 2)) * kPage + 4 * g + (r & 3);
+                    x[t][r] = cell <= last_cell[t] ? x[t][r] : -INFINITY;
+                }
+        }
+    };
+
+    // Their softmax: weights as hi + lo f16, and what the accumulators have to be scaled by; in 16 parts, which go
+    // between the products of the next pair's scores.
+    h8 ph[TILES], pl[TILES];
+    float w_[TILES][8], x_[TILES][8], pm[TILES], m_was[TILES], m_at[TILES], psum[TILES], ref[TILES], ref_at[TILES], l_new[TILES];
+    bool moved[TILES];
+    const auto softmax_part = [&](int buf, int part) {
+        if (part == 0) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+                // q8_0 V: the softmax runs over logit + E of the cell
+#pragma unroll
+                for (int r = 0; r < 8; ++r) w_[t][r] = x[t][r];
+                if constexpr (Q8V) {
+                    const f4 ea = *reinterpret_cast<const f4*>(&L.e[buf][0][4 * g]);
+                    const f4 eb = *reinterpret_cast<const f4*>(&L.e[buf][1][4 * g]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) w_[t][r] += ea[r], w_[t][r + 4] += eb[r];
+                }
+                pm[t] = max_of(max_of(max_of(w_[t][0], w_[t][1]), max_of(w_[t][2], w_[t][3])),
+                               max_of(max_of(w_[t][4], w_[t][5]), max_of(w_[t][6], w_[t][7])));
+            }
+        }
+        if (part == 1 || part == 2) {
+            if (part - 1 < TILES) pm[part - 1] = max_over_groups(pm[part - 1]);
+        }
+        if (part == 3) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+                // Cell 0 is live for every query, so from the first pair on the reference m_run is finite.
+                // It follows the running maximum lazily: it moves only when a pair's maximum passes it by
+                // more than kSlack (weights then reach 2^kSlack at most, far inside f16 and f32), which after
+                // the first pairs is rare -- and every move costs a rescale of the 64 accumulators.  (q8_0 weights
+                // multiply values of up to 2^8: products of up to 2^14, summed in f32.)
+                constexpr float kSlack = 6.0f;
+                moved[t] = pm[t] > m_run[t] + kSlack;  // m_run = -inf at the start: any finite maximum moves it
+                m_was[t] = m_run[t];
+                m_run[t] = moved[t] ? pm[t] : m_run[t];
+                // a range may hold no live cell for a row (it begins past the row's position): its reference
+                // stays at -inf, and the weights of its dead cells are taken against 0
+                m_at[t] = SPLIT && m_run[t] == -INFINITY ? 0.0f : m_run[t];
+                ref[t] = Q8V ? fmaxf(l_ref[t], m_run[t]) : m_run[t];
+                ref_at[t] = SPLIT && ref[t] == -INFINITY ? 0.0f : ref[t];
+                psum[t] = 0.0f;
+            }
+        }
+        constexpr int kPairs = 4 * TILES;
+        if (part >= 4 && part < 4 + kPairs) {
+            const int t = (part - 4) >> 2, r0 = ((part - 4) & 3) * 2;
+#pragma unroll
+            for (int r = r0; r < r0 + 2; ++r) {
+                w_[t][r] = __builtin_amdgcn_exp2f(w_[t][r] - m_at[t]);
+                stay(w_[t][r]);
+                if constexpr (Q8V) x_[t][r] = __builtin_amdgcn_exp2f(x[t][r] - ref_at[t]);
+            }
+        }
+        if (part >= 6 && part < 6 + kPairs) {
+            // p = hi + lo, both rounded to nearest (the matrix cores read f16 subnormals as the numbers
+            // they are, so small weights keep their low parts' few bits)
+            const int t = (part - 6) >> 2, r0 = ((part - 6) & 3) * 2;
+            psum[t] += Q8V ? x_[t][r0] : w_[t][r0];
+            psum[t] += Q8V ? x_[t][r0 + 1] : w_[t][r0 + 1];
+            const h2m hi = to_f16(w_[t][r0], w_[t][r0 + 1]);
+            const h2m lo = to_f16(remainder_of(w_[t][r0], hi[0], minus_one), remainder_of(w_[t][r0 + 1], hi[1], minus_one));
+            ph[t][r0] = hi[0], ph[t][r0 + 1] = hi[1];
+            pl[t][r0] = lo[0], pl[t][r0 + 1] = lo[1];
+        }
+        if (part == 15) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+                l_new[t] = l_run[t] + psum[t];
+                stay(ph[t]);
+                stay(pl[t]);
+            }
+        }
+    };
+    const auto rescale = [&]() {
+        bool any = false;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) any = any || moved[t] || (Q8V && l_new[t] > kMostL);
+        if (__builtin_amdgcn_ballot_w64(any) != 0) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) {
+                const float alpha = __builtin_amdgcn_exp2f(m_was[t] - m_at[t]);  // 1, or 0 at the start
+#pragma unroll
+                for (int d = 0; d < 16; ++d) o[t][d] *= alpha;
+                if constexpr (Q8V) {
+                    l_new[t] = l_run[t] * __builtin_amdgcn_exp2f(l_ref[t] - ref_at[t]) + psum[t];
+                    const float l_was = l_ref[t];
+                    l_ref[t] = ref[t];
+                    if (l_new[t] > kMostL) {
+                        // up to the pair's largest logit (its terms are then 1 at most), and by 2^64 at least
+                        float up = ref_at[t] + 64.0f;
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) up = fmaxf(up, x[t][r]);
+                        l_new[t] = 0.0f;
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) l_new[t] += __builtin_amdgcn_exp2f(x[t][r] - up);
+                        l_new[t] += l_run[t] * __builtin_amdgcn_exp2f(l_was - up);
+                        l_ref[t] = up;
+                    }
+                } else {
+                    l_new[t] = l_run[t] * alpha + psum[t];
                 }
             }
         }
-        // q8_0 V: the softmax runs over logit + E of the cell (wa, wb); dead cells stay at -inf
-        float wa[4], wb[4];
-        if constexpr (Q8V) {
-            const f4 ea = *reinterpret_cast<const f4*>(&L.e[buf][4 * g]);
-            f4 eb = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (second) eb = *reinterpret_cast<const f4*>(&L.e[buf + 1][4 * g]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                wa[r] = ta[r] + ea[r];
-                wb[r] = tb[r] + eb[r];
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) wa[r] = ta[r], wb[r] = tb[r];
-        }
+        for (int t = 0; t < TILES; ++t) l_run[t] = l_new[t];
+    };
 
-        // ---- online softmax for this lane's query, over the pair's 32 cells ---------------------------
-        // Cell 0 is live for every query, so from the first pair on the reference m_run is finite.
-        // It follows the running maximum lazily: it moves only when a pair's maximum passes it by
-        // more than kSlack (weights then reach 2^kSlack at most, far inside f16 and f32), which after
-        // the first pairs is rare -- and every move costs a rescale of the 64 accumulators.  (q8_0 weights
-        // multiply values of up to 2^8: products of up to 2^14, summed in f32.)
-        constexpr float kSlack = 6.0f;
-        float pm = fmaxf(fmaxf(fmaxf(wa[0], wa[1]), fmaxf(wa[2], wa[3])), fmaxf(fmaxf(wb[0], wb[1]), fmaxf(wb[2], wb[3])));
-        pm = max_over_lane_groups(pm);
-        const bool moved = pm > m_run + kSlack;  // m_run = -inf at the start: any finite maximum moves it
-        const float m_new = moved ? pm : m_run;
-        // a range may hold no live cell for a row (it begins past the row's position): its reference
-        // stays at -inf, and the weights of its dead cells are taken against 0
-        const float m_at = SPLIT && m_new == -INFINITY ? 0.0f : m_new;
-        float pv[8];
-        float psum = 0.0f;
-        const float ref = Q8V ? fmaxf(l_ref, m_new) : m_new;
-        const float ref_at = SPLIT && ref == -INFINITY ? 0.0f : ref;
-        const auto tt = [&](int r) { return r < 4 ? ta[r & 3] : tb[r & 3]; };
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            pv[r] = __builtin_amdgcn_exp2f((r < 4 ? wa[r & 3] : wb[r & 3]) - m_at);
-            psum += Q8V ? __builtin_amdgcn_exp2f(tt(r) - ref_at) : pv[r];
-        }
-        // p = hi + lo, both rounded to nearest (the matrix cores read f16 subnormals as the numbers
-        // they are, so small weights keep their low parts' few bits)
-        h8 ph, pl;  // slots 0..3: the first page's cells 4 g + r, slots 4..7: the second page's
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            _Float16 hi, lo;
-            split_f16(pv[r], hi, lo);
-            ph[r] = hi;
-            pl[r] = lo;
-        }
-        float l_new = l_run + psum;
-        const bool high = Q8V && l_new > kMostL;
-        if (__builtin_amdgcn_ballot_w64(moved || high) != 0) {
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_at);  // 1, or 0 at the start
-#pragma unroll
-            for (int t = 0; t < 16; ++t) o[t] *= alpha;
-            if constexpr (Q8V) {
-                l_new = l_run * __builtin_amdgcn_exp2f(l_ref - ref_at) + psum;
-                const float l_was = l_ref;
-                l_ref = ref;
-                if (l_new > kMostL) {
-                    // up to the pair's largest logit (its terms are then 1 at most), and by 2^64 at least
-                    float up = ref_at + 64.0f;
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) up = fmaxf(up, tt(r));
-                    l_new = 0.0f;
-#pragma unroll
-                    for (int r = 0; r < 8; ++r) l_new += __builtin_amdgcn_exp2f(tt(r) - up);
-                    l_new += l_run * __builtin_amdgcn_exp2f(l_was - up);
-                    l_ref = up;
-                }
-            } else {
-                l_new = l_run * alpha + psum;
-            }
-        }
-        l_run = l_new;
-        m_run = m_new;
-
-        // ---- O^T += V^T . P^T over the 32 cells of the pair ----------------------------------------
-        // Per tile of 16 output columns one transposing read from either page's image: lane (c, g)
-        // receives column 16 tile + c of cells 4 g .. 4 g + 3 -- slots 0..3 and 4..7 of the operand,
-        // the order P^T has.  Rows past the work-group's last position are zeros in the image.  A
-        // second page past this wave's last one meets zero probabilities: its buffer holds a page of
-        // the work-group all the same (the last one again, past the end), never nothing, so the
-        // reads need no condition and the 32 of them can be issued ahead of the MFMAs.
-        // quantised V: the image of high parts meets p's high and low parts, the image of low parts
-        // p's high parts
+    // O^T += V^T . P^T over the 32 cells of the pair: per tile of 16 output columns one transposing read from either
+    // page's image: lane (c, g) receives column 16 d + c of cells 4 g .. 4 g + 3 -- slots 0..3 and 4..7 of the operand,
+    // the order P^T has.  Quantised V: the image of high parts meets p's high and low parts, the image of low
+    // parts p's high parts.
+    h8 vf[WIDE ? 32 : 16];
+    const auto read_v = [&](int buf, int d) {
 #pragma unroll
         for (int img = 0; img < (WIDE ? 2 : 1); ++img) {
-            const _Float16* va_s = &L.vimg[buf][img][0][0] + tr_off;
-            const _Float16* vb_s = &L.vimg[buf + 1][img][0][0] + tr_off;
+            const int at = v_piece + (d & 1 ? v_odd : 0) + (d >> 1) * 64;
+            const tr_s4 fa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(&L.vimg[buf][0][img][0][0] + at));
+            const tr_s4 fb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(&L.vimg[buf][1][img][0][0] + at));
+            vf[img * 16 + d] = __builtin_bit_cast(h8, __builtin_shufflevector(fa, fb, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    };
+    const auto multiply_v = [&](int d) {
 #pragma unroll
-            for (int t = 0; t < 16; ++t) {
-                const tr_s4 fa = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(va_s + t * 16));
-                const tr_s4 fb = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_ptr)(vb_s + t * 16));
-                const h8 vv = __builtin_bit_cast(h8, __builtin_shufflevector(fa, fb, 0, 1, 2, 3, 4, 5, 6, 7));
-                o[t] = mfma32(vv, ph, o[t]);
-                if (img == 0) o[t] = mfma32(vv, pl, o[t]);
-            }
+        for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[d], ph[t], o[t][d]);
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[d], pl[t], o[t][d]);
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[16 + d], ph[t], o[t][d]);
         }
     };
 
-    // Two pairs are in flight behind the one being multiplied: one in the other two LDS buffers,
-    // one in the staging registers (past the end they carry the last page again).
-    PageStage<LAY> stage_a, stage_b;
-    const int last_pg = wg_pages - 1;
-    fetch(first_pg, stage_a);
-    fetch(min(first_pg + 1, last_pg), stage_b);
-    deposit(0, stage_a);
-    deposit(1, stage_b);
-    fetch(min(first_pg + 2, last_pg), stage_a);
-    fetch(min(first_pg + 3, last_pg), stage_b);
+    const auto keep_q_in_agprs = [&]() {
+        if constexpr (TILES == 2) {
+#pragma unroll
+            for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    v4u a = __builtin_bit_cast(v4u, qhi[t][m]), b = __builtin_bit_cast(v4u, qlo[t][m]);
+                    asm("" : "+a"(a), "+a"(b));
+                    qhi[t][m] = __builtin_bit_cast(h8, a), qlo[t][m] = __builtin_bit_cast(h8, b);
+                }
+        }
+    };
+    constexpr int kAhead = 3;  // fragments asked for ahead of their products
+
+    if constexpr (I8H) {
+        deposit_k(0, stage_k, 0);
+        deposit_k(0, stage_k, 1);
+        load_pair_k(1, ids_v);
+    }
+    if constexpr (WIDE) {
+        deposit_v(0, stage_v, 0);
+        deposit_v(0, stage_v, 1);
+        load_pair_v(1, ids_v);
+    }
+    if constexpr (I8H) {
+        deposit_k(1, stage_k, 0);
+        deposit_k(1, stage_k, 1);
+        load_pair_k(0, ids_k);
+    }
+    if constexpr (!I8H) wait_for_loads();
+    clear_dead_v(0, first_pg);
     __syncthreads();
-    for (int pg = first_pg; pg < wg_pages; pg += 2) {
-        const int buf = (pg - first_pg) & 2;  // 0 or 2
-        if (pg < n_pages) process_pair(pg, buf);
-        deposit(buf ^ 2, stage_a);  // pages pg + 2, pg + 3
-        deposit((buf ^ 2) + 1, stage_b);
-        fetch(min(pg + 4, last_pg), stage_a);
-        fetch(min(pg + 5, last_pg), stage_b);
-        // after the barrier the other pair of buffers is complete, and nobody reads this one any more
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        read_k(0, i);
+        multiply_k(i);
+    }
+    __syncthreads();
+    // At the head of the step for pair j: K of pair j + 1 and V of pair j in LDS; quantised rows: K of pair j + 2 and V of
+    // pair j + 1 in registers.  The step brings both into LDS, over K of pair j, whose scores are there already, and V of
+    // pair j - 1.
+    int pg = first_pg, buf = 0;
+    for (; pg + 2 < wg_pages; pg += 2, buf ^= 1) {
+        keep_q_in_agprs();
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) read_k(buf ^ 1, i);
+        const int ids_next = table_pair(pg + 6);
+        logits(pg);
+        const uint64_t k_at_pages = k_pages(ids_k), v_at_pages = v_pages(ids_v);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if (i + kAhead < 16) read_k(buf ^ 1, i + kAhead);
+            if (!I8H && i >= 1 && i < 5) load_k(buf, page_of(k_at_pages, (i - 1) >> 1), (i - 1) >> 1, (i - 1) & 1);
+            if (!WIDE && i >= 5 && i < 9) load_v(buf ^ 1, page_of(v_at_pages, (i - 5) >> 1), (i - 5) >> 1, (i - 5) & 1);
+            multiply_k(i);
+            if (I8H && i < 2 * kPutParts) deposit_k_part(buf, stage_k, i / kPutParts, i % kPutParts);
+            softmax_part(buf, i);
+        }
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) read_v(buf, d);
+        rescale();
+        ids_v = ids_k, ids_k = ids_next;
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+            if (d + kAhead < 16) read_v(buf, d + kAhead);
+            multiply_v(d);
+            if constexpr (WIDE) {
+                if (d < 2 * kPutParts) deposit_v_part(buf ^ 1, stage_v, d / kPutParts, d % kPutParts);
+                if (Q8V && d == 14) wait_for_loads();  // K of pair j + 2, asked for ahead of the scores
+                if (d == 14) load_pair_v(0, ids_v);
+                if (I8H && d == 15) load_pair_k(0, ids_k);
+                // left to itself the scheduler does the deposit first and the products behind it
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (LAY == BKV_LAYOUT_F16) wait_for_loads();
+        clear_dead_v(buf ^ 1, pg + 2);
         __syncthreads();
+    }
+    logits(pg);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) softmax_part(buf, i);
+    rescale();
+#pragma unroll
+    for (int d = 0; d < 16; ++d) {
+        read_v(buf, d);
+        multiply_v(d);
     }
 
     // ---- normalise, gate, store ---------------------------------------------------------------------
-    if constexpr (Q8V) {
-        // the row's four lanes to one reference, the outputs to it too (nearly always M: nothing to do)
-        const float ref = max_over_lane_groups(l_ref);
-        const float ref_at = ref == -INFINITY ? 0.0f : ref;
-        l_run *= __builtin_amdgcn_exp2f(l_ref - ref_at);
-        if (__builtin_amdgcn_ballot_w64(m_run != ref) != 0) {
-            const float down = __builtin_amdgcn_exp2f(m_run - ref_at);
 #pragma unroll
-            for (int t = 0; t < 16; ++t) o[t] *= down;
+    for (int t = 0; t < TILES; ++t) {
+        if constexpr (Q8V) {
+            // the row's four lanes to one reference, the outputs to it too (nearly always M: nothing to do)
+            const float ref = max_over_lane_groups(l_ref[t]);
+            const float ref_at = ref == -INFINITY ? 0.0f : ref;
+            l_run[t] *= __builtin_amdgcn_exp2f(l_ref[t] - ref_at);
+            if (__builtin_amdgcn_ballot_w64(m_run[t] != ref) != 0) {
+                const float down = __builtin_amdgcn_exp2f(m_run[t] - ref_at);
+#pragma unroll
+                for (int d = 0; d < 16; ++d) o[t][d] *= down;
+            }
+            m_run[t] = ref;
         }
-        m_run = ref;
-    }
-    l_run = sum_over_lane_groups(l_run);
-    if (!row_live) return;
-    if constexpr (SPLIT) {
-        if (cut) {
-            const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
-            const size_t at = slot * kRowsPerWg + wave * kRowsPerWave + c;
-            float* po = P.part_o + at * kHd + 4 * g;
+        const float l = sum_over_lane_groups(l_run[t]);
+        if (!row_live[t]) continue;
+        if constexpr (SPLIT) {
+            if (cut) {
+                const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
+                const size_t at = slot * kRowsPerWg + wave * kRows + t * kRowsPerWave + c;
+                float* po = P.part_o + at * kHd + 4 * g;
 #pragma unroll
-            for (int t = 0; t < 16; ++t) *reinterpret_cast<f4*>(po + 16 * t) = o[t];
-            if (g == 0) *reinterpret_cast<float2*>(P.part_ml + at * 2) = make_float2(m_run, l_run);
-            return;
+                for (int d = 0; d < 16; ++d) *reinterpret_cast<f4*>(po + 16 * d) = o[t][d];
+                if (g == 0) *reinterpret_cast<float2*>(P.part_ml + at * 2) = make_float2(m_run[t], l);
+                continue;
+            }
         }
-    }
-    const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
-    float* op = P.out + ((size_t)(P.b.src0[e] + tok) * P.n_q + head) * kHd;
-    const float* gp = P.gate ? P.gate + (size_t)(P.b.src0[e] + tok) * P.gate_tok_stride +
-                                   (size_t)head * P.gate_head_stride
-                             : nullptr;
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        float* op = P.out + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd;
+        const float* gp = P.gate ? P.gate + (size_t)(P.b.src0[e] + tok[t]) * P.gate_tok_stride +
+                                       (size_t)head[t] * P.gate_head_stride
+                                 : nullptr;
+        // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
+        // chain of 64 trips to memory
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        const int d0 = 16 * t + 4 * g;
-        float y[4];
+        for (int half = 0; half < 2; ++half) {
+            f4 y[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            y[r] = o[t][r] * inv;
-            if (gp) y[r] *= sigmoid(gp[d0 + r]);
+            for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
+            if (gp) {
+                f4 z[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) z[i][r] = gp[16 * (half * 8 + i) + 4 * g + r];
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) y[i][r] *= sigmoid(z[i][r]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) *reinterpret_cast<f4*>(op + 16 * (half * 8 + i) + 4 * g) = y[i];
         }
-        *reinterpret_cast<float4*>(op + d0) = make_float4(y[0], y[1], y[2], y[3]);
     }
 }
 
@@ -723,11 +932,11 @@ __global__ __launch_bounds__(64 * kMergeWaves, 4) void prefill_merge_kernel(cons
     *reinterpret_cast<float4*>(P.out + (out_row * P.n_q + head) * kHd + 4 * lane) = y;
 }
 
-template <int LAY, int WAVES>
+template <int LAY, int TILES>
 hipError_t launch_split(bkv_pool* p, const PrefillSplitParams& kp, hipStream_t stream) {
-    constexpr int kRows = WAVES * kRowsPerWave;
-    launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<LAY, WAVES, true>,
-                  dim3((unsigned)kp.s.wg_base[kp.b.n]), dim3(64 * WAVES), 0, stream, kp);
+    constexpr int kRows = 4 * TILES * kRowsPerWave;
+    launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<LAY, TILES, true>,
+                  dim3((unsigned)kp.s.wg_base[kp.b.n]), dim3(256), 0, stream, kp);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     const unsigned rows = (unsigned)kp.s.unit_base[kp.b.n] * kRows;
@@ -763,9 +972,9 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
         sp.s = *split;
         sp.part_o = ws->o;
         sp.part_ml = ws->ml;
-        if (p->g.layout == BKV_LAYOUT_Q8V) return launch_split<BKV_LAYOUT_Q8V, 8>(p, sp, stream);
-        if (p->g.layout == BKV_LAYOUT_I8H) return launch_split<BKV_LAYOUT_I8H, 8>(p, sp, stream);
-        return launch_split<BKV_LAYOUT_F16, 4>(p, sp, stream);
+        if (p->g.layout == BKV_LAYOUT_Q8V) return launch_split<BKV_LAYOUT_Q8V, 2>(p, sp, stream);
+        if (p->g.layout == BKV_LAYOUT_I8H) return launch_split<BKV_LAYOUT_I8H, 2>(p, sp, stream);
+        return launch_split<BKV_LAYOUT_F16, 1>(p, sp, stream);
     }
     // Deal the work-groups to the dies by unit where that costs little: the grid then holds 8 x the
     // longest die's share, and work-groups past a shorter die's share leave at once.
@@ -776,16 +985,16 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
         grid = (int32_t)(share * kXcds);
     }
     if (p->g.layout == BKV_LAYOUT_Q8V)
-        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_Q8V>, dim3((unsigned)grid), dim3(512), 0,
+        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_Q8V, 2>, dim3((unsigned)grid), dim3(256), 0,
                       stream, kp);
     else if (p->g.layout == BKV_LAYOUT_I8H)
-        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_I8H>, dim3((unsigned)grid), dim3(512), 0,
+        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_I8H, 2>, dim3((unsigned)grid), dim3(256), 0,
                       stream, kp);
     else if (rows_per_wg == 8 * kRowsPerWave)
-        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_F16, 8>, dim3((unsigned)grid), dim3(512), 0,
+        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_F16, 2>, dim3((unsigned)grid), dim3(256), 0,
                       stream, kp);
     else
-        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_F16, 4>, dim3((unsigned)grid), dim3(256), 0,
+        launch_staged(p, BKV_STAGE_PREFILL_ATTN, prefill_attn_kernel<BKV_LAYOUT_F16, 1>, dim3((unsigned)grid), dim3(256), 0,
                       stream, kp);
     return hipGetLastError();
 }

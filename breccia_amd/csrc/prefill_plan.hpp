@@ -106,7 +106,7 @@ BKV_HD inline int split_ranges(int pages, int pps, int max_splits, int& each) {
     return (pages + each - 1) / each;
 }
 
-// Query rows one work-group owns.  f16 pools: 128 when the chunks make more 64-row work-groups than
+// Query rows one work-group of four waves owns, in tiles of 16: two tiles a wave or one.  f16 pools: 128 when the chunks make more 64-row work-groups than
 // fit the chip at two per compute unit (then sharing the page images among more rows is worth more
 // than spreading out), else 64.
 inline int32_t prefill_rows_per_wg(bool f16, int64_t wgs_of_64_rows, int32_t n_cu) {

@@ -248,11 +248,38 @@ def test_the_largest_batch_of_chunks_in_one_call(layout):
         z.free()
 
 
+@pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H])
+def test_short_walks_of_wide_work_groups(layout):
+    # Work-groups of 128 rows (on f16 pools: 544 and more of 64 rows) whose walks are 1 to 9 pairs of pages, odd page counts
+    # among them, with waves and lanes that have no query row; every byte that was not written is 0xFF.
+    rng = np.random.Generator(np.random.PCG64(1040 + layout))
+    befores = [0, 1, 14, 15, 16, 17, 30, 31, 32, 33, 47, 48, 63, 64, 100, 111]
+    with Twin(n_pages=320, max_seqs=16, layout=layout) as tw:
+        tw.pool.fill(0xFF)
+        for img in tw.images:
+            img.k[:] = 0xFF
+            img.v[:] = 0xFF
+        tw.pool.set_free_order(rng.permutation(320).astype(np.int32))
+        lens = [int(x) for x in rng.integers(130, 151, size=16)]
+        seqs = [tw.pool.seq_create() for _ in befores]
+        for s, before, t in zip(seqs, befores, lens):
+            fill(tw, s, before + t, rng, chunk=512)
+        qs = [rng.standard_normal((t, 16, 256)).astype(np.float32) for t in lens]
+        gates = [rng.standard_normal((t, 16, 256)).astype(np.float32) for t in lens]
+        outs = prefill(tw, 0, seqs, befores, qs, 16, gates)
+        for s, before, t, q, g, out in zip(seqs, befores, lens, qs, gates, outs):
+            assert np.all(np.isfinite(out))
+            for i in sorted({0, 15, 16, int(rng.integers(17, t - 1)), t - 1}):
+                want = tw.oracle_attend(0, s, before + i, q[i], 16, gate=g[i])
+                _, rel = check_attn(out[i], want, "chunk at %d, token %d" % (before, i))
+                assert rel <= REF_BAR_MAX_REL, (before, i, rel)
+
+
 def test_work_group_width_does_not_change_a_bit():
-    # On f16 pools a call whose chunks fill the chip runs work-groups of eight waves (128 query rows
-    # share each page image), a smaller one work-groups of four.  A wave's sixteen rows are computed
-    # the same way in both, so three chunks in one call (566 work-groups of 64 rows: eight waves) and
-    # the same chunks one call each (four waves; each keeps more than half of the chip busy, so that
+    # On f16 pools a call whose chunks fill the chip runs work-groups of 128 query rows (two tiles of
+    # sixteen a wave), a smaller one work-groups of 64 (one tile).  A tile's rows are computed
+    # the same way in both, so three chunks in one call (566 work-groups of 64 rows: two tiles a wave) and
+    # the same chunks one call each (one; each keeps more than half of the chip busy, so that
     # none has its walks cut) must agree in every bit; the oracle checks a sample.
     rng = np.random.Generator(np.random.PCG64(1234))
     cases = [(100, 700), (37, 650), (515, 900)]
