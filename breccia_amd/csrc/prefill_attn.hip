@@ -75,6 +75,8 @@ constexpr int kRowsPerWave = kPrefillRowsPerWave;
 constexpr int kQ8vRow = kHd / 32 * 36;  // bytes of a q8_0 row
 constexpr int kI8hRow = kHd + kHd / 32 * 2;  // bytes of an int8 row: codes, then 8 f16 scales
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLog2eLo = (float)(1.4426950408889634 - (double)kLog2e);
+constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kLoDown = 1.0f / 2048.0f;  // q's low parts enter the products times 2^11
 // Two rows of a page image in LDS: 1024 bytes in one piece, as one load of a wave delivers them, and padding.  In the
 // second row neighbouring 16-byte chunks (V: 32-byte pairs of them) have changed places.  With the padding, the rows
@@ -101,6 +103,8 @@ struct PrefillKernelParams {
     int64_t gate_tok_stride, gate_head_stride;
     int32_t max_pages_per_seq, n_kv, n_q, group;
     float scale_log2e;
+    uint32_t group_inverse, n_kv_inverse;  // floor((2^32 - 1) / n), for divided_by
+    int32_t gate_in_fours;                 // four gate values can be read at once
     int32_t by_xcd;  // work-groups are dealt to the chip's 8 dies so that each die sees few (entry, kv head) units
 };
 
@@ -129,9 +133,28 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
     lo = (_Float16)(x - (float)hi);
 }
 
-// sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91)
+// x / n and the rest, for x >= 0: the inverse is below 2^32 / n by less than 1, so the product's quotient is right or one
+// too small.  (A division by a number that only the launch knows is some 40 instructions.)
+__device__ __forceinline__ int divided_by(int x, int n, uint32_t inverse, int& rest) {
+    int q = (int)__umulhi((uint32_t)x, inverse);
+    rest = x - q * n;
+    if (rest >= n) ++q, rest -= n;
+    return q;
+}
+__device__ __forceinline__ int divided_by(int x, int n, uint32_t inverse) {
+    int rest;
+    return divided_by(x, n, inverse, rest);
+}
+
+// sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91).  exp(-|x|) is 2^t (1 + r ln 2), t + r being the
+// product with log2(e) to twice f32's precision.
 __device__ __forceinline__ float sigmoid(float x) {
-    const float ex = expf(-fabsf(x));
+    float a = -fabsf(x);
+    a = a < -150.0f ? -150.0f : a;  // 0 either way, and r stays a number
+    const float t = a * kLog2e;
+    const float r = __builtin_fmaf(a, kLog2eLo, __builtin_fmaf(a, kLog2e, -t));
+    float ex = __builtin_amdgcn_exp2f(t);
+    ex = __builtin_fmaf(ex, r * kLn2, ex);
     const float d = 1.0f + ex;  // 1 .. 2: nothing of a general division's scaling is needed
     float inv = __builtin_amdgcn_rcpf(d);
     inv = __builtin_fmaf(__builtin_fmaf(-d, inv, 1.0f), inv, inv);
@@ -227,8 +250,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             range = rem % P.s.splits[e];
             rem /= P.s.splits[e];
         }
-        kvh = rem % P.n_kv;
-        idx = rem / P.n_kv + (cut ? 0 : P.s.n_cut[e]);
+        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh) + (cut ? 0 : P.s.n_cut[e]);
     } else if (P.by_xcd) {
         const int units = P.b.n * P.n_kv;
         const int x = (int)blockIdx.x % kXcds;
@@ -238,7 +260,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             u = x;
             for (;;) {
                 if (u >= units) return;  // this die's share of the grid is shorter than the longest
-                const int nb = (P.b.n_tok[u / P.n_kv] * P.group + kRowsPerWg - 1) / kRowsPerWg;
+                const int nb = (P.b.n_tok[divided_by(u, P.n_kv, P.n_kv_inverse)] * P.group + kRowsPerWg - 1) / kRowsPerWg;
                 if (j < nb) break;
                 j -= nb;
                 u += kXcds;
@@ -249,13 +271,11 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             const int dies = (kXcds - u + units - 1) / units;  // dies x with x % units == u
             idx = j * dies + x / units;
         }
-        e = u / P.n_kv;
-        kvh = u - e * P.n_kv;
+        e = divided_by(u, P.n_kv, P.n_kv_inverse, kvh);
     } else {
         while (e + 1 < P.b.n && (int)blockIdx.x >= P.b.wg_base[e + 1]) ++e;
         const int rem = (int)blockIdx.x - P.b.wg_base[e];
-        kvh = rem % P.n_kv;
-        idx = rem / P.n_kv;
+        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh);
     }
     const int n_rows = P.b.n_tok[e] * P.group;  // query rows of this kv head
     const int n_blocks = (n_rows + kRowsPerWg - 1) / kRowsPerWg;
@@ -272,7 +292,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
 
     // pages the work-group walks: those of its last row
     const int wg_last_row = min(rb * kRowsPerWg + kRowsPerWg, n_rows) - 1;
-    const int wg_pos_max = P.b.pos0[e] + wg_last_row / P.group;
+    const int wg_pos_max = P.b.pos0[e] + divided_by(wg_last_row, P.group, P.group_inverse);
     int wg_pages = wg_pos_max / kPage + 1;
     int first_pg = 0;
     if constexpr (SPLIT) {
@@ -291,14 +311,15 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     for (int t = 0; t < TILES; ++t) {
         const int row = row0 + t * kRowsPerWave + c;
         row_live[t] = row < n_rows;
-        tok[t] = row_live[t] ? row / P.group : 0;
-        head[t] = kvh * P.group + (row_live[t] ? row % P.group : 0);
+        int h;
+        tok[t] = divided_by(row_live[t] ? row : 0, P.group, P.group_inverse, h);
+        head[t] = kvh * P.group + h;
         // a lane without a query row (past the end of the chunk) walks along with q = 0: its column of
         // the products is its own, and nothing of it is stored
         last_cell[t] = min(row_live[t] ? P.b.pos0[e] + tok[t] : 0x7fffffff, wg_pages * kPage - 1);
     }
     // the last cell that every row of this wave attends: pages wholly at or below it need no mask
-    const int all_live = min(P.b.pos0[e] + (wave_live ? row0 / P.group : 0), wg_pages * kPage - 1);
+    const int all_live = min(P.b.pos0[e] + (wave_live ? divided_by(row0, P.group, P.group_inverse) : 0), wg_pages * kPage - 1);
 
     constexpr int kKRow = I8H ? kI8hRow : kHd * 2;  // bytes of a row in the K pool and in the V pool
     constexpr int kVRow = I8H ? kI8hRow : Q8V ? kQ8vRow : kHd * 2;
@@ -307,7 +328,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     const size_t v_page_bytes = (size_t)P.n_kv * kPage * kVRow;
     const size_t v_head_off = (size_t)kvh * kPage * kVRow;
 
-    // ---- requests of the prologue ----------------------------------------------------------------
+    // ---- table entries, on which everything waits ----------------------------------------------------------------
     __shared__ __attribute__((aligned(16))) PrefillLds<LAY> L;
     const int tid = threadIdx.x;
     const int last_pg = wg_pages - 1;
@@ -325,17 +346,6 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
         const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(pages >> 32), w);
         return (page_ptr)((uint64_t)hi << 32 | lo);
     };
-
-    // q: lane (c, g) holds q[row][32 m + 8 g + 0..7], m = 0..7.  All of the row is requested at once (a lane without a row
-    // reads the chunk's first one and drops it): behind a branch a fragment, each was waited for before the next was
-    // asked for, a trip to memory each.
-    f4 raw[TILES][16];
-#pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        const float* qp = P.q + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd + g * 8;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
-    }
 
     // ---- pages into LDS --------------------------------------------------------------------------
     // f16 rows go there by themselves: wave w moves rows 4 w .. 4 w + 3 of a page, two rows a load; lane l delivers
@@ -493,6 +503,18 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     load_pair_k(0, ids_0);
     load_pair_v(0, ids_0);
     if constexpr (!I8H) load_pair_k(1, ids_v);
+
+    // q: lane (c, g) holds q[row][32 m + 8 g + 0..7], m = 0..7.  All of the row is requested at once (a lane without a row
+    // reads the chunk's first one and drops it): behind a branch a fragment, each was waited for before the next was
+    // asked for, a trip to memory each.  Behind the first pages' requests: a wave's 16 or 32, which touch 16 rows each, keep
+    // the path to memory busy for 3 us.
+    f4 raw[TILES][16];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const float* qp = P.q + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd + g * 8;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
+    }
 
     // ---- q as hi + lo f16 --------------------------------------------------------------------------
     float minus_one = -1.0f;
@@ -853,10 +875,16 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
             if (gp) {
                 f4 z[8];
+                const float* at = gp + 128 * half + 4 * g;
+                if (P.gate_in_fours) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                    for (int i = 0; i < 8; ++i) z[i] = *reinterpret_cast<const f4*>(at + 16 * i);
+                } else {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) z[i][r] = gp[16 * (half * 8 + i) + 4 * g + r];
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) z[i][r] = at[16 * i + r];
+                }
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -890,7 +918,7 @@ __global__ __launch_bounds__(64 * kMergeWaves, 4) void prefill_merge_kernel(cons
     if (row >= n_rows) return;
     const int wg_last_row = min(rb * rows_per_wg + rows_per_wg, n_rows) - 1;
     int each;
-    const int ranges = split_ranges((P.b.pos0[e] + wg_last_row / P.group) / kPage + 1, P.s.pps, P.s.splits[e], each);
+    const int ranges = split_ranges((P.b.pos0[e] + divided_by(wg_last_row, P.group, P.group_inverse)) / kPage + 1, P.s.pps, P.s.splits[e], each);
     const size_t at = ((size_t)P.s.slot_base[e] + (size_t)unit * P.s.splits[e]) * rows_per_wg + r;
     const float* po = P.part_o + at * kHd + 4 * lane;
     const size_t step = (size_t)rows_per_wg * kHd;
@@ -901,7 +929,9 @@ __global__ __launch_bounds__(64 * kMergeWaves, 4) void prefill_merge_kernel(cons
     for (int u = 0; u < kMergeInFlight; ++u) v[u] = part_row(u);
     float2 ml = *reinterpret_cast<const float2*>(P.part_ml + (at + (size_t)min(lane, ranges - 1) * rows_per_wg) * 2);
     if (lane >= ranges) ml = make_float2(-INFINITY, 0.0f);
-    const int tok = row / P.group, head = kvh * P.group + row % P.group;
+    int head;
+    const int tok = divided_by(row, P.group, P.group_inverse, head);
+    head += kvh * P.group;
     const size_t out_row = (size_t)(P.b.src0[e] + tok);
     float4 gt = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (P.gate) {
@@ -964,6 +994,9 @@ hipError_t launch_prefill_attn(bkv_pool* p, int32_t layer, const PrefillBatch& b
     kp.n_kv = p->g.n_kv;
     kp.n_q = a.n_q_head;
     kp.group = a.n_q_head / p->g.n_kv;
+    kp.group_inverse = 0xffffffffu / (uint32_t)kp.group;
+    kp.n_kv_inverse = 0xffffffffu / (uint32_t)kp.n_kv;
+    kp.gate_in_fours = (((uint64_t)(uintptr_t)a.gate | (uint64_t)a.gate_seq_stride * 4 | (uint64_t)a.gate_head_stride * 4) & 15) == 0;
     kp.scale_log2e = a.scale * kLog2e;
     int32_t grid = b.wg_base[b.n];
     if (grid == 0) return hipSuccess;

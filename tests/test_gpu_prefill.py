@@ -248,6 +248,33 @@ def test_the_largest_batch_of_chunks_in_one_call(layout):
         z.free()
 
 
+@pytest.mark.parametrize("first,head_stride,tok_extra", [(1, 256, 0), (0, 257, 0), (0, 256, 2), (4, 260, 8)])
+def test_gate_values_at_any_alignment(first, head_stride, tok_extra):
+    # gate values that can be read four at a time, and those that cannot (by their first address, by either stride): the
+    # same numbers, so the same bits
+    n_q, t = 6, 37
+    rng = np.random.Generator(np.random.PCG64(1050))
+    tok_stride = n_q * head_stride + tok_extra
+    with Twin(n_pages=16, max_seqs=1) as tw:
+        s = tw.pool.seq_create()
+        fill(tw, s, t, rng, chunk=64)
+        q = rng.standard_normal((t, n_q, 256)).astype(np.float32)
+        gate = rng.standard_normal((t, n_q, 256)).astype(np.float32) * 3
+        want = prefill(tw, 0, [s], [0], [q], n_q, [gate])[0]
+        spread = np.zeros(first + t * tok_stride + 4, np.float32)
+        for i in range(t):
+            for h in range(n_q):
+                at = first + i * tok_stride + h * head_stride
+                spread[at:at + 256] = gate[i, h]
+        qd, gd, od = DeviceBuffer.from_numpy(q), DeviceBuffer.from_numpy(spread), DeviceBuffer(q.nbytes)
+        tw.pool.prefill_attn(0, [s], [0], [t], n_q, qd, od, 1.0 / 16.0, gate_dev=gd.ptr.value + 4 * first,
+                             gate_tok_stride=tok_stride, gate_head_stride=head_stride)
+        got = od.download(np.float32, q.size).reshape(q.shape)
+        for b in (qd, gd, od):
+            b.free()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H])
 def test_short_walks_of_wide_work_groups(layout):
     # Work-groups of 128 rows (on f16 pools: 544 and more of 64 rows) whose walks are 1 to 9 pairs of pages, odd page counts
