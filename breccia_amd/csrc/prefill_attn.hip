@@ -161,6 +161,22 @@ __device__ __forceinline__ float sigmoid(float x) {
     return (x >= 0.0f ? 1.0f : ex) * inv;
 }
 
+// The arguments' cache lines, asked for at once as a kernel begins: left to where each field is used, they are a chain of
+// trips to memory (a kernel of 13 us spent 0.4 of them ahead of its first own request and 1 ahead of its last store).
+template <typename S>
+__device__ __forceinline__ void now(const PrefillBatch& b, int n_kv, const S& at_end) {
+    asm volatile("" : : "s"(b.row[0]), "s"(b.pos0[0]), "s"(b.n_tok[0]), "s"(b.src0[0]), "s"(b.wg_base[0]), "s"(n_kv), "s"(at_end));
+}
+__device__ __forceinline__ void now(const PrefillSplit& s) {
+    asm volatile("" : : "s"(s.pps), "s"(s.splits[0]), "s"(s.wg_base[0]), "s"(s.unit_base[0]), "s"(s.slot_base[0]));
+}
+// keeps an argument in registers from here on instead of asking for it again
+template <typename T>
+__device__ __forceinline__ T held(T x) {
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
 // two f32 numbers as f16, rounded to nearest
 __device__ __forceinline__ h2m to_f16(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));
@@ -234,6 +250,8 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     constexpr int kWavesPerWg = 4;
     constexpr int kRows = kRowsPerWave * TILES;
     constexpr int kRowsPerWg = kRows * kWavesPerWg;
+    now(P.b, P.n_kv, P.by_xcd);
+    if constexpr (SPLIT) now(P.s);
     // ---- which (entry, kv head, block of query rows) ---------------------------------
     int e = 0, kvh, idx;  // idx: which of the unit's blocks, in dispatch order
     int range = 0;       // which range of the block's pages
@@ -472,6 +490,13 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
         }
     };
 
+    // for the last lines of the kernel
+    const float* const gate = held(P.gate);
+    float* const out = held(P.out);
+    const int64_t gate_tok_stride = held(P.gate_tok_stride), gate_head_stride = held(P.gate_head_stride);
+    const int n_q = held(P.n_q), src0 = held(P.b.src0[e]);
+    const int gate_in_fours = held(P.gate_in_fours);
+
     CodeStage stage_k, stage_v;
     // the first two pairs of K and the first of V; the next of either (quantised rows) in registers
     const auto load_pair_k = [&](int buf, int ids) {
@@ -511,7 +536,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     f4 raw[TILES][16];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        const float* qp = P.q + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd + g * 8;
+        const float* qp = P.q + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd + g * 8;
 #pragma unroll
         for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
     }
@@ -862,10 +887,8 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             }
         }
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        float* op = P.out + ((size_t)(P.b.src0[e] + tok[t]) * P.n_q + head[t]) * kHd;
-        const float* gp = P.gate ? P.gate + (size_t)(P.b.src0[e] + tok[t]) * P.gate_tok_stride +
-                                       (size_t)head[t] * P.gate_head_stride
-                                 : nullptr;
+        float* op = out + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
+        const float* gp = gate + (size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride;
         // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
         // chain of 64 trips to memory
 #pragma unroll
@@ -873,10 +896,10 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             f4 y[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
-            if (gp) {
+            if (gate) {
                 f4 z[8];
                 const float* at = gp + 128 * half + 4 * g;
-                if (P.gate_in_fours) {
+                if (gate_in_fours) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) z[i] = *reinterpret_cast<const f4*>(at + 16 * i);
                 } else {
@@ -903,6 +926,8 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
 constexpr int kMergeWaves = 4;
 constexpr int kMergeInFlight = 8;
 __global__ __launch_bounds__(64 * kMergeWaves, 4) void prefill_merge_kernel(const PrefillSplitParams P, int32_t rows_per_wg) {
+    now(P.b, P.n_kv, P.part_ml);
+    now(P.s);
     const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kMergeWaves + (int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     int unit = w / rows_per_wg;
