@@ -839,7 +839,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
                 if (d < 2 * kPutParts) deposit_v_part(buf ^ 1, stage_v, d / kPutParts, d % kPutParts);
                 if (Q8V && d == 14) wait_for_loads();  // K of pair j + 2, asked for ahead of the scores
                 if (d == 14) load_pair_v(0, ids_v);
-                if (I8H && d == 15) load_pair_k(0, ids_k);
+                if (I8H && d == 1) load_pair_k(0, ids_k);  // half a step ahead of their deposit, as V's codes are
                 // left to itself the scheduler does the deposit first and the products behind it
                 __builtin_amdgcn_sched_barrier(0);
             }
