@@ -133,28 +133,29 @@ inline int32_t last_done(const std::vector<int32_t>& runs, int32_t units) {
 }
 
 // Cuts the page walks of a small call's row blocks into ranges; false where the call is better off
-// uncut.  A row block's walk is a serial chain: 1.4 us a page pair on f16 pools when the compute unit
-// has nothing else (2.3-3.6 us on the quantised ones), and a call of a few blocks is as long as its longest
-// chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups, 34 us).  Cutting
-// pays for a second kernel (4-9 us, by the partial rows it reads), so:
+// uncut.  A row block's walk is a serial chain: 0.9 us a page pair on f16 pools when the compute unit
+// has nothing else (2.1-2.4 us on the quantised ones, whose blocks are twice as long), and a call of a few blocks is as
+// long as its longest chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups).  Cutting
+// pays for a second kernel (4-9 us, by the partial rows it reads), so (us of a layer: append and attention):
 // - a call that leaves half of the compute units idle is cut if
 //   - a range keeps at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several, and
-//   - the chain loses 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured 31.1 us
-//     uncut and 31.2 cut, 300 behind 200 cells (16 to 4) 35.0 and 34.5;
+//   - the chain loses 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured 24.4 us
+//     uncut and 24.2 cut, 300 behind 200 cells (16 to 4) 25.4 and 25.8;
 //   - into one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer
-//     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8;
+//     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8
+//     (these four with the kernel of one tile a wave in all calls: 24.2 and 45.4 us now);
 // - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) of up to
 //   two work-groups a compute unit may be cut, into ranges of an even share of the pairs;
 // - either way the chain has to lose a pair for every 32 partial results the second kernel reads; in the larger calls,
 //   where the ranges come on top of a chip that is nearly busy, for every 24, and for every 20 if they don't all find a
-//   compute unit at once (the chain of a cut call is then the schedule's).  260 calls a layout, random and at the
-//   edges, each measured cut and uncut: a pair less gains 2.5 us (f16 1.4), a partial result costs 0.04 (f16 0.03),
-//   in the larger calls 0.17.  With these lines no call loses more than 4 %, but for 60 chunks of 8 tokens
-//   behind 600 cells (7 %); with a ratio of longest walk to even share (1.7) some lost 41 %: four chunks of 270 from
-//   scratch 38 us uncut, 52 cut; 600 with 48 heads 70 and 79; 32 chunks of 8 behind 250 28 and 31; on the other
-//   side two chunks of 530 60 and 48, 1900 169 and 151, 400 with 48 heads 51 and 45.
-// Before / after, us a layer: 41 tokens behind 517 cells 37 / 24, 100 behind 8000 374 / 55, 200 behind
-// 3000 with q8_0 V 262 / 59, 300 behind 1000 on an int8 pool 125 / 48.
+//   compute unit at once (the chain of a cut call is then the schedule's).  The ratios come from 260 calls a layout, random
+//   and at the edges, each measured cut and uncut with a kernel of eight waves a work-group: a pair less gained 2.5 us (f16
+//   1.4), a partial result cost 0.04 (f16 0.03), in the larger calls 0.17.  They hold for the present one, uncut and cut:
+//   four chunks of 270 from scratch, left uncut, 38 and, with a ratio of longest walk to even share, 52; 600 with 48
+//   heads, left uncut, 59; two chunks of 530 54 / 44 (int8 59 / 46), 1900 144 / 130 (162 / 137), 400 with 48 heads 46 / 41
+//   (49 / 43), two of 530 behind 700 100 / 97.
+// Uncut / cut, us a layer: 41 tokens behind 517 cells 25.9 / 19.3, 100 behind 8000 237 / 45, 200 behind
+// 3000 with q8_0 V 223 / 55, 300 behind 1000 on an int8 pool 110 / 43, 900 behind 2000 226 / 136.
 // chain: page pairs of the cut call's longest chain, where it was worked out.
 inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s,
                                int32_t& chain) {
