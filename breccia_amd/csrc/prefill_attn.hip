@@ -30,8 +30,8 @@
 // - every instruction counts, a wave issues one at a time (4 cycles): packed conversions, mixed-precision remainders, page
 //   addresses worked out lane by lane.
 // Against work-groups of eight waves with a tile each, whose steps were not pipelined: 4 chunks of 1024 behind 2048 cells,
-// 16 heads, f16, 334 -> 286 us; a prompt of 4096, 24 heads, q8_0 V, 650 -> 538; three ragged chunks, int8, 175 -> 160; 41
-// tokens behind 517 cells through 12 layers 274 -> 235.  A step takes 3120 cycles on f16 pools, 4930 with q8_0 V; its products
+// 16 heads, f16, 336 -> 286 us; a prompt of 4096, 24 heads, q8_0 V, 648 -> 535; three ragged chunks, int8, 175 -> 158; 41
+// tokens behind 517 cells through 12 layers 274 -> 217.  A step takes 3120 cycles on f16 pools, 4930 with q8_0 V; its products
 // alone would take 2048 and 2560.  On f16 pools the clock falls to 2.0 GHz (1200 TFLOP/s issued; registers alone, no
 // loads, reach 1430 there): power is the next bound.  Tried and slower: all of a step as one block, the output a step
 // later (305 us f16); a third pair of pages in LDS (290, 582); chunks of one fragment fenced off from each other (299).
@@ -781,7 +781,9 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
                 }
         }
     };
-    constexpr int kAhead = 3;  // fragments asked for ahead of their products
+    // Fragments asked for ahead of their products.  1 to 3 of K and 3 to 6 of V were measured: f16 271 us with 3 and 3 (others 273
+    // to 281), q8_0 V 521 with 3 and 5 (525 to 535, 528 with 3 and 3), int8 348 with 2 and 5 (351 to 360, 359 with 3 and 3).
+    constexpr int kAheadK = I8H ? 2 : 3, kAheadV = WIDE ? 5 : 3;
 
     if constexpr (I8H) {
         deposit_k(0, stage_k, 0);
@@ -814,13 +816,13 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     for (; pg + 2 < wg_pages; pg += 2, buf ^= 1) {
         keep_q_in_agprs();
 #pragma unroll
-        for (int i = 0; i < kAhead; ++i) read_k(buf ^ 1, i);
+        for (int i = 0; i < kAheadK; ++i) read_k(buf ^ 1, i);
         const int ids_next = table_pair(pg + 6);
         logits(pg);
         const uint64_t k_at_pages = k_pages(ids_k), v_at_pages = v_pages(ids_v);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            if (i + kAhead < 16) read_k(buf ^ 1, i + kAhead);
+            if (i + kAheadK < 16) read_k(buf ^ 1, i + kAheadK);
             if (!I8H && i >= 1 && i < 5) load_k(buf, page_of(k_at_pages, (i - 1) >> 1), (i - 1) >> 1, (i - 1) & 1);
             if (!WIDE && i >= 5 && i < 9) load_v(buf ^ 1, page_of(v_at_pages, (i - 5) >> 1), (i - 5) >> 1, (i - 5) & 1);
             multiply_k(i);
@@ -828,12 +830,12 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             softmax_part(buf, i);
         }
 #pragma unroll
-        for (int d = 0; d < kAhead; ++d) read_v(buf, d);
+        for (int d = 0; d < kAheadV; ++d) read_v(buf, d);
         rescale();
         ids_v = ids_k, ids_k = ids_next;
 #pragma unroll
         for (int d = 0; d < 16; ++d) {
-            if (d + kAhead < 16) read_v(buf, d + kAhead);
+            if (d + kAheadV < 16) read_v(buf, d + kAheadV);
             multiply_v(d);
             if constexpr (WIDE) {
                 if (d < 2 * kPutParts) deposit_v_part(buf ^ 1, stage_v, d / kPutParts, d % kPutParts);
