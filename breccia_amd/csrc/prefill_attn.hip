@@ -162,7 +162,7 @@ __device__ __forceinline__ float sigmoid(float x) {
 }
 
 // The arguments' cache lines, asked for at once as a kernel begins: left to where each field is used, they are a chain of
-// trips to memory (a kernel of 13 us spent 0.4 of them ahead of its first own request and 1 ahead of its last store).
+// trips to memory (41 tokens behind 517 cells through 12 layers: 234 us, 218 with this and `held`).
 template <typename S>
 __device__ __forceinline__ void now(const PrefillBatch& b, int n_kv, const S& at_end) {
     asm volatile("" : : "s"(b.row[0]), "s"(b.pos0[0]), "s"(b.n_tok[0]), "s"(b.src0[0]), "s"(b.wg_base[0]), "s"(n_kv), "s"(at_end));
