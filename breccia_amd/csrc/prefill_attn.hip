@@ -223,8 +223,10 @@ __device__ __forceinline__ float max_over_groups(float x) {
 // What a thread carries of one pair of quantised pages between its fetch and its deposit into LDS: of row tid / 16,
 // block tid / 2 % 8, the codes of two 16-byte chunks of the f16 images.
 struct CodeStage {
-    uint2 c[2][2];      // [page][chunk]
-    unsigned scale[2];  // q8_0: the f32; int8 pools: the f16's bits
+    uint2 c[2][2];                 // [page][chunk]
+    unsigned scale[2];             // q8_0: the f32
+    unsigned short half_scale[2];  // int8 pools: the f16's bits.  (As 32 bits they would be widened, and waited for, where
+                                   // they were requested)
 };
 
 template <int LAY>
@@ -305,7 +307,6 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     const int c = lane & 15;  // query row of the tile / cell of the page / output column group
     const int g = lane >> 4;  // which quarter of the contraction index this lane feeds
     const int row0 = rb * kRowsPerWg + wave * kRows;
-    // a wave whose rows lie past the end still helps to fetch pages and joins the barriers
     const bool wave_live = row0 < n_rows;
 
     // pages the work-group walks: those of its last row
@@ -335,6 +336,16 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
         // a lane without a query row (past the end of the chunk) walks along with q = 0: its column of
         // the products is its own, and nothing of it is stored
         last_cell[t] = min(row_live[t] ? P.b.pos0[e] + tok[t] : 0x7fffffff, wg_pages * kPage - 1);
+    }
+    // Where the walk of each tile ends: behind the last page that a row of it attends.  Not later: a page may hold values
+    // of V that are not finite, which a weight of 0 would not keep away from the tile's rows.  A wave that is done, or whose
+    // rows lie past the chunk's end, still brings pages into LDS and joins the barriers.
+    int end_pg[TILES], wave_end = 0;
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+        const int first = row0 + t * kRowsPerWave, last = min(first + kRowsPerWave, n_rows) - 1;
+        end_pg[t] = first < n_rows ? min((P.b.pos0[e] + divided_by(last, P.group, P.group_inverse)) / kPage + 1, wg_pages) : 0;
+        wave_end = max(wave_end, end_pg[t]);
     }
     // the last cell that every row of this wave attends: pages wholly at or below it need no mask
     const int all_live = min(P.b.pos0[e] + (wave_live ? divided_by(row0, P.group, P.group_inverse) : 0), wg_pages * kPage - 1);
@@ -391,14 +402,14 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             st.c[w][h].y = *(const __attribute__((address_space(1))) unsigned*)(page + (at + 4));
         }
         if (q8) st.scale[w] = *(const __attribute__((address_space(1))) unsigned*)(page + (row + c_blk * 36));
-        else st.scale[w] = *(const __attribute__((address_space(1))) unsigned short*)(page + (row + kHd + c_blk * 2));
+        else st.half_scale[w] = *(const __attribute__((address_space(1))) unsigned short*)(page + (row + kHd + c_blk * 2));
     };
     const auto eight = [](const h2m (&x)[4]) {
         return h8{x[0][0], x[0][1], x[1][0], x[1][1], x[2][0], x[2][1], x[3][0], x[3][1]};
     };
     // code * scale (7 + 11 significant bits) as hi = f16(code * scale) and the exact remainder (times `up`).  A scale
     // with exponent field 0 reads as zero, as everywhere.
-    const auto i8h_scale = [](unsigned bits) {
+    const auto i8h_scale = [](unsigned short bits) {
         return __builtin_bit_cast(_Float16, (unsigned short)((bits & 0x7c00u) == 0 ? 0u : bits));
     };
     const auto half_of = [&](unsigned codes, h2m s_hi, h2m s_lo, h2m* hi, h2m* lo) {
@@ -424,7 +435,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     // the low parts of K times 2^11, like those of q: their products with q's high parts join those of q's low parts
     const auto deposit_k_part = [&](int buf, const CodeStage& st, int w, int part) {
         if (part == 0) {
-            const _Float16 scale = i8h_scale(st.scale[w]);
+            const _Float16 scale = i8h_scale(st.half_scale[w]);
             put_sh = h2m{scale, scale};
         } else if (part % 3 != 0) {
             const int h = part / 4, k = (part - 1) % 3;
@@ -438,7 +449,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     const auto deposit_v_part = [&](int buf, const CodeStage& st, int w, int part) {
         if (part == 0) {
             if constexpr (I8H) {
-                const _Float16 scale = i8h_scale(st.scale[w]);
+                const _Float16 scale = i8h_scale(st.half_scale[w]);
                 put_sh = h2m{scale, scale};
             } else {
                 // the largest scale of the row: over the lanes that differ in the block bits (1..3).  (Scales are not
@@ -758,14 +769,14 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             vf[img * 16 + d] = __builtin_bit_cast(h8, __builtin_shufflevector(fa, fb, 0, 1, 2, 3, 4, 5, 6, 7));
         }
     };
-    const auto multiply_v = [&](int d) {
+    const auto multiply_v = [&](int d, int first) {  // first: of the tiles
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[d], ph[t], o[t][d]);
+        for (int t = first; t < TILES; ++t) o[t][d] = mfma32(vf[d], ph[t], o[t][d]);
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[d], pl[t], o[t][d]);
+        for (int t = first; t < TILES; ++t) o[t][d] = mfma32(vf[d], pl[t], o[t][d]);
         if constexpr (WIDE) {
 #pragma unroll
-            for (int t = 0; t < TILES; ++t) o[t][d] = mfma32(vf[16 + d], ph[t], o[t][d]);
+            for (int t = first; t < TILES; ++t) o[t][d] = mfma32(vf[16 + d], ph[t], o[t][d]);
         }
     };
 
@@ -809,11 +820,37 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
         multiply_k(i);
     }
     __syncthreads();
+    // What a step brings into LDS and requests, without products to put between
+    const auto bring = [&](int pg, int buf) {
+        const int ids_next = table_pair(pg + 6);
+        const uint64_t k_at_pages = k_pages(ids_k), v_at_pages = v_pages(ids_v);
+        if constexpr (!I8H) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_k(buf, page_of(k_at_pages, i >> 1), i >> 1, i & 1);
+        }
+        if constexpr (!WIDE) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_v(buf ^ 1, page_of(v_at_pages, i >> 1), i >> 1, i & 1);
+        }
+        ids_v = ids_k, ids_k = ids_next;
+        if constexpr (I8H) {
+            deposit_k(buf, stage_k, 0);
+            deposit_k(buf, stage_k, 1);
+            load_pair_k(0, ids_k);
+        }
+        if constexpr (WIDE) {
+            deposit_v(buf ^ 1, stage_v, 0);
+            deposit_v(buf ^ 1, stage_v, 1);
+            if constexpr (Q8V) wait_for_loads();  // of K, ahead of the next codes
+            load_pair_v(0, ids_v);
+        }
+    };
     // At the head of the step for pair j: K of pair j + 1 and V of pair j in LDS; quantised rows: K of pair j + 2 and V of
     // pair j + 1 in registers.  The step brings both into LDS, over K of pair j, whose scores are there already, and V of
     // pair j - 1.
     int pg = first_pg, buf = 0;
-    for (; pg + 2 < wg_pages; pg += 2, buf ^= 1) {
+    const int stop = min(wg_pages - 2, end_pg[0]);
+    for (; pg < stop; pg += 2, buf ^= 1) {
         keep_q_in_agprs();
 #pragma unroll
         for (int i = 0; i < kAheadK; ++i) read_k(buf ^ 1, i);
@@ -836,7 +873,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
 #pragma unroll
         for (int d = 0; d < 16; ++d) {
             if (d + kAheadV < 16) read_v(buf, d + kAheadV);
-            multiply_v(d);
+            multiply_v(d, 0);
             if constexpr (WIDE) {
                 if (d < 2 * kPutParts) deposit_v_part(buf ^ 1, stage_v, d / kPutParts, d % kPutParts);
                 if (Q8V && d == 14) wait_for_loads();  // K of pair j + 2, asked for ahead of the scores
@@ -850,14 +887,38 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
         clear_dead_v(buf ^ 1, pg + 2);
         __syncthreads();
     }
-    logits(pg);
+    // Left are the walk's last pair or, where the first tile is done earlier, one that only the second tile attends (its
+    // rows reach at most 16 cells further); then the work-group's other steps, without products.  A step has one barrier
+    // for every wave, at its end, whichever loop the wave is in.  (With every wave in all steps: 4 chunks of 1024 behind 2048
+    // cells, f16, 289 us against 292, append included; the other layouts the same: what the compiler makes of the loop above.)
+    bool more = pg + 2 < wg_pages;
+    if (pg < wave_end) {
+        logits(pg);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) softmax_part(buf, i);
-    rescale();
+        for (int i = 0; i < 16; ++i) softmax_part(buf, i);
+        rescale();
+        if (pg < end_pg[0]) {
 #pragma unroll
-    for (int d = 0; d < 16; ++d) {
-        read_v(buf, d);
-        multiply_v(d);
+            for (int d = 0; d < 16; ++d) {
+                read_v(buf, d);
+                multiply_v(d, 0);
+            }
+        } else if constexpr (TILES == 2) {
+#pragma unroll
+            for (int d = 0; d < 16; ++d) {
+                read_v(buf, d);
+                multiply_v(d, 1);
+            }
+        }
+    }
+    if (more) bring(pg, buf);
+    while (more) {
+        if constexpr (LAY == BKV_LAYOUT_F16) wait_for_loads();
+        clear_dead_v(buf ^ 1, pg + 2);
+        __syncthreads();
+        pg += 2, buf ^= 1;
+        more = pg + 2 < wg_pages;
+        if (more) bring(pg, buf);
     }
 
     // ---- normalise, gate, store ---------------------------------------------------------------------

@@ -302,6 +302,39 @@ def test_short_walks_of_wide_work_groups(layout):
                 assert rel <= REF_BAR_MAX_REL, (before, i, rel)
 
 
+@pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H])
+@pytest.mark.parametrize("n_q, before, tokens, bad", [
+    (16, 24, 40, 32),     # rows of the first waves end a pair of pages before the work-group does
+    (16, 26, 40, 32),     # and those of a wave's first sixteen rows before its others
+    (2, 5, 130, 64),      # 128 tokens to a work-group: four pairs of pages between its first rows and its last
+    (16, 528 + 26, 41, 576),   # cut
+    (16, 26, 2100, 32 * 51),   # f16: 1051 work-groups of 64 rows, so two tiles a wave
+])
+def test_values_that_are_not_finite_stay_with_later_rows(n_q, before, tokens, bad, layout):
+    # V of cell `bad` overflows.  A weight of 0 does not undo that, so rows must not meet the cell's pair of pages at all
+    # where the last of their sixteen rows lies before it: the same bits as with an ordinary row there.
+    rng = np.random.Generator(np.random.PCG64(1070))
+    with Twin(n_pages=(before + tokens) // 16 + 2, max_seqs=1, layout=layout) as tw:
+        s = tw.pool.seq_create()
+        fill(tw, s, before + tokens, rng, chunk=1024)
+        q = rng.standard_normal((tokens, n_q, 256)).astype(np.float32)
+        want = prefill(tw, 0, [s], [before], [q], n_q)[0]
+        assert np.all(np.isfinite(want))
+        kd = DeviceBuffer.from_numpy(rng.standard_normal((1, 2, 256)).astype(np.float32))
+        vd = DeviceBuffer.from_numpy(np.full((1, 2, 256), np.inf, np.float32))
+        tw.pool.append(0, [s], [bad], [1], kd, vd)
+        got = prefill(tw, 0, [s], [before], [q], n_q)[0]
+        kd.free()
+        vd.free()
+        group = n_q // 2
+        rows = np.arange(tokens * group)
+        last = np.minimum(rows // 16 * 16 + 15, rows[-1]) // group + before  # of the row's sixteen
+        clear = (last < bad // 32 * 32).reshape(tokens, group)
+        clear = np.concatenate([clear, clear], axis=1)  # two kv heads
+        assert np.any(clear) and not np.all(np.isfinite(got))
+        assert np.array_equal(got[clear].view(np.uint32), want[clear].view(np.uint32))
+
+
 def test_work_group_width_does_not_change_a_bit():
     # On f16 pools a call whose chunks fill the chip runs work-groups of 128 query rows (two tiles of
     # sixteen a wave), a smaller one work-groups of 64 (one tile).  A tile's rows are computed
