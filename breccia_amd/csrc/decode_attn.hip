@@ -13,6 +13,7 @@
 #include <atomic>
 
 #include "decode_attn_common.hpp"
+#include "gate.hpp"
 
 namespace bkv {
 
@@ -143,17 +144,7 @@ __global__ __launch_bounds__(64 * kMergeGroups) void decode_attn_merge_kernel(co
         lt += red_l[k];
     }
     r = lt > 0.0f ? r / lt : 0.0f;
-    if (P.gate) {
-        // sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91)
-        float sg;
-        if (gt >= 0.0f) {
-            sg = 1.0f / (1.0f + expf(-gt));
-        } else {
-            const float t = expf(gt);
-            sg = t / (1.0f + t);
-        }
-        r *= sg;
-    }
+    if (P.gate) r *= sigmoid(gt);
     P.out[((size_t)e * P.n_q + h) * kHd + d] = r;
 }
 

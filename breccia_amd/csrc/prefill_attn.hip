@@ -62,6 +62,7 @@
 #include <type_traits>
 
 #include "bkv_internal.hpp"
+#include "gate.hpp"
 #include "lane_groups.hpp"
 #include "quant_decode.hpp"
 
@@ -75,8 +76,6 @@ constexpr int kRowsPerWave = kPrefillRowsPerWave;
 constexpr int kQ8vRow = kHd / 32 * 36;  // bytes of a q8_0 row
 constexpr int kI8hRow = kHd + kHd / 32 * 2;  // bytes of an int8 row: codes, then 8 f16 scales
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLog2eLo = (float)(1.4426950408889634 - (double)kLog2e);
-constexpr float kLn2 = 0.6931471805599453f;
 constexpr float kLoDown = 1.0f / 2048.0f;  // q's low parts enter the products times 2^11
 // Two rows of a page image in LDS: 1024 bytes in one piece, as one load of a wave delivers them, and padding.  In the
 // second row neighbouring 16-byte chunks (V: 32-byte pairs of them) have changed places.  With the padding, the rows
@@ -144,21 +143,6 @@ __device__ __forceinline__ int divided_by(int x, int n, uint32_t inverse, int& r
 __device__ __forceinline__ int divided_by(int x, int n, uint32_t inverse) {
     int rest;
     return divided_by(x, n, inverse, rest);
-}
-
-// sigmoid in the overflow-free form of the reference (qsa/cpu.rs:84-91).  exp(-|x|) is 2^t (1 + r ln 2), t + r being the
-// product with log2(e) to twice f32's precision.
-__device__ __forceinline__ float sigmoid(float x) {
-    float a = -fabsf(x);
-    a = a < -150.0f ? -150.0f : a;  // 0 either way, and r stays a number
-    const float t = a * kLog2e;
-    const float r = __builtin_fmaf(a, kLog2eLo, __builtin_fmaf(a, kLog2e, -t));
-    float ex = __builtin_amdgcn_exp2f(t);
-    ex = __builtin_fmaf(ex, r * kLn2, ex);
-    const float d = 1.0f + ex;  // 1 .. 2: nothing of a general division's scaling is needed
-    float inv = __builtin_amdgcn_rcpf(d);
-    inv = __builtin_fmaf(__builtin_fmaf(-d, inv, 1.0f), inv, inv);
-    return (x >= 0.0f ? 1.0f : ex) * inv;
 }
 
 // The arguments' cache lines, asked for at once as a kernel begins: left to where each field is used, they are a chain of

@@ -302,6 +302,43 @@ def test_short_walks_of_wide_work_groups(layout):
                 assert rel <= REF_BAR_MAX_REL, (before, i, rel)
 
 
+@pytest.mark.parametrize("before, tokens, cut", [(0, 37, 0), (517, 41, 1)])
+def test_gates_of_any_size_act_as_in_the_decode_kernel(before, tokens, cut):
+    # sigmoid(gate) where its exponential is subnormal or 0 (below -87.3, -103.9), saturated, infinite or NaN, and 160000
+    # ordinary gates: a row's output is the same bits as its output without a gate times what the decode kernel multiplies by
+    # (read off a sequence of one cell whose V is 1).
+    n_q = 16
+    edges = np.float32([0.0, -0.0, 1e-30, -1e-30, 17.3, -17.3, 87.0, -87.0, -87.3, -87.4, 88.0, -88.0, -88.8, 100.0, -100.0,
+                        -103.2, -103.9, -104.5, -110.0, 150.5, -150.5, -3e38, 3e38, np.inf, -np.inf, np.nan])
+    rng = np.random.Generator(np.random.PCG64(1060))
+    with Twin(n_pages=48, max_seqs=2) as tw:
+        s, one = tw.pool.seq_create(), tw.pool.seq_create()
+        fill(tw, s, before + tokens, rng, chunk=64)
+        tw.pool.seq_reserve(one, 1)
+        tw.append(0, [one], [0], [np.zeros((1, 2, 256), np.float32)], [np.ones((1, 2, 256), np.float32)])
+        q = rng.standard_normal((tokens, n_q, 256)).astype(np.float32)
+        gate = (rng.standard_normal((tokens, n_q, 256)) * 20).astype(np.float32)
+        gate[:, :, 3:3 + edges.size] = edges
+        sig = tw.decode_attn(0, [one] * tokens, [0] * tokens, q, n_q, scale=1.0 / 16.0, gate=gate)
+        # expf is good to 1 ulp (2^-23), the sum and the quotient add 2^-24 each; subnormal results have steps of 2^-149
+        with np.errstate(over="ignore", invalid="ignore"):
+            g = gate.astype(np.float64)
+            want = np.where(g >= 0, 1.0 / (1.0 + np.exp(-g)), np.exp(g) / (1.0 + np.exp(g)))
+            want[g == np.inf] = 1.0
+            off = np.abs(sig.astype(np.float64) - want) <= want * 2.0 ** -22 + 2.0 ** -148
+        assert np.all(off | np.isnan(g)) and np.all(np.isnan(sig) == np.isnan(g))
+        plain = prefill(tw, 0, [s], [before], [q], n_q)[0]
+        tw.pool.timing_enable(True)
+        gated = prefill(tw, 0, [s], [before], [q], n_q, [gate])[0]
+        device_sync()
+        tw.pool.timing_enable(False)
+        assert tw.pool.timing_read(L.STAGE_ATTN_MERGE)[0] == cut
+        same = gated.view(np.uint32) == (plain * sig).view(np.uint32)
+        bad = np.argwhere(~(same | np.isnan(g)))
+        assert bad.size == 0, (len(bad), [float(gate[tuple(i)]) for i in bad[:8]])
+        assert np.all(np.isnan(gated) == np.isnan(g))
+
+
 @pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H])
 @pytest.mark.parametrize("n_q, before, tokens, bad", [
     (16, 24, 40, 32),     # rows of the first waves end a pair of pages before the work-group does
