@@ -160,6 +160,12 @@ __device__ __forceinline__ T held(T x) {
     asm volatile("" : "+s"(x));
     return x;
 }
+// A pointer that came through `held` is not known to be to global memory any more: used as it is, each access is a flat one,
+// which LDS counts too and which are waited for together.
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* in_global(T* p) {
+    return (__attribute__((address_space(1))) T*)p;
+}
 
 // two f32 numbers as f16, rounded to nearest
 __device__ __forceinline__ h2m to_f16(float a, float b) {
@@ -934,8 +940,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             }
         }
         const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        float* op = out + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
-        const float* gp = gate + (size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride;
+        const auto op = in_global(out) + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
         // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
         // chain of 64 trips to memory
 #pragma unroll
@@ -945,10 +950,10 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
             if (gate) {
                 f4 z[8];
-                const float* at = gp + 128 * half + 4 * g;
+                const auto at = in_global(gate) + ((size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride + 128 * half + 4 * g);
                 if (gate_in_fours) {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) z[i] = *reinterpret_cast<const f4*>(at + 16 * i);
+                    for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)(at + 16 * i);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
@@ -961,7 +966,7 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
                     for (int r = 0; r < 4; ++r) y[i][r] *= sigmoid(z[i][r]);
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) *reinterpret_cast<f4*>(op + 16 * (half * 8 + i) + 4 * g) = y[i];
+            for (int i = 0; i < 8; ++i) *(__attribute__((address_space(1))) f4*)(op + 16 * (half * 8 + i) + 4 * g) = y[i];
         }
     }
 }

@@ -1,25 +1,36 @@
 """Registers of the attention kernels, as the compiler reports them: a kernel that spills pays for it on every page
 it walks.  No device is needed."""
+import functools
 import os
 import re
 import shutil
 import subprocess
+import tempfile
 
 import pytest
 
 from breccia_amd import build
 
 
-def scratch_of_kernels(source):
+@functools.lru_cache(maxsize=None)
+def compiled(source):
+    """-> what the compiler says of each kernel's resources, and its assembly"""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc here")
-    proc = subprocess.run([hipcc] + build.HIP_FLAGS + build.FILE_FLAGS.get(source, []) +
-                          ["--cuda-device-only", "-Rpass-analysis=kernel-resource-usage",
-                           "-I", os.path.join(build.HERE, "..", "include"), "-c", os.path.join(build.CSRC, source),
-                           "-o", os.devnull], capture_output=True, text=True)
-    assert proc.returncode == 0, proc.stderr[-2000:]
-    return dict(re.findall(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", proc.stderr, re.S))
+    with tempfile.TemporaryDirectory() as tmp:
+        asm = os.path.join(tmp, "kernels.s")
+        proc = subprocess.run([hipcc] + build.HIP_FLAGS + build.FILE_FLAGS.get(source, []) +
+                              ["--cuda-device-only", "-Rpass-analysis=kernel-resource-usage",
+                               "-I", os.path.join(build.HERE, "..", "include"), "-S", os.path.join(build.CSRC, source),
+                               "-o", asm], capture_output=True, text=True)
+        assert proc.returncode == 0, proc.stderr[-2000:]
+        with open(asm) as f:
+            return proc.stderr, f.read()
+
+
+def scratch_of_kernels(source):
+    return dict(re.findall(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", compiled(source)[0], re.S))
 
 
 def test_step_kernels_do_not_spill():
@@ -36,3 +47,12 @@ def test_chunk_kernels_do_not_spill():
     chunk = {k: int(v) for k, v in scratch.items() if "prefill_attn_kernel" in k}
     assert len(chunk) == 7, sorted(scratch)
     assert not any(chunk.values()), chunk
+
+
+@pytest.mark.parametrize("source", ["decode_attn_mfma.hip", "prefill_attn.hip", "kv_move.hip", "select.hip"])
+def test_kernels_know_which_memory_they_access(source):
+    # a pointer that the compiler has lost sight of (it went through integers or asm) makes flat accesses: LDS counts them
+    # too, and what waits for one waits for all LDS reads
+    text = compiled(source)[1]
+    assert re.search(r"^\s+global_load", text, re.M)
+    assert not re.findall(r"^\s+flat_\w+", text, re.M)
