@@ -197,7 +197,7 @@ __device__ __forceinline__ void load_to_lds(unsigned lds, page_ptr base, unsigne
     asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
                  : "=&s"(at)
                  : "s"(lds), "v"(lane_off), "s"(base)
-                 : "memory");
+                 : "m0", "memory");
 }
 __device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

@@ -56,3 +56,19 @@ def test_kernels_know_which_memory_they_access(source):
     text = compiled(source)[1]
     assert re.search(r"^\s+global_load", text, re.M)
     assert not re.findall(r"^\s+flat_\w+", text, re.M)
+
+
+def test_inline_assembly_declares_the_registers_it_names():
+    # m0, vcc and the like, written inside a block and not among its clobbers, would be lost to a compiler that keeps a value there
+    blocks = 0
+    for name in sorted(os.listdir(build.CSRC)):
+        with open(os.path.join(build.CSRC, name)) as f:
+            text = f.read()
+        for stmt in re.findall(r"\basm(?:\s+volatile)?\s*\((.*?)\);", text, re.S):
+            parts = re.split(r":(?=(?:[^\"]*\"[^\"]*\")*[^\"]*$)", stmt)  # at the colons outside of strings
+            clobbers = parts[3] if len(parts) > 3 else ""
+            for line in re.split(r"\\n\\t|\\n", "".join(re.findall(r'"((?:[^"\\]|\\.)*)"', parts[0]))):
+                written = re.match(r"\s*[sv]_\w+\s+(m0|vcc\w*|exec\w*|scc)\b", line)
+                blocks += 1
+                assert not written or '"%s"' % written.group(1) in clobbers, (name, line)
+    assert blocks > 10
