@@ -194,10 +194,15 @@ __device__ __forceinline__ void load_to_lds(unsigned lds, page_ptr base, unsigne
     // (the base came from a VALU instruction, which a vector-memory one must not follow closely: the copy is a scalar
     // instruction, and the wait state that m0 wants)
     uint64_t at;
+    // (m0 is reserved: the compiler keeps nothing there of its own accord, and warns that it would not; what it must not do is
+    // let a value that it puts there for an instruction of its own live across this)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
     asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
                  : "=&s"(at)
                  : "s"(lds), "v"(lane_off), "s"(base)
                  : "m0", "memory");
+#pragma clang diagnostic pop
 }
 __device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
