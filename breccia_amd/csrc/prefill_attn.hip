@@ -236,67 +236,17 @@ struct PrefillLds {
 __device__ __forceinline__ int k_at(int row, int chunk) { return (row >> 1) * kLdsRowsK + (row & 1) * 512 + (chunk ^ (row & 1)) * 16; }
 __device__ __forceinline__ int v_at(int row, int chunk) { return (row >> 1) * kLdsRowsV + (row & 1) * 512 + (chunk ^ 2 * (row & 1)) * 16; }
 
-// TILES: tiles of 16 query rows a wave owns.
-// SPLIT: a work-group walks one range of its block's pages and leaves a partial result.
-template <int LAY, int TILES, bool SPLIT = false>
-__global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
-    const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams> P) {
+// A row block's walk, or one range of it.  TILES: tiles of 16 query rows a wave owns; the block's n_rows - rb * WG_ROWS first
+// rows are dealt to the waves in that size.
+template <int LAY, int TILES, int WG_ROWS, bool SPLIT>
+__device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams>& P,
+                                           PrefillLds<LAY>& L, int e, int kvh, int idx, int rb, int range, bool cut) {
     constexpr bool Q8V = LAY == BKV_LAYOUT_Q8V;
     constexpr bool I8H = LAY == BKV_LAYOUT_I8H;
     constexpr bool WIDE = LAY != BKV_LAYOUT_F16;  // V (int8 pools: K too) as two f16 images
-    constexpr int kWavesPerWg = 4;
     constexpr int kRows = kRowsPerWave * TILES;
-    constexpr int kRowsPerWg = kRows * kWavesPerWg;
-    now(P.b, P.n_kv, P.by_xcd);
-    if constexpr (SPLIT) now(P.s);
-    // ---- which (entry, kv head, block of query rows) ---------------------------------
-    int e = 0, kvh, idx;  // idx: which of the unit's blocks, in dispatch order
-    int range = 0;       // which range of the block's pages
-    bool cut = false;    // the block is cut at all
-    if constexpr (SPLIT) {
-        while (e + 1 < P.b.n && (int)blockIdx.x >= P.s.wg_base[e + 1]) ++e;
-        int rem = (int)blockIdx.x - P.s.wg_base[e];
-        // uncut blocks first: the longest of them are longer than a range
-        const int blocks = (P.b.n_tok[e] * P.group + kRowsPerWg - 1) / kRowsPerWg;
-        const int uncut = (blocks - P.s.n_cut[e]) * P.n_kv;
-        cut = rem >= uncut;
-        if (cut) {
-            rem -= uncut;
-            range = rem % P.s.splits[e];
-            rem /= P.s.splits[e];
-        }
-        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh) + (cut ? 0 : P.s.n_cut[e]);
-    } else if (P.by_xcd) {
-        const int units = P.b.n * P.n_kv;
-        const int x = (int)blockIdx.x % kXcds;
-        int j = (int)blockIdx.x / kXcds;
-        int u;
-        if (units >= kXcds) {
-            u = x;
-            for (;;) {
-                if (u >= units) return;  // this die's share of the grid is shorter than the longest
-                const int nb = (P.b.n_tok[divided_by(u, P.n_kv, P.n_kv_inverse)] * P.group + kRowsPerWg - 1) / kRowsPerWg;
-                if (j < nb) break;
-                j -= nb;
-                u += kXcds;
-            }
-            idx = j;
-        } else {
-            u = x % units;
-            const int dies = (kXcds - u + units - 1) / units;  // dies x with x % units == u
-            idx = j * dies + x / units;
-        }
-        e = divided_by(u, P.n_kv, P.n_kv_inverse, kvh);
-    } else {
-        while (e + 1 < P.b.n && (int)blockIdx.x >= P.b.wg_base[e + 1]) ++e;
-        const int rem = (int)blockIdx.x - P.b.wg_base[e];
-        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh);
-    }
+    constexpr int kRowsPerWg = WG_ROWS;
     const int n_rows = P.b.n_tok[e] * P.group;  // query rows of this kv head
-    const int n_blocks = (n_rows + kRowsPerWg - 1) / kRowsPerWg;
-    if (idx >= n_blocks) return;
-    // later rows attend more cells: the heaviest blocks are dispatched first
-    const int rb = n_blocks - 1 - idx;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int c = lane & 15;  // query row of the tile / cell of the page / output column group
@@ -353,7 +303,6 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
     const size_t v_head_off = (size_t)kvh * kPage * kVRow;
 
     // ---- table entries, on which everything waits ----------------------------------------------------------------
-    __shared__ __attribute__((aligned(16))) PrefillLds<LAY> L;
     const int tid = threadIdx.x;
     const int last_pg = wg_pages - 1;
     // The table's entries come through the vector path (lane parity picks the page of a pair, past the end the last page
@@ -787,9 +736,10 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
                 }
         }
     };
-    // Fragments asked for ahead of their products.  1 to 3 of K and 3 to 6 of V were measured: f16 271 us with 3 and 3 (others 273
-    // to 281), q8_0 V 521 with 3 and 5 (525 to 535, 528 with 3 and 3), int8 348 with 2 and 5 (351 to 360, 359 with 3 and 3).
-    constexpr int kAheadK = I8H ? 2 : 3, kAheadV = WIDE ? 5 : 3;
+    // Fragments asked for ahead of their products, K and V.  Measured with two tiles a wave, append included: 4 chunks of 1024
+    // behind 2048 cells, f16, 288 us with 4 and 3 (289 with 4 and 4, 291 with 3 and 3, 4 and 5).  The kernel alone, same chunks:
+    // q8_0 V 521 us with 3 and 5 (525 to 535, 528 with 3 and 3), int8 348 with 2 and 5 (351 to 360, 359 with 3 and 3).
+    constexpr int kAheadK = I8H ? 2 : LAY == BKV_LAYOUT_F16 && TILES == 2 ? 4 : 3, kAheadV = WIDE ? 5 : 3;
 
     if constexpr (I8H) {
         deposit_k(0, stage_k, 0);
@@ -974,6 +924,72 @@ __global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
             for (int i = 0; i < 8; ++i) *(__attribute__((address_space(1))) f4*)(op + 16 * (half * 8 + i) + 4 * g) = y[i];
         }
     }
+}
+
+// SPLIT: a work-group walks one range of its block's pages and leaves a partial result.
+template <int LAY, int TILES, bool SPLIT = false>
+__global__ __launch_bounds__(256, TILES == 2 ? 1 : 2) void prefill_attn_kernel(
+    const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams> P) {
+    constexpr int kRowsPerWg = 4 * TILES * kRowsPerWave;
+    __shared__ __attribute__((aligned(16))) PrefillLds<LAY> L;
+    now(P.b, P.n_kv, P.by_xcd);
+    if constexpr (SPLIT) now(P.s);
+    // ---- which (entry, kv head, block of query rows) ---------------------------------
+    int e = 0, kvh, idx;  // idx: which of the unit's blocks, in dispatch order
+    int range = 0;       // which range of the block's pages
+    bool cut = false;    // the block is cut at all
+    if constexpr (SPLIT) {
+        while (e + 1 < P.b.n && (int)blockIdx.x >= P.s.wg_base[e + 1]) ++e;
+        int rem = (int)blockIdx.x - P.s.wg_base[e];
+        // uncut blocks first: the longest of them are longer than a range
+        const int blocks = (P.b.n_tok[e] * P.group + kRowsPerWg - 1) / kRowsPerWg;
+        const int uncut = (blocks - P.s.n_cut[e]) * P.n_kv;
+        cut = rem >= uncut;
+        if (cut) {
+            rem -= uncut;
+            range = rem % P.s.splits[e];
+            rem /= P.s.splits[e];
+        }
+        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh) + (cut ? 0 : P.s.n_cut[e]);
+    } else if (P.by_xcd) {
+        const int units = P.b.n * P.n_kv;
+        const int x = (int)blockIdx.x % kXcds;
+        int j = (int)blockIdx.x / kXcds;
+        int u;
+        if (units >= kXcds) {
+            u = x;
+            for (;;) {
+                if (u >= units) return;  // this die's share of the grid is shorter than the longest
+                const int nb = (P.b.n_tok[divided_by(u, P.n_kv, P.n_kv_inverse)] * P.group + kRowsPerWg - 1) / kRowsPerWg;
+                if (j < nb) break;
+                j -= nb;
+                u += kXcds;
+            }
+            idx = j;
+        } else {
+            u = x % units;
+            const int dies = (kXcds - u + units - 1) / units;  // dies x with x % units == u
+            idx = j * dies + x / units;
+        }
+        e = divided_by(u, P.n_kv, P.n_kv_inverse, kvh);
+    } else {
+        while (e + 1 < P.b.n && (int)blockIdx.x >= P.b.wg_base[e + 1]) ++e;
+        const int rem = (int)blockIdx.x - P.b.wg_base[e];
+        idx = divided_by(rem, P.n_kv, P.n_kv_inverse, kvh);
+    }
+    const int n_rows = P.b.n_tok[e] * P.group;  // query rows of this kv head
+    const int n_blocks = (n_rows + kRowsPerWg - 1) / kRowsPerWg;
+    if (idx >= n_blocks) return;
+    // later rows attend more cells: the heaviest blocks are dispatched first
+    const int rb = n_blocks - 1 - idx;
+    // Few rows in a block (a short chunk, a chunk's end): a tile a wave, all four at work.  With two, half of the waves had all
+    // of the products.  us of a call, two tiles / one (eight waves of one tile, before there were two): 64 chunks of 9 tokens
+    // behind 2000 cells, 4 kv heads of 4 heads each, int8 167 / 129 (139), q8_0 V 139 / 118 (132); 32 chunks of 8 behind 250,
+    // 2 kv heads of 8, int8 30.0 / 23.8 (26.7).
+    if (TILES == 2 && n_rows - rb * kRowsPerWg <= 4 * kRowsPerWave)
+        walk_block<LAY, 1, kRowsPerWg, SPLIT>(P, L, e, kvh, idx, rb, range, cut);
+    else
+        walk_block<LAY, TILES, kRowsPerWg, SPLIT>(P, L, e, kvh, idx, rb, range, cut);
 }
 
 // The ranges of a cut block's rows put together: one wave per row, lane d4 owns head-dim elements

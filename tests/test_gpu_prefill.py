@@ -372,6 +372,38 @@ def test_values_that_are_not_finite_stay_with_later_rows(n_q, before, tokens, ba
         assert np.array_equal(got[clear].view(np.uint32), want[clear].view(np.uint32))
 
 
+@pytest.mark.parametrize("layout", [L.LAYOUT_Q8V, L.LAYOUT_I8H])
+@pytest.mark.parametrize("n_q, tokens", [(16, 1), (16, 3), (16, 8), (6, 20), (2, 64)])
+def test_blocks_of_few_rows_give_the_same_bits(n_q, tokens, layout):
+    # Up to 64 rows of a block of 128 (8, 24, 64, 60, 64 here): a tile of sixteen a wave instead of two.  The same rows in a
+    # full block, which takes two, must agree in every bit; the oracle checks a sample.  (f16 pools take blocks of 64 here;
+    # their blocks of 128 are those of test_short_walks_of_wide_work_groups.)
+    rng = np.random.Generator(np.random.PCG64(1080 + n_q))
+    full = 128 // (n_q // 2)
+    with Twin(n_pages=48, max_seqs=4, layout=layout) as tw:
+        tw.pool.fill(0xFF)
+        for img in tw.images:
+            img.k[:] = 0xFF
+            img.v[:] = 0xFF
+        befores = [0, 15, 31, 60]  # at most 188 cells, 6 pairs of pages: a walk of 7 may be cut, and sums in another order
+        seqs = [tw.pool.seq_create() for _ in befores]
+        q = [rng.standard_normal((full, n_q, 256)).astype(np.float32) for _ in befores]
+        for s, before in zip(seqs, befores):
+            fill(tw, s, before + tokens, rng, chunk=512)
+        few = prefill(tw, 0, seqs, befores, [x[:tokens] for x in q], n_q)
+        for s, before, x, out in zip(seqs, befores, q, few):
+            _, rel = check_attn(out[-1], tw.oracle_attend(0, s, before + tokens - 1, x[tokens - 1], n_q), "behind %d" % before)
+            assert rel <= REF_BAR_MAX_REL, (before, rel)
+            fill(tw, s, before + full, rng, chunk=512)
+        tw.pool.timing_enable(True)
+        full_blocks = prefill(tw, 0, seqs, befores, q, n_q)
+        device_sync()
+        tw.pool.timing_enable(False)
+        assert tw.pool.timing_read(L.STAGE_ATTN_MERGE)[0] == 0, "no walk was meant to be cut"
+        for out, wide in zip(few, full_blocks):
+            assert np.array_equal(out.view(np.uint32), wide[:tokens].view(np.uint32))
+
+
 def test_work_group_width_does_not_change_a_bit():
     # On f16 pools a call whose chunks fill the chip runs work-groups of 128 query rows (two tiles of
     # sixteen a wave), a smaller one work-groups of 64 (one tile).  A tile's rows are computed
