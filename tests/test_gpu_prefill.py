@@ -320,7 +320,7 @@ def test_gates_of_any_size_act_as_in_the_decode_kernel(before, tokens, cut):
         gate = (rng.standard_normal((tokens, n_q, 256)) * 20).astype(np.float32)
         gate[:, :, 3:3 + edges.size] = edges
         sig = tw.decode_attn(0, [one] * tokens, [0] * tokens, q, n_q, scale=1.0 / 16.0, gate=gate)
-        # expf is good to 1 ulp (2^-23), the sum and the quotient add 2^-24 each; subnormal results have steps of 2^-149
+        # the exponential is good to 1 ulp (2^-23), the sum and the quotient add 2^-24 each; subnormal results have steps of 2^-149
         with np.errstate(over="ignore", invalid="ignore"):
             g = gate.astype(np.float64)
             want = np.where(g >= 0, 1.0 / (1.0 + np.exp(-g)), np.exp(g) / (1.0 + np.exp(g)))
