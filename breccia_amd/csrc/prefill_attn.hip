@@ -736,10 +736,13 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
                 }
         }
     };
-    // Fragments asked for ahead of their products, K and V.  Measured with two tiles a wave, append included: 4 chunks of 1024
-    // behind 2048 cells, f16, 288 us with 4 and 3 (289 with 4 and 4, 291 with 3 and 3, 4 and 5).  The kernel alone, same chunks:
-    // q8_0 V 521 us with 3 and 5 (525 to 535, 528 with 3 and 3), int8 348 with 2 and 5 (351 to 360, 359 with 3 and 3).
-    constexpr int kAheadK = I8H ? 2 : LAY == BKV_LAYOUT_F16 && TILES == 2 ? 4 : 3, kAheadV = WIDE ? 5 : 3;
+    // Fragments asked for ahead of their products, K and V, as measured with two tiles a wave (us a call, append included; what
+    // counts is less the distance than the registers that it leaves): f16, 4 chunks of 1024 behind 2048 cells, 288 with 4 and 3
+    // (289 with 4 and 4, 291 with 3 and 3 or 4 and 5); int8, 1204 tokens behind 495, 32 heads, 145.5 with 2 and 4 (151 with 2
+    // and 5, 147 with 1 and 5, 148 with 2 and 3, 152 with 3 and 4: codes of the next pair then move through the upper half of
+    // the register file, and are waited for there).  q8_0 V, a prompt of 4096, 24 heads with gate, in an earlier form of this loop: 521
+    // with 3 and 5 (525 to 535 with others).
+    constexpr int kAheadK = I8H ? 2 : LAY == BKV_LAYOUT_F16 && TILES == 2 ? 4 : 3, kAheadV = I8H ? 4 : WIDE ? 5 : 3;
 
     if constexpr (I8H) {
         deposit_k(0, stage_k, 0);
