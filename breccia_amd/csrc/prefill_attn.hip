@@ -8,7 +8,8 @@
 // used by every query row behind it), so it goes to MFMA -- unlike the decode kernel, which
 // is a GEMV per sequence.  A work-group of four waves owns 128 consecutive query rows ((token, head) pairs of one kv
 // head), two tiles of 16 a wave, and walks the pages 0..page(pos) together, two at a time.  (Small calls on f16 pools:
-// one tile a wave, 64 rows a work-group, two work-groups a compute unit.)  Per page of 16 cells and per tile:
+// one tile a wave, 64 rows a work-group, two work-groups a compute unit.  Blocks that have no more than 64 rows: one tile a
+// wave.)  Per page of 16 cells and per tile:
 //   S^T[cell][query] = K[cell][:] . Q[query][:]        v_mfma_f32_16x16x32_f16, A = K, B = Q
 //   online softmax per query (base 2), P^T in the layout S^T came out in
 //   O^T[d][query]   += V^T[d][cell] . P^T[cell][query]  v_mfma_f32_16x16x32_f16 over the 32 cells of
@@ -24,17 +25,19 @@
 // parts of each of its tiles.  With one tile a wave that is two products, and LDS has to deliver its 128 bytes a clock
 // for the matrix cores to be busy; two tiles halve it.  They need 256 registers for q and the accumulators, so a wave has
 // a SIMD (512 registers) to itself: q in the upper half of the register file, which only matrix products read, everything
-// else in the lower.  Nobody fills such a wave's gaps, hence
+// else in the lower (quantised layouts: 60 to 68 values that a step needs once or not at all share the upper half).  Nobody
+// fills such a wave's gaps, hence
 // - a pair's scores are computed a step ahead of their softmax, whose instructions stand between those products;
 // - f16 pages go from memory to LDS without passing through registers (load_to_lds);
 // - every instruction counts, a wave issues one at a time (4 cycles): packed conversions, mixed-precision remainders, page
 //   addresses worked out lane by lane.
-// Against work-groups of eight waves with a tile each, whose steps were not pipelined: 4 chunks of 1024 behind 2048 cells,
-// 16 heads, f16, 336 -> 286 us; a prompt of 4096, 24 heads, q8_0 V, 648 -> 535; three ragged chunks, int8, 175 -> 158; 41
-// tokens behind 517 cells through 12 layers 274 -> 217.  A step takes 3120 cycles on f16 pools, 4930 with q8_0 V; its products
-// alone would take 2048 and 2560.  On f16 pools the clock falls to 2.0 GHz (1200 TFLOP/s issued; registers alone, no
-// loads, reach 1430 there): power is the next bound.  Tried and slower: all of a step as one block, the output a step
-// later (305 us f16); a third pair of pages in LDS (290, 582); chunks of one fragment fenced off from each other (299).
+// Against work-groups of eight waves with a tile each, whose steps were not pipelined (us of a call, append included): 4
+// chunks of 1024 behind 2048 cells, 16 heads, f16, 332 -> 281; a prompt of 4096, 24 heads with gate, q8_0 V, 643 -> 530; three
+// ragged chunks, int8, 174 -> 157; 41 tokens behind 517 cells through 12 layers 273 -> 218.  A step takes 3140 cycles on f16
+// pools, 4860 with q8_0 V, 5450 with int8; its products alone would take 2048, 2560 and 3072.  On f16 pools the clock falls to
+// 2.1 GHz (1200 TFLOP/s issued; registers alone, no loads, reach 1430 there): power is the next bound.  Tried on the f16 case
+// and slower, 286 to 291 then: all of a step as one block, the output a step later (305); a third pair of pages in LDS (290);
+// chunks of one fragment fenced off from each other (299).
 // The V operand needs, per lane, four cells of one head-dim column of either page: a column of
 // the row-major page image.  gfx950's transposing LDS read (ds_read_b64_tr_b16) delivers exactly
 // that: within a group of 16 lanes, lane L receives element L % 4 of the 8-byte pieces that lanes
@@ -83,7 +86,6 @@ constexpr float kLoDown = 1.0f / 2048.0f;  // q's low parts enter the products t
 constexpr int kLdsRowsK = 1024 + 32;
 constexpr int kLdsRowsV = 1024 + 64;
 
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -132,7 +134,7 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
     lo = (_Float16)(x - (float)hi);
 }
 
-// x / n and the rest, for x >= 0: the inverse is below 2^32 / n by less than 1, so the product's quotient is right or one
+// x / n and the rest, for x >= 0: the inverse is below 2^32 / n by 1 at most, so the product's quotient is right or one
 // too small.  (A division by a number that only the launch knows is some 40 instructions.)
 __device__ __forceinline__ int divided_by(int x, int n, uint32_t inverse, int& rest) {
     int q = (int)__umulhi((uint32_t)x, inverse);

@@ -106,9 +106,9 @@ BKV_HD inline int split_ranges(int pages, int pps, int max_splits, int& each) {
     return (pages + each - 1) / each;
 }
 
-// Query rows one work-group of four waves owns, in tiles of 16: two tiles a wave or one.  f16 pools: 128 when the chunks make more 64-row work-groups than
-// fit the chip at two per compute unit (then sharing the page images among more rows is worth more
-// than spreading out), else 64.
+// Query rows one work-group of four waves owns, in tiles of 16: two tiles a wave or one.  f16 pools: 128 when the chunks
+// make more 64-row work-groups than fit the chip at two per compute unit (then sharing the page images among more rows is
+// worth more than spreading out), else 64.
 inline int32_t prefill_rows_per_wg(bool f16, int64_t wgs_of_64_rows, int32_t n_cu) {
     if (!f16) return 8 * kPrefillRowsPerWave;
     return wgs_of_64_rows > 2 * (int64_t)(n_cu > 0 ? n_cu : 256) ? 8 * kPrefillRowsPerWave : 4 * kPrefillRowsPerWave;
@@ -134,28 +134,29 @@ inline int32_t last_done(const std::vector<int32_t>& runs, int32_t units) {
 
 // Cuts the page walks of a small call's row blocks into ranges; false where the call is better off
 // uncut.  A row block's walk is a serial chain: 0.9 us a page pair on f16 pools when the compute unit
-// has nothing else (2.1-2.4 us on the quantised ones, whose blocks are twice as long), and a call of a few blocks is as
+// has nothing else (2.1-2.3 us on the quantised ones, whose blocks are twice as long), and a call of a few blocks is as
 // long as its longest chain while most of the chip idles (41 tokens behind 517 cells: 12 work-groups).  Cutting
-// pays for a second kernel (4-9 us, by the partial rows it reads), so (us of a layer: append and attention):
+// pays for a second kernel (4-9 us, by the partial rows it reads), so:
 // - a call that leaves half of the compute units idle is cut if
 //   - a range keeps at least 3 pairs (quantised: 2), the fixed cost of a work-group being worth several, and
-//   - the chain loses 10 pairs (quantised: 5): 400 tokens from scratch (13 pairs to 5) measured 24.4 us
-//     uncut and 24.2 cut, 300 behind 200 cells (16 to 4) 25.4 and 25.8;
+//   - the chain loses 10 pairs (quantised: 5): 300 tokens behind 200 cells (16 pairs to 4) 22.9 us uncut, 22.4 cut;
 //   - into one work-group per compute unit, or on f16 pools two (what fits) where a range would still be longer
 //     than 8 pairs: 64 tokens behind 2000 cells 30.4 us with one, 35.0 with two; 100 behind 8000: 66.0 and 56.8
-//     (these four with the kernel of one tile a wave in all calls: 24.2 and 45.4 us now);
+//     (append included, with eight-wave work-groups; 20.3 and 43.2 without the append now);
 // - a larger call on a quantised pool (f16 pools take work-groups half as long there, two a compute unit) of up to
 //   two work-groups a compute unit may be cut, into ranges of an even share of the pairs;
 // - either way the chain has to lose a pair for every 32 partial results the second kernel reads; in the larger calls,
 //   where the ranges come on top of a chip that is nearly busy, for every 24, and for every 20 if they don't all find a
-//   compute unit at once (the chain of a cut call is then the schedule's).  The ratios come from 260 calls a layout, random
-//   and at the edges, each measured cut and uncut with a kernel of eight waves a work-group: a pair less gained 2.5 us (f16
-//   1.4), a partial result cost 0.04 (f16 0.03), in the larger calls 0.17.  They hold for the present one, uncut and cut:
-//   four chunks of 270 from scratch, left uncut, 38 and, with a ratio of longest walk to even share, 52; 600 with 48
-//   heads, left uncut, 59; two chunks of 530 54 / 44 (int8 59 / 46), 1900 144 / 130 (162 / 137), 400 with 48 heads 46 / 41
-//   (49 / 43), two of 530 behind 700 100 / 97.
-// Uncut / cut, us a layer: 41 tokens behind 517 cells 25.9 / 19.3, 100 behind 8000 237 / 45, 200 behind
-// 3000 with q8_0 V 223 / 55, 300 behind 1000 on an int8 pool 110 / 43, 900 behind 2000 226 / 136.
+//   compute unit at once (the chain of a cut call is then the schedule's).
+// The ratios were fitted to a kernel of eight waves a work-group: a pair less gained 2.5 us (f16 1.4), a partial result cost
+// 0.04 (f16 0.03), in the larger calls 0.17.  A pair is a third cheaper now and they have not been fitted again; what they do
+// was measured, though: of 258 calls, random ones and those named here, on the three layouts, 107 are cut and take 0.38 of
+// their time uncut on average; two of them on either quantised layout are slower for it: 60 chunks of 8 tokens behind 600
+// cells, q8_0 V 38.4 uncut and 43.4 cut (int8 43.1 and 45.8), and nine unequal ones with 64 heads, 60.4 and 65.3 (64.5
+// and 68.6).  What is left uncut and might pay was not looked at.
+// us, uncut / cut: 41 tokens behind 517 cells 24.2 / 15.0, 100 behind 8000 249 / 43, 200 behind 3000 with q8_0 V 214 / 48,
+// 300 behind 1000 on an int8 pool 103 / 39, 900 behind 2000 218 / 130; two chunks of 530 q8_0 V 48 / 39 (int8 52 / 41), 1900
+// from scratch 134 / 123 (148 / 130), 400 with 48 heads 40 / 37 (44 / 38), two of 530 behind 700 92 / 87 (101 / 92).
 // chain: page pairs of the cut call's longest chain, where it was worked out.
 inline bool plan_prefill_split(const PrefillPlanLimits& lim, const PrefillBatch& b, int32_t rows, int32_t group, PrefillSplit& s,
                                int32_t& chain) {

@@ -42,11 +42,25 @@ def test_step_kernels_do_not_spill():
 
 
 def test_chunk_kernels_do_not_spill():
-    # 512 registers of a lone wave, q in the upper half: f16 with one tile a wave and two, both quantised layouts, cut and not
+    # 512 registers of a lone wave: f16 with one tile a wave and two, both quantised layouts, cut and not
     scratch = scratch_of_kernels("prefill_attn.hip")
     chunk = {k: int(v) for k, v in scratch.items() if "prefill_attn_kernel" in k}
     assert len(chunk) == 7, sorted(scratch)
     assert not any(chunk.values()), chunk
+
+
+def test_chunk_kernels_hold_little_beside_q_in_the_upper_registers():
+    # Before a wave of 512 registers spills to memory it moves values through its upper half, which the VALU cannot read.
+    # q of two tiles takes 128 there.  Quantised pages: what else lives there is needed once a step or less, fewer than 72
+    # values; more, and codes that were just requested are among them (and waited for).
+    remarks, text = compiled("prefill_attn.hip")
+    upper = {k: int(v) for k, v in re.findall(r"Function Name: (\S+).*?AGPRs: (\d+)", remarks, re.S) if "prefill_attn_kernel" in k}
+    assert len(upper) == 7, sorted(upper)
+    for name, count in upper.items():
+        layout, tiles = map(int, re.search(r"prefill_attn_kernelILi(\d)ELi(\d)", name).groups())
+        body = text[text.index("\n" + name + ":"):]
+        back = len(re.findall(r"^\s+v_accvgpr_read", body[:body.index(".Lfunc_end")], re.M))
+        assert (count, back) == (0, 0) if tiles == 1 else (count, back) == (128, 0) if layout == 0 else count < 128 + 72, (name, count, back)
 
 
 @pytest.mark.parametrize("source", ["decode_attn_mfma.hip", "prefill_attn.hip", "kv_move.hip", "select.hip"])
