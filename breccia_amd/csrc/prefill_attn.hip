@@ -238,8 +238,8 @@ struct PrefillLds {
 __device__ __forceinline__ int k_at(int row, int chunk) { return (row >> 1) * kLdsRowsK + (row & 1) * 512 + (chunk ^ (row & 1)) * 16; }
 __device__ __forceinline__ int v_at(int row, int chunk) { return (row >> 1) * kLdsRowsV + (row & 1) * 512 + (chunk ^ 2 * (row & 1)) * 16; }
 
-// A row block's walk, or one range of it.  TILES: tiles of 16 query rows a wave owns; the block's n_rows - rb * WG_ROWS first
-// rows are dealt to the waves in that size.
+// A row block's walk, or one range of it, by the four waves of a work-group.  TILES: tiles of 16 query rows a wave owns, the
+// block's rows dealt to the waves in order.  WG_ROWS: rows of a full block, 64 per tile or more.
 template <int LAY, int TILES, int WG_ROWS, bool SPLIT>
 __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, PrefillSplitParams, PrefillKernelParams>& P,
                                            PrefillLds<LAY>& L, int e, int kvh, int idx, int rb, int range, bool cut) {
@@ -742,8 +742,8 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     // counts is less the distance than the registers that it leaves): f16, 4 chunks of 1024 behind 2048 cells, 288 with 4 and 3
     // (289 with 4 and 4, 291 with 3 and 3 or 4 and 5); int8, 1204 tokens behind 495, 32 heads, 145.5 with 2 and 4 (151 with 2
     // and 5, 147 with 1 and 5, 148 with 2 and 3, 152 with 3 and 4: codes of the next pair then move through the upper half of
-    // the register file, and are waited for there).  q8_0 V, a prompt of 4096, 24 heads with gate, in an earlier form of this loop: 521
-    // with 3 and 5 (525 to 535 with others).
+    // the register file, and are waited for there).  q8_0 V, a prompt of 4096, 24 heads with gate, in an earlier form of this
+    // loop: 521 with 3 and 5 (525 to 535 with others).
     constexpr int kAheadK = I8H ? 2 : LAY == BKV_LAYOUT_F16 && TILES == 2 ? 4 : 3, kAheadV = I8H ? 4 : WIDE ? 5 : 3;
 
     if constexpr (I8H) {
@@ -910,7 +910,8 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
             for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
             if (gate) {
                 f4 z[8];
-                const auto at = in_global(gate) + ((size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride + 128 * half + 4 * g);
+                const auto at = in_global(gate) + ((size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride +
+                                                   128 * half + 4 * g);
                 if (gate_in_fours) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)(at + 16 * i);
