@@ -11,9 +11,11 @@
 // folded in LDS and written as one partial per work-group; the merge kernel combines the page
 // ranges of a head and applies sigmoid(gate).
 #include <atomic>
+#include <type_traits>
 
 #include "decode_attn_common.hpp"
 #include "gate.hpp"
+#include "lane_groups.hpp"
 
 namespace bkv {
 
@@ -31,27 +33,70 @@ struct MergeParams {
     uint32_t inv_group16;  // small_divisor_inverse(group)
 };
 
-constexpr int kMergeGroups = 16;   // waves of a work-group; wave g sums splits g, g + 16, ...
-constexpr int kMergeInFlight = 8;  // partial rows (16 bytes a lane) a wave requests per round
+constexpr int kMergeWaves = 4;
+constexpr int kMergeCols = 64;                  // columns of a work-group
+constexpr int kMergeGroups = kMergeWaves * 4;   // 16 lanes, 4 columns each, sum splits i, i + kMergeGroups, ...
+constexpr int kMergeInFlight = 6;               // partial rows a lane requests at most per round
 
-// One work-group per (entry, q head): 16 waves.  Lane d4 of wave g owns head-dim elements
-// 4 d4 .. 4 d4 + 3 of splits g, g + 16, ...; it requests its first 8 partial rows straight away,
-// and only then are the per-split (m, l) pairs staged in LDS and the maximum agreed, so the two
-// round trips to memory overlap.  One round covers 128 splits.
+// A lane's share of a head: splits at, at + kMergeGroups, ... under a maximum of its own.
+struct MergeSum {
+    f4 o = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    float l = 0.0f, m = -INFINITY;
+};
+// exp2(x - ref), and 0 where nothing has been attended yet (both -inf)
+__device__ __forceinline__ float weight_of(float x, float ref) { return __builtin_amdgcn_exp2f(x - (ref == -INFINITY ? 0.0f : ref)); }
+
+// N rounds of kMergeGroups splits from split s0 on, everything requested before the first use and without branches:
+// past the end the last split is requested again and gets no weight.
+template <int N>
+__device__ __forceinline__ void merge_rounds(const float* po, const float* pml, uint32_t lane_at, uint32_t ostride, uint32_t mlstride, int s0, int splits,
+                                             MergeSum& a) {
+    float m[N], l[N];
+    f4 v[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const uint32_t s = (uint32_t)min(s0 + u * kMergeGroups, splits - 1);
+        const float2 ml = *reinterpret_cast<const float2*>(pml + s * mlstride);
+        m[u] = ml.x, l[u] = ml.y;
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const uint32_t s = (uint32_t)min(s0 + u * kMergeGroups, splits - 1);
+        v[u] = *reinterpret_cast<const f4*>(po + (s * ostride + lane_at));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float mx = a.m;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        m[u] = s0 + u * kMergeGroups < splits ? m[u] : -INFINITY;
+        mx = fmaxf(mx, m[u]);
+    }
+    const float keep = weight_of(a.m, mx);
+    a.o *= keep;
+    a.l *= keep;
+    a.m = mx;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const float f = weight_of(m[u], mx);
+        a.o += v[u] * f;
+        a.l = fmaf(f, l[u], a.l);
+    }
+}
+
+// One work-group per (entry, q head, quarter of the columns).  The kernel is a chain of trips -- arguments, partial
+// results, output -- and what stands between them.  With a work-group of 16 waves a head, (m, l) staged in LDS and the
+// maximum agreed ahead of the sums, it was 6900 cycles for one sequence of 4096 cells (65 splits), 5400 for four of up to
+// 2048 and 6100 for eight of up to 32k.  Every 16 lanes now keep a maximum of their own and everything meets once, at the
+// end, and a quarter of a head is what one compute unit takes in a quarter of the time (64 bytes a clock): 4000, 3400, 3600.
 template <bool DESC>
-__global__ __launch_bounds__(64 * kMergeGroups) void decode_attn_merge_kernel(const MergeParams P) {
-    constexpr int kMaxStaged = 1024;
-    constexpr int kThreads = 64 * kMergeGroups;
-    __shared__ float sm[kMaxStaged];
-    __shared__ float sl[kMaxStaged];
-    __shared__ __attribute__((aligned(16))) float red[kMergeGroups][kHd];
-    __shared__ float red_l[kMergeGroups];
-    __shared__ float wave_max[kMergeGroups];
-    // grid (q heads, entries): no division at the head of a kernel that is all latency
+__global__ __launch_bounds__(64 * kMergeWaves) void decode_attn_merge_kernel(const MergeParams P) {
+    __shared__ __attribute__((aligned(16))) float red[kMergeWaves][kMergeCols];
+    __shared__ __attribute__((aligned(16))) float red_m[kMergeWaves], red_l[kMergeWaves];
+    // grid (q heads x quarters, entries): no division at the head of a kernel that is all latency, and every argument
+    // is asked for at once
     const int e = blockIdx.y;
-    const int h = blockIdx.x;
-    const int kvh = small_div(h, P.inv_group16);
-    const int hl = h - kvh * P.group;
+    const int h = blockIdx.x / (kHd / kMergeCols);
+    const int col = blockIdx.x % (kHd / kMergeCols) * kMergeCols;
     int splits, base;
     if constexpr (DESC) {
         const batch_desc_ptr D = (batch_desc_ptr)(uintptr_t)P.bd;
@@ -61,91 +106,61 @@ __global__ __launch_bounds__(64 * kMergeGroups) void decode_attn_merge_kernel(co
         splits = P.b.splits[e];
         base = P.b.wg_base[e];
     }
-    const int wg0 = base + kvh;
-    const int d4 = threadIdx.x & 63;
-    const int g = threadIdx.x >> 6;
-    const size_t ostride = (size_t)P.n_kv * P.group * kHd;  // floats between consecutive splits
-    const float* po = P.part_o + ((size_t)wg0 * P.group + hl) * kHd + 4 * d4;
-    const float* pml = P.part_ml + ((size_t)wg0 * P.group + hl) * 2;
-    const size_t mlstride = (size_t)P.n_kv * P.group * 2;
-
-    f4 v[kMergeInFlight];
-#pragma unroll
-    for (int u = 0; u < kMergeInFlight; ++u) {
-        const int s = g + u * kMergeGroups;
-        v[u] = s < splits ? *reinterpret_cast<const f4*>(po + (size_t)s * ostride) : f4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    asm volatile("" ::"s"(splits), "s"(base), "s"(P.part_o), "s"(P.part_ml), "s"(P.gate), "s"(P.out), "s"(P.gate_seq_stride), "s"(P.gate_head_stride),
+                 "s"(P.n_kv), "s"(P.n_q), "s"(P.group), "s"(P.inv_group16));
+    const int kvh = small_div(h, P.inv_group16);
+    const int hl = h - kvh * P.group;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // the gate of the element this thread writes at the end is requested with the partial rows, not after
     // the sums (a trip to memory at the tail of a kernel that is all latency)
     float gt = 0.0f;
-    if (P.gate && threadIdx.x < kHd)
-        gt = P.gate[(size_t)e * P.gate_seq_stride + (size_t)h * P.gate_head_stride + threadIdx.x];
-    // stage (m, l) and agree on the maximum: per-thread max over its splits, wave reduction,
-    // then one LDS slot per wave (a serial scan over the splits would cost a dependent LDS
-    // round trip per split)
-    float my_m = -INFINITY;
-    for (int s = threadIdx.x; s < splits; s += kThreads) {
-        const float ms = pml[(size_t)s * mlstride];
-        if (s < kMaxStaged) {
-            sm[s] = ms;
-            sl[s] = pml[(size_t)s * mlstride + 1];
-        }
-        my_m = fmaxf(my_m, ms);
+    if (P.gate && wave == 0) gt = P.gate[(size_t)e * P.gate_seq_stride + (size_t)h * P.gate_head_stride + col + lane];
+    const size_t head = ((size_t)(base + kvh) * P.group + hl);  // the first split's row
+    // floats between consecutive splits; the workspace is 33.6 MB, 32 bits hold any offset in it
+    const uint32_t ostride = (uint32_t)(P.n_kv * P.group * kHd), mlstride = (uint32_t)(P.n_kv * P.group * 2);
+    static_assert((uint64_t)kMaxWgs * 8 * kHd * sizeof(float) < (1ull << 32), "32-bit offsets");
+    const float* const po = P.part_o + head * kHd + col;
+    const float* const pml = P.part_ml + head * 2;
+    const uint32_t lane_at = 4u * (uint32_t)(lane & 15);
+    const int at = threadIdx.x >> 4;
+    MergeSum a;
+    const auto rounds = [&](auto n, int s0) { merge_rounds<decltype(n)::value>(po, pml, lane_at, ostride, mlstride, s0, splits, a); };
+    if (splits <= kMergeGroups) {
+        rounds(std::integral_constant<int, 1>(), at);
+    } else if (splits <= 2 * kMergeGroups) {
+        rounds(std::integral_constant<int, 2>(), at);
+    } else if (splits <= 4 * kMergeGroups) {
+        rounds(std::integral_constant<int, 4>(), at);
+    } else {
+        for (int s0 = 0; s0 < splits; s0 += kMergeInFlight * kMergeGroups) rounds(std::integral_constant<int, kMergeInFlight>(), s0 + at);
     }
+    // the four 16-lane groups of a wave, then the waves
+    const float m_wave = max_over_lane_groups(a.m);
+    const float f = weight_of(a.m, m_wave);
+    f4 o;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) my_m = fmaxf(my_m, __shfl_xor(my_m, off, 64));
-    if ((threadIdx.x & 63) == 0) wave_max[g] = my_m;
+    for (int k = 0; k < 4; ++k) o[k] = sum_over_lane_groups(a.o[k] * f);
+    const float l_wave = sum_over_lane_groups(a.l * f);
+    if (lane < 16) *reinterpret_cast<f4*>(&red[wave][4 * lane]) = o;
+    if (lane == 0) {
+        red_m[wave] = m_wave;
+        red_l[wave] = l_wave;
+    }
     __syncthreads();
-    const auto m_of = [&](int s) { return s < kMaxStaged ? sm[s] : pml[(size_t)s * mlstride]; };
-    const auto l_of = [&](int s) { return s < kMaxStaged ? sl[s] : pml[(size_t)s * mlstride + 1]; };
-    float mx = wave_max[0];
-#pragma unroll
-    for (int w = 1; w < kMergeGroups; ++w) mx = fmaxf(mx, wave_max[w]);
-    f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    float lsum = 0.0f;
-#pragma unroll
-    for (int u = 0; u < kMergeInFlight; ++u) {
-        const int s = g + u * kMergeGroups;
-        if (s < splits) {
-            const float ms = m_of(s);
-            const float f = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - mx);
-            acc += v[u] * f;
-            lsum = fmaf(f, l_of(s), lsum);
-        }
-    }
-    // further rounds for split lists beyond 128
-    for (int s0 = g + kMergeInFlight * kMergeGroups; s0 < splits; s0 += kMergeInFlight * kMergeGroups) {
-#pragma unroll
-        for (int u = 0; u < kMergeInFlight; ++u) {
-            const int s = s0 + u * kMergeGroups;
-            v[u] = s < splits ? *reinterpret_cast<const f4*>(po + (size_t)s * ostride) : f4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (int u = 0; u < kMergeInFlight; ++u) {
-            const int s = s0 + u * kMergeGroups;
-            if (s < splits) {
-                const float ms = m_of(s);
-                const float f = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - mx);
-                acc += v[u] * f;
-                lsum = fmaf(f, l_of(s), lsum);
-            }
-        }
-    }
-    *reinterpret_cast<f4*>(&red[g][4 * d4]) = acc;
-    if (d4 == 0) red_l[g] = lsum;
-    __syncthreads();
-    // the first four waves fold the 16 rows: thread d sums element d
-    if (threadIdx.x >= kHd) return;
-    const int d = threadIdx.x;
+    if (wave != 0) return;
+    const f4 m = *reinterpret_cast<const f4*>(red_m), l = *reinterpret_cast<const f4*>(red_l);
+    const float mx = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
     float r = 0.0f, lt = 0.0f;
 #pragma unroll
-    for (int k = 0; k < kMergeGroups; ++k) {
-        r += red[k][d];
-        lt += red_l[k];
+    for (int w = 0; w < kMergeWaves; ++w) {
+        const float fw = weight_of(m[w], mx);
+        r = fmaf(red[w][lane], fw, r);
+        lt = fmaf(l[w], fw, lt);
     }
     r = lt > 0.0f ? r / lt : 0.0f;
     if (P.gate) r *= sigmoid(gt);
-    P.out[((size_t)e * P.n_q + h) * kHd + d] = r;
+    P.out[((size_t)e * P.n_q + h) * kHd + col + lane] = r;
 }
 
 }  // namespace
@@ -268,7 +283,7 @@ hipError_t launch_decode_attn(bkv_pool* p, int32_t layer, const AttnBatch& b, co
     mp.n_q = a.n_q_head;
     mp.group = group;
     mp.inv_group16 = small_divisor_inverse(group);
-    const dim3 mgrid((unsigned)a.n_q_head, (unsigned)b.n), mblock(64 * kMergeGroups);
+    const dim3 mgrid((unsigned)a.n_q_head * (kHd / kMergeCols), (unsigned)b.n), mblock(64 * kMergeWaves);
     if (a.desc)
         hipLaunchKernelGGL(decode_attn_merge_kernel<true>, mgrid, mblock, 0, stream, mp);
     else if (a.timed)
