@@ -58,32 +58,36 @@ __device__ __forceinline__ int small_div(int x, uint32_t inv16) { return (int)((
 // (page range x kv head), and the entry's position, block-table row and pages per range.  With DESC the
 // batch is read from device memory through the constant address space (uniform addresses: scalar
 // loads), and a work-group past the end of the current cut reports false: such a launch has a fixed grid.
+//
+// Finding the entry must not be a chain of loads at the head of a launch that may last five microseconds: lane i reads
+// entry i, the work-group's entry is found with a ballot, and the scalar arguments are asked for at the same time, one
+// trip to memory for any batch (cycles from a work-group's first instruction to here: searched entry by entry, with what
+// was found and the pointers loaded after that, 900 for one entry, 1200 for four and 100 more with each; now 900).
 typedef const __attribute__((address_space(4))) AttnBatch* batch_desc_ptr;
-template <bool DESC>
+__device__ __forceinline__ int lane_of_wave() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+template <bool STEP, bool DESC, typename Batch>
+__device__ __forceinline__ bool find_unit(const AttnKernelParams& P, const Batch& B, int unit, int& e, int& rem, int& pos, int& row, int& pps) {
+    static_assert(kMaxBatch <= 64, "one lane per entry");
+    const int lane = lane_of_wave();  // not kept for later: the kernels have no register to spare for it
+    const int first = B.wg_base[lane], my_pos = B.pos[lane], my_row = B.row[lane], my_pps = B.pps[lane];
+    const int n = B.n;
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(n), "s"(P.kpool), "s"(P.vpool), "s"(P.tables), "s"(P.q), "s"(P.max_pages_per_seq), "s"(P.n_kv), "s"(P.n_q),
+                 "s"(P.group), "s"(P.inv_kv16), "s"(P.part_o), "s"(P.part_ml), "s"(P.scale_log2e));
+    if constexpr (STEP) asm volatile("" ::"s"(P.new_k), "s"(P.new_v), "s"(P.kpool_w), "s"(P.vpool_w));
+    if (DESC && unit >= B.wg_base[n]) return false;
+    e = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < n && unit >= first)) - 1;
+    rem = unit - __builtin_amdgcn_readlane(first, e);
+    pos = __builtin_amdgcn_readlane(my_pos, e);
+    row = __builtin_amdgcn_readlane(my_row, e);
+    pps = __builtin_amdgcn_readlane(my_pps, e);
+    return true;
+}
+template <bool STEP, bool DESC>
 __device__ __forceinline__ bool unit_of_work_group(const AttnKernelParams& P, int unit, int& e, int& rem, int& pos,
                                                    int& row, int& pps) {
-    if constexpr (DESC) {
-        const batch_desc_ptr D = (batch_desc_ptr)(uintptr_t)P.bd;
-        const int n = D->n;
-        if (unit >= D->wg_base[n]) return false;
-        e = 0;
-        while (e + 1 < n && unit >= D->wg_base[e + 1]) ++e;
-        rem = unit - D->wg_base[e];
-        pos = D->pos[e];
-        row = D->row[e];
-        pps = D->pps[e];
-    } else {
-        // entry 0's fields are asked for alongside n: their cache lines (sixteen entries each) are then on
-        // their way before the entry is known
-        asm volatile("" ::"s"(P.b.pos[0]), "s"(P.b.pps[0]), "s"(P.b.row[0]), "s"(P.b.wg_base[0]));
-        e = 0;
-        while (e + 1 < P.b.n && unit >= P.b.wg_base[e + 1]) ++e;
-        rem = unit - P.b.wg_base[e];
-        pos = P.b.pos[e];
-        row = P.b.row[e];
-        pps = P.b.pps[e];
-    }
-    return true;
+    if constexpr (DESC) return find_unit<STEP, true>(P, *(batch_desc_ptr)(uintptr_t)P.bd, unit, e, rem, pos, row, pps);
+    else return find_unit<STEP, false>(P, P.b, unit, e, rem, pos, row, pps);
 }
 
 // Row encodings of the K and V pools:

@@ -30,6 +30,11 @@ namespace {
 // 128 h + 8 c of rows 4 g + r.  Every fragment register is refilled with the next page's data
 // right after its last use.
 typedef _Float16 h4m __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) uint32_t* sel_list_ptr;
+typedef const __attribute__((address_space(4))) int32_t* block_table_ptr;
+__device__ __forceinline__ uint32_t pick4(const uint32_t (&a)[4], int j) {
+    return j == 0 ? a[0] : j == 1 ? a[1] : j == 2 ? a[2] : a[3];
+}
 
 __device__ __forceinline__ void split_hi_lo(float x, _Float16& hi, _Float16& lo) {
     hi = (_Float16)x;
@@ -158,6 +163,331 @@ __device__ __forceinline__ void k_pair_home(const v4u& lo_rows, const v4u& hi_ro
     odd = __builtin_bit_cast(half8, o);
 }
 
+// Of two pointers of the argument block, k's for the lower half of the wave and v's for the upper.  Both are pinned in
+// registers first: the compiler otherwise has every lane load its own from the argument block, a trip to memory on the
+// vector side.  The address space has to be named then; a flat access would have every wait be for everything.
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* k_or_v(bool is_k, T* k, T* v) {
+    uintptr_t ka = (uintptr_t)k, va = (uintptr_t)v;
+    asm("" : "+s"(ka), "+s"(va));
+    return (__attribute__((address_space(1))) T*)(is_k ? ka : va);
+}
+
+// A new f16 row (STEP), slice by slice: 8 values, from the caller's f32 row to 16 bytes of the pool.
+struct NewSliceF16 {
+    f4 a, b;
+};
+__device__ __forceinline__ void request_new_slice(const AttnKernelParams& P, int e, int kvh, bool is_k, int slice, NewSliceF16& x) {
+    const auto src = (const __attribute__((address_space(1))) f4*)(k_or_v(is_k, P.new_k, P.new_v) +
+                                                                    ((size_t)e * P.n_kv + (size_t)kvh) * kHd + slice * 8);
+    x.a = src[0];
+    x.b = src[1];
+}
+__device__ __forceinline__ v4u store_new_slice(const AttnKernelParams& P, const NewSliceF16& x, bool is_k, size_t row_off, int slice) {
+    v4u w;
+    w.x = f16_store_pair(x.a[0], x.a[1]), w.y = f16_store_pair(x.a[2], x.a[3]);
+    w.z = f16_store_pair(x.b[0], x.b[1]), w.w = f16_store_pair(x.b[2], x.b[3]);
+    *(__attribute__((address_space(1))) v4u*)(k_or_v(is_k, P.kpool_w, P.vpool_w) + row_off + (size_t)slice * 16) = w;
+    return w;
+}
+
+// ---- ranges of one page a wave -----------------------------------------------------------------
+// A range of kWaves pages (pps == kWaves: all of a context's while the batch leaves the chip room) is walked in one go,
+// and what bounds it is the chain arguments -> table -> rows -> products -> partial result, a wave's own instructions
+// included.  There the four waves split the columns, not the pages: wave w multiplies columns 64 w .. 64 w + 63 of all
+// four pages' K by the two q fragments it has split itself, the partial scores meet in LDS, each wave takes the softmax
+// of one page, and the probabilities, again through LDS, meet columns 64 w .. 64 w + 63 of the four pages' V.  As many
+// products as with a page a wave; in place of all q fragments (64 KiB read from LDS) and four outputs to be summed
+// (64 KiB written, 64 read) go 16 KiB of partial scores and 4 of probabilities.  Cycles of a work-group, four sequences
+// of up to 2048 cells: 12500, now 8800 (arguments 900, table 900, rows 2900; f16, stamped).
+struct OnePageLds {
+    f4 s[kWaves][kWaves][64];  // [page][wave][lane (c, g)]: that wave's columns' share of q[head c] . k[cell 4 g + r]
+    v4u p[kWaves][64];         // [page][lane]: high, then low parts of head c's probabilities of cells 4 g .. 4 g + 3
+    float m[16][kWaves];
+    float l[16][kWaves];
+    v4u new_row[kWaves][16];   // [wave]: its 128 bytes of the new K row, then of the new V row
+};
+__device__ __forceinline__ float max4(f4 x) { return fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])); }
+
+// From the waves' shares of the scores to the probabilities of all four pages: p[j] of lane (c, g) holds the high, then
+// the low parts of head c's probabilities of cells 4 g + r of page j.  live: of cells 4 g + r of page `wave`.  Writes
+// the work-group's (m, l).  Without a cell to attend: zeros, m = -inf and l = 0.
+// ex, down: q8_0 V only (null otherwise): what its rows' exponents take out of the values (see that kernel).
+__device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OnePageLds& L, const f4 (&part)[kWaves], const bool (&live)[4], int wg,
+                                                 int wave, int lane, v4u (&p_out)[kWaves], const int* ex = nullptr, const float* down = nullptr) {
+    const int c = lane & 15, g = lane >> 4;
+    const float scale = P.scale_log2e;
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) L.s[j][wave][lane] = part[j];
+    __syncthreads();
+    const f4 s = (L.s[wave][0][lane] + L.s[wave][1][lane]) + (L.s[wave][2][lane] + L.s[wave][3][lane]);
+    f4 t;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r] = live[r] ? s[r] * scale + (ex ? (float)ex[r] : 0.0f) : -INFINITY;
+    const float pm = max_over_lane_groups(max4(t));
+    if (g == 0) L.m[c][wave] = pm;
+    __syncthreads();
+    const float m = max4(*reinterpret_cast<const f4*>(L.m[c]));
+    const bool none = m == -INFINITY;
+    h4m phi, plo;
+    float psum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float p = none ? 0.0f : __builtin_amdgcn_exp2f(t[r] - m);
+        psum = down ? fmaf(p, down[r], psum) : psum + p;
+        _Float16 h, l;
+        split_hi_lo(p, h, l);
+        phi[r] = h;
+        plo[r] = l;
+    }
+    L.p[wave][lane] = __builtin_bit_cast(v4u, half8{phi[0], phi[1], phi[2], phi[3], plo[0], plo[1], plo[2], plo[3]});
+    psum = sum_over_lane_groups(psum);
+    if (g == 0) L.l[c][wave] = psum;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) p_out[j] = L.p[j][lane];
+    if (wave == 0 && g == 0 && c < P.group) {
+        const f4 l = *reinterpret_cast<const f4*>(L.l[c]);
+        float* const ml = P.part_ml + ((size_t)wg * P.group + c) * 2;
+        ml[0] = m;
+        ml[1] = (l[0] + l[1]) + (l[2] + l[3]);
+    }
+}
+// o[t][r] of lane (c, g) is out[head c][64 wave + 16 g + 4 r + t]
+__device__ __forceinline__ void one_page_store(const AttnKernelParams& P, int wg, int wave, int c, int g, const f4 (&o)[4]) {
+    if (c < P.group) {
+        float* const d = P.part_o + ((size_t)wg * P.group + c) * kHd + 64 * wave + 16 * g;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) *reinterpret_cast<f4*>(d + 4 * r) = f4{o[0][r], o[1][r], o[2][r], o[3][r]};
+    }
+}
+// this wave's two q fragments, high and low parts
+__device__ __forceinline__ void split_q(const QRaw& q, bool head_live, half8 (&qhi)[kQFragsPerWave], half8 (&qlo)[kQFragsPerWave]) {
+#pragma unroll
+    for (int i = 0; i < kQFragsPerWave; ++i) {
+        const float x[8] = {q.x[i][0].x, q.x[i][0].y, q.x[i][0].z, q.x[i][0].w,
+                            q.x[i][1].x, q.x[i][1].y, q.x[i][1].z, q.x[i][1].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            _Float16 hi, lo;
+            split_hi_lo(head_live ? x[j] : 0.0f, hi, lo);
+            qhi[i][j] = hi;
+            qlo[i][j] = lo;
+        }
+    }
+}
+
+// The 16 listed blocks of a range (SEL), lane by lane: lane i < 16 looks up block i (block i % 4 of page i / 4), and
+// takes its turn through slot -> id -> page; the others repeat lanes 0..15.
+struct ListedBlock {
+    uint32_t id;   // 0xffffffff past the list's end
+    uint32_t row;  // page * 4 + block of the page, clamped to the sequence's own blocks whatever the list holds
+};
+__device__ __forceinline__ ListedBlock listed_block_of_lane(const AttnKernelParams& P, const int32_t* table, int e, int pos, int pg0, int lane) {
+    const uint32_t at = (uint32_t)pg0 * 4u + (uint32_t)(lane & 15);
+    // read whether or not the list reaches the slot (the buffer holds max_ids slots per entry): nothing here waits
+    // for the list's length
+    const uint32_t raw = P.ids[(size_t)e * (size_t)P.id_stride + min(at, (uint32_t)P.max_ids - 1u)];
+    const uint32_t n_sel = min(P.counts[e], (uint32_t)P.max_ids);
+    const uint32_t b = min(raw, (uint32_t)pos >> 2);
+    const uint32_t page = (uint32_t)table[b >> 2];
+    return ListedBlock{at < n_sel ? raw : 0xffffffffu, page * 4u + (b & 3u)};
+}
+
+// f16 K: the four pages' scores, this wave's columns' share.  kf[j]: rows c % 8 and 8 + c % 8 of page j, segment
+// g + 4 (c / 8) of the wave's 128-byte line
+__device__ __forceinline__ void one_page_scores_f16(const v4u (&kf)[kWaves][2], const half8 (&qhi)[kQFragsPerWave], const half8 (&qlo)[kQFragsPerWave],
+                                                    f4 (&part)[kWaves]) {
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        half8 ka, kb;
+        k_pair_home(kf[j][0], kf[j][1], ka, kb);
+        f4 a = f4{0.0f, 0.0f, 0.0f, 0.0f}, b = a;
+        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi[0], a, 0, 0, 0);
+        b = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo[0], b, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qhi[1], a, 0, 0, 0);
+        b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qlo[1], b, 0, 0, 0);
+        part[j] = a + b;
+    }
+}
+// the new K row's line (8 slices) in place of the stale one: row r sits in the lanes with c % 8 == r % 8, in the
+// register of rows 0..7 or of rows 8..15
+__device__ __forceinline__ void one_page_take_new_k(const v4u* line, int new_page, int r, int c, int g, v4u (&kf)[kWaves][2]) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const v4u w = line[g + 4 * (c >> 3)];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j)
+        if (j == new_page && (c & 7) == (r & 7)) {
+            if (r < 8) kf[j][0] = w; else kf[j][1] = w;
+        }
+}
+
+// f16 rows of a listed block, and the lane's K rows of page j (c % 8 and 8 + c % 8)
+__device__ __forceinline__ size_t listed_f16_rows(const ListedBlock& listed, int block, size_t page_bytes, size_t head_off) {
+    const uint32_t row = (uint32_t)__shfl((int)listed.row, block, 64);
+    return (size_t)(row >> 2) * page_bytes + head_off + (size_t)(row & 3u) * 4u * (kHd * 2);
+}
+__device__ __forceinline__ void one_page_k_rows_listed(const ListedBlock& listed, int j, int c7, size_t page_bytes, size_t head_off, const uint8_t* base,
+                                                       const uint8_t*& lo, const uint8_t*& hi) {
+    lo = base + listed_f16_rows(listed, 4 * j + (c7 >> 2), page_bytes, head_off) + (size_t)(c7 & 3) * (kHd * 2);
+    hi = base + listed_f16_rows(listed, 4 * j + 2 + (c7 >> 2), page_bytes, head_off) + (size_t)(c7 & 3) * (kHd * 2);
+}
+
+// A unit of 16 rows of ROW bytes on its way through registers: 64 lanes x (4 x 16 bytes + what is left).  Of a
+// selection list, page `wave` of the range, whose rows 4 j .. 4 j + 3 are listed block 4 wave + j (rows are multiples
+// of 16 bytes long, so no lane's piece straddles blocks).
+template <bool SEL, int ROW, typename Tail>
+__device__ __forceinline__ void fetch_unit(const uint8_t* pool, size_t page_off, const ListedBlock& listed, int wave, size_t page_bytes, size_t head_off,
+                                           int lane, v4u (&q)[4], Tail& tail) {
+    static_assert(16 * ROW == 64 * (64 + (int)sizeof(Tail)), "a unit");
+    const auto at = [&](int off) {
+        if constexpr (SEL) {
+            const int j = (off >= 4 * ROW) + (off >= 8 * ROW) + (off >= 12 * ROW);
+            const uint32_t row = (uint32_t)__shfl((int)listed.row, 4 * wave + j, 64);
+            return pool + ((size_t)(row >> 2) * page_bytes + head_off + (size_t)(row & 3u) * 4u * ROW) + (off - j * 4 * ROW);
+        } else {
+            return pool + page_off + off;
+        }
+    };
+#pragma unroll
+    for (int n = 0; n < 4; ++n) q[n] = *reinterpret_cast<const v4u*>(at(n * 1024 + lane * 16));
+    tail = *reinterpret_cast<const Tail*>(at(4096 + lane * (int)sizeof(Tail)));
+}
+
+template <bool STEP, bool SEL>
+__device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageLds& L, int e, int kvh, int wg, int pos, const int32_t* table,
+                                             int pg0, int wave, int lane) {
+    const int c = lane & 15, g = lane >> 4, c7 = c & 7;
+    const size_t page_bytes = (size_t)P.n_kv * kPage * kHd * 2;
+    const size_t head_off = (size_t)kvh * kPage * kHd * 2;
+    const int n_pages = pos / kPage + 1;  // dense
+    // STEP: every wave takes its own columns of the new row, lanes 0..7 of K and 8..15 of V.  They are requested ahead
+    // of everything else: what is requested in a branch has to come first, or the waits behind it are for all that
+    // may be in flight
+    const int new_page = n_pages - 1 - pg0, new_r = pos & (kPage - 1);
+    const bool takes_new_row = STEP && new_page < kWaves;
+    NewSliceF16 x;
+    if constexpr (STEP) {
+        if (takes_new_row) request_new_slice(P, e, kvh, c < 8, 8 * wave + c7, x);
+    }
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // K rows c % 8 and 8 + c % 8 of every page, bytes 128 wave .. + 127 (a whole line a row: eight lanes, as in the
+    // kernel below); of V, columns 64 wave + 4 c .. + 3 of rows 4 g .. 4 g + 3 of every page
+    const uint8_t *k_lo[kWaves], *k_hi[kWaves], *v_rows[kWaves];
+    uint32_t id[kWaves];  // SEL: block g of page j
+    size_t new_row_off = 0;
+    const int k_at = 128 * wave + 16 * (g + 4 * (c >> 3)), v_at = (64 * wave + 4 * c) * 2;
+    if constexpr (SEL) {
+        const ListedBlock listed = listed_block_of_lane(P, table, e, pos, pg0, lane);
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) {
+            one_page_k_rows_listed(listed, j, c7, page_bytes, head_off, P.kpool + k_at, k_lo[j], k_hi[j]);
+            v_rows[j] = P.vpool + listed_f16_rows(listed, 4 * j + g, page_bytes, head_off) + v_at;
+            id[j] = (uint32_t)__shfl((int)listed.id, 4 * j + g, 64);
+        }
+    } else {
+        const block_table_ptr bt = (block_table_ptr)(uintptr_t)table;
+        int page[kWaves];
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) page[j] = bt[min(pg0 + j, n_pages - 1)];
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) {
+            const size_t off = (size_t)page[j] * page_bytes + head_off;
+            k_lo[j] = P.kpool + off + (size_t)c7 * (kHd * 2) + k_at;
+            k_hi[j] = k_lo[j] + 8 * (kHd * 2);
+            v_rows[j] = P.vpool + off + (size_t)(4 * g) * (kHd * 2) + v_at;
+            if (j == new_page) new_row_off = off + (size_t)new_r * (kHd * 2);
+        }
+    }
+    // (not as nontemporal loads, which the long walks use: these took 400 of 9200 cycles longer with them)
+    v4u kf[kWaves][2];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        kf[j][0] = *reinterpret_cast<const v4u*>(k_lo[j]);
+        kf[j][1] = *reinterpret_cast<const v4u*>(k_hi[j]);
+    }
+    v2u vf[kWaves][4];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            vf[j][r] = *reinterpret_cast<const v2u*>(v_rows[j] + r * (kHd * 2));
+    __builtin_amdgcn_sched_barrier(0);
+
+    if constexpr (STEP) {
+        if (takes_new_row) {
+            if (lane < 16) L.new_row[wave][lane] = store_new_slice(P, x, c < 8, new_row_off, 8 * wave + c7);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
+    }
+    half8 qhi[kQFragsPerWave], qlo[kQFragsPerWave];
+    split_q(q_raw, c < P.group, qhi, qlo);
+    if constexpr (STEP) {
+        if (takes_new_row) one_page_take_new_k(L.new_row[wave], new_page, new_r, c, g, kf);
+    }
+
+    f4 part[kWaves];
+    one_page_scores_f16(kf, qhi, qlo, part);
+    bool live[kWaves][4], mine[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) {
+            if constexpr (SEL) live[j][r] = block_cell_live(id[j], r, pos);
+            else live[j][r] = (pg0 + j) * kPage + 4 * g + r <= pos;
+        }
+        if constexpr (SEL) mine[r] = block_cell_live(pick4(id, wave), r, pos);
+        else mine[r] = (pg0 + wave) * kPage + 4 * g + r <= pos;
+    }
+    v4u p[kWaves];
+    one_page_softmax(P, L, part, mine, wg, wave, lane, p);
+
+    if constexpr (STEP) {
+        if (takes_new_row) {
+            const v2u w = reinterpret_cast<const v2u*>(&L.new_row[wave][8])[c];
+#pragma unroll
+            for (int j = 0; j < kWaves; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (j == new_page && 4 * g + r == new_r) vf[j][r] = w;
+        }
+    }
+    // rows that are not attended may hold anything (even NaN): exact zeros
+    if (SEL || pg0 + kWaves >= n_pages) {
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (!live[j][r]) vf[j][r] = v2u{0u, 0u};
+    }
+    f4 o[4] = {};
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        // columns 4 c + t of the cells of pages 2 j and 2 j + 1
+        const v4u p0 = p[2 * j], p1 = p[2 * j + 1];
+        const half8 phi = __builtin_bit_cast(half8, v4u{p0.x, p0.y, p1.x, p1.y});
+        const half8 plo = __builtin_bit_cast(half8, v4u{p0.z, p0.w, p1.z, p1.w});
+        v4u a[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const v2u x0 = vf[2 * j + (k >> 1)][2 * (k & 1)], x1 = vf[2 * j + (k >> 1)][2 * (k & 1) + 1];
+                a[t][k] = __builtin_amdgcn_perm(t < 2 ? x1.x : x1.y, t < 2 ? x0.x : x0.y, t & 1 ? 0x07060302u : 0x05040100u);
+            }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[t]), phi, o[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[t]), plo, o[t], 0, 0, 0);
+    }
+    one_page_store(P, wg, wave, c, g, o);
+}
+
 // STEP: the row of cell pos comes from the caller's f32 K/V (stored under the f16 rule into the
 // pool on the way): the pool ends up as bkv_append would leave it, the output as append + attend.
 // SEL: the 16 rows of an iteration are four listed 4-cell blocks instead of a page (block g
@@ -168,13 +498,13 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
     // the q fragments on their way between the waves lie where the fold staging will be
     __shared__ __attribute__((aligned(16))) MfmaFoldLds lds;
     QFragLds& q_lds = *reinterpret_cast<QFragLds*>(&lds.ow[0][0][0]);
-    static_assert(sizeof(QFragLds) <= sizeof(lds.ow), "the staging holds the q fragments");
+    static_assert(sizeof(QFragLds) <= sizeof(lds.ow) && sizeof(OnePageLds) <= sizeof(lds), "the staging holds the q fragments");
     __shared__ __attribute__((aligned(16))) v4u new_row[STEP ? 64 : 1];  // STEP: the row of cell pos, K then V
 
     // ---- which (entry, kv head, page range); one work-group per unit (no head chunks) --------
     const int unit = blockIdx.x;
     int e, rem, pos, row, pps;
-    if (!unit_of_work_group<DESC>(P, unit, e, rem, pos, row, pps)) return;
+    if (!unit_of_work_group<STEP, DESC>(P, unit, e, rem, pos, row, pps)) return;
     const int split = small_div(rem, P.inv_kv16);
     const int kvh = rem - split * P.n_kv;
     const int wg = unit;
@@ -194,6 +524,11 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
+    if (pps == kWaves) {
+        one_page_f16<STEP, SEL>(P, reinterpret_cast<OnePageLds&>(lds), e, kvh, wg, pos,
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+        return;
+    }
     const int c = lane & 15;
     const int g = lane >> 4;
     const size_t page_bytes = (size_t)P.n_kv * kPage * kHd * 2;
@@ -246,16 +581,28 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
         return reinterpret_cast<const v4u*>(rows + (size_t)r * (kHd * 2) + (size_t)(h * 128 + c * 8) * 2);
     };
 
+    // STEP: the wave that will hold the page of cell pos (in its last iteration) takes the new row while its first
+    // pages are on their way.  Fetched at the last page instead, the row would add a trip to memory to the end of
+    // that work-group's walk.  It is requested first: what is requested in a branch has to come first, or the
+    // waits behind it are for all that may be in flight.
+    const int last = n_pages - 1;
+    const bool takes_new_row = STEP && last >= pg0 && last < pg1 && ((last - pg0) & (kWaves - 1)) == wave;
+    NewSliceF16 x;  // lane l < 32: slice l of the K row, lane 32 + l: slice l of the V row
+    if constexpr (STEP) {
+        if (takes_new_row) request_new_slice(P, e, kvh, lane < 32, lane & 31, x);
+    }
     QRaw q_raw;
     request_q(P, e, kvh, wave, c, g, q_raw);
     __builtin_amdgcn_sched_barrier(0);
     int pg = pg0 + wave;
     v4u kf[8], vf[2][4];
     RowRuns<SEL> cur{};
-    // a selection list's first rows are requested before its length is known (every address is clamped
-    // to the sequence's own blocks, so rows past the list's end are merely unused)
-    if (SEL || pg < pg1) {
-        locate(pg, cur);
+    // A wave without pages of its own requests the range's last one, which nothing reads: in a branch, these
+    // requests would have every wait for q wait for the pages too.  A selection list's first rows are requested
+    // before its length is known (every address is clamped to the sequence's own blocks, so rows past the list's
+    // end are merely unused).
+    {
+        locate(SEL ? pg : min(pg, pg1 - 1), cur);
         const uint8_t* kp_lo = k_row_of(cur, c7);
         const uint8_t* kp_hi = k_row_of(cur, 8 + c7);
         const uint8_t* vp = v_rows(cur);
@@ -269,33 +616,18 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
 #pragma unroll
             for (int r = 0; r < 4; ++r) vf[h][r] = __builtin_nontemporal_load(v_addr(vp, h, r));
     }
+    __builtin_amdgcn_sched_barrier(0);
 
-    half8 qhi[8], qlo[8];
-    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
-    __syncthreads();  // a wave without pages goes straight to the fold
-
-    // STEP: the wave that will hold the page of cell pos (in its last iteration) takes the new row now,
-    // while its first pages are on their way: lane l < 32 converts slice l (8 values) of the K row, lane
-    // 32 + l slice l of the V row, stores it into the pool (whole rows, 16 bytes a lane) and parks it in
-    // LDS.  Fetched at the last page instead, the row would add a trip to memory to the end of that
-    // work-group's walk.
     if constexpr (STEP) {
-        const int last = n_pages - 1;
-        if (last >= pg0 && last < pg1 && ((last - pg0) & (kWaves - 1)) == wave) {
-            const bool is_k = lane < 32;
-            const int sl = lane & 31;
-            const float* src = (is_k ? P.new_k : P.new_v) + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + sl * 8;
-            const float4 a = *reinterpret_cast<const float4*>(src);
-            const float4 b = *reinterpret_cast<const float4*>(src + 4);
-            v4u w;
-            w.x = f16_store_pair(a.x, a.y), w.y = f16_store_pair(a.z, a.w);
-            w.z = f16_store_pair(b.x, b.y), w.w = f16_store_pair(b.z, b.w);
+        if (takes_new_row) {
             const size_t here = (size_t)bt[last] * page_bytes + head_off + (size_t)(pos & (kPage - 1)) * (kHd * 2);
-            *reinterpret_cast<v4u*>((is_k ? P.kpool_w : P.vpool_w) + here + (size_t)sl * 16) = w;
-            new_row[lane] = w;
+            new_row[lane] = store_new_slice(P, x, lane < 32, here, lane & 31);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         }
     }
+    half8 qhi[8], qlo[8];
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
+    __syncthreads();  // a wave without pages goes straight to the fold
 
     // O^T accumulators: o[h][t][r] = out[head c][128 h + 8 (4 g + r) + t]
     f4 o[2][8];
@@ -507,8 +839,6 @@ __device__ __forceinline__ const uint8_t* unit_piece(const UnitSrc<SEL>& u, int 
 // (0xffffffff past the end of the list) and, clamped to the blocks at or below `pos` before any
 // address is formed, the byte offset of each block's rows inside a pool whose pages are
 // `page_bytes` long and whose rows are `row_bytes` long.
-typedef const __attribute__((address_space(4))) uint32_t* sel_list_ptr;
-typedef const __attribute__((address_space(4))) int32_t* block_table_ptr;
 __device__ __forceinline__ void listed_blocks(sel_list_ptr sel, uint32_t n_sel, uint32_t max_ids, block_table_ptr bt,
                                               int it, int pos, size_t page_bytes, size_t head_off, int row_bytes,
                                               uint32_t (&id)[4], size_t (&off)[4]) {
@@ -522,9 +852,6 @@ __device__ __forceinline__ void listed_blocks(sel_list_ptr sel, uint32_t n_sel, 
         const uint32_t idc = min(raw, (uint32_t)pos >> 2);
         off[j] = (size_t)bt[idc >> 2] * page_bytes + head_off + (size_t)(idc & 3u) * 4u * (size_t)row_bytes;
     }
-}
-__device__ __forceinline__ uint32_t pick4(const uint32_t (&a)[4], int j) {
-    return j == 0 ? a[0] : j == 1 ? a[1] : j == 2 ? a[2] : a[3];
 }
 
 // One unit between memory and LDS: 4352 bytes = 64 lanes x (4 x 16 + 4).
@@ -546,6 +873,150 @@ __device__ __forceinline__ void i8h_unit_deposit(const I8hUnitRegs& r, uint8_t* 
     *reinterpret_cast<unsigned*>(dst + 4096 + lane * 4) = r.tail;
 }
 
+// Ranges of one page a wave (see OnePageLds): a wave fetches and stages one page, as below, and multiplies columns
+// 64 wave .. + 63 (two scale blocks) of all four.
+struct OnePageI8hLds {
+    uint8_t slot[kWaves][kI8hSlot];
+    OnePageLds x;
+};
+// the halves of a dword whose exponent field is 0 read as zero
+__device__ __forceinline__ unsigned zero_exponent_as_zero(unsigned two_halves) {
+    const unsigned lo = two_halves & 0x7c00u ? two_halves & 0xffffu : 0u;
+    const unsigned hi = two_halves & 0x7c000000u ? two_halves & 0xffff0000u : 0u;
+    return lo | hi;
+}
+template <bool STEP, bool SEL>
+__device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI8hLds& L, int e, int kvh, int wg, int pos, const int32_t* table,
+                                             int pg0, int wave, int lane) {
+    constexpr int kRow = row_bytes_of(kRowI8H);
+    const int c = lane & 15, g = lane >> 4;
+    const size_t page_bytes = (size_t)P.n_kv * kI8hUnit;
+    const size_t head_off = (size_t)kvh * kI8hUnit;
+    const int n_pages = pos / kPage + 1;  // dense
+    const block_table_ptr bt = (block_table_ptr)(uintptr_t)table;
+    const bool takes_new_row = STEP && n_pages - 1 - pg0 == wave;
+    NewSliceF16 x;
+    if constexpr (STEP) {
+        if (takes_new_row) request_new_slice(P, e, kvh, lane < 32, lane & 31, x);  // ahead of everything else, as there
+    }
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
+    ListedBlock listed{};
+    size_t page_off = 0;
+    if constexpr (SEL) listed = listed_block_of_lane(P, table, e, pos, pg0, lane);
+    else page_off = (size_t)bt[min(pg0 + wave, n_pages - 1)] * page_bytes + head_off;
+    I8hUnitRegs k_regs, v_regs;
+    fetch_unit<SEL, kRow>(P.kpool, page_off, listed, wave, page_bytes, head_off, lane, k_regs.q, k_regs.tail);
+    fetch_unit<SEL, kRow>(P.vpool, page_off, listed, wave, page_bytes, head_off, lane, v_regs.q, v_regs.tail);
+    __builtin_amdgcn_sched_barrier(0);
+
+    const int li = lane & 31, new_r = pos & (kPage - 1);
+    uint32_t new_codes[2] = {0, 0}, new_scale = 0;
+    if constexpr (STEP) {
+        // encoded 8 values a lane as in the append kernel, into the pool; into LDS once the page is there
+        if (takes_new_row) {
+            const float v[8] = {x.a[0], x.a[1], x.a[2], x.a[3], x.b[0], x.b[1], x.b[2], x.b[3]};
+            new_scale = i8h_scale_bits(quad_max(amax8(v)));
+            i8h_codes8(v, f16_load(new_scale), new_codes[0], new_codes[1]);
+            const auto row = k_or_v(lane < 32, P.kpool_w, P.vpool_w) + page_off + (size_t)new_r * kRow;
+            *(__attribute__((address_space(1))) v2u*)(row + li * 8) = v2u{new_codes[0], new_codes[1]};
+            if ((li & 3) == 0) *(__attribute__((address_space(1))) unsigned short*)(row + kHd + 2 * (li >> 2)) = (unsigned short)new_scale;
+        }
+    }
+    half8 qhi[kQFragsPerWave], qlo[kQFragsPerWave];
+    split_q(q_raw, c < P.group, qhi, qlo);
+
+    uint8_t* const slot = L.slot[wave];
+    i8h_unit_deposit(k_regs, slot, lane);
+    i8h_unit_deposit(v_regs, slot + kI8hUnit, lane);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (STEP) {
+        if (takes_new_row) {
+            uint8_t* const row = slot + (lane < 32 ? 0 : kI8hUnit) + new_r * kRow;
+            *reinterpret_cast<v2u*>(row + li * 8) = v2u{new_codes[0], new_codes[1]};
+            if ((li & 3) == 0) *reinterpret_cast<unsigned short*>(row + kHd + 2 * (li >> 2)) = (unsigned short)new_scale;
+        }
+    }
+    {
+        // The page's scales, one dword a lane: with exponent field 0 they read as zero, and rows that are not attended
+        // may hold anything: a zero scale keeps a NaN from them (any code is a finite number).  Written back only
+        // where something changed.
+        const int row = lane >> 2;
+        bool row_live;
+        if constexpr (SEL) row_live = block_cell_live((uint32_t)__shfl((int)listed.id, 4 * wave + (row >> 2), 64), row & 3, pos);
+        else row_live = (pg0 + wave) * kPage + row <= pos;
+        unsigned* const ks = reinterpret_cast<unsigned*>(slot + row * kRow + kHd + 4 * (lane & 3));
+        unsigned* const vs = ks + kI8hUnit / 4;
+        const unsigned k = *ks, v = *vs, k_clean = zero_exponent_as_zero(k), v_clean = row_live ? zero_exponent_as_zero(v) : 0u;
+        if (__builtin_amdgcn_ballot_w64(k != k_clean || v != v_clean) != 0) {
+            *ks = k_clean;
+            *vs = v_clean;
+        }
+    }
+    __syncthreads();
+
+    f4 part[kWaves];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        const uint8_t* const ks = L.slot[j];
+        part[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        h2m sc[4];  // of the wave's two blocks
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[r] = *reinterpret_cast<const h2m*>(ks + (4 * g + r) * kRow + kHd + 4 * wave);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const half8 ka = codes8_to_f16(*reinterpret_cast<const v2u*>(ks + c * kRow + (2 * wave + i) * 32 + g * 8));
+            f4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qhi[i], f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qlo[i], s, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[j][r] = fmaf((float)sc[r][i], s[r], part[j][r]);
+        }
+    }
+    bool mine[4];
+    const uint32_t id = SEL ? (uint32_t)__shfl((int)listed.id, 4 * wave + g, 64) : 0u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if constexpr (SEL) mine[r] = block_cell_live(id, r, pos);
+        else mine[r] = (pg0 + wave) * kPage + 4 * g + r <= pos;
+    }
+    v4u p[kWaves];
+    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p);
+
+    f4 o[4] = {};
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        // lane (c, g): columns 64 wave + 4 c + t of rows 4 g + r, in block 2 wave + c / 8
+        const uint8_t* const vs = L.slot[j] + kI8hUnit + 4 * g * kRow;
+        unsigned codes[4], col[4], sb[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            codes[r] = *reinterpret_cast<const unsigned*>(vs + r * kRow + 64 * wave + 4 * c) ^ 0x80808080u;
+            sb[r] = *reinterpret_cast<const unsigned short*>(vs + r * kRow + kHd + 2 * (2 * wave + (c >> 3)));
+        }
+        transpose4x4_bytes(codes, col);
+        const h2m s01 = __builtin_bit_cast(h2m, sb[0] | (sb[1] << 16)), s23 = __builtin_bit_cast(h2m, sb[2] | (sb[3] << 16));
+        const half8 phh = __builtin_bit_cast(half8, v4u{p[j].x, p[j].y, p[j].x, p[j].y});
+        const half8 pll = __builtin_bit_cast(half8, v4u{p[j].z, p[j].w, p[j].z, p[j].w});
+        half8 a[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            h2m c01, c23;
+            biased_to_f16(col[t], c01, c23);
+            const h2m hi01 = c01 * s01, hi23 = c23 * s23;
+            const h2m lo01 = __builtin_elementwise_fma(c01, s01, -hi01), lo23 = __builtin_elementwise_fma(c23, s23, -hi23);
+            a[t] = half8{hi01[0], hi01[1], hi23[0], hi23[1], lo01[0], lo01[1], lo23[0], lo23[1]};
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], phh, o[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], pll, o[t], 0, 0, 0);
+    }
+    one_page_store(P, wg, wave, c, g, o);
+}
+
 // SEL: an iteration's 16 rows are four listed 4-cell blocks (see decode_attn_mfma_kernel); the
 // work is planned for max_ids blocks, a work-group past the end of the list has nothing to do.
 template <bool STEP, bool DESC = false, bool SEL = false>
@@ -563,7 +1034,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 
     const int unit = blockIdx.x;
     int e, rem, pos, row, pps;
-    if (!unit_of_work_group<DESC>(P, unit, e, rem, pos, row, pps)) return;
+    if (!unit_of_work_group<STEP, DESC>(P, unit, e, rem, pos, row, pps)) return;
     const int split = small_div(rem, P.inv_kv16);
     const int kvh = rem - split * P.n_kv;
     const int wg = unit;
@@ -581,6 +1052,12 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
+    if (pps == kWaves) {
+        static_assert(sizeof(OnePageI8hLds) <= kRing, "the fold staging holds it");
+        one_page_i8h<STEP, SEL>(P, *reinterpret_cast<OnePageI8hLds*>(ring), e, kvh, wg, pos,
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+        return;
+    }
     const int c = lane & 15;
     const int g = lane >> 4;
     const int my_block = c >> 2;  // which of the 4 blocks of a half this lane's 8 columns lie in
@@ -604,7 +1081,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 #pragma unroll
             for (int j = 0; j < 4; ++j) u.run[j] = pool + off[j];
         } else {
-            u.run[0] = pool + (n_steps > 0 ? unit_off(i) : 0);
+            u.run[0] = pool + unit_off(i);
         }
     };
     // the page in flight: requested while the page before is multiplied
@@ -616,13 +1093,9 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
         unit_src(i, P.vpool, u);
         i8h_unit_fetch<SEL>(u, lane, v_regs);
     };
-    QRaw q_raw;
-    request_q(P, e, kvh, wave, c, g, q_raw);
-    __builtin_amdgcn_sched_barrier(0);
-    if (SEL || n_steps > 0) fetch(0);  // a selection list's first units before its length is known
-
     // STEP: the wave that will hold the page of cell pos (in its last step) takes the new rows before the
-    // loop, behind the request of its first units: lanes 0..31 encode the K row and lanes 32..63 the V row, 8
+    // loop, requested ahead of its first units (what is requested in a branch has to come first, or the waits behind
+    // it are for all that may be in flight): lanes 0..31 encode the K row and lanes 32..63 the V row, 8
     // values a lane as in the append kernel, into the pool and into two parking rows in LDS.  In its last step
     // the wave copies a parked row into the unit that has just landed (an LDS move instead of a trip to memory
     // and an encode at the end of the work-group's walk).  With 32 values in each of 16 lanes, encoded behind the
@@ -630,15 +1103,17 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     // layer with the merge, one sequence of 4096 cells 12.3 -> 11.0, four short ones 12.5 -> 11.3, 64 of 512 to
     // 4096 45.7 -> 43.9.
     const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
-    float new_x[8];
+    NewSliceF16 x;
     if constexpr (STEP) {
-        if (takes_new_row) {
-            const float* src = (lane < 32 ? P.new_k : P.new_v) + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + (lane & 31) * 8;
-            const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-            new_x[0] = a.x, new_x[1] = a.y, new_x[2] = a.z, new_x[3] = a.w;
-            new_x[4] = b.x, new_x[5] = b.y, new_x[6] = b.z, new_x[7] = b.w;
-        }
+        if (takes_new_row) request_new_slice(P, e, kvh, lane < 32, lane & 31, x);
     }
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
+    // a selection list's first units before its length is known; a wave without pages requests the range's last one,
+    // which nothing reads
+    fetch(0);
+    __builtin_amdgcn_sched_barrier(0);
 
     const auto wave_lds_fence = [&]() {
         // the wave's own LDS writes are in order with its later reads; keep the compiler from
@@ -649,17 +1124,18 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     };
     if constexpr (STEP) {
         if (takes_new_row) {
+            const float new_x[8] = {x.a[0], x.a[1], x.a[2], x.a[3], x.b[0], x.b[1], x.b[2], x.b[3]};
             const uint32_t hb = i8h_scale_bits(quad_max(amax8(new_x)));
             uint32_t w0, w1;
             i8h_codes8(new_x, f16_load(hb), w0, w1);
             const int li = lane & 31;
             const size_t at = unit_off(n_steps - 1) + (size_t)(pos & (kPage - 1)) * kRow;
-            uint8_t* const pool_row = (lane < 32 ? P.kpool_w : P.vpool_w) + at;
+            const auto pool_row = k_or_v(lane < 32, P.kpool_w, P.vpool_w) + at;
             uint8_t* const park = parked + (lane < 32 ? 0 : kRow);
-            *reinterpret_cast<v2u*>(pool_row + li * 8) = v2u{w0, w1};
+            *(__attribute__((address_space(1))) v2u*)(pool_row + li * 8) = v2u{w0, w1};
             *reinterpret_cast<v2u*>(park + li * 8) = v2u{w0, w1};
             if ((li & 3) == 0) {
-                *reinterpret_cast<unsigned short*>(pool_row + kHd + 2 * (li >> 2)) = (unsigned short)hb;
+                *(__attribute__((address_space(1))) unsigned short*)(pool_row + kHd + 2 * (li >> 2)) = (unsigned short)hb;
                 *reinterpret_cast<unsigned short*>(park + kHd + 2 * (li >> 2)) = (unsigned short)hb;
             }
             wave_lds_fence();
@@ -852,7 +1328,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     // every wave is done with its slot before the fold staging takes their place
     __syncthreads();
     // the lane's place from the hardware again: kept over the loop, it was one register too many
-    const int again = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int again = lane_of_wave();
     mfma_fold_and_store(P, *reinterpret_cast<MfmaFoldLds*>(ring), wg, wave, again & 15, again >> 4, o, m_run, l_run);
 }
 
@@ -877,6 +1353,33 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 constexpr int kQ8vRow = row_bytes_of(kRowQ8);  // 288
 constexpr int kQ8vUnit = kPage * kQ8vRow;      // 4608
 
+// A new V row (STEP), 8 values a lane, four lanes to a block, as in the append kernel: encoded and stored into the pool;
+// the caller puts the codes (and the first lane of a block the scale) where its own V rows are.
+__device__ __forceinline__ void q8v_new_slice(const AttnKernelParams& P, const NewSliceF16& x, int slice, size_t row_off, float& scale, uint32_t (&codes)[2]) {
+    const float v[8] = {x.a[0], x.a[1], x.a[2], x.a[3], x.b[0], x.b[1], x.b[2], x.b[3]};
+    scale = q8v_scale(quad_max(amax8(v)));
+    q8_codes8(v, scale, codes[0], codes[1]);
+    const auto blk = (__attribute__((address_space(1))) unsigned*)(uintptr_t)(P.vpool_w + row_off + (size_t)(slice >> 2) * 36);
+    if ((slice & 3) == 0) blk[0] = __builtin_bit_cast(unsigned, scale);
+    blk[1 + 2 * (slice & 3)] = codes[0];
+    blk[2 + 2 * (slice & 3)] = codes[1];
+}
+// Exponents of rows 4 g + r of a page, and 2^-E, from the larger of two block scales of row 4 g + c % 4 in every lane
+// (blocks 2 (c / 4) and 2 (c / 4) + 1): the row's maximum over the lanes c, c ^ 4, c ^ 8, c ^ 12, then the four rows'
+// from the lanes of the quad.
+__device__ __forceinline__ void q8v_row_exponents(float smax, int (&ex)[4], float (&down)[4]) {
+    smax = fmaxf(smax, dpp_mov<0x124>(smax));  // row_ror:4
+    smax = fmaxf(smax, dpp_mov<0x128>(smax));  // row_ror:8
+    const float mr[4] = {dpp_mov<0x00>(smax), dpp_mov<0x55>(smax), dpp_mov<0xAA>(smax), dpp_mov<0xFF>(smax)};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        int ee = (int)((__builtin_bit_cast(unsigned, mr[r]) >> 23) & 0xffu) - 127;
+        ee = min(max(ee, -120), 120);
+        ex[r] = ee;
+        down[r] = __builtin_bit_cast(float, (unsigned)(127 - ee) << 23);
+    }
+}
+
 // A V unit: 4608 bytes = 64 lanes x (4 x 16 + 8).
 struct Q8vUnitRegs {
     v4u q[4];
@@ -896,6 +1399,156 @@ __device__ __forceinline__ void q8v_unit_deposit(const Q8vUnitRegs& r, uint8_t* 
     *reinterpret_cast<v2u*>(dst + 4096 + lane * 8) = r.tail;
 }
 
+// Ranges of one page a wave (see OnePageLds): K as on the f16 pool, V staged as below, one page a wave; the wave that
+// stages a page works out its rows' exponents.
+struct OnePageQ8vLds {
+    uint8_t slot[kWaves][kQ8vUnit];
+    float down[kWaves][kPage];  // 2^-E
+    OnePageLds x;
+};
+template <bool STEP, bool SEL>
+__device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ8vLds& L, int e, int kvh, int wg, int pos, const int32_t* table,
+                                             int pg0, int wave, int lane) {
+    const int c = lane & 15, g = lane >> 4, c7 = c & 7;
+    const size_t k_page_bytes = (size_t)P.n_kv * kPage * kHd * 2, k_head_off = (size_t)kvh * kPage * kHd * 2;
+    const size_t v_page_bytes = (size_t)P.n_kv * kQ8vUnit, v_head_off = (size_t)kvh * kQ8vUnit;
+    const int n_pages = pos / kPage + 1;  // dense
+    // STEP: lanes 0..7 take the wave's columns of the new K row, and in the wave of its page lanes 32..63 the V row;
+    // requested ahead of everything else, as on the f16 pool
+    const int new_page = n_pages - 1 - pg0, new_r = pos & (kPage - 1), li = lane & 31;
+    const bool takes_new_row = STEP && new_page < kWaves;
+    NewSliceF16 x;
+    if constexpr (STEP) {
+        if (takes_new_row) request_new_slice(P, e, kvh, lane < 32, lane < 32 ? 8 * wave + c7 : li, x);
+    }
+    QRaw q_raw;
+    request_q(P, e, kvh, wave, c, g, q_raw);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t *k_lo[kWaves], *k_hi[kWaves];
+    const int k_at = 128 * wave + 16 * (g + 4 * (c >> 3));
+    size_t new_k_off = 0, v_off = 0;
+    ListedBlock listed{};
+    if constexpr (SEL) {
+        listed = listed_block_of_lane(P, table, e, pos, pg0, lane);
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) one_page_k_rows_listed(listed, j, c7, k_page_bytes, k_head_off, P.kpool + k_at, k_lo[j], k_hi[j]);
+    } else {
+        const block_table_ptr bt = (block_table_ptr)(uintptr_t)table;
+        int page[kWaves];
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) page[j] = bt[min(pg0 + j, n_pages - 1)];
+#pragma unroll
+        for (int j = 0; j < kWaves; ++j) {
+            const size_t off = (size_t)page[j] * k_page_bytes + k_head_off;
+            k_lo[j] = P.kpool + off + (size_t)c7 * (kHd * 2) + k_at;
+            k_hi[j] = k_lo[j] + 8 * (kHd * 2);
+            if (j == new_page) new_k_off = off + (size_t)new_r * (kHd * 2);
+            if (j == wave) v_off = (size_t)page[j] * v_page_bytes + v_head_off;
+        }
+    }
+    v4u kf[kWaves][2];
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        kf[j][0] = *reinterpret_cast<const v4u*>(k_lo[j]);
+        kf[j][1] = *reinterpret_cast<const v4u*>(k_hi[j]);
+    }
+    Q8vUnitRegs v_regs;
+    fetch_unit<SEL, kQ8vRow>(P.vpool, v_off, listed, wave, v_page_bytes, v_head_off, lane, v_regs.q, v_regs.tail);
+    __builtin_amdgcn_sched_barrier(0);
+
+    const bool takes_new_v = takes_new_row && new_page == wave && lane >= 32;
+    uint32_t new_codes[2] = {0, 0};
+    float new_scale = 0.0f;
+    if constexpr (STEP) {
+        if (takes_new_row) {
+            if (lane < 8) L.x.new_row[wave][lane] = store_new_slice(P, x, true, new_k_off, 8 * wave + lane);
+            if (takes_new_v) q8v_new_slice(P, x, li, v_off + (size_t)new_r * kQ8vRow, new_scale, new_codes);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
+    }
+    half8 qhi[kQFragsPerWave], qlo[kQFragsPerWave];
+    split_q(q_raw, c < P.group, qhi, qlo);
+    if constexpr (STEP) {
+        if (takes_new_row) one_page_take_new_k(L.x.new_row[wave], new_page, new_r, c, g, kf);
+    }
+    f4 part[kWaves];
+    one_page_scores_f16(kf, qhi, qlo, part);
+
+    uint8_t* const slot = L.slot[wave];
+    q8v_unit_deposit(v_regs, slot, lane);
+    if constexpr (STEP) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if (takes_new_v) {
+            unsigned* const blk = reinterpret_cast<unsigned*>(slot + new_r * kQ8vRow + (li >> 2) * 36);
+            if ((li & 3) == 0) blk[0] = __builtin_bit_cast(unsigned, new_scale);
+            blk[1 + 2 * (li & 3)] = new_codes[0];
+            blk[2 + 2 * (li & 3)] = new_codes[1];
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    bool mine[4], mine_scale;  // of cells 4 g + r, and of cell 4 g + c % 4
+    const uint32_t id = SEL ? (uint32_t)__shfl((int)listed.id, 4 * wave + g, 64) : 0u;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if constexpr (SEL) mine[r] = block_cell_live(id, r, pos);
+        else mine[r] = (pg0 + wave) * kPage + 4 * g + r <= pos;
+    }
+    mine_scale = c & 2 ? (c & 1 ? mine[3] : mine[2]) : (c & 1 ? mine[1] : mine[0]);
+    int ex[4];
+    float down[4];
+    {
+        // scales of blocks 2 (c / 4), + 1 of row 4 g + c % 4.  Rows that are not attended may hold anything: they count
+        // as scale 1 here and are zeroed for whoever multiplies them
+        float* const rp = reinterpret_cast<float*>(slot + (4 * g + (c & 3)) * kQ8vRow + (c >> 2) * 72);
+        float smax = fmaxf(rp[0], rp[9]);
+        if (!mine_scale) {
+            smax = 1.0f;
+            rp[0] = 0.0f;
+            rp[9] = 0.0f;
+        }
+        q8v_row_exponents(smax, ex, down);
+        if (c == 0) *reinterpret_cast<f4*>(&L.down[wave][4 * g]) = f4{down[0], down[1], down[2], down[3]};
+    }
+    // (the barriers of the softmax stand between these writes and the waves that read them)
+    v4u p[kWaves];
+    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, ex, down);
+
+    f4 o[4] = {};
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+        // lane (c, g): columns 64 wave + 4 c + t of rows 4 g + r, in block 2 wave + c / 8
+        const uint8_t* const vs = L.slot[j] + 4 * g * kQ8vRow + (2 * wave + (c >> 3)) * 36;
+        const f4 dn = *reinterpret_cast<const f4*>(&L.down[j][4 * g]);
+        unsigned codes[4], col[4];
+        _Float16 shi[4], slo[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            codes[r] = *reinterpret_cast<const unsigned*>(vs + r * kQ8vRow + 4 + 4 * c7) ^ 0x80808080u;
+            split_hi_lo(*reinterpret_cast<const float*>(vs + r * kQ8vRow) * dn[r], shi[r], slo[r]);
+        }
+        transpose4x4_bytes(codes, col);
+        const h2m s01 = h2m{shi[0], shi[1]}, s23 = h2m{shi[2], shi[3]}, l01 = h2m{slo[0], slo[1]}, l23 = h2m{slo[2], slo[3]};
+        const half8 whh = __builtin_bit_cast(half8, v4u{p[j].x, p[j].y, p[j].x, p[j].y});
+        const half8 wll = __builtin_bit_cast(half8, v4u{p[j].z, p[j].w, p[j].z, p[j].w});
+        half8 a[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            h2m c01, c23, hi01, hi23, lo01, lo23;
+            biased_to_f16(col[t], c01, c23);
+            scaled_hi_lo(c01, s01, l01, hi01, lo01);
+            scaled_hi_lo(c23, s23, l23, hi23, lo23);
+            a[t] = half8{hi01[0], hi01[1], hi23[0], hi23[1], lo01[0], lo01[1], lo23[0], lo23[1]};
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], whh, o[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], wll, o[t], 0, 0, 0);
+    }
+    one_page_store(P, wg, wave, c, g, o);
+}
+
 // SEL: an iteration's 16 rows are four listed 4-cell blocks, as in the int8 kernel.
 template <bool STEP, bool DESC = false, bool SEL = false>
 __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const AttnKernelParams P) {
@@ -912,7 +1565,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
 
     const int unit = blockIdx.x;
     int e, rem, pos, row, pps;
-    if (!unit_of_work_group<DESC>(P, unit, e, rem, pos, row, pps)) return;
+    if (!unit_of_work_group<STEP, DESC>(P, unit, e, rem, pos, row, pps)) return;
     const int split = small_div(rem, P.inv_kv16);
     const int kvh = rem - split * P.n_kv;
     const int wg = unit;
@@ -929,6 +1582,12 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
+    if (pps == kWaves) {
+        static_assert(sizeof(OnePageQ8vLds) <= kLds, "the fold staging holds it");
+        one_page_q8v<STEP, SEL>(P, *reinterpret_cast<OnePageQ8vLds*>(smem), e, kvh, wg, pos,
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+        return;
+    }
     const int c = lane & 15;
     const int g = lane >> 4;
     const size_t k_page_bytes = (size_t)P.n_kv * kPage * kHd * 2;
@@ -954,8 +1613,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
 #pragma unroll
             for (int j = 0; j < 4; ++j) u.run[j] = pool + off[j];
         } else {
-            u.run[0] = n_steps > 0 ? pool + phys(i) * (is_k ? k_page_bytes : v_page_bytes) + (is_k ? k_head_off : v_head_off)
-                                   : pool;
+            u.run[0] = pool + phys(i) * (is_k ? k_page_bytes : v_page_bytes) + (is_k ? k_head_off : v_head_off);
         }
     };
     // K rows are fetched in whole 128-byte lines, as in decode_attn_mfma_kernel: for the pair of fragments
@@ -977,12 +1635,25 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     };
     // the page in flight: K in the fragment registers, refilled as they are used up; the V unit requested
     // while the page before is multiplied
+    // STEP: the wave that will hold the page of cell pos (in its last step) encodes the new row before the loop, while
+    // its first units are on their way, 8 values a lane as the append kernel does -- lanes 0..31 K under the f16 rule,
+    // lanes 32..63 V as q8_0 blocks -- into the pool and into a parking row in LDS; in its last step it copies the parked
+    // row into the unit that has just landed (two LDS moves instead of a trip to memory and an encode at the end of the
+    // work-group's walk).  Requested ahead of everything else: what is requested in a branch has to come first, or the
+    // waits behind it are for all that may be in flight.
+    const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
+    NewSliceF16 x;
+    if constexpr (STEP) {
+        if (takes_new_row) request_new_slice(P, e, kvh, lane < 32, lane & 31, x);
+    }
     QRaw q_raw;
     request_q(P, e, kvh, wave, c, g, q_raw);
     __builtin_amdgcn_sched_barrier(0);
     v4u kf[8];
     Q8vUnitRegs v_regs;
-    if (SEL || n_steps > 0) {  // a selection list's first units before its length is known
+    // a selection list's first units before its length is known; a wave without pages requests the range's last one,
+    // which nothing reads
+    {
         UnitSrc<SEL> u;
         const uint8_t *lo, *hi;
         unit_src(0, true, u);
@@ -996,67 +1667,33 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
         q8v_unit_fetch<SEL>(u, lane, v_regs);
     }
 
-    // STEP: the wave that will hold the page of cell pos (in its last step) encodes the new row before
-    // the loop, while its first units are on their way, as the append kernel does -- K under the f16
-    // rule, 8 values a lane; V as q8_0 blocks, one lane per block -- into the pool and into a parking
-    // row in LDS; in its last step it copies the parked row into the unit that has just landed (two LDS
-    // moves instead of a trip to memory and an encode at the end of the work-group's walk).
+    __builtin_amdgcn_sched_barrier(0);
     const auto wave_lds_fence = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    // the raw values are requested behind the first units and encoded once the q fragments are traded
-    const bool takes_new_row = STEP && n_steps > 0 && pg0 + wave + kWaves * (n_steps - 1) == n_pages - 1;
-    float new_x[32];
     if constexpr (STEP) {
         if (takes_new_row) {
+            const int r = pos & (kPage - 1), li = lane & 31;
             if (lane < 32) {
-                const float* src = P.new_k + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + lane * 8;
-                const float4 a = *reinterpret_cast<const float4*>(src);
-                const float4 b = *reinterpret_cast<const float4*>(src + 4);
-                new_x[0] = a.x, new_x[1] = a.y, new_x[2] = a.z, new_x[3] = a.w;
-                new_x[4] = b.x, new_x[5] = b.y, new_x[6] = b.z, new_x[7] = b.w;
-            } else if (lane < 40) {
-                const float* src = P.new_v + ((size_t)e * P.n_kv + (size_t)kvh) * kHd + (lane - 32) * 32;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float4 a = *reinterpret_cast<const float4*>(src + 4 * j);
-                    new_x[4 * j] = a.x, new_x[4 * j + 1] = a.y, new_x[4 * j + 2] = a.z, new_x[4 * j + 3] = a.w;
-                }
-            }
-        }
-    }
-
-    half8 qhi[8], qlo[8];
-    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
-
-    if constexpr (STEP) {
-        if (takes_new_row) {
-            const int r = pos & (kPage - 1);
-            const int i = n_steps - 1;
-            if (lane < 32) {
-                v4u w;
-                w.x = f16_store_pair(new_x[0], new_x[1]), w.y = f16_store_pair(new_x[2], new_x[3]);
-                w.z = f16_store_pair(new_x[4], new_x[5]), w.w = f16_store_pair(new_x[6], new_x[7]);
-                *reinterpret_cast<v4u*>(parked + lane * 16) = w;
-                *reinterpret_cast<v4u*>(P.kpool_w + phys(i) * k_page_bytes + k_head_off + (size_t)r * 512 + lane * 16) = w;
-            } else if (lane < 40) {
-                const int blk = lane - 32;
-                uint32_t w[9];
-                q8v_block_words(new_x, w);
-                uint32_t* const ld = reinterpret_cast<uint32_t*>(parked + 512 + blk * 36);
-                uint32_t* const gd = reinterpret_cast<uint32_t*>(P.vpool_w + phys(i) * v_page_bytes + v_head_off +
-                                                                  (size_t)r * kQ8vRow + blk * 36);
-#pragma unroll
-                for (int j = 0; j < 9; ++j) {
-                    ld[j] = w[j];
-                    gd[j] = w[j];
-                }
+                *reinterpret_cast<v4u*>(parked + li * 16) =
+                    store_new_slice(P, x, true, phys(n_steps - 1) * k_page_bytes + k_head_off + (size_t)r * 512, li);
+            } else {
+                float scale;
+                uint32_t codes[2];
+                q8v_new_slice(P, x, li, phys(n_steps - 1) * v_page_bytes + v_head_off + (size_t)r * kQ8vRow, scale, codes);
+                unsigned* const blk = reinterpret_cast<unsigned*>(parked + 512 + (li >> 2) * 36);
+                if ((li & 3) == 0) blk[0] = __builtin_bit_cast(unsigned, scale);
+                blk[1 + 2 * (li & 3)] = codes[0];
+                blk[2 + 2 * (li & 3)] = codes[1];
             }
             wave_lds_fence();
         }
     }
+    half8 qhi[8], qlo[8];
+    trade_q(q_raw, q_lds, wave, lane, c < P.group, qhi, qlo);
+
     // K registers hold rows as fetched: row r sits in the lanes with c % 8 == r % 8, in the register of
     // rows 0..7 or of rows 8..15, segment g + 4 (c / 8) of each 128-byte line
     const auto take_new_k = [&]() {
@@ -1154,23 +1791,10 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
             smax = fmaxf(a, b);
             // rows past `pos` may hold anything: they count as scale 1 here and as zeros below
             if (last_page && !live_mine) smax = 1.0f;
-            smax = fmaxf(smax, dpp_mov<0x124>(smax));  // row_ror:4
-            smax = fmaxf(smax, dpp_mov<0x128>(smax));  // row_ror:8
         }
         int ex[4];
         float down[4];  // 2^-E
-        {
-            const float m0 = dpp_mov<0x00>(smax), m1 = dpp_mov<0x55>(smax);
-            const float m2 = dpp_mov<0xAA>(smax), m3 = dpp_mov<0xFF>(smax);
-            const float mr[4] = {m0, m1, m2, m3};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int ee = (int)((__builtin_bit_cast(unsigned, mr[r]) >> 23) & 0xffu) - 127;
-                ee = min(max(ee, -120), 120);
-                ex[r] = ee;
-                down[r] = __builtin_bit_cast(float, (unsigned)(127 - ee) << 23);
-            }
-        }
+        q8v_row_exponents(smax, ex, down);
 
         // ---- online softmax of head c over logit + E ------------------------------------------------
         float t4[4], tw[4];
