@@ -9,12 +9,16 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libbreccia_kv.so")
 BENCH_LIB = os.path.join(HERE, "libbreccia_kv_bench.so")
+
+# the calls of a serving loop for Python callers, past ctypes (csrc/hot_calls.cpp)
+HOT_MODULE = os.path.join(HERE, "_hot" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 SOURCES = ["allocator.cpp", "prefix_tree.cpp", "api.hip", "kv_move.hip", "decode_attn.hip", "decode_attn_mfma.hip", "prefill_attn.hip", "select.hip"]
 ARCH = "gfx950"
@@ -66,7 +70,21 @@ def build(verbose: bool = False) -> str:
     _run([hipcc] + HIP_FLAGS + ["-I", os.path.join(HERE, "..", "include"), "-c",
                                 os.path.join(CSRC, "bench_support.hip"), "-o", obj])
     _run([hipcc, "-shared", "-fPIC", "--offload-arch=" + ARCH, obj, "-o", BENCH_LIB])
+    build_hot_calls(verbose)
     return LIB
+
+
+def build_hot_calls(verbose: bool = False) -> str:
+    """The CPython module that kv.py makes its per-layer calls through; host code, links the library."""
+    import numpy
+
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-I", sysconfig.get_paths()["include"],
+           "-I", numpy.get_include(), os.path.join(CSRC, "hot_calls.cpp"), "-o", HOT_MODULE, "-L" + HERE, "-lbreccia_kv",
+           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath,/opt/rocm/lib"]
+    if verbose:
+        print(" ".join(cmd))
+    _run(cmd)
+    return HOT_MODULE
 
 
 def build_cpp_mirror_test(verbose: bool = False) -> str:

@@ -175,6 +175,8 @@ AllocErr PageAllocator::retain_fresh_page(int32_t* page_out, std::string& err) {
 bool PageAllocator::seq_resident(int32_t seq, int64_t n_cells) const {
     const int64_t pages = (n_cells + page_cells_ - 1) / page_cells_;
     if (pages > seqs_[(size_t)seq].n_pages) return false;
+    // asked for every entry of every attention call: no look at up to 8192 entries where none is out
+    if (seqs_[(size_t)seq].away == 0) return true;
     const int32_t* row = seq_table(seq);
     for (int64_t c = 0; c < pages; ++c)
         if (row[c] < 0) return false;
@@ -352,6 +354,7 @@ AllocErr PageAllocator::seq_detach_pages(int32_t seq, int32_t lp0, int32_t n,
         drop_page(row[c]);
         set_entry(seq, c, -1);
     }
+    q.away += n;
     return AllocErr::Ok;
 }
 
@@ -384,6 +387,7 @@ AllocErr PageAllocator::seq_attach_pages(int32_t seq, int32_t lp0, int32_t n,
         phys_out.push_back(p);
         set_entry(seq, c, p);
     }
+    q.away -= n;
     return AllocErr::Ok;
 }
 
@@ -392,6 +396,7 @@ bool PageAllocator::check(std::string& err) const {
     for (int32_t s = 0; s < max_seqs_; ++s) {
         const Seq& q = seqs_[(size_t)s];
         const int32_t* row = seq_table(s);
+        int32_t away = 0;
         for (int32_t c = 0; c < max_pages_per_seq_; ++c) {
             const int32_t p = row[c];
             if (!q.live || c >= q.n_pages) {
@@ -406,6 +411,11 @@ bool PageAllocator::check(std::string& err) const {
                 return false;
             }
             if (p >= 0) ++seen[(size_t)p];
+            else ++away;
+        }
+        if (q.live && away != q.away) {
+            err = fmt("sequence %lld: %lld pages out, %lld counted", s, away, q.away);
+            return false;
         }
         if (q.live && q.len > (int64_t)q.n_pages * page_cells_) {
             err = fmt("sequence %lld: length %lld exceeds its %lld pages", s, q.len, q.n_pages);

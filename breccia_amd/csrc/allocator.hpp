@@ -90,6 +90,7 @@ private:
         bool live = false;
         int64_t len = 0;
         int32_t n_pages = 0;
+        int32_t away = 0;  // of them, entries of -1: pages that were swapped out
     };
 
     int32_t take_page();

@@ -11,6 +11,11 @@ import os
 import numpy as np
 
 from . import lib as L
+
+try:
+    from . import _hot
+except ImportError as e:
+    raise ImportError("breccia_amd._hot is not built or does not load (%s). Build it with `python -m breccia_amd.build`" % e) from e
 from .lib import BkvError, PagePair, PoolDesc, check, lib  # noqa: F401
 
 
@@ -260,6 +265,9 @@ class Pool:
 
     def seq_reserve(self, seq: int, new_len: int, cow_capacity: int = 4):
         """Returns the list of (src, dst) copy-on-write pairs the caller must page_copy."""
+        done = _hot.seq_reserve(self.handle, seq, new_len, cow_capacity)
+        if done is not NotImplemented:
+            return done if type(done) is list else check(done)
         pairs = (PagePair * max(cow_capacity, 1))()
         n = C.c_int32()
         check(lib.bkv_seq_reserve(self.handle, seq, new_len, pairs, cow_capacity, n))
@@ -370,9 +378,14 @@ class Pool:
         return tuple(int(x) for x in nodes), tuple(int(x) for x in moved)
 
     # -- hot path
+    # Plain arguments go through the _hot module, which makes the same C call and returns its status; whatever it does
+    # not take (NotImplemented, nothing done) goes through ctypes.
     def append(self, layer: int, seqs, pos0, n_tokens, k_dev, v_dev, stream=None,
                f16_rows: bool = False) -> None:
         """k_dev / v_dev hold f32 rows, or raw binary16 rows when f16_rows is set."""
+        done = _hot.append(self.handle, layer, seqs, pos0, n_tokens, k_dev, v_dev, stream, f16_rows)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos0, pp = _i64(pos0)
         n_tokens, pn = _i32(n_tokens)
@@ -383,6 +396,10 @@ class Pool:
     def append_kprep(self, layer: int, seqs, pos0, n_tokens, k_dev, v_dev, gamma_dev, eps: float,
                      table_dev, n_rot: int, max_pos: int, positions_dev=None, stream=None) -> None:
         """RMSNorm(k) * gamma -> rotary at the token's position -> append, in one launch."""
+        done = _hot.append_kprep(self.handle, layer, seqs, pos0, n_tokens, k_dev, v_dev, gamma_dev, eps, table_dev, n_rot, max_pos,
+                                 positions_dev, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos0, pp = _i64(pos0)
         n_tokens, pn = _i32(n_tokens)
@@ -395,6 +412,10 @@ class Pool:
     def decode_attn(self, layer: int, seqs, pos, n_q_head: int, q_dev, out_dev, scale: float,
                     gate_dev=None, gate_seq_stride: int = 0, gate_head_stride: int = 0,
                     stream=None) -> None:
+        done = _hot.decode_attn(self.handle, layer, seqs, pos, n_q_head, q_dev, out_dev, scale, gate_dev, gate_seq_stride,
+                                gate_head_stride, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos, pp = _i64(pos)
         assert seqs.size == pos.size
@@ -415,6 +436,10 @@ class Pool:
     def prefill_attn(self, layer: int, seqs, pos0, n_tokens, n_q_head: int, q_dev, out_dev, scale: float,
                      gate_dev=None, gate_tok_stride: int = 0, gate_head_stride: int = 0, stream=None) -> None:
         """Causal attention of whole chunks (token t of chunk i sees cells 0..pos0[i]+t), on MFMA."""
+        done = _hot.prefill_attn(self.handle, layer, seqs, pos0, n_tokens, n_q_head, q_dev, out_dev, scale, gate_dev,
+                                 gate_tok_stride, gate_head_stride, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos0, pp = _i64(pos0)
         n_tokens, pn = _i32(n_tokens)
@@ -427,6 +452,10 @@ class Pool:
                     scale: float, gate_dev=None, gate_seq_stride: int = 0, gate_head_stride: int = 0,
                     stream=None) -> None:
         """Append one token per sequence at pos and attend 0..pos, in one call."""
+        done = _hot.decode_step(self.handle, layer, seqs, pos, k_new_dev, v_new_dev, n_q_head, q_dev, out_dev, scale, gate_dev,
+                                gate_seq_stride, gate_head_stride, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos, pp = _i64(pos)
         assert seqs.size == pos.size
@@ -438,6 +467,10 @@ class Pool:
                            ids_dev, id_stride: int, counts_dev, max_ids: int, gate_dev=None,
                            gate_seq_stride: int = 0, gate_head_stride: int = 0, stream=None) -> None:
         """Attention over per-entry lists of selected 4-cell blocks (device u32 ids / counts)."""
+        done = _hot.decode_attn_select(self.handle, layer, seqs, pos, n_q_head, q_dev, out_dev, scale, ids_dev, id_stride,
+                                       counts_dev, max_ids, gate_dev, gate_seq_stride, gate_head_stride, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         seqs, ps = _i32(seqs)
         pos, pp = _i64(pos)
         assert seqs.size == pos.size
@@ -450,6 +483,10 @@ class Pool:
                       topk_blocks: int, ids_dev, id_stride: int, counts_dev, max_ids: int,
                       stream=None) -> None:
         """Indexer score + top-k: leaves ids / counts on the device for decode_attn_select."""
+        done = _hot.select_blocks(self.handle, pos, idx_q_dev, pooled_devs, n_blocks, idx_n_head, idx_dim, topk_blocks, ids_dev,
+                                  id_stride, counts_dev, max_ids, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         pos, pp = _i64(pos)
         n_blocks, pn = _i32(n_blocks)
         assert pos.size == n_blocks.size == len(pooled_devs)
@@ -461,6 +498,10 @@ class Pool:
     def idx_pool(self, pooled_dev, max_blocks: int, tail_dev, idx_k_dev, pos0: int, tokens: int, gamma_dev,
                  eps: float, table_dev, n_rot: int, max_pos: int, idx_dim: int = 128, stream=None) -> None:
         """Pool the indexer keys of every block this call completes; keep the incomplete tail."""
+        done = _hot.idx_pool(self.handle, pooled_dev, max_blocks, tail_dev, idx_k_dev, pos0, tokens, gamma_dev, eps, table_dev,
+                             n_rot, max_pos, idx_dim, stream)
+        if done is not NotImplemented:
+            return check(done) if done else None
         check(lib.bkv_idx_pool(self.handle, _ptr(pooled_dev), max_blocks, _ptr(tail_dev), _ptr(idx_k_dev), pos0,
                                tokens, _ptr(gamma_dev), eps, _ptr(table_dev), n_rot, max_pos, idx_dim,
                                _sh(stream)))
@@ -608,3 +649,6 @@ def _ptr(x):
     if isinstance(x, DeviceBuffer):
         return x.ptr
     return x
+
+
+_hot.bind(C.c_void_p, DeviceBuffer, Stream)
