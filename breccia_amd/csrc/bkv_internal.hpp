@@ -185,13 +185,20 @@ inline void launch_staged(bkv_pool* p, int stage, K kernel, dim3 grid, dim3 bloc
 }
 
 // ---- kernel launchers (each validates nothing: callers have checked) ---------
-struct AppendBatch {
+// Entries of a batch that travels in the smaller of a kernel's argument structs: what a launch costs the host grows
+// with its arguments (measured at AttnKernelArgs, decode_attn_common.hpp).
+constexpr int32_t kFewEntries = 16;
+static_assert((kFewEntries & (kFewEntries - 1)) == 0 && kFewEntries < BKV_MAX_BATCH, "a power of two");
+
+template <int N>
+struct AppendBatchOf {
     int32_t n;
-    int32_t row[BKV_MAX_BATCH];      // block-table row of the sequence
-    int32_t pos0[BKV_MAX_BATCH];     // first cell
-    int32_t n_tok[BKV_MAX_BATCH];    // tokens of this sequence
-    int32_t src0[BKV_MAX_BATCH];     // first source row in k/v
+    int32_t row[N];      // block-table row of the sequence
+    int32_t pos0[N];     // first cell
+    int32_t n_tok[N];    // tokens of this sequence
+    int32_t src0[N];     // first source row in k/v
 };
+using AppendBatch = AppendBatchOf<BKV_MAX_BATCH>;
 hipError_t launch_append(bkv_pool* p, int32_t layer, const AppendBatch& b, int32_t max_tok,
                          const void* k, const void* v, bool src_is_f16, hipStream_t stream);
 

@@ -22,7 +22,6 @@ namespace bkv {
 namespace {
 
 struct MergeParams {
-    AttnBatch b;
     const AttnBatch* bd;  // DESC: the batch is read from this device-resident copy
     const float* part_o;
     const float* part_ml;
@@ -32,6 +31,21 @@ struct MergeParams {
     int32_t n_kv, n_q, group;
     uint32_t inv_group16;  // small_divisor_inverse(group)
 };
+// What the merge needs of a batch, as an argument (kFewEntries: why there are two).
+template <int N>
+struct MergeArgs : MergeParams {
+    int32_t splits[N], wg_base[N];
+};
+template <int N>
+static MergeArgs<N> merge_args(const MergeParams& mp, const AttnBatch& b) {
+    MergeArgs<N> args{};
+    static_cast<MergeParams&>(args) = mp;
+    for (int i = 0; i < b.n; ++i) {
+        args.splits[i] = b.splits[i];
+        args.wg_base[i] = b.wg_base[i];
+    }
+    return args;
+}
 
 constexpr int kMergeWaves = 4;
 constexpr int kMergeCols = 64;                  // columns of a work-group
@@ -88,8 +102,10 @@ __device__ __forceinline__ void merge_rounds(const float* po, const float* pml, 
 // maximum agreed ahead of the sums, it was 6900 cycles for one sequence of 4096 cells (65 splits), 5400 for four of up to
 // 2048 and 6100 for eight of up to 32k.  Every 16 lanes now keep a maximum of their own and everything meets once, at the
 // end, and a quarter of a head is what one compute unit takes in a quarter of the time (64 bytes a clock): 4000, 3400, 3600.
-template <bool DESC>
-__global__ __launch_bounds__(64 * kMergeWaves) void decode_attn_merge_kernel(const MergeParams P) {
+// N: entries of the batch in the arguments, 0: the batch is in device memory (DESC).
+template <int N>
+__global__ __launch_bounds__(64 * kMergeWaves) void decode_attn_merge_kernel(const std::conditional_t<N == 0, MergeParams, MergeArgs<N>> P) {
+    constexpr bool DESC = N == 0;
     __shared__ __attribute__((aligned(16))) float red[kMergeWaves][kMergeCols];
     __shared__ __attribute__((aligned(16))) float red_m[kMergeWaves], red_l[kMergeWaves];
     // grid (q heads x quarters, entries): no division at the head of a kernel that is all latency, and every argument
@@ -103,8 +119,8 @@ __global__ __launch_bounds__(64 * kMergeWaves) void decode_attn_merge_kernel(con
         splits = D->splits[e];
         base = D->wg_base[e];
     } else {
-        splits = P.b.splits[e];
-        base = P.b.wg_base[e];
+        splits = P.splits[e];
+        base = P.wg_base[e];
     }
     asm volatile("" ::"s"(splits), "s"(base), "s"(P.part_o), "s"(P.part_ml), "s"(P.gate), "s"(P.out), "s"(P.gate_seq_stride), "s"(P.gate_head_stride),
                  "s"(P.n_kv), "s"(P.n_q), "s"(P.group), "s"(P.inv_group16));
@@ -239,7 +255,6 @@ hipError_t launch_decode_attn(bkv_pool* p, int32_t layer, const AttnBatch& b, co
     const int32_t n_kv = p->g.n_kv;
     const int32_t group = a.n_q_head / n_kv;
     AttnKernelParams kp;
-    kp.b = b;
     kp.bd = a.desc;
     kp.kpool = p->k_layer[(size_t)layer];
     kp.vpool = p->v_layer[(size_t)layer];
@@ -268,10 +283,9 @@ hipError_t launch_decode_attn(bkv_pool* p, int32_t layer, const AttnBatch& b, co
     // the events ride on the dispatch
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     if (a.timed) (void)timer_dispatch_events(p, BKV_STAGE_ATTN_SPLIT, &ev_start, &ev_stop);
-    hipError_t err = launch_decode_attn_mfma(kp, p->g.layout, step, sel, total, stream, ev_start, ev_stop);
+    hipError_t err = launch_decode_attn_mfma(kp, b, p->g.layout, step, sel, total, stream, ev_start, ev_stop);
     if (err != hipSuccess) return err;
     MergeParams mp;
-    mp.b = b;
     mp.bd = a.desc;
     mp.part_o = kp.part_o;
     mp.part_ml = kp.part_ml;
@@ -284,12 +298,15 @@ hipError_t launch_decode_attn(bkv_pool* p, int32_t layer, const AttnBatch& b, co
     mp.group = group;
     mp.inv_group16 = small_divisor_inverse(group);
     const dim3 mgrid((unsigned)a.n_q_head * (kHd / kMergeCols), (unsigned)b.n), mblock(64 * kMergeWaves);
-    if (a.desc)
-        hipLaunchKernelGGL(decode_attn_merge_kernel<true>, mgrid, mblock, 0, stream, mp);
-    else if (a.timed)
-        launch_staged(p, BKV_STAGE_ATTN_MERGE, decode_attn_merge_kernel<false>, mgrid, mblock, 0, stream, mp);
-    else
-        hipLaunchKernelGGL(decode_attn_merge_kernel<false>, mgrid, mblock, 0, stream, mp);
+    const auto merge = [&](auto kernel, const auto& args) {
+        if (a.timed && !a.desc)
+            launch_staged(p, BKV_STAGE_ATTN_MERGE, kernel, mgrid, mblock, 0, stream, args);
+        else
+            hipLaunchKernelGGL(kernel, mgrid, mblock, 0, stream, args);
+    };
+    if (a.desc) merge(decode_attn_merge_kernel<0>, mp);
+    else if (b.n <= kFewEntries) merge(decode_attn_merge_kernel<kFewEntries>, merge_args<kFewEntries>(mp, b));
+    else merge(decode_attn_merge_kernel<kMaxBatch>, merge_args<kMaxBatch>(mp, b));
     return hipGetLastError();
 }
 

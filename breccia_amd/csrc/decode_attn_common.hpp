@@ -3,6 +3,8 @@
 // live.
 #pragma once
 
+#include <type_traits>
+
 #include "bkv_internal.hpp"
 
 namespace bkv {
@@ -17,8 +19,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 struct AttnKernelParams {
-    AttnBatch b;
-    // kernels instantiated with DESC read the batch from this device-resident copy instead of `b`: a
+    // kernels instantiated with DESC read the batch from this device-resident copy instead of their arguments: a
     // launch recorded once (in a graph) then serves whatever batch the descriptor holds when it runs
     const AttnBatch* bd;
     const uint8_t* kpool;
@@ -45,6 +46,22 @@ struct AttnKernelParams {
     uint8_t* vpool_w;
 };
 
+// The batch as a kernel argument.  What a launch costs the host grows with its arguments (2.8 us up to 100 bytes, 3.3 at
+// 500, 3.9 at 1500), and the short steps of a decode loop are bound by that: a batch of few entries travels in a
+// smaller struct, in kernels of their own.  12 layers of one sequence of 4096 cells 113 -> 104 us, of four
+// short ones 113 -> 101; where the kernels are what bounds a step (eight sequences of 1k to 32k, 191.9) it makes no difference.
+// The append with K preparation keeps the one struct: with the smaller one its four launches in 159 us took 1.3 longer.  16 entries: from 200 bytes to 500 there is little between.
+struct AttnBatchFew {
+    int32_t n;
+    int32_t row[kFewEntries], pos[kFewEntries], wg_base[kFewEntries], pps[kFewEntries];
+};
+template <typename Batch>
+struct AttnKernelArgs : AttnKernelParams {
+    Batch b;
+};
+template <bool DESC>
+using AttnArgsOf = std::conditional_t<DESC, AttnKernelParams, AttnKernelArgs<AttnBatch>>;
+
 // x / d for the small numbers of this launch geometry, as a multiplication by ceil(2^16 / d): exact while
 // x * d < 2^16 (work-group indices stay below kMaxWgs = 4096, head indices below 256, divisors are kv head
 // counts and head groups of at most 16).  An integer division by a run-time value is some forty dependent
@@ -69,7 +86,9 @@ template <bool STEP, bool DESC, typename Batch>
 __device__ __forceinline__ bool find_unit(const AttnKernelParams& P, const Batch& B, int unit, int& e, int& rem, int& pos, int& row, int& pps) {
     static_assert(kMaxBatch <= 64, "one lane per entry");
     const int lane = lane_of_wave();  // not kept for later: the kernels have no register to spare for it
-    const int first = B.wg_base[lane], my_pos = B.pos[lane], my_row = B.row[lane], my_pps = B.pps[lane];
+    constexpr bool kFew = std::is_same<Batch, AttnBatchFew>::value;
+    const int at = kFew ? lane & (kFewEntries - 1) : lane;
+    const int first = B.wg_base[at], my_pos = B.pos[at], my_row = B.row[at], my_pps = B.pps[at];
     const int n = B.n;
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::"s"(n), "s"(P.kpool), "s"(P.vpool), "s"(P.tables), "s"(P.q), "s"(P.max_pages_per_seq), "s"(P.n_kv), "s"(P.n_q),
@@ -83,9 +102,9 @@ __device__ __forceinline__ bool find_unit(const AttnKernelParams& P, const Batch
     pps = __builtin_amdgcn_readlane(my_pps, e);
     return true;
 }
-template <bool STEP, bool DESC>
-__device__ __forceinline__ bool unit_of_work_group(const AttnKernelParams& P, int unit, int& e, int& rem, int& pos,
-                                                   int& row, int& pps) {
+// Args: AttnKernelArgs of the batch's kind; with DESC the AttnKernelParams alone.
+template <bool STEP, bool DESC, typename Args>
+__device__ __forceinline__ bool unit_of_work_group(const Args& P, int unit, int& e, int& rem, int& pos, int& row, int& pps) {
     if constexpr (DESC) return find_unit<STEP, true>(P, *(batch_desc_ptr)(uintptr_t)P.bd, unit, e, rem, pos, row, pps);
     else return find_unit<STEP, false>(P, P.b, unit, e, rem, pos, row, pps);
 }
@@ -124,7 +143,7 @@ __device__ __forceinline__ bool block_cell_live(uint32_t id, int r, int pos) {
 // (entry, kv head, page range).
 // `start` / `stop`: optional events attached to the dispatch (its own begin and end time stamps)
 // kp.bd != nullptr: the step kernels that read the batch from the descriptor (`total` is then the fixed grid).
-hipError_t launch_decode_attn_mfma(const AttnKernelParams& kp, int layout, bool step, bool sel, int32_t total,
+hipError_t launch_decode_attn_mfma(const AttnKernelParams& kp, const AttnBatch& b, int layout, bool step, bool sel, int32_t total,
                                    hipStream_t stream, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
 }  // namespace bkv

@@ -492,8 +492,8 @@ __device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageL
 // pool on the way): the pool ends up as bkv_append would leave it, the output as append + attend.
 // SEL: the 16 rows of an iteration are four listed 4-cell blocks instead of a page (block g
 // supplies the V rows of lane group g, block c / 4 the K row of lane c).
-template <bool STEP, bool SEL = false, bool DESC = false>
-__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnKernelParams P) {
+template <bool STEP, bool SEL, bool DESC, typename Args>
+__device__ __forceinline__ void split_f16(const Args& P) {
     static_assert(!(STEP && SEL), "the fused step attends the dense selection");
     // the q fragments on their way between the waves lie where the fold staging will be
     __shared__ __attribute__((aligned(16))) MfmaFoldLds lds;
@@ -779,6 +779,15 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnK
 
     mfma_fold_and_store(P, lds, wg, wave, c, g, o, m_run, l_run);
 }
+template <bool STEP, bool SEL = false, bool DESC = false>
+__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_kernel(const AttnArgsOf<DESC> P) {
+    split_f16<STEP, SEL, DESC>(P);
+}
+// A batch of few entries.  f16 pools only: with a body that is a function of its own the int8 kernels spill.
+template <bool STEP, bool SEL>
+__global__ __launch_bounds__(kBlock, 2) void decode_attn_few_kernel(const AttnKernelArgs<AttnBatchFew> P) {
+    split_f16<STEP, SEL, false>(P);
+}
 
 // ---- decode attention on the matrix cores, int8 rows with f16 block scales ---------------------
 // The I8H layout ([256 x i8][8 x f16 scale] per row) through the same MFMA decomposition as
@@ -1020,7 +1029,7 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
 // SEL: an iteration's 16 rows are four listed 4-cell blocks (see decode_attn_mfma_kernel); the
 // work is planned for max_ids blocks, a work-group past the end of the list has nothing to do.
 template <bool STEP, bool DESC = false, bool SEL = false>
-__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const AttnKernelParams P) {
+__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const AttnArgsOf<DESC> P) {
     static_assert(!(STEP && SEL), "the fused step attends the dense selection");
     // one slot per wave; the fold staging of the epilogue reuses the memory
     constexpr int kRing = kWaves * kI8hSlot > (int)sizeof(MfmaFoldLds) ? kWaves * kI8hSlot : (int)sizeof(MfmaFoldLds);
@@ -1551,7 +1560,7 @@ __device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ
 
 // SEL: an iteration's 16 rows are four listed 4-cell blocks, as in the int8 kernel.
 template <bool STEP, bool DESC = false, bool SEL = false>
-__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const AttnKernelParams P) {
+__global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const AttnArgsOf<DESC> P) {
     static_assert(!(STEP && SEL), "the fused step attends the dense selection");
     // per wave one V slot during the loop, the fold staging after it
     constexpr int kWaveLds = kQ8vUnit;
@@ -1880,16 +1889,15 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
 
 // With `start` / `stop` the two events are attached to the dispatch itself (they take the kernel's
 // own begin and end time stamps, what a profiler's kernel trace reports), otherwise a plain launch.
-template <typename K>
-static void launch_one(K kernel, const AttnKernelParams& kp, int32_t total, hipStream_t stream, hipEvent_t start,
-                       hipEvent_t stop) {
+template <typename K, typename Args>
+static void launch_one(K kernel, const Args& args, int32_t total, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
     if (start && stop)
-        hipExtLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(kBlock), 0, stream, start, stop, 0, kp);
+        hipExtLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(kBlock), 0, stream, start, stop, 0, args);
     else
-        kernel<<<total, kBlock, 0, stream>>>(kp);
+        kernel<<<total, kBlock, 0, stream>>>(args);
 }
 
-hipError_t launch_decode_attn_mfma(const AttnKernelParams& kp, int layout, bool step, bool sel, int32_t total,
+hipError_t launch_decode_attn_mfma(const AttnKernelParams& kp, const AttnBatch& b, int layout, bool step, bool sel, int32_t total,
                                    hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
     if (kp.bd) {
         // the batch comes from the device-resident descriptor: the fused step only
@@ -1902,26 +1910,47 @@ hipError_t launch_decode_attn_mfma(const AttnKernelParams& kp, int layout, bool 
             launch_one(decode_attn_mfma_kernel<true, false, true>, kp, total, stream, start, stop);
         return hipGetLastError();
     }
+    if (layout == BKV_LAYOUT_F16 && b.n <= kFewEntries) {
+        AttnKernelArgs<AttnBatchFew> args{};
+        static_cast<AttnKernelParams&>(args) = kp;
+        args.b.n = b.n;
+        for (int i = 0; i < b.n; ++i) {
+            args.b.row[i] = b.row[i];
+            args.b.pos[i] = b.pos[i];
+            args.b.wg_base[i] = b.wg_base[i];
+            args.b.pps[i] = b.pps[i];
+        }
+        if (step)
+            launch_one(decode_attn_few_kernel<true, false>, args, total, stream, start, stop);
+        else if (sel)
+            launch_one(decode_attn_few_kernel<false, true>, args, total, stream, start, stop);
+        else
+            launch_one(decode_attn_few_kernel<false, false>, args, total, stream, start, stop);
+        return hipGetLastError();
+    }
+    AttnKernelArgs<AttnBatch> args;
+    static_cast<AttnKernelParams&>(args) = kp;
+    args.b = b;
     if (layout == BKV_LAYOUT_I8H) {
         if (step)
-            launch_one(decode_attn_mfma_i8h_kernel<true>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_i8h_kernel<true>, args, total, stream, start, stop);
         else if (sel)
-            launch_one(decode_attn_mfma_i8h_kernel<false, false, true>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_i8h_kernel<false, false, true>, args, total, stream, start, stop);
         else
-            launch_one(decode_attn_mfma_i8h_kernel<false>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_i8h_kernel<false>, args, total, stream, start, stop);
     } else if (layout == BKV_LAYOUT_Q8V) {
         if (step)
-            launch_one(decode_attn_mfma_q8v_kernel<true>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_q8v_kernel<true>, args, total, stream, start, stop);
         else if (sel)
-            launch_one(decode_attn_mfma_q8v_kernel<false, false, true>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_q8v_kernel<false, false, true>, args, total, stream, start, stop);
         else
-            launch_one(decode_attn_mfma_q8v_kernel<false>, kp, total, stream, start, stop);
+            launch_one(decode_attn_mfma_q8v_kernel<false>, args, total, stream, start, stop);
     } else if (step)
-        launch_one(decode_attn_mfma_kernel<true, false>, kp, total, stream, start, stop);
+        launch_one(decode_attn_mfma_kernel<true, false>, args, total, stream, start, stop);
     else if (sel)
-        launch_one(decode_attn_mfma_kernel<false, true>, kp, total, stream, start, stop);
+        launch_one(decode_attn_mfma_kernel<false, true>, args, total, stream, start, stop);
     else
-        launch_one(decode_attn_mfma_kernel<false, false>, kp, total, stream, start, stop);
+        launch_one(decode_attn_mfma_kernel<false, false>, args, total, stream, start, stop);
     return hipGetLastError();
 }
 

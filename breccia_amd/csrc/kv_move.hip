@@ -117,7 +117,8 @@ __device__ __forceinline__ RowOfSeq split_row(uint64_t r, unsigned n_kv, bool fi
     return RowOfSeq{t, (unsigned)(r - (uint64_t)t * n_kv)};
 }
 // the pool row of (sequence s of the call, token t, kv head)
-__device__ __forceinline__ size_t pool_row_of(const AppendBatch& b, const MoveGeom& g, const int32_t* tables, int s,
+template <typename Batch>
+__device__ __forceinline__ size_t pool_row_of(const Batch& b, const MoveGeom& g, const int32_t* tables, int s,
                                               RowOfSeq rs) {
     // cells are below 2^31 (pos0 and the token count are int32 and their sum is checked on the host)
     const unsigned cell = (unsigned)b.pos0[s] + rs.t;
@@ -129,8 +130,8 @@ __device__ __forceinline__ size_t pool_row_of(const AppendBatch& b, const MoveGe
 // One lane converts 8 consecutive elements of one (token, kv head) row of K and of V:
 // two 16-byte loads and one 16-byte store per pool.  grid.y = sequence of the call; the rows of a
 // sequence are contiguous in the source, so unit u of a sequence is simply its u-th 8-element group.
-template <typename SrcT, int HD>
-__global__ __launch_bounds__(kBlock) void append_f16_kernel(AppendBatch b, MoveGeom g,
+template <typename SrcT, int HD, typename Batch>
+__global__ __launch_bounds__(kBlock) void append_f16_kernel(Batch b, MoveGeom g,
                                                             uint16_t* __restrict__ kpool,
                                                             uint16_t* __restrict__ vpool,
                                                             const int32_t* __restrict__ tables,
@@ -202,8 +203,8 @@ __device__ __forceinline__ void image_rows_out(const uint8_t* image, uint8_t* po
 // leave as whole contiguous rows, one 16-byte piece a lane (4-byte pieces when the head dim
 // makes rows that are not 16-byte multiples).  A work-group owns 256 / (hd / 8) consecutive
 // rows of one sequence of the call (grid.y).
-template <int LAYOUT, typename SrcT, int HD>
-__global__ __launch_bounds__(kBlock) void append_quant_kernel(AppendBatch b, MoveGeom g,
+template <int LAYOUT, typename SrcT, int HD, typename Batch>
+__global__ __launch_bounds__(kBlock) void append_quant_kernel(Batch b, MoveGeom g,
                                                               uint8_t* __restrict__ kpool,
                                                               uint8_t* __restrict__ vpool,
                                                               const int32_t* __restrict__ tables,
@@ -769,8 +770,23 @@ PoolPtrs pool_ptrs(const bkv_pool* p) {
 
 }  // namespace
 
-template <typename SrcT>
-static hipError_t launch_append_from(bkv_pool* p, int32_t layer, const AppendBatch& b,
+// f of the batch, in the smaller argument struct where it fits (kFewEntries)
+template <typename F>
+static void with_batch(const AppendBatch& b, F f) {
+    if (b.n > kFewEntries) return f(b);
+    AppendBatchOf<kFewEntries> few{};
+    few.n = b.n;
+    for (int i = 0; i < b.n; ++i) {
+        few.row[i] = b.row[i];
+        few.pos0[i] = b.pos0[i];
+        few.n_tok[i] = b.n_tok[i];
+        few.src0[i] = b.src0[i];
+    }
+    f(few);
+}
+
+template <typename SrcT, typename Batch>
+static hipError_t launch_append_from(bkv_pool* p, int32_t layer, const Batch& b,
                                      int32_t max_tok, const SrcT* k, const SrcT* v,
                                      hipStream_t stream) {
     const MoveGeom g = move_geom(p);
@@ -781,10 +797,10 @@ static hipError_t launch_append_from(bkv_pool* p, int32_t layer, const AppendBat
         const int64_t lanes = (int64_t)max_tok * (g.n_kv * g.hd / 8);
         dim3 grid((unsigned)((lanes + kBlock - 1) / kBlock), (unsigned)b.n);
         if (g.hd == 256)
-            launch_staged(p, BKV_STAGE_APPEND, append_f16_kernel<SrcT, 256>, grid, dim3(kBlock), 0, stream, b, g,
+            launch_staged(p, BKV_STAGE_APPEND, append_f16_kernel<SrcT, 256, Batch>, grid, dim3(kBlock), 0, stream, b, g,
                           (uint16_t*)kp, (uint16_t*)vp, tables, k, v);
         else
-            launch_staged(p, BKV_STAGE_APPEND, append_f16_kernel<SrcT, 0>, grid, dim3(kBlock), 0, stream, b, g,
+            launch_staged(p, BKV_STAGE_APPEND, append_f16_kernel<SrcT, 0, Batch>, grid, dim3(kBlock), 0, stream, b, g,
                           (uint16_t*)kp, (uint16_t*)vp, tables, k, v);
         return hipGetLastError();
     }
@@ -792,22 +808,25 @@ static hipError_t launch_append_from(bkv_pool* p, int32_t layer, const AppendBat
     const int64_t rows = (int64_t)max_tok * g.n_kv;
     dim3 grid((unsigned)((rows + rows_wg - 1) / rows_wg), (unsigned)b.n);
     if (p->g.layout == BKV_LAYOUT_I8H)  // pools of this layout have head dim 256
-        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_I8H, SrcT, 256>, grid, dim3(kBlock), 0,
+        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_I8H, SrcT, 256, Batch>, grid, dim3(kBlock), 0,
                       stream, b, g, kp, vp, tables, k, v);
     else if (g.hd == 256)
-        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_Q8V, SrcT, 256>, grid, dim3(kBlock), 0,
+        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_Q8V, SrcT, 256, Batch>, grid, dim3(kBlock), 0,
                       stream, b, g, kp, vp, tables, k, v);
     else
-        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_Q8V, SrcT, 0>, grid, dim3(kBlock), 0,
+        launch_staged(p, BKV_STAGE_APPEND, append_quant_kernel<BKV_LAYOUT_Q8V, SrcT, 0, Batch>, grid, dim3(kBlock), 0,
                       stream, b, g, kp, vp, tables, k, v);
     return hipGetLastError();
 }
 
 hipError_t launch_append(bkv_pool* p, int32_t layer, const AppendBatch& b, int32_t max_tok,
                          const void* k, const void* v, bool src_is_f16, hipStream_t stream) {
-    if (src_is_f16)
-        return launch_append_from(p, layer, b, max_tok, (const uint16_t*)k, (const uint16_t*)v, stream);
-    return launch_append_from(p, layer, b, max_tok, (const float*)k, (const float*)v, stream);
+    hipError_t err = hipSuccess;
+    with_batch(b, [&](const auto& batch) {
+        err = src_is_f16 ? launch_append_from(p, layer, batch, max_tok, (const uint16_t*)k, (const uint16_t*)v, stream)
+                         : launch_append_from(p, layer, batch, max_tok, (const float*)k, (const float*)v, stream);
+    });
+    return err;
 }
 
 hipError_t launch_append_kprep(bkv_pool* p, int32_t layer, const AppendBatch& b, int32_t max_tok,

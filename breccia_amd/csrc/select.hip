@@ -16,6 +16,7 @@
 // in LDS and written out.  Everything is deterministic: no atomic decides an
 // order (the histogram counts are order-independent).
 #include <algorithm>
+#include <type_traits>
 
 #include "bkv_internal.hpp"
 
@@ -35,8 +36,10 @@ constexpr int kRankKeys = 256;    // keys of a radix bin that are ranked directl
 constexpr int kBuckets = kTopkThreads;  // buckets the selected keys are ordered through (one per thread)
 constexpr int kBucketCap = 64;    // a fuller bucket sends the list to the sorting network instead
 
+template <int N>  // lists that the arguments have room for (kFewEntries)
 struct ScoreParams {
-    SelectBatch b;
+    int32_t pos[N], n_blocks[N];
+    const float* pooled[N];
     const float* q;      // [n][idx_n_head][idx_dim]
     double* scores;      // [n][score_stride]
     int64_t score_stride;
@@ -49,22 +52,22 @@ struct ScoreParams {
 // at a time (pooled and q must be 16-byte aligned); DIM = 0: any width, element by element (the
 // index arithmetic of its loops divides by the run-time width).  The products and the sum keep
 // the CPU's order in both.
-template <int DIM>
-__global__ __launch_bounds__(kScoreThreads) void idx_score_kernel(const ScoreParams P) {
+template <int DIM, int N>
+__global__ __launch_bounds__(kScoreThreads) void idx_score_kernel(const ScoreParams<N> P) {
     // rows DIM + 4 (16-byte aligned, 4 banks apart: 16-byte reads of 64 rows do not collide) or
     // D + 1 floats apart (odd: lanes walking one column of 64 rows hit 64 banks)
     __shared__ __attribute__((aligned(16))) float pooled_s[kScoreTile * (kMaxIdxDim + 4)];
     __shared__ __attribute__((aligned(16))) float q_s[kMaxIdxHead * kMaxIdxDim];
     __shared__ double part_s[kMaxIdxHead][kScoreTile];
     const int e = blockIdx.y;
-    const int n_blocks = P.b.n_blocks[e];
+    const int n_blocks = P.n_blocks[e];
     const int b0 = (int)blockIdx.x * kScoreTile;
     if (b0 >= n_blocks) return;
     const int nb = min(kScoreTile, n_blocks - b0);
     const int D = DIM ? DIM : P.idx_dim, H = P.idx_n_head;
     const int stride = DIM ? DIM + 4 : D + 1;
     const int tid = threadIdx.x;
-    const float* pooled = P.b.pooled[e] + (size_t)b0 * D;
+    const float* pooled = P.pooled[e] + (size_t)b0 * D;
     if constexpr (DIM != 0) {
         constexpr int kRow4 = DIM / 4;
         for (int i = tid; i < nb * kRow4; i += kScoreThreads)
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(kScoreThreads) void idx_score_kernel(const ScorePar
         for (int h = 0; h < H; ++h) acc += part_s[h][tid];
         const int64_t first_cell = (int64_t)(b0 + tid) * P.idx_block;
         P.scores[(size_t)e * P.score_stride + b0 + tid] =
-            first_cell > (int64_t)P.b.pos[e] ? -INFINITY : acc;
+            first_cell > (int64_t)P.pos[e] ? -INFINITY : acc;
     }
 }
 
@@ -257,8 +260,9 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* wave_sums, int* 
     return before + inc - v;
 }
 
+template <int N>
 struct TopkParams {
-    SelectBatch b;
+    int32_t pos[N], n_blocks[N];
     const void* scores;   // [n][score_stride] of T
     int64_t score_stride;
     uint32_t* ids;        // [n][id_stride]
@@ -269,8 +273,8 @@ struct TopkParams {
 
 // kRegKeys = keys a thread keeps in registers: 8 serves lists of up to 8192 blocks (a 32k
 // context), 32 up to 32768 (128k); longer lists re-read their scores on every pass.
-template <typename T, int kRegKeys>
-__global__ __launch_bounds__(kTopkThreads) void topk_blocks_kernel(const TopkParams P) {
+template <typename T, int kRegKeys, int kRoom>
+__global__ __launch_bounds__(kTopkThreads) void topk_blocks_kernel(const TopkParams<kRoom> P) {
     // kHistCopies copies of the 256 bins, a lane adds to copy lane % kHistCopies: scores cluster in a
     // few bins of the first digit (its top bits are exponent bits), and LDS atomics of one wave on
     // one address run one after the other.  257 ints per copy put equal bins of different copies in
@@ -290,8 +294,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_blocks_kernel(const TopkPar
 
     const int e = blockIdx.x;
     const int tid = threadIdx.x;
-    const int N = P.b.n_blocks[e];
-    const uint32_t own = (uint32_t)(P.b.pos[e] / P.idx_block);
+    const int N = P.n_blocks[e];
+    const uint32_t own = (uint32_t)(P.pos[e] / P.idx_block);
     uint32_t* ids = P.ids + (size_t)e * P.id_stride;
 
     if (P.dense) {
@@ -744,24 +748,35 @@ __global__ __launch_bounds__(kTopkThreads) void topk_blocks_kernel(const TopkPar
 
 }  // namespace
 
+// f of the number of entries that the arguments of a launch for b have room for
+template <typename F>
+static void with_room_for(const SelectBatch& b, F f) {
+    if (b.n <= kFewEntries) f(std::integral_constant<int, kFewEntries>{});
+    else f(std::integral_constant<int, BKV_MAX_BATCH>{});
+}
+
 hipError_t launch_idx_score(bkv_pool* p, const SelectBatch& b, const float* q, int32_t idx_n_head, int32_t idx_dim,
                             int32_t idx_block, double* scores, int64_t score_stride, int32_t max_blocks,
                             hipStream_t stream) {
-    ScoreParams sp;
-    sp.b = b;
-    sp.q = q;
-    sp.scores = scores;
-    sp.score_stride = score_stride;
-    sp.idx_n_head = idx_n_head;
-    sp.idx_dim = idx_dim;
-    sp.idx_block = idx_block;
     dim3 grid((unsigned)((max_blocks + kScoreTile - 1) / kScoreTile), (unsigned)b.n);
     bool wide = idx_dim == 128 && (reinterpret_cast<uintptr_t>(q) & 15u) == 0;
     for (int i = 0; i < b.n && wide; ++i) wide = (reinterpret_cast<uintptr_t>(b.pooled[i]) & 15u) == 0;
-    if (wide)
-        launch_staged(p, BKV_STAGE_IDX_SCORE, idx_score_kernel<128>, grid, dim3(kScoreThreads), 0, stream, sp);
-    else
-        launch_staged(p, BKV_STAGE_IDX_SCORE, idx_score_kernel<0>, grid, dim3(kScoreThreads), 0, stream, sp);
+    with_room_for(b, [&](auto room) {
+        constexpr int N = decltype(room)::value;
+        ScoreParams<N> sp{};
+        std::copy(b.pos, b.pos + b.n, sp.pos);
+        std::copy(b.n_blocks, b.n_blocks + b.n, sp.n_blocks);
+        std::copy(b.pooled, b.pooled + b.n, sp.pooled);
+        sp.q = q;
+        sp.scores = scores;
+        sp.score_stride = score_stride;
+        sp.idx_n_head = idx_n_head;
+        sp.idx_dim = idx_dim;
+        sp.idx_block = idx_block;
+        const auto launch = [&](auto kernel) { launch_staged(p, BKV_STAGE_IDX_SCORE, kernel, grid, dim3(kScoreThreads), 0, stream, sp); };
+        if (wide) launch(idx_score_kernel<128, N>);
+        else launch(idx_score_kernel<0, N>);
+    });
     return hipGetLastError();
 }
 
@@ -769,31 +784,34 @@ hipError_t launch_topk_blocks(bkv_pool* p, const SelectBatch& b, const void* sco
                               int64_t score_stride, int32_t topk_blocks, int32_t idx_block, bool dense,
                               uint32_t* ids, int64_t id_stride, uint32_t* counts, int32_t max_ids,
                               hipStream_t stream) {
-    TopkParams tp;
-    tp.b = b;
-    tp.scores = scores;
-    tp.score_stride = score_stride;
-    tp.ids = ids;
-    tp.id_stride = id_stride;
-    tp.counts = counts;
-    tp.topk_blocks = topk_blocks;
-    tp.max_ids = max_ids;
-    tp.idx_block = idx_block;
-    tp.dense = dense ? 1 : 0;
     int32_t longest = 0;
     for (int i = 0; i < b.n; ++i) longest = std::max(longest, b.n_blocks[i]);
     const bool few = longest <= 8 * kTopkThreads;
-    if (scores_f64) {
-        if (few)
-            launch_staged(p, BKV_STAGE_TOPK, topk_blocks_kernel<double, 8>, dim3((unsigned)b.n), dim3(kTopkThreads), 0, stream, tp);
-        else
-            launch_staged(p, BKV_STAGE_TOPK, topk_blocks_kernel<double, 32>, dim3((unsigned)b.n), dim3(kTopkThreads), 0, stream, tp);
-    } else {
-        if (few)
-            launch_staged(p, BKV_STAGE_TOPK, topk_blocks_kernel<float, 8>, dim3((unsigned)b.n), dim3(kTopkThreads), 0, stream, tp);
-        else
-            launch_staged(p, BKV_STAGE_TOPK, topk_blocks_kernel<float, 32>, dim3((unsigned)b.n), dim3(kTopkThreads), 0, stream, tp);
-    }
+    with_room_for(b, [&](auto room) {
+        constexpr int N = decltype(room)::value;
+        TopkParams<N> tp{};
+        std::copy(b.pos, b.pos + b.n, tp.pos);
+        std::copy(b.n_blocks, b.n_blocks + b.n, tp.n_blocks);
+        tp.scores = scores;
+        tp.score_stride = score_stride;
+        tp.ids = ids;
+        tp.id_stride = id_stride;
+        tp.counts = counts;
+        tp.topk_blocks = topk_blocks;
+        tp.max_ids = max_ids;
+        tp.idx_block = idx_block;
+        tp.dense = dense ? 1 : 0;
+        const auto launch = [&](auto kernel) {
+            launch_staged(p, BKV_STAGE_TOPK, kernel, dim3((unsigned)b.n), dim3(kTopkThreads), 0, stream, tp);
+        };
+        if (scores_f64) {
+            if (few) launch(topk_blocks_kernel<double, 8, N>);
+            else launch(topk_blocks_kernel<double, 32, N>);
+        } else {
+            if (few) launch(topk_blocks_kernel<float, 8, N>);
+            else launch(topk_blocks_kernel<float, 32, N>);
+        }
+    });
     return hipGetLastError();
 }
 
