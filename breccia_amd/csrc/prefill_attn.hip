@@ -234,6 +234,11 @@ struct PrefillLds {
     uint8_t vimg[2][2][LAY == BKV_LAYOUT_F16 ? 1 : 2][kPage / 2][kLdsRowsV];
     float e[LAY == BKV_LAYOUT_Q8V ? 2 : 1][2][kPage];  // q8_0 V: E of the cells
 };
+// The waves' tiles of outputs on their way to memory; rows 16 bytes apart in the banks.
+constexpr int kOutRow = kHd + 4;
+struct OutLds {
+    float row[4][kRowsPerWave][kOutRow];
+};
 // byte of 16-byte chunk `chunk` of row `row` in a page image
 __device__ __forceinline__ int k_at(int row, int chunk) { return (row >> 1) * kLdsRowsK + (row & 1) * 512 + (chunk ^ (row & 1)) * 16; }
 __device__ __forceinline__ int v_at(int row, int chunk) { return (row >> 1) * kLdsRowsV + (row & 1) * 512 + (chunk ^ 2 * (row & 1)) * 16; }
@@ -872,6 +877,18 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     }
 
     // ---- normalise, gate, store ---------------------------------------------------------------------
+    // A lane holds 16 bytes of each 64 of its row: a store (or a request for the gate) straight from here touches 16 rows
+    // 16 bytes at a time, and the path to memory takes them row by row, 64 cycles an instruction.  The wave's tile goes
+    // through LDS instead (the images are done with) and leaves row by row, 1 KiB an instruction.  Cycles of the
+    // epilogue, before / now: one tile 4100 / 2900, two 8300 / 6100; 41 tokens behind 517 cells through 12 layers 217 ->
+    // 210 us.  Not so f16 pools with two tiles a wave: their calls fill the chip and are at its power limit, where
+    // cycles saved beside the products save no time, and the walk's registers come out worse (285 against 284 us).
+    constexpr bool kStaged = LAY != BKV_LAYOUT_F16 || TILES == 1;
+    if constexpr (kStaged) __syncthreads();
+    static_assert(sizeof(OutLds) <= sizeof(PrefillLds<LAY>), "the tiles of four waves in the memory of the images");
+    float* const mine = &reinterpret_cast<OutLds*>(&L)->row[wave][0][0];
+    // worked out again: the walk has no register to spare for them
+    const int lane_out = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), c_out = lane_out & 15, g_out = lane_out >> 4;
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
         if constexpr (Q8V) {
@@ -887,47 +904,100 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
             m_run[t] = ref;
         }
         const float l = sum_over_lane_groups(l_run[t]);
-        if (!row_live[t]) continue;
-        if constexpr (SPLIT) {
-            if (cut) {
-                const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
-                const size_t at = slot * kRowsPerWg + wave * kRows + t * kRowsPerWave + c;
-                float* po = P.part_o + at * kHd + 4 * g;
+        if constexpr (!kStaged) {
+            if (!row_live[t]) continue;
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            const auto op = in_global(out) + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
+            // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
+            // chain of 64 trips to memory
 #pragma unroll
-                for (int d = 0; d < 16; ++d) *reinterpret_cast<f4*>(po + 16 * d) = o[t][d];
-                if (g == 0) *reinterpret_cast<float2*>(P.part_ml + at * 2) = make_float2(m_run[t], l);
-                continue;
-            }
-        }
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        const auto op = in_global(out) + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
-        // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
-        // chain of 64 trips to memory
+            for (int half = 0; half < 2; ++half) {
+                f4 y[8];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            f4 y[8];
+                for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
+                if (gate) {
+                    f4 z[8];
+                    const auto at = in_global(gate) + ((size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride +
+                                                       128 * half + 4 * g);
+                    if (gate_in_fours) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) y[i] = o[t][half * 8 + i] * inv;
-            if (gate) {
-                f4 z[8];
-                const auto at = in_global(gate) + ((size_t)(src0 + tok[t]) * gate_tok_stride + (size_t)head[t] * gate_head_stride +
-                                                   128 * half + 4 * g);
-                if (gate_in_fours) {
+                        for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)(at + 16 * i);
+                    } else {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)(at + 16 * i);
-                } else {
+                        for (int i = 0; i < 8; ++i)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) z[i][r] = at[16 * i + r];
+                    }
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) z[i][r] = at[16 * i + r];
+                        for (int r = 0; r < 4; ++r) y[i][r] *= sigmoid(z[i][r]);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) *(__attribute__((address_space(1))) f4*)(op + 16 * (half * 8 + i) + 4 * g) = y[i];
+            }
+        } else {
+            const int live = min(n_rows - (row0 + t * kRowsPerWave), kRowsPerWave);  // rows of the tile
+            if (live <= 0) continue;
+            const bool parts = SPLIT && cut;
+            // rows of output and gate: worked out by lane r for row r (past the chunk's end: the last row's)
+            int head;
+            const int row = row0 + t * kRowsPerWave + min(c_out, live - 1), tok = src0 + divided_by(row, P.group, P.group_inverse, head);
+            head += kvh * P.group;
+            const uint64_t out_at = (uint64_t)(uintptr_t)out + ((uint64_t)tok * (uint64_t)n_q + (uint64_t)head) * (kHd * 4);
+            const uint64_t gate_at = (uint64_t)(uintptr_t)gate + (uint64_t)((int64_t)tok * gate_tok_stride + (int64_t)head * gate_head_stride) * 4;
+            const auto row_at = [](uint64_t at, int r) {
+                const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)at, r);
+                const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(at >> 32), r);
+                return (uint64_t)hi << 32 | lo;
+            };
+            typedef __attribute__((address_space(1))) float* out_ptr;
+            typedef const __attribute__((address_space(1))) float* gate_ptr;
+            const float inv = parts ? 1.0f : l > 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+            for (int d = 0; d < 16; ++d) *reinterpret_cast<f4*>(mine + c_out * kOutRow + 16 * d + 4 * g_out) = o[t][d] * inv;
+            // from here on lane l has elements 4 l .. 4 l + 3 of every row
+            const auto staged = [&](int r) { return *reinterpret_cast<const f4*>(mine + r * kOutRow + 4 * lane_out); };
+            if constexpr (SPLIT) {
+                if (cut) {
+                    const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
+                    const size_t at = slot * kRowsPerWg + wave * kRows + t * kRowsPerWave;
+                    float* po = P.part_o + at * kHd + 4 * lane_out;
+#pragma unroll
+                    for (int r = 0; r < kRowsPerWave; ++r)
+                        if (r < live) *reinterpret_cast<f4*>(po + r * kHd) = staged(r);
+                    if (lane_out < live) *reinterpret_cast<float2*>(P.part_ml + (at + lane_out) * 2) = make_float2(m_run[t], l);
+                    continue;
+                }
+            }
+            // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
+            // chain of trips to memory
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                f4 y[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) y[i] = staged(half * 8 + i);
+                if (gate) {
+                    f4 z[8];
+                    const auto gate_row = [&](int i) { return (gate_ptr)row_at(gate_at, half * 8 + i) + 4 * lane_out; };
+                    if (gate_in_fours) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)gate_row(i);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) z[i][r] = gate_row(i)[r];
+                    }
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) y[i][r] *= sigmoid(z[i][r]);
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) y[i][r] *= sigmoid(z[i][r]);
+                    if (half * 8 + i < live) *(__attribute__((address_space(1))) f4*)((out_ptr)row_at(out_at, half * 8 + i) + 4 * lane_out) = y[i];
             }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) *(__attribute__((address_space(1))) f4*)(op + 16 * (half * 8 + i) + 4 * g) = y[i];
         }
     }
 }
