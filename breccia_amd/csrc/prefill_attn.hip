@@ -169,6 +169,13 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* in_global(T* p) 
     return (__attribute__((address_space(1))) T*)p;
 }
 
+// what lane i has in x
+__device__ __forceinline__ uint64_t lane_value(uint64_t x, int i) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, i);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), i);
+    return (uint64_t)hi << 32 | lo;
+}
+
 // two f32 numbers as f16, rounded to nearest
 __device__ __forceinline__ h2m to_f16(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));
@@ -259,6 +266,8 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     const int c = lane & 15;  // query row of the tile / cell of the page / output column group
     const int g = lane >> 4;  // which quarter of the contraction index this lane feeds
     const int row0 = rb * kRowsPerWg + wave * kRows;
+    // q and the outputs pass through LDS between memory and the lanes (where not, and why: there)
+    constexpr bool kStaged = LAY == BKV_LAYOUT_F16 && TILES == 1;
     const bool wave_live = row0 < n_rows;
 
     // pages the work-group walks: those of its last row
@@ -309,6 +318,25 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     const size_t v_page_bytes = (size_t)P.n_kv * kPage * kVRow;
     const size_t v_head_off = (size_t)kvh * kPage * kVRow;
 
+    // ---- q, row by row ---------------------------------------------------------------------------
+    // Lane (c, g) is to hold q[row][32 m + 8 g + 0..7], m = 0..7.  Requested like that each instruction touches 16 rows 16
+    // bytes at a time, 64 cycles of the path to memory.  Requested here is a row an instruction, ahead of the table; its
+    // pieces find their lanes through the memory of the V images.  41 tokens behind 517 cells through 12 layers 210 ->
+    // 202 us (cycles to the first scores 8500 -> 7500).  f16 pools with one tile a wave only, whose calls may leave most of the
+    // chip idle: where every compute unit asks for 128 KiB at once, memory is what q waits for (two tiles, int8, three
+    // ragged chunks: 18900 cycles of prologue instead of 15700), and the quantised kernels have their walk of one tile in the
+    // same kernel, whose registers came out worse for the other (158 -> 162 us).
+    // (A lane without a row has the chunk's first row, and drops it.)  All of it is requested at once: behind a branch a
+    // fragment, each was waited for before the next was asked for, a trip to memory each.
+    const int src_q = P.b.src0[e], heads_q = P.n_q;
+    f4 raw[TILES][16];
+    if constexpr (kStaged) {
+        const uint64_t at = (uint64_t)(uintptr_t)P.q + ((uint64_t)(src_q + tok[0]) * (uint64_t)heads_q + (uint64_t)head[0]) * (kHd * 4);
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            raw[0][i] = *(const __attribute__((address_space(1))) f4*)((const __attribute__((address_space(1))) float*)lane_value(at, i) + 4 * lane);
+    }
+
     // ---- table entries, on which everything waits ----------------------------------------------------------------
     const int tid = threadIdx.x;
     const int last_pg = wg_pages - 1;
@@ -321,11 +349,7 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     // addresses of a pair's pages, lane by lane as the entries came; pages are then picked from them
     const auto k_pages = [&](int ids) { return (uint64_t)(uintptr_t)(P.kpool + head_off) + (uint64_t)(unsigned)ids * (unsigned)page_bytes; };
     const auto v_pages = [&](int ids) { return (uint64_t)(uintptr_t)(P.vpool + v_head_off) + (uint64_t)(unsigned)ids * (unsigned)v_page_bytes; };
-    const auto page_of = [](uint64_t pages, int w) {
-        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)pages, w);
-        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(pages >> 32), w);
-        return (page_ptr)((uint64_t)hi << 32 | lo);
-    };
+    const auto page_of = [](uint64_t pages, int w) { return (page_ptr)lane_value(pages, w); };
 
     // ---- pages into LDS --------------------------------------------------------------------------
     // f16 rows go there by themselves: wave w moves rows 4 w .. 4 w + 3 of a page, two rows a load; lane l delivers
@@ -487,20 +511,40 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
             }
         }
     };
-    load_pair_k(0, ids_0);
-    load_pair_v(0, ids_0);
-    if constexpr (!I8H) load_pair_k(1, ids_v);
-
-    // q: lane (c, g) holds q[row][32 m + 8 g + 0..7], m = 0..7.  All of the row is requested at once (a lane without a row
-    // reads the chunk's first one and drops it): behind a branch a fragment, each was waited for before the next was
-    // asked for, a trip to memory each.  Behind the first pages' requests: a wave's 16 or 32, which touch 16 rows each, keep
-    // the path to memory busy for 3 us.
-    f4 raw[TILES][16];
+    if constexpr (kStaged) {
+        // q's rows are waited for ahead of pages that go to LDS by themselves: of those the compiler has no count, and
+        // would have them arrive first
+        stay(raw[0][15]);
+        load_pair_k(0, ids_0);
+        load_pair_k(1, ids_v);
+        // eight rows of a wave at a time, as the V images have room for
+        constexpr int kAtOnce = 8;
+        static_assert(4 * kAtOnce * kOutRow * sizeof(float) <= sizeof(L.vimg), "q's rows in the memory of the V images");
+        float* const mine = reinterpret_cast<float*>(&L.vimg) + wave * (kAtOnce * kOutRow);
+        f4 q_row[16];
 #pragma unroll
-    for (int t = 0; t < TILES; ++t) {
-        const float* qp = P.q + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd + g * 8;
+        for (int i = 0; i < 16; ++i) q_row[i] = raw[0][i];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
+        for (int part = 0; part < 2; ++part) {
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) *reinterpret_cast<f4*>(mine + i * kOutRow + 4 * lane) = q_row[part * kAtOnce + i];
+            if ((c >> 3) == part) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    raw[0][i] = *reinterpret_cast<const f4*>(mine + (c & (kAtOnce - 1)) * kOutRow + (i >> 1) * 32 + g * 8 + (i & 1) * 4);
+            }
+        }
+    } else {
+        load_pair_k(0, ids_0);
+        load_pair_v(0, ids_0);
+        if constexpr (!I8H) load_pair_k(1, ids_v);
+        // behind the first pages' requests: q's keep the path to memory busy for 3 us
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const float* qp = P.q + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd + g * 8;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) raw[t][i] = *reinterpret_cast<const f4*>(qp + (i >> 1) * 32 + (i & 1) * 4);
+        }
     }
 
     // ---- q as hi + lo f16 --------------------------------------------------------------------------
@@ -767,12 +811,17 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
         load_pair_k(0, ids_k);
     }
     if constexpr (!I8H) wait_for_loads();
-    clear_dead_v(0, first_pg);
+    if constexpr (!kStaged) clear_dead_v(0, first_pg);
     __syncthreads();
+    if constexpr (kStaged) load_pair_v(0, ids_0);  // to where q's rows were
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         read_k(0, i);
         multiply_k(i);
+    }
+    if constexpr (kStaged) {
+        wait_for_loads();
+        clear_dead_v(0, first_pg);
     }
     __syncthreads();
     // What a step brings into LDS and requests, without products to put between
@@ -880,10 +929,10 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
     // A lane holds 16 bytes of each 64 of its row: a store (or a request for the gate) straight from here touches 16 rows
     // 16 bytes at a time, and the path to memory takes them row by row, 64 cycles an instruction.  The wave's tile goes
     // through LDS instead (the images are done with) and leaves row by row, 1 KiB an instruction.  Cycles of the
-    // epilogue, before / now: one tile 4100 / 2900, two 8300 / 6100; 41 tokens behind 517 cells through 12 layers 217 ->
-    // 210 us.  Not so f16 pools with two tiles a wave: their calls fill the chip and are at its power limit, where
-    // cycles saved beside the products save no time, and the walk's registers come out worse (285 against 284 us).
-    constexpr bool kStaged = LAY != BKV_LAYOUT_F16 || TILES == 1;
+    // epilogue, before / now: 4100 / 2900; 41 tokens behind 517 cells through 12 layers 217 -> 210 us.  f16 pools with one tile
+    // a wave only: with two tiles (8300 / 6100) calls fill the chip and are at its power limit, where cycles saved
+    // beside the products save no time, and the walk's registers come out worse (f16 285 against 284 us, a prompt of 4096
+    // with q8_0 V 544 against 542.5).
     if constexpr (kStaged) __syncthreads();
     static_assert(sizeof(OutLds) <= sizeof(PrefillLds<LAY>), "the tiles of four waves in the memory of the images");
     float* const mine = &reinterpret_cast<OutLds*>(&L)->row[wave][0][0];
@@ -906,6 +955,17 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
         const float l = sum_over_lane_groups(l_run[t]);
         if constexpr (!kStaged) {
             if (!row_live[t]) continue;
+            if constexpr (SPLIT) {
+                if (cut) {
+                    const size_t slot = (size_t)P.s.slot_base[e] + (size_t)(idx * P.n_kv + kvh) * P.s.splits[e] + range;
+                    const size_t at = slot * kRowsPerWg + wave * kRows + t * kRowsPerWave + c;
+                    float* po = P.part_o + at * kHd + 4 * g;
+#pragma unroll
+                    for (int d = 0; d < 16; ++d) *reinterpret_cast<f4*>(po + 16 * d) = o[t][d];
+                    if (g == 0) *reinterpret_cast<float2*>(P.part_ml + at * 2) = make_float2(m_run[t], l);
+                    continue;
+                }
+            }
             const float inv = l > 0.0f ? 1.0f / l : 0.0f;
             const auto op = in_global(out) + ((size_t)(src0 + tok[t]) * n_q + head[t]) * kHd;
             // the gate's values in two batches of requests: one by one, each waited for before its product, they were a
@@ -946,11 +1006,6 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
             head += kvh * P.group;
             const uint64_t out_at = (uint64_t)(uintptr_t)out + ((uint64_t)tok * (uint64_t)n_q + (uint64_t)head) * (kHd * 4);
             const uint64_t gate_at = (uint64_t)(uintptr_t)gate + (uint64_t)((int64_t)tok * gate_tok_stride + (int64_t)head * gate_head_stride) * 4;
-            const auto row_at = [](uint64_t at, int r) {
-                const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)at, r);
-                const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(at >> 32), r);
-                return (uint64_t)hi << 32 | lo;
-            };
             typedef __attribute__((address_space(1))) float* out_ptr;
             typedef const __attribute__((address_space(1))) float* gate_ptr;
             const float inv = parts ? 1.0f : l > 0.0f ? 1.0f / l : 0.0f;
@@ -979,7 +1034,7 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
                 for (int i = 0; i < 8; ++i) y[i] = staged(half * 8 + i);
                 if (gate) {
                     f4 z[8];
-                    const auto gate_row = [&](int i) { return (gate_ptr)row_at(gate_at, half * 8 + i) + 4 * lane_out; };
+                    const auto gate_row = [&](int i) { return (gate_ptr)lane_value(gate_at, half * 8 + i) + 4 * lane_out; };
                     if (gate_in_fours) {
 #pragma unroll
                         for (int i = 0; i < 8; ++i) z[i] = *(const __attribute__((address_space(1))) f4*)gate_row(i);
@@ -996,7 +1051,7 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
                 }
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    if (half * 8 + i < live) *(__attribute__((address_space(1))) f4*)((out_ptr)row_at(out_at, half * 8 + i) + 4 * lane_out) = y[i];
+                    if (half * 8 + i < live) *(__attribute__((address_space(1))) f4*)((out_ptr)lane_value(out_at, half * 8 + i) + 4 * lane_out) = y[i];
             }
         }
     }
