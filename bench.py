@@ -318,7 +318,7 @@ def main() -> int:
                 "traffic_source": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE profile of this command (seed %d), "
                                   "profiles/hbm_traffic_all_kernels.md; a constant of this file, not measured "
                                   "by this run" % MEASURED_TRAFFIC["seed"],
-                "kernel": "decode_attn_mfma_kernel<true, false, false> (f16 K/V, all 8 q heads of a kv head per pass on the "
+                "kernel": "decode_attn_few_kernel<true, false> (f16 K/V, all 8 q heads of a kv head per pass on the "
                           "matrix cores, new row taken in flight)",
                 "avg_us": round(split_us, 2),
                 "launches": n_split, "algorithmic_bytes": attn_bytes}
