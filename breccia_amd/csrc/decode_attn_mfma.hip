@@ -210,11 +210,17 @@ struct OnePageLds {
 __device__ __forceinline__ float max4(f4 x) { return fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])); }
 
 // From the waves' shares of the scores to the probabilities of all four pages: p[j] of lane (c, g) holds the high, then
-// the low parts of head c's probabilities of cells 4 g + r of page j.  live: of cells 4 g + r of page `wave`.  Writes
-// the work-group's (m, l).  Without a cell to attend: zeros, m = -inf and l = 0.
+// the low parts of head c's probabilities of cells 4 g + r of page j, relative to that page's own maximum, and f[j] is
+// what a sum over page j is multiplied by.  Each page keeps the maximum of its own, as each wave of a longer walk does:
+// relative to the largest of all 64 cells, the weights of a quieter page slide into the subnormals of f16, whose low
+// parts end at 2^-24, and V that is loud there shows the missing bits (10000 times as loud, 14 bits below: 1.1e-4 of the
+// output, now 2.7e-7).
+// live: of cells 4 g + r of page `wave`.  Writes the work-group's (m, l).  Without a cell to attend: zeros, m = -inf
+// and l = 0.
 // ex, down: q8_0 V only (null otherwise): what its rows' exponents take out of the values (see that kernel).
 __device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OnePageLds& L, const f4 (&part)[kWaves], const bool (&live)[4], int wg,
-                                                 int wave, int lane, v4u (&p_out)[kWaves], const int* ex = nullptr, const float* down = nullptr) {
+                                                 int wave, int lane, v4u (&p_out)[kWaves], f4& f, const int* ex = nullptr,
+                                                 const float* down = nullptr) {
     const int c = lane & 15, g = lane >> 4;
     const float scale = P.scale_log2e;
 #pragma unroll
@@ -225,15 +231,12 @@ __device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OneP
 #pragma unroll
     for (int r = 0; r < 4; ++r) t[r] = live[r] ? s[r] * scale + (ex ? (float)ex[r] : 0.0f) : -INFINITY;
     const float pm = max_over_lane_groups(max4(t));
-    if (g == 0) L.m[c][wave] = pm;
-    __syncthreads();
-    const float m = max4(*reinterpret_cast<const f4*>(L.m[c]));
-    const bool none = m == -INFINITY;
+    const bool none = pm == -INFINITY;
     h4m phi, plo;
     float psum = 0.0f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const float p = none ? 0.0f : __builtin_amdgcn_exp2f(t[r] - m);
+        const float p = none ? 0.0f : __builtin_amdgcn_exp2f(t[r] - pm);
         psum = down ? fmaf(p, down[r], psum) : psum + p;
         _Float16 h, l;
         split_hi_lo(p, h, l);
@@ -242,15 +245,22 @@ __device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OneP
     }
     L.p[wave][lane] = __builtin_bit_cast(v4u, half8{phi[0], phi[1], phi[2], phi[3], plo[0], plo[1], plo[2], plo[3]});
     psum = sum_over_lane_groups(psum);
-    if (g == 0) L.l[c][wave] = psum;
+    if (g == 0) {
+        L.m[c][wave] = pm;
+        L.l[c][wave] = psum;
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kWaves; ++j) p_out[j] = L.p[j][lane];
+    const f4 m = *reinterpret_cast<const f4*>(L.m[c]);
+    const float mx = max4(m);
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) f[j] = m[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[j] - mx);
     if (wave == 0 && g == 0 && c < P.group) {
         const f4 l = *reinterpret_cast<const f4*>(L.l[c]);
         float* const ml = P.part_ml + ((size_t)wg * P.group + c) * 2;
-        ml[0] = m;
-        ml[1] = (l[0] + l[1]) + (l[2] + l[3]);
+        ml[0] = mx;
+        ml[1] = fmaf(f[3], l[3], fmaf(f[2], l[2], fmaf(f[1], l[1], f[0] * l[0])));
     }
 }
 // o[t][r] of lane (c, g) is out[head c][64 wave + 16 g + 4 r + t]
@@ -443,7 +453,8 @@ __device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageL
         else mine[r] = (pg0 + wave) * kPage + 4 * g + r <= pos;
     }
     v4u p[kWaves];
-    one_page_softmax(P, L, part, mine, wg, wave, lane, p);
+    f4 f;
+    one_page_softmax(P, L, part, mine, wg, wave, lane, p, f);
 
     if constexpr (STEP) {
         if (takes_new_row) {
@@ -465,25 +476,19 @@ __device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageL
     }
     f4 o[4] = {};
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        // columns 4 c + t of the cells of pages 2 j and 2 j + 1
-        const v4u p0 = p[2 * j], p1 = p[2 * j + 1];
-        const half8 phi = __builtin_bit_cast(half8, v4u{p0.x, p0.y, p1.x, p1.y});
-        const half8 plo = __builtin_bit_cast(half8, v4u{p0.z, p0.w, p1.z, p1.w});
-        v4u a[4];
+    for (int j = 0; j < kWaves; ++j) {
+        // columns 4 c + t of the page's 16 cells, against the high and the low parts of p
+        const half8 phl = __builtin_bit_cast(half8, p[j]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const v2u x0 = vf[2 * j + (k >> 1)][2 * (k & 1)], x1 = vf[2 * j + (k >> 1)][2 * (k & 1) + 1];
-                a[t][k] = __builtin_amdgcn_perm(t < 2 ? x1.x : x1.y, t < 2 ? x0.x : x0.y, t & 1 ? 0x07060302u : 0x05040100u);
-            }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[t]), phi, o[t], 0, 0, 0);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a[t]), plo, o[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) {
+            const auto column = [&](int r) {
+                const v2u x0 = vf[j][r], x1 = vf[j][r + 1];
+                return __builtin_amdgcn_perm(t < 2 ? x1.x : x1.y, t < 2 ? x0.x : x0.y, t & 1 ? 0x07060302u : 0x05040100u);
+            };
+            const unsigned r01 = column(0), r23 = column(2);
+            o[t] += __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, v4u{r01, r23, r01, r23}), phl,
+                                                           f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0) * f[j];
+        }
     }
     one_page_store(P, wg, wave, c, g, o);
 }
@@ -992,7 +997,8 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
         else mine[r] = (pg0 + wave) * kPage + 4 * g + r <= pos;
     }
     v4u p[kWaves];
-    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p);
+    f4 f;
+    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, f);
 
     f4 o[4] = {};
 #pragma unroll
@@ -1018,10 +1024,11 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
             const h2m lo01 = __builtin_elementwise_fma(c01, s01, -hi01), lo23 = __builtin_elementwise_fma(c23, s23, -hi23);
             a[t] = half8{hi01[0], hi01[1], hi23[0], hi23[1], lo01[0], lo01[1], lo23[0], lo23[1]};
         }
+        f4 s[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], phh, o[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], phh, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], pll, o[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) o[t] += __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], pll, s[t], 0, 0, 0) * f[j];
     }
     one_page_store(P, wg, wave, c, g, o);
 }
@@ -1522,7 +1529,8 @@ __device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ
     }
     // (the barriers of the softmax stand between these writes and the waves that read them)
     v4u p[kWaves];
-    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, ex, down);
+    f4 f;
+    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, f, ex, down);
 
     f4 o[4] = {};
 #pragma unroll
@@ -1550,10 +1558,11 @@ __device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ
             scaled_hi_lo(c23, s23, l23, hi23, lo23);
             a[t] = half8{hi01[0], hi01[1], hi23[0], hi23[1], lo01[0], lo01[1], lo23[0], lo23[1]};
         }
+        f4 s[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], whh, o[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], whh, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], wll, o[t], 0, 0, 0);
+        for (int t = 0; t < 4; ++t) o[t] += __builtin_amdgcn_mfma_f32_16x16x32_f16(a[t], wll, s[t], 0, 0, 0) * f[j];
     }
     one_page_store(P, wg, wave, c, g, o);
 }

@@ -1,0 +1,38 @@
+"""Values that decode attention meets seldom, in ranges of one page a wave as in longer walks."""
+import numpy as np
+import pytest
+
+from breccia_amd import lib as L
+from gpu_common import REF_BAR_MAX_REL, Twin, check_attn
+from test_gpu_attn_select import oracle_select, select_attn
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [L.LAYOUT_F16, L.LAYOUT_Q8V, L.LAYOUT_I8H]
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("below", [14, 20])
+@pytest.mark.parametrize("cells", [64, 150])
+def test_a_quiet_page_keeps_its_bits(layout, below, cells):
+    """Cells 32..47 have weights `below` powers of two under the others' and V 10000 times theirs.  A weight is carried as two
+    f16 numbers relative to its own page's largest: off by 2^-22 of itself or 2^-25 of that, at most 16 x 5 x 10^4 x 2^-(25 +
+    below) of the output.  Relative to the largest weight of four pages it would be 2^-25 of that one: 2e-2 of the output
+    at worst, 1e-4 with these values."""
+    rng = np.random.Generator(np.random.PCG64(6100 + 10 * layout + below + cells))
+    k, v = rng.standard_normal((2, cells, 2, 256)).astype(np.float32)
+    q = rng.standard_normal((1, 16, 256)).astype(np.float32)
+    k *= 0.3
+    q[..., 0], k[..., 0] = 16.0, 0.0  # times the scale of 1/16: a logit of k's first element
+    k[32:48, :, 0] = -below * np.log(2.0)
+    v[32:48] *= 1e4
+    with Twin(n_pages=16, max_seqs=1, layout=layout) as tw:
+        s = tw.pool.seq_create()
+        tw.pool.seq_reserve(s, cells)
+        tw.append(0, [s], [0], [k], [v])
+        blocks = list(range((cells + 3) // 4))
+        for what, got, want in [
+                ("dense", tw.decode_attn(0, [s], [cells - 1], q, 16, scale=1.0 / 16.0), tw.oracle_attend(0, s, cells - 1, q[0], 16)),
+                ("list", select_attn(tw, 0, [s], [cells - 1], q, 16, [blocks]), oracle_select(tw, 0, s, cells - 1, q[0], 16, blocks))]:
+            _, rel = check_attn(got[0], want, what)
+            assert rel <= REF_BAR_MAX_REL, (what, rel)
