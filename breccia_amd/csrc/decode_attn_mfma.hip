@@ -216,10 +216,13 @@ __device__ __forceinline__ float max4(f4 x) { return fmaxf(fmaxf(x[0], x[1]), fm
 // parts end at 2^-24, and V that is loud there shows the missing bits (10000 times as loud, 14 bits below: 1.1e-4 of the
 // output, now 2.7e-7).
 // live: of cells 4 g + r of page `wave`.  Writes the work-group's (m, l).  Without a cell to attend: zeros, m = -inf
-// and l = 0.
+// and l = 0.  dead: page `wave` is behind the last one.  A dense page that is not has a cell, and where all its scores are
+// NaN the sum has to become NaN as well (with zeros for it a NaN key alone in its range would be passed over); a group of
+// listed blocks may have none, as in the walk below.
 // ex, down: q8_0 V only (null otherwise): what its rows' exponents take out of the values (see that kernel).
-__device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OnePageLds& L, const f4 (&part)[kWaves], const bool (&live)[4], int wg,
-                                                 int wave, int lane, v4u (&p_out)[kWaves], f4& f, const int* ex = nullptr,
+template <bool SEL>
+__device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OnePageLds& L, const f4 (&part)[kWaves], const bool (&live)[4], bool dead,
+                                                 int wg, int wave, int lane, v4u (&p_out)[kWaves], f4& f, const int* ex = nullptr,
                                                  const float* down = nullptr) {
     const int c = lane & 15, g = lane >> 4;
     const float scale = P.scale_log2e;
@@ -230,8 +233,8 @@ __device__ __forceinline__ void one_page_softmax(const AttnKernelParams& P, OneP
     f4 t;
 #pragma unroll
     for (int r = 0; r < 4; ++r) t[r] = live[r] ? s[r] * scale + (ex ? (float)ex[r] : 0.0f) : -INFINITY;
-    const float pm = max_over_lane_groups(max4(t));
-    const bool none = pm == -INFINITY;
+    const float pm = max_over_lane_groups(fmaxf(max4(t), -INFINITY));
+    const bool none = SEL ? pm == -INFINITY : dead;
     h4m phi, plo;
     float psum = 0.0f;
 #pragma unroll
@@ -454,7 +457,7 @@ __device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageL
     }
     v4u p[kWaves];
     f4 f;
-    one_page_softmax(P, L, part, mine, wg, wave, lane, p, f);
+    one_page_softmax<SEL>(P, L, part, mine, pg0 + wave >= n_pages, wg, wave, lane, p, f);
 
     if constexpr (STEP) {
         if (takes_new_row) {
@@ -998,7 +1001,7 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
     }
     v4u p[kWaves];
     f4 f;
-    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, f);
+    one_page_softmax<SEL>(P, L.x, part, mine, pg0 + wave >= n_pages, wg, wave, lane, p, f);
 
     f4 o[4] = {};
 #pragma unroll
@@ -1530,7 +1533,7 @@ __device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ
     // (the barriers of the softmax stand between these writes and the waves that read them)
     v4u p[kWaves];
     f4 f;
-    one_page_softmax(P, L.x, part, mine, wg, wave, lane, p, f, ex, down);
+    one_page_softmax<SEL>(P, L.x, part, mine, pg0 + wave >= n_pages, wg, wave, lane, p, f, ex, down);
 
     f4 o[4] = {};
 #pragma unroll

@@ -36,3 +36,22 @@ def test_a_quiet_page_keeps_its_bits(layout, below, cells):
                 ("list", select_attn(tw, 0, [s], [cells - 1], q, 16, [blocks]), oracle_select(tw, 0, s, cells - 1, q[0], 16, blocks))]:
             _, rel = check_attn(got[0], want, what)
             assert rel <= REF_BAR_MAX_REL, (what, rel)
+
+
+@pytest.mark.parametrize("layout", [L.LAYOUT_F16, L.LAYOUT_Q8V])
+@pytest.mark.parametrize("cells,at", [(65, 64), (65, 10), (64, 63), (1, 0), (300, 256), (300, 40)])
+def test_a_score_that_is_not_a_number(layout, cells, at):
+    """A key of infinities (what the cache makes of NaN) has scores of NaN.  A head with one among them has no sum, and its
+    output is zeros, whether that cell shares its range with others or is alone in it."""
+    rng = np.random.Generator(np.random.PCG64(6200 + 10 * layout + cells + at))
+    k, v = rng.standard_normal((2, cells, 2, 256)).astype(np.float32)
+    k[at, 1] = np.nan
+    q = rng.standard_normal((1, 16, 256)).astype(np.float32)
+    with Twin(n_pages=24, max_seqs=1, layout=layout) as tw:
+        s = tw.pool.seq_create()
+        tw.pool.seq_reserve(s, cells)
+        tw.append(0, [s], [0], [k], [v])
+        got = tw.decode_attn(0, [s], [cells - 1], q, 16, scale=1.0 / 16.0)[0]
+        want = tw.oracle_attend(0, s, cells - 1, q[0], 16)
+        check_attn(got[:8], want[:8], "the other kv head")
+        assert not got[8:].any()
