@@ -61,7 +61,7 @@ struct MergeSum {
 __device__ __forceinline__ float weight_of(float x, float ref) { return __builtin_amdgcn_exp2f(x - (ref == -INFINITY ? 0.0f : ref)); }
 
 // N rounds of kMergeGroups splits from split s0 on, everything requested before the first use and without branches:
-// past the end the last split is requested again and gets no weight.
+// past the end the last split is requested again and counts as zeros (not by its weight alone: 0 x inf is NaN).
 template <int N>
 __device__ __forceinline__ void merge_rounds(const float* po, const float* pml, uint32_t lane_at, uint32_t ostride, uint32_t mlstride, int s0, int splits,
                                              MergeSum& a) {
@@ -82,7 +82,10 @@ __device__ __forceinline__ void merge_rounds(const float* po, const float* pml, 
     float mx = a.m;
 #pragma unroll
     for (int u = 0; u < N; ++u) {
-        m[u] = s0 + u * kMergeGroups < splits ? m[u] : -INFINITY;
+        const bool mine = s0 + u * kMergeGroups < splits;
+        m[u] = mine ? m[u] : -INFINITY;
+        l[u] = mine ? l[u] : 0.0f;
+        v[u] = mine ? v[u] : f4{0.0f, 0.0f, 0.0f, 0.0f};
         mx = fmaxf(mx, m[u]);
     }
     const float keep = weight_of(a.m, mx);

@@ -55,3 +55,25 @@ def test_a_score_that_is_not_a_number(layout, cells, at):
         want = tw.oracle_attend(0, s, cells - 1, q[0], 16)
         check_attn(got[:8], want[:8], "the other kv head")
         assert not got[8:].any()
+
+
+@pytest.mark.parametrize("cells", [2, 40, 64, 130, 1100])
+def test_infinite_v(cells):
+    """An output over one infinite V value is that infinity, in its own column only and however many ranges are merged.  The
+    cell's weight is exp(-1/2) of its page's largest, whose f16 parts are both positive (0.60645 + 0.00009)."""
+    rng = np.random.Generator(np.random.PCG64(6300 + cells))
+    k, v = np.zeros((cells, 2, 256), np.float32), rng.standard_normal((cells, 2, 256)).astype(np.float32)
+    at = cells - 1
+    k[at, :, 0] = -0.5
+    v[at, 0, 17], v[at, 1, 200] = np.inf, -np.inf
+    q = np.zeros((1, 16, 256), np.float32)
+    q[..., 0] = 16.0
+    with Twin(n_pages=80, max_seqs=1) as tw:
+        s = tw.pool.seq_create()
+        tw.pool.seq_reserve(s, cells)
+        tw.append(0, [s], [0], [k], [v])
+        got = tw.decode_attn(0, [s], [cells - 1], q, 16, scale=1.0 / 16.0)[0]
+        want = tw.oracle_attend(0, s, cells - 1, q[0], 16)
+        assert np.all(got[:8, 17] == np.inf) and np.all(got[8:, 200] == -np.inf)
+        got[:8, 17], got[8:, 200], want[:8, 17], want[8:, 200] = 0.0, 0.0, 0.0, 0.0
+        check_attn(got, want, "the other columns")
