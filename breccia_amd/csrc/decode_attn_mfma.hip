@@ -173,6 +173,14 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* k_or_v(bool is_k
     return (__attribute__((address_space(1))) T*)(is_k ? ka : va);
 }
 
+// The wave's own LDS writes are in order with its later reads; keeps the compiler from moving either across, whichever lane
+// and type they are of.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A new f16 row (STEP), slice by slice: 8 values, from the caller's f32 row to 16 bytes of the pool.
 struct NewSliceF16 {
     f4 a, b;
@@ -956,6 +964,8 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
             *reinterpret_cast<v2u*>(row + li * 8) = v2u{new_codes[0], new_codes[1]};
             if ((li & 3) == 0) *reinterpret_cast<unsigned short*>(row + kHd + 2 * (li >> 2)) = (unsigned short)new_scale;
         }
+        // the scales go in 16 bits at a time and are read 32 at a time below, by other lanes
+        wave_lds_fence();
     }
     {
         // The page's scales, one dword a lane: with exponent field 0 they read as zero, and rows that are not attended
@@ -1134,13 +1144,6 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     fetch(0);
     __builtin_amdgcn_sched_barrier(0);
 
-    const auto wave_lds_fence = [&]() {
-        // the wave's own LDS writes are in order with its later reads; keep the compiler from
-        // moving those reads up
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     if constexpr (STEP) {
         if (takes_new_row) {
             const float new_x[8] = {x.a[0], x.a[1], x.a[2], x.a[3], x.b[0], x.b[1], x.b[2], x.b[3]};
@@ -1689,11 +1692,6 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     }
 
     __builtin_amdgcn_sched_barrier(0);
-    const auto wave_lds_fence = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     if constexpr (STEP) {
         if (takes_new_row) {
             const int r = pos & (kPage - 1), li = lane & 31;
