@@ -173,14 +173,6 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* k_or_v(bool is_k
     return (__attribute__((address_space(1))) T*)(is_k ? ka : va);
 }
 
-// The wave's own LDS writes are in order with its later reads; keeps the compiler from moving either across, whichever lane
-// and type they are of.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A new f16 row (STEP), slice by slice: 8 values, from the caller's f32 row to 16 bytes of the pool.
 struct NewSliceF16 {
     f4 a, b;

@@ -1,5 +1,6 @@
-// Reductions across the four 16-lane groups of a wave64, for kernels whose lane (c = lane % 16,
-// g = lane / 16) keeps one value per (c, g) and needs the combination over g in every lane.
+// What the lanes of a wave64 tell each other: reductions across its four 16-lane groups, for kernels whose lane
+// (c = lane % 16, g = lane / 16) keeps one value per (c, g) and needs the combination over g in every lane, and the fence
+// for what goes through LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,6 +36,14 @@ __device__ __forceinline__ float sum_over_lane_groups(float x) {
     const LanePair p = swap_halves(x);
     const LanePair q = swap_rows(p.a + p.b);
     return q.a + q.b;
+}
+
+// The wave's own LDS writes are in order with its later reads; keeps the compiler from moving either across, whichever lane
+// and type they are of.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // x of the lane a DPP control names (row_ror:4 = 0x124, row_ror:8 = 0x128, quad_perm broadcasts

@@ -528,11 +528,13 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
         for (int part = 0; part < 2; ++part) {
 #pragma unroll
             for (int i = 0; i < kAtOnce; ++i) *reinterpret_cast<f4*>(mine + i * kOutRow + 4 * lane) = q_row[part * kAtOnce + i];
+            wave_lds_fence();
             if ((c >> 3) == part) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
                     raw[0][i] = *reinterpret_cast<const f4*>(mine + (c & (kAtOnce - 1)) * kOutRow + (i >> 1) * 32 + g * 8 + (i & 1) * 4);
             }
+            wave_lds_fence();
         }
     } else {
         load_pair_k(0, ids_0);
@@ -1011,6 +1013,7 @@ __device__ __forceinline__ void walk_block(const std::conditional_t<SPLIT, Prefi
             const float inv = parts ? 1.0f : l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
             for (int d = 0; d < 16; ++d) *reinterpret_cast<f4*>(mine + c_out * kOutRow + 16 * d + 4 * g_out) = o[t][d] * inv;
+            wave_lds_fence();
             // from here on lane l has elements 4 l .. 4 l + 3 of every row
             const auto staged = [&](int r) { return *reinterpret_cast<const f4*>(mine + r * kOutRow + 4 * lane_out); };
             if constexpr (SPLIT) {
