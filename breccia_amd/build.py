@@ -75,12 +75,11 @@ def build(verbose: bool = False) -> str:
 
 
 def build_hot_calls(verbose: bool = False) -> str:
-    """The CPython module that kv.py makes its per-layer calls through; host code, links the library."""
+    """The CPython module that kv.py makes its per-layer calls through; host code, handed the library's entry points."""
     import numpy
 
     cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-I", sysconfig.get_paths()["include"],
-           "-I", numpy.get_include(), os.path.join(CSRC, "hot_calls.cpp"), "-o", HOT_MODULE, "-L" + HERE, "-lbreccia_kv",
-           "-Wl,-rpath,$ORIGIN", "-Wl,-rpath,/opt/rocm/lib"]
+           "-I", numpy.get_include(), os.path.join(CSRC, "hot_calls.cpp"), "-o", HOT_MODULE]
     if verbose:
         print(" ".join(cmd))
     _run(cmd)

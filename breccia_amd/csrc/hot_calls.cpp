@@ -9,12 +9,17 @@
 // return NotImplemented, having done nothing, and kv.py makes the call as it always could, with ctypes' conversions and
 // its own errors.  Otherwise they return the library's status (seq_reserve: the list of pairs on success).  The
 // library is called without the GIL, as ctypes does.
+//
+// The module is not linked against the library: kv.py hands it the entry points of the one that ctypes has loaded
+// (bind).  A dependency is looked for along LD_LIBRARY_PATH first, and with another copy of the library there, pools
+// made by one were read by the other.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #define NPY_NO_DEPRECATED_API NPY_1_7_API_VERSION
 #include <numpy/arrayobject.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/breccia_kv.h"
 
@@ -26,10 +31,22 @@ PyObject* g_stream = nullptr;    // kv.Stream, its address in .handle
 PyObject* g_ptr_name = nullptr;
 PyObject* g_handle_name = nullptr;
 
+// The library's entry points; null until bind().
+#define ENTRY_POINTS(X) \
+    X(bkv_append) X(bkv_append_f16) X(bkv_append_kprep) X(bkv_decode_attn) X(bkv_decode_step) X(bkv_decode_attn_select) \
+    X(bkv_prefill_attn) X(bkv_idx_pool) X(bkv_select_blocks) X(bkv_seq_reserve)
+#define POINTER(name) decltype(&::name) name = nullptr;
+struct Library {
+    ENTRY_POINTS(POINTER)
+};
+#undef POINTER
+Library g_lib;
+bool g_bound = false;
+
 // Reads the positional arguments of one call in turn; `ok` falls, and stays down, at the first that is not plain.
 class Reader {
    public:
-    Reader(PyObject* const* args, Py_ssize_t n, Py_ssize_t want) : at_(args), ok(n == want) {}
+    Reader(PyObject* const* args, Py_ssize_t n, Py_ssize_t want) : at_(args), ok(n == want && g_bound) {}
 
     int32_t i32() {
         const int64_t v = i64();
@@ -156,9 +173,9 @@ PyObject* append(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     const bool f16_rows = r.flag();
     if (!r.ok || n != n1 || n != n2 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return f16_rows ? bkv_append_f16(pool, layer, (int32_t)n, seqs, pos0, n_tokens, static_cast<const uint16_t*>(k),
+        return f16_rows ? g_lib.bkv_append_f16(pool, layer, (int32_t)n, seqs, pos0, n_tokens, static_cast<const uint16_t*>(k),
                                          static_cast<const uint16_t*>(v), stream)
-                        : bkv_append(pool, layer, (int32_t)n, seqs, pos0, n_tokens, static_cast<const float*>(k),
+                        : g_lib.bkv_append(pool, layer, (int32_t)n, seqs, pos0, n_tokens, static_cast<const float*>(k),
                                      static_cast<const float*>(v), stream);
     });
 }
@@ -179,7 +196,7 @@ PyObject* append_kprep(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok || n != n1 || n != n2 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return bkv_append_kprep(pool, layer, (int32_t)n, seqs, pos0, n_tokens, k, v, gamma, eps, table, n_rot, max_pos, positions,
+        return g_lib.bkv_append_kprep(pool, layer, (int32_t)n, seqs, pos0, n_tokens, k, v, gamma, eps, table, n_rot, max_pos, positions,
                                 stream);
     });
 }
@@ -200,7 +217,7 @@ PyObject* decode_attn(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok || n != n1 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return bkv_decode_attn(pool, layer, (int32_t)n, seqs, pos, n_q, q, gate, seq_stride, head_stride, scale, out, stream);
+        return g_lib.bkv_decode_attn(pool, layer, (int32_t)n, seqs, pos, n_q, q, gate, seq_stride, head_stride, scale, out, stream);
     });
 }
 
@@ -221,7 +238,7 @@ PyObject* decode_step(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok || n != n1 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return bkv_decode_step(pool, layer, (int32_t)n, seqs, pos, k, v, n_q, q, gate, seq_stride, head_stride, scale, out, stream);
+        return g_lib.bkv_decode_step(pool, layer, (int32_t)n, seqs, pos, k, v, n_q, q, gate, seq_stride, head_stride, scale, out, stream);
     });
 }
 
@@ -245,7 +262,7 @@ PyObject* decode_attn_select(PyObject*, PyObject* const* args, Py_ssize_t n_args
     void* stream = r.stream();
     if (!r.ok || n != n1 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return bkv_decode_attn_select(pool, layer, (int32_t)n, seqs, pos, n_q, q, gate, seq_stride, head_stride, scale, ids, id_stride,
+        return g_lib.bkv_decode_attn_select(pool, layer, (int32_t)n, seqs, pos, n_q, q, gate, seq_stride, head_stride, scale, ids, id_stride,
                                       counts, max_ids, out, stream);
     });
 }
@@ -267,7 +284,7 @@ PyObject* prefill_attn(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok || n != n1 || n != n2 || n > INT32_MAX) return not_plain();
     return status_of([&] {
-        return bkv_prefill_attn(pool, layer, (int32_t)n, seqs, pos0, n_tokens, n_q, q, gate, tok_stride, head_stride, scale, out, stream);
+        return g_lib.bkv_prefill_attn(pool, layer, (int32_t)n, seqs, pos0, n_tokens, n_q, q, gate, tok_stride, head_stride, scale, out, stream);
     });
 }
 
@@ -287,7 +304,7 @@ PyObject* idx_pool(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok) return not_plain();
     return status_of([&] {
-        return bkv_idx_pool(pool, pooled, max_blocks, tail, idx_k, pos0, tokens, gamma, eps, table, n_rot, max_pos, idx_dim, stream);
+        return g_lib.bkv_idx_pool(pool, pooled, max_blocks, tail, idx_k, pos0, tokens, gamma, eps, table, n_rot, max_pos, idx_dim, stream);
     });
 }
 
@@ -308,7 +325,7 @@ PyObject* select_blocks(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     void* stream = r.stream();
     if (!r.ok || n != n1 || n != n2) return not_plain();
     return status_of([&] {
-        return bkv_select_blocks(pool, (int32_t)n, pos, idx_q, pooled, n_blocks, n_head, idx_dim, topk, ids, id_stride, counts, max_ids,
+        return g_lib.bkv_select_blocks(pool, (int32_t)n, pos, idx_q, pooled, n_blocks, n_head, idx_dim, topk, ids, id_stride, counts, max_ids,
                                  stream);
     });
 }
@@ -325,7 +342,7 @@ PyObject* seq_reserve(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     int32_t n = 0;
     bkv_status st;
     Py_BEGIN_ALLOW_THREADS;
-    st = bkv_seq_reserve(pool, seq, new_len, pairs, capacity, &n);
+    st = g_lib.bkv_seq_reserve(pool, seq, new_len, pairs, capacity, &n);
     Py_END_ALLOW_THREADS;
     if (st != BKV_OK) return PyLong_FromLong((long)st);
     PyObject* list = PyList_New(n);
@@ -340,17 +357,32 @@ PyObject* seq_reserve(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     return list;
 }
 
-// bind(c_void_p, DeviceBuffer, Stream): the classes whose objects are read as addresses
+// bind(c_void_p, DeviceBuffer, Stream, {name: address}): the classes whose objects are read as addresses, and the
+// library's entry points
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
-    if (n_args != 3) {
-        PyErr_SetString(PyExc_TypeError, "bind takes three classes");
+    if (n_args != 4 || !PyDict_Check(args[3])) {
+        PyErr_SetString(PyExc_TypeError, "bind takes three classes and the entry points' addresses");
         return nullptr;
     }
+    Library found;
+    const auto take = [&](const char* name, auto& entry) {
+        PyObject* at = PyDict_GetItemString(args[3], name);
+        void* p = at ? PyLong_AsVoidPtr(at) : nullptr;
+        if (!p && !PyErr_Occurred()) PyErr_Format(PyExc_ValueError, "no address of %s", name);
+        entry = reinterpret_cast<std::remove_reference_t<decltype(entry)>>(p);
+        return p != nullptr;
+    };
+#define TAKE(name) \
+    if (!take(#name, found.name)) return nullptr;
+    ENTRY_POINTS(TAKE)
+#undef TAKE
     PyObject** const kept[3] = {&g_c_void_p, &g_buffer, &g_stream};
     for (int i = 0; i < 3; ++i) {
         Py_INCREF(args[i]);
         Py_XSETREF(*kept[i], args[i]);
     }
+    g_lib = found;
+    g_bound = true;
     Py_RETURN_NONE;
 }
 

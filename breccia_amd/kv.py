@@ -651,4 +651,5 @@ def _ptr(x):
     return x
 
 
-_hot.bind(C.c_void_p, DeviceBuffer, Stream)
+_hot.bind(C.c_void_p, DeviceBuffer, Stream,
+          {name: C.cast(getattr(lib, name), C.c_void_p).value for name in L.HOT_ENTRY_POINTS})

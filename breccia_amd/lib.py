@@ -161,6 +161,10 @@ _BENCH_SIGNATURES = {
     "bkv_read_probe": (C.c_int, [_vp, _u64, _i32, _vp, _vp]),
 }
 
+# entry points that kv.py also calls past ctypes (csrc/hot_calls.cpp)
+HOT_ENTRY_POINTS = ("bkv_append", "bkv_append_f16", "bkv_append_kprep", "bkv_decode_attn", "bkv_decode_step",
+                    "bkv_decode_attn_select", "bkv_prefill_attn", "bkv_idx_pool", "bkv_select_blocks", "bkv_seq_reserve")
+
 _bench_error = None   # message of the last failed call into the bench library, until check() takes it
 
 

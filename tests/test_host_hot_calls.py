@@ -1,6 +1,10 @@
 """The per-layer calls past ctypes (breccia_amd._hot): what they take, what they leave to ctypes, and that both ways
 come to the same."""
 import ctypes as C
+import os
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -130,3 +134,44 @@ def test_pages_that_are_out_are_counted():
         p.seq_reserve(s, 20)
         p.check()
         assert attend(p, 19) == L.ERR_NO_DEVICE
+
+
+def test_the_library_that_is_called_is_the_one_that_was_loaded(tmp_path):
+    """Another copy of the library on LD_LIBRARY_PATH: pools are made and read by one of them."""
+    shutil.copy(L.LIB_PATH, tmp_path)
+    script = """
+import numpy as np
+from breccia_amd.kv import BkvError, Pool, _hot
+with Pool(n_pages=4, host_only=True) as p:
+    said = []
+    for seqs in (np.ones(1, np.int32), [1]):
+        try:
+            p.decode_attn(0, seqs, np.zeros(1, np.int64), 16, 0x1000, 0x1000, 0.5)
+        except BkvError as e:
+            said.append((e.status, e.message))
+assert len(said) == 2 and said[0] == said[1] and said[0][1], said
+maps = {line.split()[-1] for line in open("/proc/self/maps") if line.rstrip().endswith("libbreccia_kv.so")}
+assert len(maps) == 1, maps
+"""
+    env = dict(os.environ, LD_LIBRARY_PATH=str(tmp_path))
+    subprocess.run([sys.executable, "-c", script], check=True, env=env, cwd=os.path.dirname(os.path.dirname(L.LIB_PATH)), timeout=100)
+
+
+def test_not_bound_yet_means_not_taken():
+    """In a fresh interpreter, before kv.py has handed over the classes and the entry points."""
+    script = """
+import importlib.util
+spec = importlib.util.spec_from_file_location("_hot", %r)
+hot = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(hot)
+assert hot.seq_reserve(0, 0, 1, 4) is NotImplemented
+for wrong in [(), (int, int, int), (int, int, int, {}), (int, int, int, {"bkv_append": 0}), (int, int, int, {"bkv_append": "x"})]:
+    try:
+        hot.bind(*wrong)
+    except (TypeError, ValueError):
+        pass
+    else:
+        raise AssertionError(wrong)
+assert hot.seq_reserve(0, 0, 1, 4) is NotImplemented
+""" % _hot.__file__
+    subprocess.run([sys.executable, "-c", script], check=True, timeout=100)
