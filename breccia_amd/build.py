@@ -74,12 +74,22 @@ def build(verbose: bool = False) -> str:
     return LIB
 
 
-def build_hot_calls(verbose: bool = False) -> str:
-    """The CPython module that kv.py makes its per-layer calls through; host code, handed the library's entry points."""
-    import numpy
-
-    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-I", sysconfig.get_paths()["include"],
-           "-I", numpy.get_include(), os.path.join(CSRC, "hot_calls.cpp"), "-o", HOT_MODULE]
+def build_hot_calls(verbose: bool = False) -> str | None:
+    """The CPython module that kv.py makes its per-layer calls through; host code, handed the library's entry points.
+    Without a compiler and headers for it there is none (None), and the calls go through ctypes."""
+    python_h = os.path.join(sysconfig.get_paths()["include"], "Python.h")
+    cxx = shutil.which("g++") or shutil.which("c++") or shutil.which("clang++")
+    try:
+        from numpy import get_include
+    except ImportError:
+        get_include = None
+    if not (cxx and get_include and os.path.exists(python_h)):
+        if os.path.exists(HOT_MODULE):
+            os.remove(HOT_MODULE)  # of other sources
+        sys.stderr.write("breccia_amd._hot is not built (C++ compiler, %s and numpy needed): calls go through ctypes\n" % python_h)
+        return None
+    cmd = [cxx, "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-I", os.path.dirname(python_h), "-I", get_include(),
+           os.path.join(CSRC, "hot_calls.cpp"), "-o", HOT_MODULE]
     if verbose:
         print(" ".join(cmd))
     _run(cmd)

@@ -7,16 +7,23 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import warnings
 
 import numpy as np
 
 from . import lib as L
+from .lib import BkvError, PagePair, PoolDesc, check, lib  # noqa: F401
 
 try:
     from . import _hot
 except ImportError as e:
-    raise ImportError("breccia_amd._hot is not built or does not load (%s). Build it with `python -m breccia_amd.build`" % e) from e
-from .lib import BkvError, PagePair, PoolDesc, check, lib  # noqa: F401
+    # not built, or for another interpreter or numpy: the library needs neither, and ctypes reaches all of it
+    warnings.warn("breccia_amd._hot is not built or does not load (%s): calls go through ctypes, 2 to 4 us more each" % e, RuntimeWarning)
+
+    class _hot:  # noqa: N801
+        """Takes no call."""
+        append = append_kprep = decode_attn = decode_step = decode_attn_select = prefill_attn = idx_pool = select_blocks = \
+            seq_reserve = bind = staticmethod(lambda *args: NotImplemented)
 
 
 _I32, _I64 = np.dtype(np.int32), np.dtype(np.int64)

@@ -9,6 +9,7 @@ import sys
 import numpy as np
 import pytest
 
+from breccia_amd import build
 from breccia_amd import lib as L
 from breccia_amd.kv import BkvError, Pool, _hot
 
@@ -175,3 +176,40 @@ for wrong in [(), (int, int, int), (int, int, int, {}), (int, int, int, {"bkv_ap
 assert hot.seq_reserve(0, 0, 1, 4) is NotImplemented
 """ % _hot.__file__
     subprocess.run([sys.executable, "-c", script], check=True, timeout=100)
+
+
+def test_without_the_module_calls_go_through_ctypes():
+    script = """
+import sys, warnings
+sys.modules["breccia_amd._hot"] = None  # as if it were not built
+import numpy as np
+with warnings.catch_warnings(record=True) as said:
+    warnings.simplefilter("always")
+    from breccia_amd.kv import BkvError, Pool
+assert any("ctypes" in str(w.message) for w in said)
+with Pool(n_pages=4, host_only=True) as p:
+    s = p.seq_create()
+    assert p.seq_reserve(s, 17) == []
+    one, at = np.ones(1, np.int32), np.zeros(1, np.int64)
+    calls = [lambda: p.append(0, [s], at, one, 64, 64), lambda: p.append_kprep(0, [s], at, one, 64, 64, 64, 1e-6, 64, 64, 16),
+             lambda: p.decode_attn(0, [s], at, 16, 64, 64, 0.5), lambda: p.decode_step(0, [s], at, 64, 64, 16, 64, 64, 0.5),
+             lambda: p.decode_attn_select(0, [s], at, 16, 64, 64, 0.5, 64, 4, 64, 4), lambda: p.prefill_attn(0, [s], at, one, 16, 64, 64, 0.5),
+             lambda: p.select_blocks(at, 64, [64], one, 4, 128, 16, 64, 32, 64, 32), lambda: p.idx_pool(64, 4, 64, 64, 0, 1, 64, 1e-6, 64, 64, 16)]
+    for call in calls:
+        try:
+            call()
+        except BkvError as e:
+            assert e.status == %d, e
+        else:
+            raise AssertionError("not refused")
+""" % L.ERR_NO_DEVICE
+    subprocess.run([sys.executable, "-c", script], check=True, cwd=os.path.dirname(os.path.dirname(L.LIB_PATH)), timeout=100)
+
+
+def test_a_build_without_headers_goes_on_without_the_module(monkeypatch, tmp_path, capsys):
+    stale = tmp_path / "_hot.so"
+    stale.write_bytes(b"of other sources")
+    monkeypatch.setattr(build, "HOT_MODULE", str(stale))
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path / "none")})
+    assert build.build_hot_calls() is None and not stale.exists()
+    assert "ctypes" in capsys.readouterr().err
