@@ -82,6 +82,13 @@ __device__ __forceinline__ int small_div(int x, uint32_t inv16) { return (int)((
 // was found and the pointers loaded after that, 900 for one entry, 1200 for four and 100 more with each; now 900).
 typedef const __attribute__((address_space(4))) AttnBatch* batch_desc_ptr;
 __device__ __forceinline__ int lane_of_wave() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+// The same from the hardware once more, and so that the compiler does not know it: where a kernel has a short form behind
+// a branch and a long walk beside it, a value that both know is kept (or spilled) over the whole walk.
+__device__ __forceinline__ int lane_of_wave_again() {
+    unsigned all_lanes = ~0u;
+    asm volatile("" : "+s"(all_lanes));
+    return __builtin_amdgcn_mbcnt_hi(all_lanes, __builtin_amdgcn_mbcnt_lo(all_lanes, 0u));
+}
 template <bool STEP, bool DESC, typename Batch>
 __device__ __forceinline__ bool find_unit(const AttnKernelParams& P, const Batch& B, int unit, int& e, int& rem, int& pos, int& row, int& pps) {
     static_assert(kMaxBatch <= 64, "one lane per entry");

@@ -290,6 +290,10 @@ __device__ __forceinline__ void split_q(const QRaw& q, bool head_live, half8 (&q
     }
 }
 
+// what lane i of the wave has in x (__shfl works with the lane's own index, which would be kept from the kernel's start
+// over the long walk)
+__device__ __forceinline__ uint32_t from_lane(uint32_t x, int i) { return (uint32_t)__builtin_amdgcn_ds_bpermute(i << 2, (int)x); }
+
 // The 16 listed blocks of a range (SEL), lane by lane: lane i < 16 looks up block i (block i % 4 of page i / 4), and
 // takes its turn through slot -> id -> page; the others repeat lanes 0..15.
 struct ListedBlock {
@@ -337,7 +341,7 @@ __device__ __forceinline__ void one_page_take_new_k(const v4u* line, int new_pag
 
 // f16 rows of a listed block, and the lane's K rows of page j (c % 8 and 8 + c % 8)
 __device__ __forceinline__ size_t listed_f16_rows(const ListedBlock& listed, int block, size_t page_bytes, size_t head_off) {
-    const uint32_t row = (uint32_t)__shfl((int)listed.row, block, 64);
+    const uint32_t row = from_lane(listed.row, block);
     return (size_t)(row >> 2) * page_bytes + head_off + (size_t)(row & 3u) * 4u * (kHd * 2);
 }
 __device__ __forceinline__ void one_page_k_rows_listed(const ListedBlock& listed, int j, int c7, size_t page_bytes, size_t head_off, const uint8_t* base,
@@ -356,7 +360,7 @@ __device__ __forceinline__ void fetch_unit(const uint8_t* pool, size_t page_off,
     const auto at = [&](int off) {
         if constexpr (SEL) {
             const int j = (off >= 4 * ROW) + (off >= 8 * ROW) + (off >= 12 * ROW);
-            const uint32_t row = (uint32_t)__shfl((int)listed.row, 4 * wave + j, 64);
+            const uint32_t row = from_lane(listed.row, 4 * wave + j);
             return pool + ((size_t)(row >> 2) * page_bytes + head_off + (size_t)(row & 3u) * 4u * ROW) + (off - j * 4 * ROW);
         } else {
             return pool + page_off + off;
@@ -399,7 +403,7 @@ __device__ __forceinline__ void one_page_f16(const AttnKernelParams& P, OnePageL
         for (int j = 0; j < kWaves; ++j) {
             one_page_k_rows_listed(listed, j, c7, page_bytes, head_off, P.kpool + k_at, k_lo[j], k_hi[j]);
             v_rows[j] = P.vpool + listed_f16_rows(listed, 4 * j + g, page_bytes, head_off) + v_at;
-            id[j] = (uint32_t)__shfl((int)listed.id, 4 * j + g, 64);
+            id[j] = from_lane(listed.id, 4 * j + g);
         }
     } else {
         const block_table_ptr bt = (block_table_ptr)(uintptr_t)table;
@@ -534,7 +538,7 @@ __device__ __forceinline__ void split_f16(const Args& P) {
     const int lane = threadIdx.x & 63;
     if (pps == kWaves) {
         one_page_f16<STEP, SEL>(P, reinterpret_cast<OnePageLds&>(lds), e, kvh, wg, pos,
-                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave_again());
         return;
     }
     const int c = lane & 15;
@@ -965,7 +969,7 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
         // where something changed.
         const int row = lane >> 2;
         bool row_live;
-        if constexpr (SEL) row_live = block_cell_live((uint32_t)__shfl((int)listed.id, 4 * wave + (row >> 2), 64), row & 3, pos);
+        if constexpr (SEL) row_live = block_cell_live(from_lane(listed.id, 4 * wave + (row >> 2)), row & 3, pos);
         else row_live = (pg0 + wave) * kPage + row <= pos;
         unsigned* const ks = reinterpret_cast<unsigned*>(slot + row * kRow + kHd + 4 * (lane & 3));
         unsigned* const vs = ks + kI8hUnit / 4;
@@ -995,7 +999,7 @@ __device__ __forceinline__ void one_page_i8h(const AttnKernelParams& P, OnePageI
         }
     }
     bool mine[4];
-    const uint32_t id = SEL ? (uint32_t)__shfl((int)listed.id, 4 * wave + g, 64) : 0u;
+    const uint32_t id = SEL ? from_lane(listed.id, 4 * wave + g) : 0u;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if constexpr (SEL) mine[r] = block_cell_live(id, r, pos);
@@ -1076,7 +1080,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
     if (pps == kWaves) {
         static_assert(sizeof(OnePageI8hLds) <= kRing, "the fold staging holds it");
         one_page_i8h<STEP, SEL>(P, *reinterpret_cast<OnePageI8hLds*>(ring), e, kvh, wg, pos,
-                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave_again());
         return;
     }
     const int c = lane & 15;
@@ -1341,8 +1345,8 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_i8h_kernel(const A
 
     // every wave is done with its slot before the fold staging takes their place
     __syncthreads();
-    // the lane's place from the hardware again: kept over the loop, it was one register too many
-    const int again = lane_of_wave();
+    // the lane's place: kept over the loop, it was one register too many
+    const int again = lane_of_wave_again();
     mfma_fold_and_store(P, *reinterpret_cast<MfmaFoldLds*>(ring), wg, wave, again & 15, again >> 4, o, m_run, l_run);
 }
 
@@ -1503,7 +1507,7 @@ __device__ __forceinline__ void one_page_q8v(const AttnKernelParams& P, OnePageQ
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     bool mine[4], mine_scale;  // of cells 4 g + r, and of cell 4 g + c % 4
-    const uint32_t id = SEL ? (uint32_t)__shfl((int)listed.id, 4 * wave + g, 64) : 0u;
+    const uint32_t id = SEL ? from_lane(listed.id, 4 * wave + g) : 0u;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         if constexpr (SEL) mine[r] = block_cell_live(id, r, pos);
@@ -1601,7 +1605,7 @@ __global__ __launch_bounds__(kBlock, 2) void decode_attn_mfma_q8v_kernel(const A
     if (pps == kWaves) {
         static_assert(sizeof(OnePageQ8vLds) <= kLds, "the fold staging holds it");
         one_page_q8v<STEP, SEL>(P, *reinterpret_cast<OnePageQ8vLds*>(smem), e, kvh, wg, pos,
-                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave());
+                                P.tables + (size_t)row * (size_t)P.max_pages_per_seq, pg0, wave, lane_of_wave_again());
         return;
     }
     const int c = lane & 15;
