@@ -23,8 +23,8 @@ __device__ __forceinline__ float f16_load(uint32_t h) {
 
 // ---- the encoders' primitives, on 8 consecutive values of a 32-value block ----------------
 // The append kernels give a block to four neighbouring lanes (8 values each, so that a wave's
-// loads are contiguous), and so does the int8 attention kernel that takes a new row in flight; the q8_0 V one
-// gives it to one lane.  All go through these functions, so all store the very same codes.
+// loads are contiguous), and so do the attention kernels that take a new row in flight.  All go through these functions,
+// so all store the very same codes.
 
 __device__ __forceinline__ float amax8(const float (&x)[8], float amax = 0.0f) {
 #pragma unroll
@@ -156,36 +156,6 @@ __device__ __forceinline__ void codes8_f16_on_biased_reciprocal(const float (&x)
 // the value of a binary16 code that is not a subnormal (scales never are): the hardware convert
 __device__ __forceinline__ float f16_normal_value(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
-}
-
-// ---- a whole block in one lane -------------------------------------------------------------
-__device__ __forceinline__ float amax32(const float (&x)[32]) {
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const float a = fabsf(x[i]);
-        amax = a > amax ? a : amax;
-    }
-    return amax;
-}
-
-__device__ __forceinline__ void q8_block(const float (&x)[32], float scale, uint32_t (&w)[8]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float y[8] = {x[8 * j], x[8 * j + 1], x[8 * j + 2], x[8 * j + 3],
-                            x[8 * j + 4], x[8 * j + 5], x[8 * j + 6], x[8 * j + 7]};
-        q8_codes8(y, scale, w[2 * j], w[2 * j + 1]);
-    }
-}
-
-// One q8_0 block as the V pool holds it: w[0] = f32 scale, w[1..8] = 32 x i8.
-__device__ __forceinline__ void q8v_block_words(const float (&x)[32], uint32_t (&w)[9]) {
-    const float scale = q8v_scale(amax32(x));
-    uint32_t c[8];
-    q8_block(x, scale, c);
-    w[0] = __float_as_uint(scale);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w[1 + j] = c[j];
 }
 
 }  // namespace bkv
