@@ -49,8 +49,10 @@ struct AttnKernelParams {
 // The batch as a kernel argument.  What a launch costs the host grows with its arguments (2.8 us up to 100 bytes, 3.3 at
 // 500, 3.9 at 1500), and the short steps of a decode loop are bound by that: a batch of few entries travels in a
 // smaller struct, in kernels of their own.  12 layers of one sequence of 4096 cells 113 -> 104 us, of four
-// short ones 113 -> 101; where the kernels are what bounds a step (eight sequences of 1k to 32k, 191.9) it makes no difference.
-// The append with K preparation keeps the one struct: with the smaller one its four launches in 159 us took 1.3 longer.  16 entries: from 200 bytes to 500 there is little between.
+// short ones 113 -> 101; where the kernels are what bounds a step (eight sequences of 1k to 32k, 191.9) it makes no
+// difference.  16 entries: from 200 bytes to 500 there is little between.  The append with K preparation keeps the one
+// struct: with the smaller one its four launches in 159 us took 1.3 longer.  So do the quantised attention kernels: the
+// int8 ones spilled with their body in a function of its own, and q8_0 V, which would not, was not tried.
 struct AttnBatchFew {
     int32_t n;
     int32_t row[kFewEntries], pos[kFewEntries], wg_base[kFewEntries], pps[kFewEntries];
@@ -73,12 +75,12 @@ __device__ __forceinline__ int small_div(int x, uint32_t inv16) { return (int)((
 
 // Which unit of work a work-group of the matrix-core kernels has: entry e, its rem-th work-group
 // (page range x kv head), and the entry's position, block-table row and pages per range.  With DESC the
-// batch is read from device memory through the constant address space (uniform addresses: scalar
-// loads), and a work-group past the end of the current cut reports false: such a launch has a fixed grid.
+// batch is read from device memory, and a work-group past the end of the current cut reports false: such a
+// launch has a fixed grid.
 //
-// Finding the entry must not be a chain of loads at the head of a launch that may last five microseconds: lane i reads
-// entry i, the work-group's entry is found with a ballot, and the scalar arguments are asked for at the same time, one
-// trip to memory for any batch (cycles from a work-group's first instruction to here: searched entry by entry, with what
+// Finding the entry must not be a chain of loads at the head of a launch that may last five microseconds: lane i loads
+// entry i (through the vector cache), the work-group's entry is found with a ballot, and the scalar arguments are asked for
+// at the same time, one trip to memory for any batch (cycles from a work-group's first instruction to here: searched entry by entry, with what
 // was found and the pointers loaded after that, 900 for one entry, 1200 for four and 100 more with each; now 900).
 typedef const __attribute__((address_space(4))) AttnBatch* batch_desc_ptr;
 __device__ __forceinline__ int lane_of_wave() { return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
